@@ -172,7 +172,8 @@ int  mi_mesh_num_nodes(const mi_mesh* m);
 #define MI_STAT_FWN_LEAVES 8     /* winding number: exact solid angles (48-B triangle record) */
 #define MI_STAT_SEEDS 9          /* greedy descents seeding a walk (one root-to-leaf path per wave) */
 #define MI_STAT_SEED_LEVELS 10   /* their levels (one 64-B node record each) */
-#define MI_STAT_COUNT 11
+#define MI_STAT_LANE_VISITS 11   /* lane walks: nodes visited by a lane (64-B cylinder record each) */
+#define MI_STAT_COUNT 12
 #define MI_STAT_STRIDE 16
 #define MI_STAT_LAUNCHES 3
 int  mi_mesh_set_stats(mi_mesh* m, uint64_t* d_counters);

@@ -41,7 +41,7 @@ MI_OK, MI_E_INVALID, MI_E_HIP, MI_E_CANCELED, MI_E_NOMEM, MI_E_LIMIT = 0, -1, -2
 
 # measurement counters of mi_mesh_set_stats: names of the slots and the bytes each event reads
 STAT_NAMES = ("walks", "quad_steps", "prism_reads", "leaf_tests", "keyed_steps", "keyed_tests", "fwn_visits",
-              "fwn_descents", "fwn_leaves", "seeds", "seed_levels")
+              "fwn_descents", "fwn_leaves", "seeds", "seed_levels", "lane_visits")
 STAT_STRIDE, STAT_LAUNCHES = 16, 3
 
 

@@ -30,22 +30,22 @@ std::atomic<int> g_treeBuilder{ MI_TREE_BUILDER_DEVICE };
 std::atomic<int> g_splitBudget{ MI_SPLIT_AUTO };       // signed-distance walks
 std::atomic<int> g_splitBudgetProj{ MI_SPLIT_AUTO };   // projection walks
 
-// Automatic split budgets, from sweeps on MI355X (bumpy spheres of 20 k to 5.2 M triangles, tree
-// depths 15 to 23).  Signed distance on trees of >= 18 levels: 3072 steps below 64 k waves, 6144
-// below 1 M (k=8 256^3: 99 -> 94.5 ms), none from 1 M waves on (512^3: k=8 521 -> 477 ms, k=9
-// 1031 -> 856 ms: enough waves to spread the long ones); shallower trees walk less, so the 64 subtree items of a
-// hand-over weigh more and an earlier hand-over spreads the few long waves (512 steps below 16 k
-// waves, 1024 above; 20 k triangles at 64^3: 2.7 -> 1.6 ms).  Projections: on trees of >= 20
-// levels nearly every wave is long and 64 steps is best (flat to within noise up to 2048 at 2^22
-// points); on shallower trees most waves finish alone given 1-2 k steps (2^22 points on 20 k /
-// 82 k / 328 k triangles: 36.7 / 50.8 / 54.1 ms at 64 steps, 5.0 / 10.0 / 24.0 ms at 1024-2048).
-int autoSdfBudget(int depth, int64_t waves)
+// Automatic step budgets of the keyed walks (a band: loDistLimitSq > 0 or minDistSq > 0), from sweeps on
+// MI355X (bumpy spheres of 20 k to 5.2 M triangles, tree depths 15 to 23).  Signed distance on trees of
+// >= 18 levels: 3072 steps below 64 k waves, 6144 below 1 M, none from 1 M waves on (enough waves to spread
+// the long ones); shallower trees walk less, so the 64 subtree items of a hand-over weigh more and an earlier
+// hand-over spreads the few long waves (512 steps below 16 k waves, 1024 above).  Projections: on trees of
+// >= 20 levels nearly every wave is long and 64 steps is best; on shallower trees most waves finish alone
+// given 1-2 k steps.  Without a band the lane walks need no hand-over: automatic is none.
+int autoSdfBudget(int depth, int64_t waves, bool band)
 {
+    if (!band) return 0;
     if (depth >= 18) return waves < 65536 ? 3072 : waves < (1 << 20) ? 6144 : 0;
     return waves < 16384 ? 512 : 1024;
 }
-int autoProjBudget(int depth)
+int autoProjBudget(int depth, bool band)
 {
+    if (!band) return 0;
     if (depth >= 20) return 64;
     return depth >= 17 ? 2048 : 1024;
 }
@@ -293,14 +293,14 @@ int sdfLaneBytes(const mi_dist_options* o) { return o && o->minDistSq > 0 ? 8 : 
 size_t sdfBytesPerVoxel(const mi_dist_options* o) { return o ? sizeof(float) + sdfLaneBytes(o) + 2 : sizeof(float); }
 
 // waves of a signed-distance launch over `layers` z-layers and the split budget it runs with
-int64_t sdfSplitPlan(const mi_mesh* m, const int32_t dims[3], int32_t layers, int32_t* budget)
+int64_t sdfSplitPlan(const mi_mesh* m, const int32_t dims[3], int32_t layers, bool band, int32_t* budget)
 {
     *budget = 0;
     if (layers <= 0) return 0;
     const int32_t d[3] = { dims[0], dims[1], layers };
     const int64_t waves = mi::sdfGridWaves(d, 0, layers);
     const int setting = meshMode(m, MI_MODE_SPLIT_SDF, g_splitBudget.load());
-    *budget = setting >= 0 ? setting : autoSdfBudget(m->depth, waves);
+    *budget = setting >= 0 ? setting : autoSdfBudget(m->depth, waves, band);
     return waves;
 }
 
@@ -309,7 +309,7 @@ int splitScratch(mi_mesh* m, DevBuf& buf, const int32_t dims[3], int32_t layers,
 {
     sc = mi::SplitScratch{};
     int32_t budget = 0;
-    const int64_t waves = sdfSplitPlan(m, dims, layers, &budget);
+    const int64_t waves = sdfSplitPlan(m, dims, layers, laneBytes == 8, &budget);
     if (budget <= 0) return MI_OK;
     const size_t bytes = mi::splitScratchBytes(waves, laneBytes);
     if (buf.bytes < bytes) MI_HIP(buf.alloc(bytes));
@@ -317,23 +317,23 @@ int splitScratch(mi_mesh* m, DevBuf& buf, const int32_t dims[3], int32_t layers,
     return MI_OK;
 }
 
-// split scratch of a projection launch over n points, placed at `base` (caller-sized with
-// projSplitBytes); no split when the budget is 0
-int projBudget(const mi_mesh* m)
+// split scratch of a projection launch over n points with loDistLimitSq `lo`, placed at `base`
+// (caller-sized with projSplitBytes); no split when the budget is 0
+int projBudget(const mi_mesh* m, float lo)
 {
     const int setting = meshMode(m, MI_MODE_SPLIT_PROJECTIONS, g_splitBudgetProj.load());
-    return setting >= 0 ? setting : autoProjBudget(m->depth);
+    return setting >= 0 ? setting : autoProjBudget(m->depth, lo > 0);
 }
 
-size_t projSplitBytes(const mi_mesh* m, int64_t n)
+size_t projSplitBytes(const mi_mesh* m, int64_t n, float lo)
 {
-    return projBudget(m) > 0 ? mi::splitScratchBytes(mi::projectionWaves(n), 8) : 0;
+    return projBudget(m, lo) > 0 ? mi::splitScratchBytes(mi::projectionWaves(n), 8) : 0;
 }
 
-void projSplit(const mi_mesh* m, void* base, int64_t n, mi::SplitScratch& sc)
+void projSplit(const mi_mesh* m, void* base, int64_t n, float lo, mi::SplitScratch& sc)
 {
     sc = mi::SplitScratch{};
-    const int budget = projBudget(m);
+    const int budget = projBudget(m, lo);
     if (budget <= 0 || !base) return;
     mi::splitScratchBind(base, mi::projectionWaves(n), 8, budget, sc);
 }
@@ -418,15 +418,16 @@ int32_t mi_get_split_budget(int32_t walk)
 namespace {
 
 struct ArenaLayout {
-    size_t dnode, tri, dint, dleaf, dquad, cut, prism;
-    size_t total() const { return dnode + tri + dint + dleaf + dquad + cut + prism; }
+    size_t dnode, tri, dint, dleaf, dquad, cut, prism, cyl;
+    size_t total() const { return dnode + tri + dint + dleaf + dquad + cut + prism + cyl; }
 };
 
 ArenaLayout arenaLayout(int32_t nf)
 {
     const size_t ni = nf > 0 ? (size_t)nf - 1 : 0, nl = nf > 0 ? (size_t)nf : 0;
     return { align256(ni * 64), align256(nl * 48), align256(ni * 32), align256(nl * 32), align256(ni * 128),
-             nf > 0 ? align256(mi::kMaxCut * sizeof(mi::CutEntry)) + 256 : 0, align256(nl * 80) };
+             nf > 0 ? align256(mi::kMaxCut * sizeof(mi::CutEntry)) + 256 : 0, align256(nl * 80),
+             align256(ni * 64) };
 }
 
 void bindArena(mi_mesh* m, const ArenaLayout& L)
@@ -438,6 +439,7 @@ void bindArena(mi_mesh* m, const ArenaLayout& L)
     m->dev.dleaf = reinterpret_cast<const float4*>(base + L.dnode + L.tri + L.dint);
     m->dev.dquad = reinterpret_cast<const float4*>(base + L.dnode + L.tri + L.dint + L.dleaf);
     m->dev.prism = reinterpret_cast<const float4*>(base + L.dnode + L.tri + L.dint + L.dleaf + L.dquad + L.cut);
+    m->dev.cyl = reinterpret_cast<const float4*>(base + L.total() - L.cyl);
 }
 
 // 4-wide records of the cooperative walks and the cut of the split form, from the binary records
@@ -452,6 +454,10 @@ int finishArena(mi_mesh* m, const ArenaLayout& L)
     MI_HIP(mi::buildPrisms(m->dev.tri, m->nf,
                            reinterpret_cast<float4*>(base + L.dnode + L.tri + L.dint + L.dleaf + L.dquad + L.cut),
                            m->stream));
+    DevBuf ranges;
+    MI_HIP(ranges.alloc(mi::cylinderScratchBytes(m->nf)));
+    m->dev.numFaces = m->nf;
+    MI_HIP(mi::buildCylinders(m->dev, reinterpret_cast<float4*>(base + L.total() - L.cyl), ranges.p, m->stream));
     char* cutBase = base + L.dnode + L.tri + L.dint + L.dleaf + L.dquad;
     mi::CutEntry* cut = reinterpret_cast<mi::CutEntry*>(cutBase);
     int32_t* nCutDev = reinterpret_cast<int32_t*>(cutBase + align256(mi::kMaxCut * sizeof(mi::CutEntry)));
@@ -730,7 +736,7 @@ int mi_sdf_grid_device(mi_mesh* m, const int32_t dims[3], const float xf[12], co
     mi::SplitScratch sc;
     if (int rc = splitScratch(m, m->ws, dims, zEnd - zBegin, sdfLaneBytes(opts), sc)) return rc;
     MI_HIP(mi::launchSdfGrid(callView(m), dims, toXf(xf), o, zBegin, zEnd, d_res, m->stackD, pick(m, stream), nullptr,
-                             nullptr, nullptr, &sc));
+                             nullptr, &sc));
     return MI_OK;
 }
 
@@ -772,16 +778,16 @@ int mi_proj_find_projections_device(mi_mesh* m, const float* d_pts, int64_t n, c
     MI_HIP(hipSetDevice(m->device));
     hipStream_t s = pick(m, stream);
     const size_t sortBytes = align256(mi::sortWorkspaceBytes(n));
-    if (int rc = ensureWorkspace(m, sortBytes + projSplitBytes(m, n))) return rc;
+    if (int rc = ensureWorkspace(m, sortBytes + projSplitBytes(m, n, lo))) return rc;
     mi::SplitScratch sc;
-    projSplit(m, m->ws.as<char>() + sortBytes, n, sc);
+    projSplit(m, m->ws.as<char>() + sortBytes, n, lo, sc);
     const uint32_t* perm = nullptr;
     MI_HIP(mi::sortPointsMorton(d_pts, n, m->sortLo, m->sortHi, m->ws.p, m->ws.bytes, &perm, s));
     mi::Xf px, tx;
     if (ptXf) px = toXf(ptXf);
     if (treeXf) tx = toXf(treeXf);
     MI_HIP(mi::launchProjections(callView(m), d_pts, perm, n, ptXf ? &px : nullptr, treeXf ? &tx : nullptr, up, lo,
-                                 reinterpret_cast<mi::ProjRec*>(d_res), m->stackD, s, nullptr, nullptr, nullptr, &sc));
+                                 reinterpret_cast<mi::ProjRec*>(d_res), m->stackD, s, nullptr, nullptr, &sc));
     return MI_OK;
 }
 
@@ -800,17 +806,17 @@ int mi_proj_find_projections_noalloc_device(mi_mesh* m, const float* d_pts, int6
     MI_HIP(mi::noAllocScratch(m->device, &scratch));
     // the same workspace layout as mi_proj_find_projections_device, in the fixed scratch
     const size_t sortBytes = align256(mi::sortWorkspaceBytes(n));
-    if (sortBytes + projSplitBytes(m, n) > mi::kNoAllocScratchBytes)
+    if (sortBytes + projSplitBytes(m, n, lo) > mi::kNoAllocScratchBytes)
         return fail(MI_E_LIMIT, "the no-allocation scratch is too small for this call");
     mi::SplitScratch sc;
-    projSplit(m, static_cast<char*>(scratch) + sortBytes, n, sc);
+    projSplit(m, static_cast<char*>(scratch) + sortBytes, n, lo, sc);
     const uint32_t* perm = nullptr;
     MI_HIP(mi::sortPointsMorton(d_pts, n, m->sortLo, m->sortHi, scratch, sortBytes, &perm, s));
     mi::Xf px, tx;
     if (ptXf) px = toXf(ptXf);
     if (treeXf) tx = toXf(treeXf);
     MI_HIP(mi::launchProjections(callView(m), d_pts, perm, n, ptXf ? &px : nullptr, treeXf ? &tx : nullptr, up, lo,
-                                 reinterpret_cast<mi::ProjRec*>(d_res), m->stackD, s, nullptr, nullptr, nullptr, &sc));
+                                 reinterpret_cast<mi::ProjRec*>(d_res), m->stackD, s, nullptr, nullptr, &sc));
     return MI_OK;
 }
 
@@ -825,16 +831,16 @@ int mi_proj_find_projections_bounded_device(mi_mesh* m, const float* d_pts, int6
     MI_HIP(hipSetDevice(m->device));
     hipStream_t s = pick(m, stream);
     const size_t sortBytes = align256(mi::sortWorkspaceBytes(n));
-    if (int rc = ensureWorkspace(m, sortBytes + projSplitBytes(m, n))) return rc;
+    if (int rc = ensureWorkspace(m, sortBytes + projSplitBytes(m, n, lo))) return rc;
     mi::SplitScratch sc;
-    projSplit(m, m->ws.as<char>() + sortBytes, n, sc);
+    projSplit(m, m->ws.as<char>() + sortBytes, n, lo, sc);
     const uint32_t* perm = nullptr;
     MI_HIP(mi::sortPointsMorton(d_pts, n, m->sortLo, m->sortHi, m->ws.p, m->ws.bytes, &perm, s));
     mi::Xf px, tx;
     if (ptXf) px = toXf(ptXf);
     if (treeXf) tx = toXf(treeXf);
     MI_HIP(mi::launchProjections(callView(m), d_pts, perm, n, ptXf ? &px : nullptr, treeXf ? &tx : nullptr, up, lo,
-                                 reinterpret_cast<mi::ProjRec*>(d_res), m->stackD, s, d_upSq, nullptr, nullptr, &sc));
+                                 reinterpret_cast<mi::ProjRec*>(d_res), m->stackD, s, d_upSq, nullptr, &sc));
     return MI_OK;
 }
 
@@ -848,31 +854,18 @@ int mi_proj_find_projections_capped_device(mi_mesh* m, const float* d_pts, int64
     std::lock_guard<std::mutex> lk(m->mu);
     MI_HIP(hipSetDevice(m->device));
     hipStream_t s = pick(m, stream);
-    // workspace: sort, rerun list, its counter, split scratch.  The split scratch is bound even when the
-    // step budget is 0: the waves with a failed cap hand their queries, uncapped, to the split pass, so no
-    // query is searched again after it (a separate rerun launch over scattered queries ends on its
-    // slowest single walk).  Only a tree too small to cut uses the rerun list.
+    // workspace: sort, the counter of failed caps (each such query walks again inside the launch)
     const size_t sortBytes = align256(mi::sortWorkspaceBytes(n));
-    const size_t listBytes = align256((size_t)n * 4) + 256;
-    const int64_t waves = mi::projectionWaves(n);
-    const size_t splitBytes = mi::splitScratchBytes(waves, 8);
-    if (int rc = ensureWorkspace(m, sortBytes + listBytes + splitBytes)) return rc;
-    char* base = m->ws.as<char>();
-    uint32_t* list = reinterpret_cast<uint32_t*>(base + sortBytes);
-    uint32_t* count = reinterpret_cast<uint32_t*>(base + sortBytes + align256((size_t)n * 4));
-    mi::SplitScratch sc;
-    mi::splitScratchBind(base + sortBytes + listBytes, waves, 8, projBudget(m), sc);
+    if (int rc = ensureWorkspace(m, sortBytes + 256)) return rc;
+    uint32_t* count = reinterpret_cast<uint32_t*>(m->ws.as<char>() + sortBytes);
     const uint32_t* perm = nullptr;
     MI_HIP(mi::sortPointsMorton(d_pts, n, m->sortLo, m->sortHi, m->ws.p, sortBytes, &perm, s));
     MI_HIP(mi::fillU32(count, 1, 0u, s));
     MI_HIP(mi::launchProjections(callView(m), d_pts, perm, n, nullptr, nullptr, up, 0.f,
-                                 reinterpret_cast<mi::ProjRec*>(d_res), m->stackD, s, d_capSq, list, count, &sc));
+                                 reinterpret_cast<mi::ProjRec*>(d_res), m->stackD, s, d_capSq, count));
     uint32_t h = 0;
     MI_HIP(hipMemcpyAsync(&h, count, 4, hipMemcpyDeviceToHost, s));
     MI_HIP(hipStreamSynchronize(s));
-    if (h && m->dev.nCut <= 0)
-        MI_HIP(mi::launchProjections(callView(m), d_pts, list, (int64_t)h, nullptr, nullptr, up, 0.f,
-                                     reinterpret_cast<mi::ProjRec*>(d_res), m->stackD, s));
     if (reruns) *reruns = h;
     return MI_OK;
 }
@@ -893,28 +886,16 @@ int mi_sdf_grid_capped_device(mi_mesh* m, const int32_t dims[3], const float xf[
     std::lock_guard<std::mutex> lk(m->mu);
     MI_HIP(hipSetDevice(m->device));
     hipStream_t s = pick(m, stream);
-    // workspace: rerun list, its counter, split scratch (bound even with a step budget of 0, as for the
-    // capped projections: failed caps are searched again in the split pass; only a tree too small to cut
-    // uses the rerun list)
-    const size_t listBytes = align256(nvox * 4) + 256;
-    int32_t budget = 0;
-    const int64_t waves = sdfSplitPlan(m, dims, zEnd - zBegin, &budget);
-    const size_t splitBytes = mi::splitScratchBytes(waves, sdfLaneBytes(opts));
-    if (int rc = ensureWorkspace(m, listBytes + splitBytes)) return rc;
-    uint32_t* list = m->ws.as<uint32_t>();
-    uint32_t* count = reinterpret_cast<uint32_t*>(m->ws.as<char>() + align256(nvox * 4));
-    mi::SplitScratch sc;
-    mi::splitScratchBind(m->ws.as<char>() + listBytes, waves, sdfLaneBytes(opts), budget, sc);
+    // workspace: the counter of failed caps (each such voxel walks again inside the launch)
+    if (int rc = ensureWorkspace(m, 256)) return rc;
+    uint32_t* count = m->ws.as<uint32_t>();
     mi::DistOpts o{ opts->minDistSq, opts->maxDistSq, opts->nullOutsideMinMax, opts->windingNumberThreshold,
                     opts->windingNumberBeta };
     MI_HIP(mi::fillU32(count, 1, 0u, s));
-    MI_HIP(mi::launchSdfGrid(callView(m), dims, toXf(xf), o, zBegin, zEnd, d_res, m->stackD, s, d_capSq, list, count,
-                             &sc));
+    MI_HIP(mi::launchSdfGrid(callView(m), dims, toXf(xf), o, zBegin, zEnd, d_res, m->stackD, s, d_capSq, count));
     uint32_t h = 0;
     MI_HIP(hipMemcpyAsync(&h, count, 4, hipMemcpyDeviceToHost, s));
     MI_HIP(hipStreamSynchronize(s));
-    if (h && m->dev.nCut <= 0)
-        MI_HIP(mi::launchSdfVoxels(callView(m), dims, toXf(xf), o, zBegin, list, (int64_t)h, d_res, m->stackD, s));
     if (reruns) *reruns = h;
     return MI_OK;
 }
@@ -937,7 +918,7 @@ static int gridLaunch(mi_mesh* m, const int32_t dims[3], const mi::Xf& x, const 
     if (opts) {
         mi::DistOpts o{ opts->minDistSq, opts->maxDistSq, opts->nullOutsideMinMax, opts->windingNumberThreshold,
                         opts->windingNumberBeta };
-        MI_HIP(mi::launchSdfGrid(callView(m), dims, x, o, z0, z1, out, m->stackD, s, nullptr, nullptr, nullptr, sc));
+        MI_HIP(mi::launchSdfGrid(callView(m), dims, x, o, z0, z1, out, m->stackD, s, nullptr, nullptr, sc));
     } else {
         MI_HIP(mi::launchFwnGrid(callView(m), dims, x, beta, z0, z1, out, m->stackD, s));
     }
@@ -1143,7 +1124,7 @@ constexpr size_t kPartPoints = size_t(1) << 21;
 
 template <class LaunchFn>
 static int pointsHost(mi_mesh* m, const float* pts, int64_t n, size_t outElem, void* res, LaunchFn&& launchFn,
-                      mi_progress_fn cb, void* user, bool split = false)
+                      mi_progress_fn cb, void* user, bool split = false, float lo = 0.f)
 {
     std::lock_guard<std::mutex> lk(m->mu);
     MI_HIP(hipSetDevice(m->device));
@@ -1165,9 +1146,9 @@ static int pointsHost(mi_mesh* m, const float* pts, int64_t n, size_t outElem, v
         MI_HIP(sl[i].pts.alloc(part * 12));
         MI_HIP(sl[i].res.alloc(part * outElem));
         MI_HIP(sl[i].ws.alloc(mi::sortWorkspaceBytes((int64_t)part)));
-        if (split && projSplitBytes(m, (int64_t)part)) {
-            MI_HIP(sl[i].split.alloc(projSplitBytes(m, (int64_t)part)));
-            projSplit(m, sl[i].split.p, (int64_t)part, sl[i].sc);
+        if (split && projSplitBytes(m, (int64_t)part, lo)) {
+            MI_HIP(sl[i].split.alloc(projSplitBytes(m, (int64_t)part, lo)));
+            projSplit(m, sl[i].split.p, (int64_t)part, lo, sl[i].sc);
         }
     }
     PartStreams ps;
@@ -1265,9 +1246,9 @@ int mi_proj_find_projections(mi_mesh* m, const float* pts, int64_t n, const floa
                           return mi::launchProjections(callView(m), dp, perm, sz, ptXf ? &px : nullptr,
                                                        treeXf ? &tx : nullptr, up, lo,
                                                        static_cast<mi::ProjRec*>(dr), m->stackD, st,
-                                                       nullptr, nullptr, nullptr, sc);
+                                                       nullptr, nullptr, sc);
                       },
-                      nullptr, nullptr, true);
+                      nullptr, nullptr, true, lo);
 }
 
 size_t mi_proj_heap_bytes(size_t numProjections)
@@ -1305,11 +1286,11 @@ int uploadItems(mi_batch* b, int32_t count, hipStream_t s)
 }
 
 // builds the device descriptors (sorting every item's points) and returns the unit count
-int prepareBatch(mi_batch* b, const mi_batch_item* items, int32_t count, hipStream_t s, int64_t* total, int* stackD,
+int prepareBatch(mi_batch* b, const mi_batch_item* items, int32_t count, hipStream_t s, int64_t* total, int* depth,
                  bool upload = true)
 {
     *total = 0;
-    *stackD = 8;
+    *depth = 0;
     b->host.assign((size_t)count, mi::BatchItem{});
     size_t wsTotal = 0;
     for (int32_t i = 0; i < count; ++i) {
@@ -1322,7 +1303,7 @@ int prepareBatch(mi_batch* b, const mi_batch_item* items, int32_t count, hipStre
             return fail(MI_E_INVALID, "invalid batch item grid");
         if (it.mesh->device != b->device) return fail(MI_E_INVALID, "batch items must live on the batch's device");
         wsTotal += align256(mi::sortWorkspaceBytes(it.numPts));
-        *stackD = std::max(*stackD, it.mesh->stackD);
+        *depth = std::max(*depth, (int)it.mesh->depth);
     }
     if (wsTotal && b->sortWs.bytes < wsTotal) MI_HIP(b->sortWs.alloc(wsTotal));
     // launch order: items on deeper trees first (their work units are the long ones), larger first
@@ -1372,14 +1353,14 @@ int prepareBatch(mi_batch* b, const mi_batch_item* items, int32_t count, hipStre
     return upload ? uploadItems(b, count, s) : MI_OK;
 }
 
-int launchPrepared(mi_batch* b, int32_t count, int64_t total, int stackD, const mi_dist_options* opts, float up,
+int launchPrepared(mi_batch* b, int32_t count, int64_t total, int depth, const mi_dist_options* opts, float up,
                    int blocksPerCU, int xcdSplit, hipStream_t s, bool capped = false)
 {
     mi::DistOpts o{ opts->minDistSq, opts->maxDistSq, opts->nullOutsideMinMax, opts->windingNumberThreshold,
                     opts->windingNumberBeta };
     MI_HIP(mi::fillU32(b->tickets.as<uint32_t>(), 16, 0u, s));
     MI_HIP(mi::launchBatch(b->items.as<mi::BatchItem>(), count, total, o, up,
-                           b->tickets.as<unsigned long long>(), xcdSplit, b->numCUs * blocksPerCU, stackD, capped, s));
+                           b->tickets.as<unsigned long long>(), xcdSplit, b->numCUs * blocksPerCU, depth, capped, s));
     return MI_OK;
 }
 
@@ -1437,9 +1418,9 @@ int mi_batch_run_device(mi_batch* b, const mi_batch_item* items, int32_t count, 
     MI_HIP(hipSetDevice(b->device));
     hipStream_t s = static_cast<hipStream_t>(stream);
     int64_t total = 0;
-    int stackD = 8;
-    if (int rc = prepareBatch(b, items, count, s, &total, &stackD)) return rc;
-    return launchPrepared(b, count, total, stackD, opts, upDistLimitSq, b->blocksPerCU, b->xcdSplit, s);
+    int depth = 0;
+    if (int rc = prepareBatch(b, items, count, s, &total, &depth)) return rc;
+    return launchPrepared(b, count, total, depth, opts, upDistLimitSq, b->blocksPerCU, b->xcdSplit, s);
 }
 
 int mi_batch_run_capped_device(mi_batch* b, const mi_batch_item* items, int32_t count, const float* const* d_capSdf,
@@ -1453,8 +1434,8 @@ int mi_batch_run_capped_device(mi_batch* b, const mi_batch_item* items, int32_t 
     MI_HIP(hipSetDevice(b->device));
     hipStream_t s = static_cast<hipStream_t>(stream);
     int64_t total = 0;
-    int stackD = 8;
-    if (int rc = prepareBatch(b, items, count, s, &total, &stackD, false)) return rc;
+    int depth = 0;
+    if (int rc = prepareBatch(b, items, count, s, &total, &depth, false)) return rc;
     // two counters per item: the voxels and points whose cap failed (each searched again, uncapped, by its
     // own wave inside the launch)
     const size_t cntBytes = align256((size_t)count * 8);
@@ -1469,7 +1450,7 @@ int mi_batch_run_capped_device(mi_batch* b, const mi_batch_item* items, int32_t 
     }
     MI_HIP(mi::fillU32(counts, 2 * count, 0u, s));
     if (int rc = uploadItems(b, count, s)) return rc;
-    if (int rc = launchPrepared(b, count, total, stackD, opts, upDistLimitSq, b->blocksPerCU, b->xcdSplit, s, true))
+    if (int rc = launchPrepared(b, count, total, depth, opts, upDistLimitSq, b->blocksPerCU, b->xcdSplit, s, true))
         return rc;
     std::vector<uint32_t> hc((size_t)count * 2);
     MI_HIP(hipMemcpyAsync(hc.data(), counts, hc.size() * 4, hipMemcpyDeviceToHost, s));
@@ -1494,8 +1475,8 @@ int mi_batch_autotune(mi_batch* b, const mi_batch_item* items, int32_t count, co
     MI_HIP(hipSetDevice(b->device));
     hipStream_t s = static_cast<hipStream_t>(stream);
     int64_t total = 0;
-    int stackD = 8;
-    if (int rc = prepareBatch(b, items, count, s, &total, &stackD)) return rc;
+    int depth = 0;
+    if (int rc = prepareBatch(b, items, count, s, &total, &depth)) return rc;
     hipEvent_t e0, e1;
     MI_HIP(hipEventCreate(&e0));
     MI_HIP(hipEventCreate(&e1));
@@ -1504,11 +1485,11 @@ int mi_batch_autotune(mi_batch* b, const mi_batch_item* items, int32_t count, co
     const int blocksCand[] = { 2, 3, 4, 5, 6 };
     int rc = MI_OK;
     // warm-up (caches, code object load)
-    rc = launchPrepared(b, count, total, stackD, opts, upDistLimitSq, b->blocksPerCU, b->xcdSplit, s);
+    rc = launchPrepared(b, count, total, depth, opts, upDistLimitSq, b->blocksPerCU, b->xcdSplit, s);
     for (int split = 0; split < 2 && rc == MI_OK; ++split) {
         for (int bpc : blocksCand) {
             if (hipEventRecord(e0, s) != hipSuccess) { rc = fail(MI_E_HIP, "AMD GPU error: event"); break; }
-            rc = launchPrepared(b, count, total, stackD, opts, upDistLimitSq, bpc, split, s);
+            rc = launchPrepared(b, count, total, depth, opts, upDistLimitSq, bpc, split, s);
             if (rc != MI_OK) break;
             float ms = 0.f;
             if (hipEventRecord(e1, s) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||

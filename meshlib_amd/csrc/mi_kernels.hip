@@ -10,21 +10,23 @@
 //  * queries of a wave are spatially coherent: grid voxels are mapped as 4x4x4
 //    bricks per wave; free points are Morton-sorted first, so the lanes of a wave
 //    walk mostly the same nodes and their loads hit the same cache lines;
-//  * per-lane form (kSdfGrid, kProjections, ...): each lane keeps the reference's
+//  * lane form (the default of distances and projections; mi_lane.hpp): every lane
+//    walks for itself over oriented bounds, FP64 leaf tests queued per wave;
+//  * per-lane reference form (kSdfGrid, kProjections, ...): each lane keeps the reference's
 //    depth-first order exactly (nearer child first, strict '<' on distances), with
 //    the pending far children on a per-lane stack in LDS laid out [depth][lane];
-//  * wave-cooperative form (the default; coopDistanceWalk, coopProjectWalk,
-//    coopWinding): one walk per wave over 4-wide records with wave-uniform node refs
+//  * wave-cooperative form (winding numbers; the keyed walks of a band; distances and projections
+//    when a step budget is set): one walk per wave with wave-uniform node refs
 //    (scalar loads), a stack whose uniform part is held in lanes of a few VGPRs and
 //    whose per-lane part (16-bit lower bounds of box distances) sits in LDS, and leaf
 //    tests queued and run one per lane; results equal the per-lane form's;
-//  * split form: waves past a step budget hand their queries to a second launch that
+//  * split form: wave-cooperative waves past a step budget hand their queries to a second launch that
 //    walks the tree's top subtrees for them in parallel (results merged by atomic
 //    minimum) and a third that stores them;
 //  * blocks are remapped so that each XCD (blocks are dealt round-robin over the 8
-//    XCDs) gets one contiguous range of bricks / sorted queries, keeping each L2's
+//    XCDs) gets compact ranges of bricks / one contiguous range of sorted queries, keeping each L2's
 //    working set spatially local.
-#include "mi_walk.hpp"
+#include "mi_lane.hpp"
 
 #include <hipcub/hipcub.hpp>
 
@@ -37,7 +39,7 @@ __global__ __launch_bounds__(kBlock) void kSdfGrid(MeshDev m, int dx, int dy, in
                                                    DistOpts o, float* __restrict__ out)
 {
     __shared__ int2 smem[D * kBlock];
-    const int lb = gridBlock();
+    const int lb = gridBlock<kGridChunk>();
     if (lb >= nLogical) return;
     const int lane = threadIdx.x & 63;
     const int brick = lb * (kBlock / 64) + (threadIdx.x >> 6);
@@ -66,7 +68,7 @@ __global__ __launch_bounds__(kBlock) void kFwnGrid(MeshDev m, int dx, int dy, in
                                                    float beta, float* __restrict__ out)
 {
     __shared__ int2 smem[D * kBlock];
-    const int lb = gridBlock();
+    const int lb = gridBlock<kGridChunk>();
     if (lb >= nLogical) return;
     const int lane = threadIdx.x & 63;
     const int brick = lb * (kBlock / 64) + (threadIdx.x >> 6);
@@ -114,20 +116,49 @@ __global__ __launch_bounds__(kBlock) void kSelfIntersections(MeshDev m, int nLog
     out[L.face] = (wn < 0 || wn > 1) ? 1 : 0;
 }
 
-// At most 72 VGPRs: seven waves per SIMD (the LDS of seven blocks fits a CU); the walks are bound by
-// the latency of their dependent scalar loads, and the seventh wave hides more of it than the
-// registers it costs (signed distance 105 -> 98 ms at k=8 256^3).
-// CAPPED: the capped form (bound and rerun lists given).
-template <int D, bool FILTER, bool CAPPED>
+// The lane form: every voxel of a 4x4x4 brick walks for itself (laneWalk), one wave per workgroup so that a
+// finished wave's LDS goes to the next one at once.  Measured against the wave-cooperative form with hand-over
+// (both with the winding-number sign): k=8 256^3 98.4 -> 26.4 ms, k=5 64^3 1.50 -> 0.77 ms.  CAPPED: voxels whose cap is below the plain limit and
+// finds nothing walk again without it, counted in failCount.
+template <bool CAPPED>
+__global__ __launch_bounds__(64, 4) void kSdfLane(MeshDev m, int dx, int dy, int zBegin, int zEnd, int nbx, int nby, int nbz,
+                                                  int nBricks, Xf xf, DistOpts o, const float* __restrict__ bound,
+                                                  uint32_t* __restrict__ failCount, float* __restrict__ out)
+{
+    extern __shared__ __align__(16) unsigned char laneMem[];
+    const int brick = gridBlock<64>();
+    if (brick >= nBricks) return;
+    const int lane = threadIdx.x & 63;
+    const LaneLds l = laneLds<false>(laneMem, m.depth, lane);
+    int x, y, z;
+    const bool valid = brickVoxel(brick, lane, nbx, nby, nbz, dx, dy, zBegin, zEnd, x, y, z);
+    float px = (float)x, py = (float)y, pz = (float)z;
+    xfApply(xf, px, py, pz);
+    const size_t idx = valid ? ((size_t)(z - zBegin) * dy + y) * dx + x : 0;
+    float lim = o.maxDistSq;
+    if (CAPPED && valid) { const float b = bound[idx]; lim = b < lim ? b : lim; }
+    float resSq = laneWalk<false>(m, l, px, py, pz, lim, valid, kStatQuadSteps, kStatLeafTests);
+    if (CAPPED) {
+        const bool again = valid && lim < o.maxDistSq && !(resSq < lim);
+        const uint64_t failed = waveBallot(again);
+        if (failed) {
+            if (lane == 0) atomicAdd(failCount, (uint32_t)__popcll(failed));
+            const float r = laneWalk<false>(m, l, px, py, pz, o.maxDistSq, again, kStatQuadSteps, kStatLeafTests);
+            if (again) resSq = r;
+        }
+    }
+    waveSync();
+    sdfStore(m, px, py, pz, valid, resSq, o, reinterpret_cast<uint4*>(laneMem), out, idx);
+}
+
+// The wave-cooperative form with hand-over, run when a step budget is set.
+template <int D, bool FILTER>
 __global__ __launch_bounds__(kBlock, 7) void kSdfGridCoop(MeshDev m, int dx, int dy, int zBegin, int zEnd,
                                                        int nbx, int nby, int nbz, int nLogical, Xf xf,
-                                                       DistOpts o, const float* __restrict__ bound,
-                                                       uint32_t* __restrict__ rerun,
-                                                       uint32_t* __restrict__ rerunCount,
-                                                       SplitScratch sc, float* __restrict__ out)
+                                                       DistOpts o, SplitScratch sc, float* __restrict__ out)
 {
     __shared__ DistStack<D> stkMem[kWaves];
-    const int lb = gridBlock();
+    const int lb = gridBlock<kGridChunk>();
     if (lb >= nLogical) return;
     const int lane = threadIdx.x & 63;
     const int w = threadIdx.x >> 6;
@@ -138,38 +169,20 @@ __global__ __launch_bounds__(kBlock, 7) void kSdfGridCoop(MeshDev m, int dx, int
     float px = (float)x, py = (float)y, pz = (float)z;
     xfApply(xf, px, py, pz);
     const size_t idx = valid ? ((size_t)(z - zBegin) * dy + y) * dx + x : 0;
-    float lim = o.maxDistSq;
-    if (CAPPED && valid) { const float b = bound[idx]; lim = b < lim ? b : lim; }
     bool stopped = false;
-    const float resSq = coopDistance<D, FILTER>(m, px, py, pz, valid ? lim : -1.f, &stkMem[w],
+    const float resSq = coopDistance<D, FILTER>(m, px, py, pz, valid ? o.maxDistSq : -1.f, &stkMem[w],
                                                 sc.list ? sc.budget : 0, &stopped);
-    // capped: a lane whose cap (below the plain limit) has found nothing
-    const bool uncapped = CAPPED && valid && !(resSq < lim) && lim < o.maxDistSq;
-    uint64_t failed = 0;
-    if (CAPPED) {
-        failed = waveBallot(uncapped && !stopped);      // searched to the end below a cap too small
-    }
-    if (stopped || (CAPPED && sc.list && failed)) {
-        // hand the brick to the split pass with every lane's best so far.  Capped: a lane with nothing
-        // below its cap continues uncapped from the greedy leaf (a real candidate), so every handed-over
-        // result is exact and nothing is searched a second time after the split pass.
-        float seed = resSq;
-        if (uncapped) {
-            const float g = greedyLeafDistSq(m, px, py, pz);
-            seed = g < o.maxDistSq ? g : o.maxDistSq;
-        }
+    if (stopped) {
+        // hand the brick to the split pass with every lane's best so far
         uint32_t slot = 0;
         if (lane == 0) slot = atomicAdd(&sc.counters[0], 1u);
         slot = (uint32_t)uniform((int)slot);
         if (lane == 0) sc.list[slot] = (uint32_t)brick;
-        sc.best[(size_t)slot * 64 + lane] = __float_as_uint(valid ? seed : -1.f);
+        sc.best[(size_t)slot * 64 + lane] = __float_as_uint(valid ? resSq : -1.f);
         rankCut(m, valid, px, py, pz, sc.order + (size_t)slot * 64);
         return;
     }
-    // without a split scratch (a tree too small to cut) the failed lanes go to the rerun list
-    const bool again = CAPPED && uncapped;
-    if (CAPPED) appendWave(again, (uint32_t)idx, rerun, rerunCount);
-    sdfStore(m, px, py, pz, valid && !again, resSq, o, reinterpret_cast<uint4*>(&stkMem[w]), out, idx);
+    sdfStore(m, px, py, pz, valid, resSq, o, reinterpret_cast<uint4*>(&stkMem[w]), out, idx);
 }
 
 // Second launch of the split form: persistent waves take (handed-over brick, cut subtree) pairs and
@@ -207,14 +220,11 @@ __global__ __launch_bounds__(kBlock) void kSdfSplit(MeshDev m, int dx, int dy, i
     }
 }
 
-// Third launch: the handed-over bricks' results (sign from the winding number, NaN band, store).  Every
-// handed-over search is exact: the capped form hands its failed caps over uncapped.  With caps (bound),
-// failCount counts the voxels whose cap (below maxDistSq) was below their distance.
+// Third launch: the handed-over bricks' results (sign from the winding number, NaN band, store).
 template <int D>
 __global__ __launch_bounds__(kBlock) void kSdfSplitFinish(MeshDev m, int dx, int dy, int zBegin, int zEnd,
                                                             int nbx, int nby, int nbz, Xf xf, DistOpts o,
-                                                            SplitScratch sc, const float* __restrict__ bound,
-                                                            uint32_t* __restrict__ failCount, float* __restrict__ out)
+                                                            SplitScratch sc, float* __restrict__ out)
 {
     __shared__ float4 stkMem[kWaves][2 * quadStack(D)];
     const int lane = threadIdx.x & 63;
@@ -232,37 +242,8 @@ __global__ __launch_bounds__(kBlock) void kSdfSplitFinish(MeshDev m, int dx, int
         xfApply(xf, px, py, pz);
         const size_t idx = valid ? ((size_t)(z - zBegin) * dy + y) * dx + x : 0;
         const float resSq = __uint_as_float(sc.best[(size_t)t * 64 + lane]);
-        if (bound) {
-            const float b = valid ? bound[idx] : o.maxDistSq;
-            const uint64_t f = waveBallot(valid && b < o.maxDistSq && !(resSq < b));
-            if (f && lane == 0) atomicAdd(failCount, (uint32_t)__popcll(f));
-        }
         sdfStore(m, px, py, pz, valid, resSq, o, reinterpret_cast<uint4*>(stkMem[w]), out, idx);
     }
-}
-
-// the listed voxels of a z-slab (ids relative to the slab), searched without any cap
-template <int D>
-__global__ __launch_bounds__(kBlock) void kSdfVoxelsCoop(MeshDev m, int dx, int dy, int zBegin,
-                                                         const uint32_t* __restrict__ list, int64_t count,
-                                                         int nLogical, Xf xf, DistOpts o,
-                                                         float* __restrict__ out)
-{
-    __shared__ DistStack<D> stkMem[kWaves];
-    const int lb = logicalBlock(nLogical);
-    if (lb >= nLogical) return;
-    const int64_t i = (int64_t)lb * kBlock + threadIdx.x;
-    const bool valid = i < count;
-    if (!waveBallot(valid)) return;
-    const size_t idx = valid ? list[i] : 0;
-    const size_t layer = (size_t)dx * dy;
-    const int z = zBegin + (int)(idx / layer);
-    const int rem = (int)(idx % layer);
-    float px = (float)(rem % dx), py = (float)(rem / dx), pz = (float)z;
-    xfApply(xf, px, py, pz);
-    const int w = threadIdx.x >> 6;
-    const float resSq = coopDistance<D>(m, px, py, pz, valid ? o.maxDistSq : -1.f, &stkMem[w]);
-    sdfStore(m, px, py, pz, valid, resSq, o, reinterpret_cast<uint4*>(&stkMem[w]), out, idx);
 }
 
 template <int D>
@@ -271,7 +252,7 @@ __global__ __launch_bounds__(kBlock) void kFwnGridCoop(MeshDev m, int dx, int dy
                                                        float beta, float* __restrict__ out)
 {
     __shared__ uint4 stkMem[kWaves][D];
-    const int lb = gridBlock();
+    const int lb = gridBlock<kGridChunk>();
     if (lb >= nLogical) return;
     const int lane = threadIdx.x & 63;
     const int w = threadIdx.x >> 6;
@@ -332,21 +313,16 @@ __global__ __launch_bounds__(kBlock) void kSelfIntersectionsCoop(MeshDev m, int 
 // range is cut into 8 contiguous parts, one per XCD (blocks are dealt to XCDs round-robin), and a
 // wave whose part is drained moves on to the next part: spatially adjacent units share an L2,
 // and the tail is balanced.  Every wave exits once it has seen every part drained.
-// CAPPED: the items' caps apply; a wave whose lanes found nothing below a cap smaller than the plain
-// limit walks once more for them, uncapped (persistent waves take new units meanwhile, so the retries do
-// not form a tail of their own as a separate launch over scattered queries would).
-template <int D, bool CAPPED>
-__global__ __launch_bounds__(kBlock) void kBatch(const BatchItem* __restrict__ items, int nItems, int64_t total,
-                                                 DistOpts o, float up, unsigned long long* __restrict__ tickets,
-                                                 int xcdSplit)
+// Queries walk one per lane (laneWalk).  CAPPED: the items' caps apply; lanes that found nothing below a cap
+// smaller than the plain limit walk once more, uncapped (persistent waves take new units meanwhile, so the
+// retries do not form a tail of their own as a separate launch over scattered queries would).
+template <bool CAPPED>
+__global__ __launch_bounds__(64, 4) void kBatch(const BatchItem* __restrict__ items, int nItems, int64_t total, DistOpts o,
+                                                float up, int depth, unsigned long long* __restrict__ tickets, int xcdSplit)
 {
-    union WaveStack {
-        DistStack<D> dist;
-        ProjStack<D> proj;
-        uint4 fwn[D];
-    };
-    __shared__ WaveStack stkMem[kWaves];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    extern __shared__ __align__(16) unsigned char laneMem[];
+    const int lane = threadIdx.x & 63;
+    const LaneLds l = laneLds<true>(laneMem, depth, lane);
     const int parts = xcdSplit ? kXcds : 1;
     int part = xcdSplit ? (int)(blockIdx.x % kXcds) : 0;
     int drained = 0;
@@ -377,17 +353,19 @@ __global__ __launch_bounds__(kBlock) void kBatch(const BatchItem* __restrict__ i
             xfApply(it.xf, px, py, pz);
             float lim = o.maxDistSq;
             if (CAPPED && it.capSdf && valid) { const float c = it.capSdf[idx]; lim = c < lim ? c : lim; }
-            float resSq = coopDistance<D>(it.m, px, py, pz, valid ? lim : -1.f, &stkMem[w].dist);
+            float resSq = laneWalk<false>(it.m, l, px, py, pz, lim, valid, kStatQuadSteps, kStatLeafTests);
             if (CAPPED) {
                 const bool retry = valid && !(resSq < lim) && lim < o.maxDistSq;
                 const uint64_t rm = waveBallot(retry);
                 if (rm) {
                     if (lane == 0) atomicAdd(it.rerunCount, (uint32_t)__popcll(rm));
-                    const float r = coopDistance<D>(it.m, px, py, pz, retry ? o.maxDistSq : -1.f, &stkMem[w].dist);
+                    const float r = laneWalk<false>(it.m, l, px, py, pz, o.maxDistSq, retry, kStatQuadSteps, kStatLeafTests);
                     if (retry) resSq = r;
                 }
             }
-            sdfStore(it.m, px, py, pz, valid, resSq, o, stkMem[w].fwn, it.sdf, idx);
+            waveSync();
+            sdfStore(it.m, px, py, pz, valid, resSq, o, reinterpret_cast<uint4*>(laneMem), it.sdf, idx);
+            waveSync();
         } else {
             const int64_t i = (lu - it.gridUnits) * 64 + lane;
             const bool valid = i < it.npts;
@@ -398,23 +376,19 @@ __global__ __launch_bounds__(kBlock) void kBatch(const BatchItem* __restrict__ i
                 px = it.pts[3 * q]; py = it.pts[3 * q + 1]; pz = it.pts[3 * q + 2];
                 if (CAPPED && it.capProj) { const float c = it.capProj[q]; lim = c < up ? c : up; }
             }
-            BestHit h;
-            coopProject<D>(it.m, px, py, pz, lim, valid, &stkMem[w].proj, h);
+            int leaf = -1;
+            float d = laneWalk<true>(it.m, l, px, py, pz, lim, valid, kStatKeyedSteps, kStatKeyedTests, &leaf);
             if (CAPPED) {
-                const bool retry = valid && h.face < 0 && lim < up;
+                const bool retry = valid && leaf < 0 && lim < up;
                 const uint64_t rm = waveBallot(retry);
                 if (rm) {
                     if (lane == 0) atomicAdd(it.rerunCount + 1, (uint32_t)__popcll(rm));
-                    BestHit h2;
-                    coopProject<D>(it.m, px, py, pz, up, retry, &stkMem[w].proj, h2);
-                    if (retry) h = h2;
+                    int leaf2 = -1;
+                    const float d2 = laneWalk<true>(it.m, l, px, py, pz, up, retry, kStatKeyedSteps, kStatKeyedTests, &leaf2);
+                    if (retry) { leaf = leaf2; d = d2; }
                 }
             }
-            if (valid) {
-                float4* op = reinterpret_cast<float4*>(it.proj + q);
-                op[0] = make_float4(__int_as_float(h.face), h.px, h.py, h.pz);
-                op[1] = make_float4(__int_as_float(-1), h.a, h.b, h.distSq);
-            }
+            if (valid) projStore(it.m, leaf, d, px, py, pz, it.proj + q);
         }
     }
 }
@@ -590,21 +564,16 @@ __global__ void kFillU32(uint32_t* p, int n, uint32_t v)
 } // namespace
 
 hipError_t launchBatch(const BatchItem* items, int nItems, int64_t totalUnits, const DistOpts& o, float up,
-                       unsigned long long* tickets, int xcdSplit, int blocks, int stackD, bool capped,
+                       unsigned long long* tickets, int xcdSplit, int blocks, int depth, bool capped,
                        hipStream_t s)
 {
     if (totalUnits <= 0 || nItems <= 0) return hipSuccess;
-    if (o.minDistSq > 0 || blocks <= 0) return hipErrorInvalidValue;
-    return dispatchDepth(stackD, [&](auto Dc) {
-        constexpr int D = decltype(Dc)::value;
-        if (capped)
-            hipLaunchKernelGGL((kBatch<D, true>), dim3(blocks), dim3(kBlock), 0, s, items, nItems, totalUnits, o, up,
-                               tickets, xcdSplit);
-        else
-            hipLaunchKernelGGL((kBatch<D, false>), dim3(blocks), dim3(kBlock), 0, s, items, nItems, totalUnits, o, up,
-                               tickets, xcdSplit);
-        return hipGetLastError();
-    });
+    if (o.minDistSq > 0 || blocks <= 0 || depth < 0) return hipErrorInvalidValue;
+    const size_t lds = laneSharedBytes(depth, true);
+    const auto kernel = capped ? kBatch<true> : kBatch<false>;
+    hipLaunchKernelGGL(kernel, dim3(blocks * kWaves), dim3(64), lds, s, items, nItems, totalUnits, o, up, depth, tickets,
+                       xcdSplit);
+    return hipGetLastError();
 }
 
 size_t splitScratchBytes(int64_t waves, int laneBytes)
@@ -697,19 +666,32 @@ int64_t sdfGridWaves(const int32_t dims[3], int32_t zBegin, int32_t zEnd)
 
 hipError_t launchSdfGrid(const MeshDev& m, const int32_t dims[3], const Xf& xf, const DistOpts& o,
                          int32_t zBegin, int32_t zEnd, float* out, int stackD, hipStream_t s,
-                         const float* bound, uint32_t* rerun, uint32_t* rerunCount, const SplitScratch* split)
+                         const float* bound, uint32_t* failCount, const SplitScratch* split)
 {
     const int nbx = (dims[0] + 3) / 4, nby = (dims[1] + 3) / 4, nbz = (zEnd - zBegin + 3) / 4;
     const int64_t bricks = (int64_t)nbx * nby * nbz;
     if (bricks <= 0) return hipSuccess;
     const int nLogical = (int)((bricks + 3) / 4);
-    // the wave-cooperative distance returns the minimum over candidates; with minDistSq > 0 the
-    // reference stops at the first candidate <= minDistSq in its own visit order, which the keyed walk
-    // reproduces (launchSdfGridKeyed; its split scratch holds 8 bytes per lane)
-    if (o.minDistSq > 0 && !bound && m.traversal == (int)Traversal::WaveCoop)
+    if (bound && (o.minDistSq > 0 || !failCount)) return hipErrorInvalidValue;
+    // the lane walk returns the minimum over candidates; with minDistSq > 0 the reference stops at the
+    // first candidate <= minDistSq in its own visit order, which the keyed walk reproduces
+    // (launchSdfGridKeyed; its split scratch holds 8 bytes per lane)
+    if (o.minDistSq > 0 && m.traversal == (int)Traversal::WaveCoop)
         return launchSdfGridKeyed(m, dims, xf, o, zBegin, zEnd, out, stackD, s, split);
-    const bool coop = (m.traversal == (int)Traversal::WaveCoop || bound) && !(o.minDistSq > 0);
-    if (bound && (!coop || !rerun || !rerunCount)) return hipErrorInvalidValue;
+    if (bound || (m.traversal == (int)Traversal::WaveCoop && !(split && split->list && split->budget > 0 && m.nCut > 0))) {
+        const auto kernel = bound ? kSdfLane<true> : kSdfLane<false>;
+        hipLaunchKernelGGL(kernel, dim3(chunkedGrid((int)bricks, 64)), dim3(64), laneSharedBytes(m.depth, false), s, m,
+                           dims[0], dims[1], zBegin, zEnd, nbx, nby, nbz, (int)bricks, xf, o, bound, failCount, out);
+        return hipGetLastError();
+    }
+    if (m.traversal != (int)Traversal::WaveCoop)
+        return dispatchDepth(stackD, [&](auto Dc) {
+            constexpr int D = decltype(Dc)::value;
+            hipLaunchKernelGGL(kSdfGrid<D>, dim3(chunkedGrid(nLogical, kGridChunk)), dim3(kBlock), 0, s, m, dims[0],
+                               dims[1], zBegin, zEnd, nbx, nby, nbz, nLogical, xf, o, out);
+            return hipGetLastError();
+        });
+    // A step budget was set: the wave-cooperative walks with hand-over.
     // The leaf filter saves instructions but adds a dependent load to every leaf visit.  It pays unless
     // a deep tree meets a small grid: then few waves walk long chains and nothing hides that load.
     // Measured on / off (bumpy spheres): k=5 64^3 0.89, k=7 128^3 0.87, k=8 96^3 0.96, k=8 256^3 0.87,
@@ -718,48 +700,21 @@ hipError_t launchSdfGrid(const MeshDev& m, const int32_t dims[3], const Xf& xf, 
     const int filterMode = m.leafFilter;
     const int64_t waves = sdfGridWaves(dims, zBegin, zEnd);
     const bool filter = filterMode < 0 ? waves > ((int64_t)1 << (m.depth > 8 ? m.depth - 8 : 0)) : filterMode != 0;
-    SplitScratch sc;
-    // the capped form takes the split scratch even with no step budget (its failed waves use it)
-    if (coop && split && split->list && (split->budget > 0 || bound) && m.nCut > 0) {
-        if ((int64_t)split->cap < sdfGridWaves(dims, zBegin, zEnd)) return hipErrorInvalidValue;
-        sc = *split;
-        hipError_t e = fillU32(sc.counters, 3, 0u, s);
-        if (e != hipSuccess) return e;
-    }
+    if ((int64_t)split->cap < waves) return hipErrorInvalidValue;
+    const SplitScratch sc = *split;
+    const hipError_t e = fillU32(sc.counters, 3, 0u, s);
+    if (e != hipSuccess) return e;
     return dispatchDepth(stackD, [&](auto Dc) {
         constexpr int D = decltype(Dc)::value;
-        if (coop) {
-            const auto gridKernel = bound ? (filter ? kSdfGridCoop<D, true, true> : kSdfGridCoop<D, false, true>)
-                                          : (filter ? kSdfGridCoop<D, true, false> : kSdfGridCoop<D, false, false>);
-            const auto splitKernel = filter ? kSdfSplit<D, true> : kSdfSplit<D, false>;
-            hipLaunchKernelGGL(gridKernel, dim3(chunkedGrid(nLogical)), dim3(kBlock), 0, s, m, dims[0], dims[1],
-                               zBegin, zEnd, nbx, nby, nbz, nLogical, xf, o, bound, rerun, rerunCount, sc, out);
-            if (sc.list) {
-                const int blocks = persistentBlocks();
-                hipLaunchKernelGGL(splitKernel, dim3(blocks), dim3(kBlock), 0, s, statLaunch(m, 1), dims[0], dims[1], zBegin, zEnd,
-                                   nbx, nby, nbz, xf, sc);
-                hipLaunchKernelGGL(kSdfSplitFinish<D>, dim3(blocks), dim3(kBlock), 0, s, statLaunch(m, 2), dims[0], dims[1],
-                                   zBegin, zEnd, nbx, nby, nbz, xf, o, sc, bound, rerunCount, out);
-            }
-        } else {
-            hipLaunchKernelGGL(kSdfGrid<D>, dim3(chunkedGrid(nLogical)), dim3(kBlock), 0, s, m, dims[0],
-                               dims[1], zBegin, zEnd, nbx, nby, nbz, nLogical, xf, o, out);
-        }
-        return hipGetLastError();
-    });
-}
-
-hipError_t launchSdfVoxels(const MeshDev& m, const int32_t dims[3], const Xf& xf, const DistOpts& o,
-                           int32_t zBegin, const uint32_t* list, int64_t count, float* out, int stackD,
-                           hipStream_t s)
-{
-    if (count <= 0) return hipSuccess;
-    if (o.minDistSq > 0) return hipErrorInvalidValue;
-    const int nLogical = (int)((count + kBlock - 1) / kBlock);
-    return dispatchDepth(stackD, [&](auto Dc) {
-        constexpr int D = decltype(Dc)::value;
-        hipLaunchKernelGGL(kSdfVoxelsCoop<D>, dim3(paddedGrid(nLogical)), dim3(kBlock), 0, s, m, dims[0], dims[1],
-                           zBegin, list, count, nLogical, xf, o, out);
+        const auto gridKernel = filter ? kSdfGridCoop<D, true> : kSdfGridCoop<D, false>;
+        const auto splitKernel = filter ? kSdfSplit<D, true> : kSdfSplit<D, false>;
+        hipLaunchKernelGGL(gridKernel, dim3(chunkedGrid(nLogical, kGridChunk)), dim3(kBlock), 0, s, m, dims[0], dims[1],
+                           zBegin, zEnd, nbx, nby, nbz, nLogical, xf, o, sc, out);
+        const int blocks = persistentBlocks();
+        hipLaunchKernelGGL(splitKernel, dim3(blocks), dim3(kBlock), 0, s, statLaunch(m, 1), dims[0], dims[1], zBegin, zEnd,
+                           nbx, nby, nbz, xf, sc);
+        hipLaunchKernelGGL(kSdfSplitFinish<D>, dim3(blocks), dim3(kBlock), 0, s, statLaunch(m, 2), dims[0], dims[1],
+                           zBegin, zEnd, nbx, nby, nbz, xf, o, sc, out);
         return hipGetLastError();
     });
 }
@@ -775,10 +730,10 @@ hipError_t launchFwnGrid(const MeshDev& m, const int32_t dims[3], const Xf& xf, 
     return dispatchDepth(stackD, [&](auto Dc) {
         constexpr int D = decltype(Dc)::value;
         if (coop)
-            hipLaunchKernelGGL(kFwnGridCoop<D>, dim3(chunkedGrid(nLogical)), dim3(kBlock), 0, s, m, dims[0],
+            hipLaunchKernelGGL(kFwnGridCoop<D>, dim3(chunkedGrid(nLogical, kGridChunk)), dim3(kBlock), 0, s, m, dims[0],
                                dims[1], zBegin, zEnd, nbx, nby, nbz, nLogical, xf, beta, out);
         else
-            hipLaunchKernelGGL(kFwnGrid<D>, dim3(chunkedGrid(nLogical)), dim3(kBlock), 0, s, m, dims[0],
+            hipLaunchKernelGGL(kFwnGrid<D>, dim3(chunkedGrid(nLogical, kGridChunk)), dim3(kBlock), 0, s, m, dims[0],
                                dims[1], zBegin, zEnd, nbx, nby, nbz, nLogical, xf, beta, out);
         return hipGetLastError();
     });

@@ -24,16 +24,17 @@ constexpr int kMaxCut = 1 << kCutDepth;
 // split form's last launch block 2).
 enum StatSlot : int {
     kStatWalks = 0,       // walks run (one per wave and walk)
-    kStatQuadSteps,       // distance walk: 4-wide node visits (128-B quad record each)
+    kStatQuadSteps,       // distance walk: wave steps (wave-cooperative: one 128-B quad record each)
     kStatPrismReads,      // distance walk: leaf visits reading the plane record (80 B each)
     kStatLeafTests,       // distance walk: leaf tests run (48-B triangle record each)
-    kStatKeyedSteps,      // keyed walk: node visits (128-B quad + 48-B node record each)
+    kStatKeyedSteps,      // projection walk: wave steps (wave-cooperative: one 128-B quad + 48-B node record each)
     kStatKeyedTests,      // keyed walk: leaf tests run (48-B triangle record each)
     kStatFwnVisits,       // winding number: node visits (32-B dipole record each)
     kStatFwnDescents,     // winding number: descents into an internal node's children (16-B refs)
     kStatFwnLeaves,       // winding number: exact solid angles (48-B triangle record each)
     kStatSeeds,           // greedy descents seeding a walk (one root-to-leaf path per wave)
     kStatSeedLevels,      // their levels (one 64-B node record each)
+    kStatLaneVisits,      // lane walks: nodes visited by a lane (64-B record each)
     kStatCount
 };
 constexpr int kStatStride = 16;
@@ -46,6 +47,7 @@ struct MeshDev {
     const float4* dleaf;   // 2 per leaf slot
     const float4* dquad;   // 8 per internal node: its grandchildren (4-wide records of the cooperative walks)
     const CutEntry* cut;   // nCut subtree roots covering every leaf once
+    const float4* cyl;     // 4 per internal node: its children's bounding cylinders (lane walks)
     const float4* prism;   // 5 per leaf slot: planes bounding the triangle (leaf filter of the walks)
     int32_t nCut;
     float rootMin[3], rootMax[3];
@@ -105,9 +107,9 @@ struct BatchItem {
 };
 
 // persistent launch over items[0..nItems) (device array); tickets = 8 zeroed 64-bit counters;
-// blocks = number of 256-thread workgroups to keep resident; capped: the items' caps apply
+// blocks = number of four-wave groups to keep resident; depth: of the deepest tree; capped: the items' caps apply
 hipError_t launchBatch(const BatchItem* items, int nItems, int64_t totalUnits, const DistOpts& o, float up,
-                       unsigned long long* tickets, int xcdSplit, int blocks, int stackD, bool capped,
+                       unsigned long long* tickets, int xcdSplit, int blocks, int depth, bool capped,
                        hipStream_t s);
 
 // small fill kernel (used instead of hipMemsetAsync so streams stay graph-capture safe)
@@ -119,6 +121,10 @@ int64_t projectionWaves(int64_t n);
 // 4-wide records from the binary records: internal node j's four grandchildren, a leaf child
 // standing for itself in one slot with an empty partner slot
 hipError_t buildQuads(const float4* dnode, int32_t numInternal, float4* dquad, hipStream_t s);
+// the bounding cylinders of every internal node's children (MeshDev::cyl) from the binary records;
+// scratch: cylinderScratchBytes(numFaces) device bytes
+size_t cylinderScratchBytes(int32_t numFaces);
+hipError_t buildCylinders(const MeshDev& m, float4* cyl, void* scratch, hipStream_t s);
 // the leaf-slot plane records of MeshDev::prism from the triangle records
 hipError_t buildPrisms(const float4* tri, int32_t numLeaves, float4* prism, hipStream_t s);
 
@@ -149,33 +155,28 @@ hipError_t fillU32(uint32_t* p, int n, uint32_t v, hipStream_t s);
 int stackDepthFor(int treeDepth);
 
 // z-layer slab [zBegin, zEnd) of the grid, output x-fastest
-// bound (optional): per-voxel cap on maxDistSq (indexed like out); with rerun lists given, voxels
-// whose cap found nothing are appended (slab-relative ids) instead of written
+// bound (optional): per-voxel cap on maxDistSq (indexed like out); voxels whose cap found nothing are
+// searched again without it and counted in failCount
 hipError_t launchSdfGrid(const MeshDev& m, const int32_t dims[3], const Xf& xf, const DistOpts& o,
                          int32_t zBegin, int32_t zEnd, float* out, int stackD, hipStream_t s,
-                         const float* bound = nullptr, uint32_t* rerun = nullptr, uint32_t* rerunCount = nullptr,
+                         const float* bound = nullptr, uint32_t* failCount = nullptr,
                          const SplitScratch* split = nullptr);
 // the same with minDistSq > 0 on the keyed walks (the reference's early exit at minDistSq reproduced
 // exactly); split scratch (optional) bound with 8 bytes per lane
 hipError_t launchSdfGridKeyed(const MeshDev& m, const int32_t dims[3], const Xf& xf, const DistOpts& o,
                               int32_t zBegin, int32_t zEnd, float* out, int stackD, hipStream_t s,
                               const SplitScratch* split);
-// the listed slab voxels, searched without a cap
-hipError_t launchSdfVoxels(const MeshDev& m, const int32_t dims[3], const Xf& xf, const DistOpts& o,
-                           int32_t zBegin, const uint32_t* list, int64_t count, float* out, int stackD,
-                           hipStream_t s);
 hipError_t launchFwnGrid(const MeshDev& m, const int32_t dims[3], const Xf& xf, float beta,
                          int32_t zBegin, int32_t zEnd, float* out, int stackD, hipStream_t s);
 // perm may be null (identity order)
 hipError_t launchFwnPoints(const MeshDev& m, const float* pts, const uint32_t* perm, int64_t n,
                            float beta, int32_t skipFace, float* out, int stackD, hipStream_t s);
 hipError_t launchSelfIntersections(const MeshDev& m, float beta, uint8_t* out, int stackD, hipStream_t s);
-// bound (optional): per-query cap on up (indexed by query); rerun lists as for launchSdfGrid
+// bound (optional): per-query limit below up (indexed by query); with failCount it is a cap as for launchSdfGrid
 hipError_t launchProjections(const MeshDev& m, const float* pts, const uint32_t* perm, int64_t n,
                              const Xf* ptXf, const Xf* treeXf, float up, float lo, ProjRec* out,
                              int stackD, hipStream_t s, const float* bound = nullptr,
-                             uint32_t* rerun = nullptr, uint32_t* rerunCount = nullptr,
-                             const SplitScratch* split = nullptr);
+                             uint32_t* failCount = nullptr, const SplitScratch* split = nullptr);
 
 // spatial ordering of query points: Morton codes over box [lo, hi] then a radix sort.
 // workspace layout is private; query its size first with ws == nullptr.

@@ -10,7 +10,7 @@
 //   * else the first leaf of its order at the minimum distance.
 // Both are the minimum of (max(d, loE), key), which does not depend on the visit order: the shared
 // wave walks, the split form's partial walks and their atomic merges all reproduce it exactly.
-#include "mi_walk.hpp"
+#include "mi_lane.hpp"
 
 namespace mi {
 namespace {
@@ -111,65 +111,67 @@ __device__ __forceinline__ int keyLeaf(const MeshDev& m, uint32_t key, float px,
 
 // ---------------------------------------------------------------- projections
 
-// bound (optional, indexed like the output): a per-query cap on upDistLimitSq.  With rerun lists
-// given, a query whose cap was below `up` and that found nothing below the cap is not written but
-// appended to the list, to be searched again without the cap (any cap above the true distance
-// gives the reference's record, so the combination is exact).  lo: loDistLimitSq.  CAPPED: rerun lists
-// given (the capped form); without them a bound is a plain per-query limit (the bounded form).
-template <int D, bool CAPPED>
+// The lane form (loDistLimitSq <= 0): every query walks for itself (laneWalk).  Measured against the
+// wave-cooperative form with hand-over: 2^22 points on 1.3 M triangles 64.6 -> 8.7 ms, 300 k ICP samples on
+// 328 k triangles 1.08 -> 0.53 ms, 1000 points on 20 k triangles 1.09 -> 0.23 ms.  bound (optional, indexed like
+// the output): a limit per query below `up`.  CAPPED: the bound is a guess; queries that find nothing below a
+// cap smaller than `up` walk again without it, counted in failCount (any cap above the true distance gives the
+// reference's record, so the combination is exact).
+template <bool CAPPED>
+__global__ __launch_bounds__(64, 4) void kProjectionsLane(MeshDev m, const float* __restrict__ pts,
+                                                          const uint32_t* __restrict__ perm, int64_t n, int nWaves, Xf ptXf,
+                                                          int hasPtXf, float up, const float* __restrict__ bound,
+                                                          uint32_t* __restrict__ failCount, ProjRec* __restrict__ out)
+{
+    extern __shared__ __align__(16) unsigned char laneMem[];
+    const int wv = logicalBlock(nWaves);
+    if (wv >= nWaves) return;
+    const int lane = threadIdx.x & 63;
+    const LaneLds l = laneLds<true>(laneMem, m.depth, lane);
+    int64_t q;
+    float px, py, pz, lim;
+    const bool valid = projQuery(pts, perm, n, ptXf, hasPtXf, up, bound, (uint32_t)wv, lane, q, px, py, pz, lim);
+    int leaf = -1;
+    float d = laneWalk<true>(m, l, px, py, pz, lim, valid, kStatKeyedSteps, kStatKeyedTests, &leaf);
+    if (CAPPED) {
+        const bool again = valid && leaf < 0 && lim < up;
+        const uint64_t failed = waveBallot(again);
+        if (failed) {
+            if (lane == 0) atomicAdd(failCount, (uint32_t)__popcll(failed));
+            int leaf2 = -1;
+            const float d2 = laneWalk<true>(m, l, px, py, pz, up, again, kStatKeyedSteps, kStatKeyedTests, &leaf2);
+            if (again) { leaf = leaf2; d = d2; }
+        }
+    }
+    if (valid) projStore(m, leaf, d, px, py, pz, out + q);
+}
+
+// The wave-cooperative form: bounds as plain limits per query, lo = loDistLimitSq.
+template <int D>
 __global__ __launch_bounds__(kBlock) void kProjectionsCoop(MeshDev m, const float* __restrict__ pts,
                                                            const uint32_t* __restrict__ perm, int64_t n,
                                                            int nLogical, Xf ptXf, int hasPtXf, float up, float lo,
                                                            const float* __restrict__ bound,
-                                                           uint32_t* __restrict__ rerun,
-                                                           uint32_t* __restrict__ rerunCount,
                                                            SplitScratch sc, ProjRec* __restrict__ out)
 {
     __shared__ ProjStack<D> stkMem[kWaves];
     const int lb = logicalBlock(nLogical);
     if (lb >= nLogical) return;
-    const int64_t i = (int64_t)lb * kBlock + threadIdx.x;
-    const bool valid = i < n;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const uint32_t wv = (uint32_t)(lb * kWaves + w);
+    int64_t q;
+    float px, py, pz, lim;
+    const bool valid = projQuery(pts, perm, n, ptXf, hasPtXf, up, bound, wv, lane, q, px, py, pz, lim);
     if (!waveBallot(valid)) return;
-    const int64_t q = valid ? (perm ? (int64_t)perm[i] : i) : 0;
-    float px = 0, py = 0, pz = 0;
-    float lim = up;
-    if (valid) {
-        px = pts[3 * q]; py = pts[3 * q + 1]; pz = pts[3 * q + 2];
-        if (hasPtXf) xfApply(ptXf, px, py, pz);
-        if (bound) { const float b = bound[q]; lim = b < up ? b : up; }
-    }
-    const int w = threadIdx.x >> 6;
     BestHit h;
     uint32_t key = 0;
     bool stopped = false;
     coopProject<D>(m, px, py, pz, lim, valid, &stkMem[w], h, &key, sc.list ? sc.budget : 0, &stopped, lo);
-    // capped: a lane whose cap (below up) has found nothing
-    const bool uncapped = CAPPED && valid && h.face < 0 && lim < up;
-    uint64_t failed = 0;
-    if (CAPPED) {
-        failed = waveBallot(uncapped && !stopped);      // searched to the end below a cap too small
-    }
-    if (stopped || (CAPPED && sc.list && failed)) {
-        // capped: a lane with nothing below its cap continues uncapped, from a radius just above the
-        // greedy leaf as coopProject starts, so every handed-over record is exact and nothing is searched
-        // a second time after the split pass
-        float seedE = h.distSq;
-        uint32_t seedKey = key;
-        if (uncapped) {
-            const float loE = effectiveLo(lo, up);
-            const float g = loOrder(greedyLeafDistSq(m, px, py, pz), loE);
-            const float above = g < FLT_MIN ? FLT_MIN : __uint_as_float(__float_as_uint(g) + 1u);
-            seedE = g < up && above < up ? above : up;
-            seedKey = 0;
-        }
-        handOver(m, sc, (uint32_t)(lb * kWaves + w), valid, px, py, pz, seedE, seedKey);
+    if (stopped) {
+        handOver(m, sc, wv, valid, px, py, pz, h.distSq, key);
         return;
     }
-    // without a split scratch (a tree too small to cut) the failed lanes go to the rerun list
-    const bool again = uncapped;
-    if (CAPPED) appendWave(again, (uint32_t)q, rerun, rerunCount);
-    if (!valid || again) return;
+    if (!valid) return;
     float4* o = reinterpret_cast<float4*>(out + q);
     o[0] = make_float4(__int_as_float(h.face), h.px, h.py, h.pz);
     o[1] = make_float4(__int_as_float(-1), h.a, h.b, h.distSq);
@@ -232,12 +234,10 @@ __global__ __launch_bounds__(kBlock) void kKeyedSplit(MeshDev m, Src src, SplitS
 }
 
 // Third launch of the split projections: the handed-over waves' records, from the leaf the winning
-// key names (its closest point and true squared distance recomputed exactly as the leaf test).  caps
-// (the capped form): failCount counts the queries whose cap (below up) was below their result.
+// key names (its closest point and true squared distance recomputed exactly as the leaf test).
 template <int D>
 __global__ __launch_bounds__(kBlock) void kProjSplitFinish(MeshDev m, PointSource src, SplitScratch sc,
-                                                           const float* __restrict__ caps,
-                                                           uint32_t* __restrict__ failCount, ProjRec* __restrict__ out)
+                                                           ProjRec* __restrict__ out)
 {
     const int lane = threadIdx.x & 63;
     const unsigned long long* best = reinterpret_cast<const unsigned long long*>(sc.best);
@@ -250,33 +250,11 @@ __global__ __launch_bounds__(kBlock) void kProjSplitFinish(MeshDev m, PointSourc
         int64_t q;
         float px, py, pz, lim;
         const bool valid = src.get(sc.list[t], lane, q, px, py, pz, lim);
-        const unsigned long long b = valid ? best[(size_t)t * 64 + lane] : 0ull;
-        const float e = __uint_as_float((uint32_t)(b >> 32));
-        if (caps) {
-            const float c = valid ? caps[q] : src.up;
-            const uint64_t f = waveBallot(valid && c < src.up && !(e < c));
-            if (f && lane == 0) atomicAdd(failCount, (uint32_t)__popcll(f));
-        }
         if (!valid) continue;
-        float4* o = reinterpret_cast<float4*>(out + q);
+        const unsigned long long b = best[(size_t)t * 64 + lane];
+        const float e = __uint_as_float((uint32_t)(b >> 32));
         // a winner has d < lim, i.e. order value < lim (loE < lim); otherwise the reference's empty result
-        const int leaf = e < lim ? keyLeaf(m, (uint32_t)b, px, py, pz) : -1;
-        if (leaf < 0) {
-            o[0] = make_float4(__int_as_float(-1), 0.f, 0.f, 0.f);
-            o[1] = make_float4(__int_as_float(-1), 0.f, 0.f, lim);
-            continue;
-        }
-        const Leaf L = loadLeafLanes(m.tri, leaf);
-        const double pd[3] = { px, py, pz };
-        const double ad[3] = { L.a[0], L.a[1], L.a[2] };
-        const double bd[3] = { L.b[0], L.b[1], L.b[2] };
-        const double cd[3] = { L.c[0], L.c[1], L.c[2] };
-        double pr[3], ba, bb;
-        closestPointD(pd, ad, bd, cd, pr, ba, bb);
-        const float qx = (float)pr[0], qy = (float)pr[1], qz = (float)pr[2];
-        const float dx = qx - px, dy = qy - py, dz = qz - pz;
-        o[0] = make_float4(__int_as_float(L.face), qx, qy, qz);
-        o[1] = make_float4(__int_as_float(-1), (float)ba, (float)bb, dx * dx + dy * dy + dz * dz);
+        projStore(m, e < lim ? keyLeaf(m, (uint32_t)b, px, py, pz) : -1, lim, px, py, pz, out + q);
     }
 }
 
@@ -290,7 +268,7 @@ __global__ __launch_bounds__(kBlock) void kSdfBandGrid(MeshDev m, BrickSource sr
                                                        SplitScratch sc, float* __restrict__ out)
 {
     __shared__ ProjStack<D> stkMem[kWaves];
-    const int lb = gridBlock();
+    const int lb = gridBlock<kGridChunk>();
     if (lb >= nLogical) return;
     const int lane = threadIdx.x & 63;
     const int w = threadIdx.x >> 6;
@@ -345,22 +323,29 @@ __global__ __launch_bounds__(kBlock) void kSdfBandFinish(MeshDev m, BrickSource 
 
 hipError_t launchProjections(const MeshDev& m, const float* pts, const uint32_t* perm, int64_t n,
                              const Xf* ptXf, const Xf* treeXf, float up, float lo, ProjRec* out,
-                             int stackD, hipStream_t s, const float* bound, uint32_t* rerun,
-                             uint32_t* rerunCount, const SplitScratch* split)
+                             int stackD, hipStream_t s, const float* bound, uint32_t* failCount,
+                             const SplitScratch* split)
 {
     if (n <= 0) return hipSuccess;
     const int nLogical = (int)((n + kBlock - 1) / kBlock);
     Xf px{}, tx{};
     if (ptXf) px = *ptXf;
     if (treeXf) tx = *treeXf;
-    // the keyed walk reproduces the reference's record for every loDistLimitSq; a non-rigid tree
-    // transform (applied per box) keeps the per-lane form
-    const bool coopOk = !treeXf;
-    const bool coop = coopOk && (m.traversal == (int)Traversal::WaveCoop || rerun);
-    if (rerun && (!coop || !rerunCount || !bound)) return hipErrorInvalidValue;
+    if (failCount && (treeXf || !bound || lo > 0)) return hipErrorInvalidValue;
+    const bool coop = !treeXf && m.traversal == (int)Traversal::WaveCoop;
+    const bool steps = split && split->list && split->budget > 0 && m.nCut > 0;
+    // lo > 0: the record depends on the reference's visit order, which the keyed walk reproduces; a step
+    // budget asks for the wave-cooperative form; a non-rigid tree transform (applied per box) keeps the
+    // per-lane form
+    if (failCount || (coop && !(lo > 0) && !steps)) {
+        const int nWaves = (int)((n + 63) / 64);
+        const auto kernel = failCount ? kProjectionsLane<true> : kProjectionsLane<false>;
+        hipLaunchKernelGGL(kernel, dim3(paddedGrid(nWaves)), dim3(64), laneSharedBytes(m.depth, true), s, m, pts, perm, n,
+                           nWaves, px, ptXf ? 1 : 0, up, bound, failCount, out);
+        return hipGetLastError();
+    }
     SplitScratch sc;
-    // the capped form takes the split scratch even with no step budget (its failed waves use it)
-    if (coop && split && split->list && (split->budget > 0 || rerun) && m.nCut > 0) {
+    if (coop && steps) {
         if ((int64_t)split->cap < projectionWaves(n)) return hipErrorInvalidValue;
         sc = *split;
         hipError_t e = fillU32(sc.counters, 3, 0u, s);
@@ -369,21 +354,14 @@ hipError_t launchProjections(const MeshDev& m, const float* pts, const uint32_t*
     return dispatchDepth(stackD, [&](auto Dc) {
         constexpr int D = decltype(Dc)::value;
         if (coop) {
-            if (rerun)
-                hipLaunchKernelGGL((kProjectionsCoop<D, true>), dim3(paddedGrid(nLogical)), dim3(kBlock), 0, s, m,
-                                   pts, perm, n, nLogical, px, ptXf ? 1 : 0, up, lo, bound, rerun, rerunCount, sc, out);
-            else
-                hipLaunchKernelGGL((kProjectionsCoop<D, false>), dim3(paddedGrid(nLogical)), dim3(kBlock), 0, s, m,
-                                   pts, perm, n, nLogical, px, ptXf ? 1 : 0, up, lo, bound, rerun, rerunCount, sc, out);
+            hipLaunchKernelGGL(kProjectionsCoop<D>, dim3(paddedGrid(nLogical)), dim3(kBlock), 0, s, m, pts, perm, n,
+                               nLogical, px, ptXf ? 1 : 0, up, lo, bound, sc, out);
             if (sc.list) {
-                // the capped form hands over uncapped searches (the bound no longer applies); the bounded
-                // form keeps its per-query limits
-                const PointSource src{ pts, perm, n, px, ptXf ? 1 : 0, up, lo, rerun ? nullptr : bound };
+                const PointSource src{ pts, perm, n, px, ptXf ? 1 : 0, up, lo, bound };
                 const int blocks = persistentBlocks();
                 hipLaunchKernelGGL((kKeyedSplit<D, PointSource>), dim3(blocks), dim3(kBlock), 0, s, statLaunch(m, 1),
                                    src, sc);
-                hipLaunchKernelGGL(kProjSplitFinish<D>, dim3(blocks), dim3(kBlock), 0, s, statLaunch(m, 2), src, sc,
-                                   rerun ? bound : nullptr, rerunCount, out);
+                hipLaunchKernelGGL(kProjSplitFinish<D>, dim3(blocks), dim3(kBlock), 0, s, statLaunch(m, 2), src, sc, out);
             }
         } else if (treeXf)
             hipLaunchKernelGGL((kProjections<true, D>), dim3(paddedGrid(nLogical)), dim3(kBlock), 0, s,
@@ -413,7 +391,7 @@ hipError_t launchSdfGridKeyed(const MeshDev& m, const int32_t dims[3], const Xf&
     const BrickSource src{ dims[0], dims[1], zBegin, zEnd, nbx, nby, nbz, xf, o.maxDistSq, o.minDistSq };
     return dispatchDepth(stackD, [&](auto Dc) {
         constexpr int D = decltype(Dc)::value;
-        hipLaunchKernelGGL(kSdfBandGrid<D>, dim3(chunkedGrid(nLogical)), dim3(kBlock), 0, s, m, src, nLogical, o, sc,
+        hipLaunchKernelGGL(kSdfBandGrid<D>, dim3(chunkedGrid(nLogical, kGridChunk)), dim3(kBlock), 0, s, m, src, nLogical, o, sc,
                            out);
         if (sc.list) {
             const int blocks = persistentBlocks();

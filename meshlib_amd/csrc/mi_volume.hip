@@ -1,0 +1,224 @@
+// mi_volume.hip -- bounding cylinders of the tree's nodes (MeshDev::cyl, read by the lane walks).
+//
+// A node's cylinder: axis n = its dipole's direction area, normalised; centre c = the centre of its box,
+// moved along n to the middle of its vertices' range; t = half that range, r = the largest distance of a
+// vertex from the axis.  Every vertex lies inside, hence every triangle.
+//
+// The record of internal node j is 64 bytes, 32 per child: (c, n.x), (n.y, n.z, t and r as two bf16, ref).
+// t and r are widened before they are rounded up to bf16:
+//  * 1.4 * 2^-23 * M, M the largest coordinate of a vertex: the leaf test rounds its closest point to
+//    float (half a unit of 2^-23 per coordinate, hence at most sqrt(3) / 2 of it in length), the rest is
+//    for the rounding of c and of the vertices' offsets from it;
+//  * (t + r) * 2^-19: the walk's float dot products, whose error is a few units of 2^-24 of the offset
+//    from c, and the part of that offset beyond t and r is covered by the walk's own relative slack.
+//
+// Cost on one MI355X: one pass in which every leaf goes down its own path (20 levels, 64 + 32 bytes a
+// level, shared by neighbours), reduced within the wave before the atomics.
+#include "mi_walk.hpp"
+
+namespace mi {
+namespace {
+
+struct Frame { float c[3], n[3]; };
+
+// axis and provisional centre of a node with the box [mn, mx] and the direction area (nx, ny, nz)
+__device__ __forceinline__ Frame nodeFrame(const float mn[3], const float mx[3], float nx, float ny, float nz)
+{
+    Frame f;
+    for (int i = 0; i < 3; ++i) f.c[i] = 0.5f * mn[i] + 0.5f * mx[i];
+    const float big = fmaxf(fabsf(nx), fmaxf(fabsf(ny), fabsf(nz)));
+    f.n[0] = 1.f; f.n[1] = 0.f; f.n[2] = 0.f;
+    if (big > 0 && big < INFINITY) {
+        const float x = nx / big, y = ny / big, z = nz / big;
+        const float len = sqrtf(x * x + y * y + z * z);
+        f.n[0] = x / len; f.n[1] = y / len; f.n[2] = z / len;
+    }
+    return f;
+}
+
+// offset of a vertex along the axis and its squared distance from it
+__device__ __forceinline__ void along(const Frame& f, const float* v, float& h, float& rr)
+{
+    const float x = v[0] - f.c[0], y = v[1] - f.c[1], z = v[2] - f.c[2];
+    h = x * f.n[0] + y * f.n[1] + z * f.n[2];
+    const float a = x - h * f.n[0], b = y - h * f.n[1], c = z - h * f.n[2];
+    rr = a * a + b * b + c * c;
+}
+
+// floats as unsigned integers of the same order (NaN above everything)
+__device__ __forceinline__ uint32_t ordered(float x)
+{
+    const uint32_t b = __float_as_uint(x);
+    return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
+}
+__device__ __forceinline__ float unordered(uint32_t u)
+{
+    return __uint_as_float((u & 0x80000000u) ? (u & 0x7fffffffu) : ~u);
+}
+
+// per internal node: ordered(max h), ordered(max -h), bits of max rr
+struct Range { uint32_t hi, lo, rr, pad; };
+
+__global__ __launch_bounds__(kBlock) void kCylinderRanges(MeshDev m, Range* __restrict__ range)
+{
+    const int slot = blockIdx.x * kBlock + threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    const bool valid = slot < m.numFaces;
+    Leaf L = loadLeafLanes(m.tri, valid ? slot : 0);
+    int first = 0, num = m.numFaces, node = valid ? m.rootRef : -1;
+    while (waveBallot(node >= 0)) {
+        float hi = -INFINITY, lo = -INFINITY, rr = 0.f;
+        int child = -1;
+        if (node >= 0) {
+            const float4 n0 = m.dnode[4 * (size_t)node], n1 = m.dnode[4 * (size_t)node + 1];
+            const float4 n2 = m.dnode[4 * (size_t)node + 2], n3 = m.dnode[4 * (size_t)node + 3];
+            const int h = num >> 1;
+            const bool right = slot >= first + h;
+            const float mn[3] = { right ? n1.z : n0.x, right ? n1.w : n0.y, right ? n2.x : n0.z };
+            const float mx[3] = { right ? n2.y : n0.w, right ? n2.z : n1.x, right ? n2.w : n1.y };
+            child = __float_as_int(right ? n3.y : n3.x);
+            if (right) first += h;
+            num = right ? num - h : h;
+            if (child >= 0) {
+                const float4 d = m.dint[2 * (size_t)child + 1];
+                const Frame f = nodeFrame(mn, mx, d.x, d.y, d.z);
+                const float* v[3] = { L.a, L.b, L.c };
+                for (int i = 0; i < 3; ++i) {
+                    float a, b;
+                    along(f, v[i], a, b);
+                    // a vertex without finite offsets makes the node's cylinder unbounded
+                    if (!(a - a == 0) || !(b < INFINITY)) { a = INFINITY; b = INFINITY; }
+                    hi = fmaxf(hi, a); lo = fmaxf(lo, -a); rr = fmaxf(rr, b);
+                }
+            }
+        }
+        node = child;
+        // neighbouring leaves share their ancestors: one atomic per run of equal nodes in the wave
+        for (int d = 1; d < 64; d <<= 1) {
+            const int on = __shfl_up(child, d);
+            const float oh = __shfl_up(hi, d), ol = __shfl_up(lo, d), orr = __shfl_up(rr, d);
+            if (lane >= d && on == child) { hi = fmaxf(hi, oh); lo = fmaxf(lo, ol); rr = fmaxf(rr, orr); }
+        }
+        const int next = __shfl_down(child, 1);
+        if (child >= 0 && (lane == 63 || next != child)) {
+            atomicMax(&range[child].hi, ordered(hi));
+            atomicMax(&range[child].lo, ordered(lo));
+            atomicMax(&range[child].rr, __float_as_uint(rr));
+        }
+    }
+}
+
+// the smallest bf16 not below x (x >= 0; infinity and NaN give infinity), in the upper half
+__device__ __forceinline__ uint32_t bf16Up(float x)
+{
+    if (!(x < INFINITY)) return 0x7f800000u;
+    return (__float_as_uint(x) + 0xffffu) & 0xffff0000u;
+}
+
+__device__ __forceinline__ void putCylinder(float4* out, const float c[3], const float n[3], float t, float r, float big,
+                                            int ref)
+{
+    const float wide = big * 0x1.4p-23f + (t + r) * 0x1p-19f;
+    bool ok = big < INFINITY && t < INFINITY && r < INFINITY;
+    for (int i = 0; i < 3; ++i) ok = ok && fabsf(c[i]) < INFINITY && fabsf(n[i]) < 2.f;
+    const uint32_t tr = ok ? bf16Up(t + wide) | (bf16Up(r + wide) >> 16) : 0x7f807f80u;
+    out[0] = make_float4(ok ? c[0] : 0.f, ok ? c[1] : 0.f, ok ? c[2] : 0.f, ok ? n[0] : 1.f);
+    out[1] = make_float4(ok ? n[1] : 0.f, ok ? n[2] : 0.f, __uint_as_float(tr), __int_as_float(ref));
+}
+
+// a leaf's cylinder: the triangle's normal and smallest enclosing circle (a degenerate triangle takes the
+// x axis and the middle of its longest edge)
+__device__ __forceinline__ void leafCylinder(const MeshDev& m, int slot, float4* out)
+{
+    const Leaf L = loadLeafLanes(m.tri, slot);
+    const float* v[3] = { L.a, L.b, L.c };
+    double e[3][3], len[3];       // edges v[i] -> v[i + 1]
+    for (int i = 0; i < 3; ++i) {
+        len[i] = 0;
+        for (int k = 0; k < 3; ++k) {
+            e[i][k] = (double)v[(i + 1) % 3][k] - v[i][k];
+            len[i] += e[i][k] * e[i][k];
+        }
+    }
+    const float nx = (float)(e[0][1] * e[1][2] - e[0][2] * e[1][1]);
+    const float ny = (float)(e[0][2] * e[1][0] - e[0][0] * e[1][2]);
+    const float nz = (float)(e[0][0] * e[1][1] - e[0][1] * e[1][0]);
+    int longest = 0;
+    if (len[1] > len[longest]) longest = 1;
+    if (len[2] > len[longest]) longest = 2;
+    const int i1 = (longest + 1) % 3, i2 = (longest + 2) % 3;
+    // weights of the corners: the circumcentre of an acute triangle, else the longest edge's middle
+    double w[3] = { 0, 0, 0 };
+    const double wa = len[1] * (len[0] + len[2] - len[1]), wb = len[2] * (len[0] + len[1] - len[2]);
+    const double wc = len[0] * (len[1] + len[2] - len[0]), sum = wa + wb + wc;
+    if (len[longest] < len[i1] + len[i2] && sum > 0) { w[0] = wa / sum; w[1] = wb / sum; w[2] = wc / sum; }
+    else { w[longest] = 0.5; w[i1] = 0.5; }
+    float c[3], big = 0.f;
+    for (int k = 0; k < 3; ++k) {
+        c[k] = (float)(w[0] * v[0][k] + w[1] * v[1][k] + w[2] * v[2][k]);
+        for (int i = 0; i < 3; ++i) big = fmaxf(big, fabsf(v[i][k]));
+        if (!(v[0][k] - v[0][k] == 0) || !(v[1][k] - v[1][k] == 0) || !(v[2][k] - v[2][k] == 0)) big = INFINITY;
+    }
+    Frame f = nodeFrame(c, c, nx, ny, nz);
+    for (int k = 0; k < 3; ++k) f.c[k] = c[k];
+    float t = 0.f, rr = 0.f;
+    for (int i = 0; i < 3; ++i) {
+        float h, q;
+        along(f, v[i], h, q);
+        t = fmaxf(t, fabsf(h));
+        rr = fmaxf(rr, q);
+    }
+    putCylinder(out, f.c, f.n, t, sqrtf(rr), big, ~slot);
+}
+
+__global__ __launch_bounds__(kBlock) void kCylinderRecords(MeshDev m, const Range* __restrict__ range, float4* __restrict__ cyl)
+{
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;      // child i & 1 of internal node i >> 1
+    if (i >= 2 * ((int64_t)m.numFaces - 1)) return;
+    const int j = (int)(i >> 1);
+    const float4 n0 = m.dnode[4 * (size_t)j], n1 = m.dnode[4 * (size_t)j + 1];
+    const float4 n2 = m.dnode[4 * (size_t)j + 2], n3 = m.dnode[4 * (size_t)j + 3];
+    const bool right = i & 1;
+    const int ref = __float_as_int(right ? n3.y : n3.x);
+    float4* out = cyl + 2 * (size_t)i;
+    if (ref < 0) {
+        leafCylinder(m, ~ref, out);
+        return;
+    }
+    const float mn[3] = { right ? n1.z : n0.x, right ? n1.w : n0.y, right ? n2.x : n0.z };
+    const float mx[3] = { right ? n2.y : n0.w, right ? n2.z : n1.x, right ? n2.w : n1.y };
+    const float4 d = m.dint[2 * (size_t)ref + 1];
+    Frame f = nodeFrame(mn, mx, d.x, d.y, d.z);
+    const float hi = unordered(range[ref].hi), lo = -unordered(range[ref].lo);
+    const float mid = 0.5f * hi + 0.5f * lo;
+    float big = 0.f;
+    for (int k = 0; k < 3; ++k) {
+        f.c[k] = f.c[k] + mid * f.n[k];
+        big = fmaxf(big, fmaxf(fabsf(mn[k]), fabsf(mx[k])));
+    }
+    putCylinder(out, f.c, f.n, 0.5f * hi - 0.5f * lo, sqrtf(__uint_as_float(range[ref].rr)), big, ref);
+}
+
+__global__ void kRangeInit(Range* r, int n)
+{
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < n) r[i] = Range{ 0u, 0u, 0u, 0u };
+}
+
+} // namespace
+
+size_t cylinderScratchBytes(int32_t numFaces) { return numFaces > 1 ? (size_t)(numFaces - 1) * sizeof(Range) : 0; }
+
+hipError_t buildCylinders(const MeshDev& m, float4* cyl, void* scratch, hipStream_t s)
+{
+    const int ni = m.numFaces - 1;
+    if (ni < 1) return hipSuccess;
+    Range* r = static_cast<Range*>(scratch);
+    hipLaunchKernelGGL(kRangeInit, dim3((ni + kBlock - 1) / kBlock), dim3(kBlock), 0, s, r, ni);
+    hipLaunchKernelGGL(kCylinderRanges, dim3((m.numFaces + kBlock - 1) / kBlock), dim3(kBlock), 0, s, m, r);
+    hipLaunchKernelGGL(kCylinderRecords, dim3((unsigned)((2 * (int64_t)ni + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, m, r,
+                       cyl);
+    return hipGetLastError();
+}
+
+} // namespace mi

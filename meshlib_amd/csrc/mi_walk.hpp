@@ -39,6 +39,14 @@ __device__ __forceinline__ float4 cload(const float4* p, size_t i)
     return make_float4(f[0], f[1], f[2], f[3]);
 }
 
+// a float4 through a global (not generic) load, also where the pointer itself came from memory
+typedef float lane4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ float4 gload(const float4* p, size_t i)
+{
+    const lane4 v = ((const __attribute__((address_space(1))) lane4*)p)[i];
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+
 __device__ __forceinline__ CutEntry loadCut(const MeshDev& m, uint32_t c)
 {
     const cint* e = (const cint*)(m.cut + c);
@@ -58,21 +66,22 @@ __device__ __forceinline__ int logicalBlock(int nLogical)
     return (b % kXcds) * per + b / kXcds;
 }
 
-// Grid kernels instead deal chunks of kGridChunk consecutive logical blocks (64 bricks) to the XCDs
+// Grid kernels instead deal chunks of consecutive logical blocks (64 bricks: 16 blocks of four waves) to the XCDs
 // in turn: each L2 still sees spatially compact runs, and the costly middle of a grid (voxels deep
 // inside the mesh) is spread over all eight XCDs instead of landing on two of them.  The launch
 // covers whole rounds of chunks (chunkedGrid), so the mapping is a bijection onto its blocks.
 constexpr int kGridChunk = 16;
+template <int CHUNK>
 __device__ __forceinline__ int gridBlock()
 {
     const int b = blockIdx.x;
     const int x = b % kXcds, r = b / kXcds;
-    return ((r / kGridChunk) * kXcds + x) * kGridChunk + r % kGridChunk;
+    return ((r / CHUNK) * kXcds + x) * CHUNK + r % CHUNK;
 }
 
-inline int chunkedGrid(int nLogical)
+inline int chunkedGrid(int nLogical, int chunk)
 {
-    const int round = kXcds * kGridChunk;
+    const int round = kXcds * chunk;
     return (nLogical + round - 1) / round * round;
 }
 
@@ -221,7 +230,7 @@ __device__ __forceinline__ float leafDistSq(const Leaf& L, float px, float py, f
 // The leaf record through vector loads: for per-lane leaf indices.
 __device__ __forceinline__ Leaf loadLeafLanes(const float4* __restrict__ tri, int k)
 {
-    const float4 t0 = tri[3 * (size_t)k], t1 = tri[3 * (size_t)k + 1], t2 = tri[3 * (size_t)k + 2];
+    const float4 t0 = gload(tri, 3 * (size_t)k), t1 = gload(tri, 3 * (size_t)k + 1), t2 = gload(tri, 3 * (size_t)k + 2);
     Leaf L;
     L.a[0] = t0.x; L.a[1] = t0.y; L.a[2] = t0.z;
     L.b[0] = t0.w; L.b[1] = t1.x; L.b[2] = t1.y;
@@ -1062,19 +1071,6 @@ __device__ __forceinline__ void rankCut(const MeshDev& m, bool valid, float px, 
     if (lane < m.nCut) order[rank] = (uint8_t)lane;
 }
 
-// appends `value` of every lane with p set to list[] (one atomic per wave)
-__device__ __forceinline__ void appendWave(bool p, uint32_t value, uint32_t* list, uint32_t* count)
-{
-    const uint64_t mask = waveBallot(p);
-    if (!mask) return;
-    const int lane = threadIdx.x & 63;
-    const int leader = __builtin_ctzll(mask);
-    uint32_t base = 0;
-    if (lane == leader) base = atomicAdd(count, (uint32_t)__popcll(mask));
-    base = (uint32_t)__builtin_amdgcn_readlane((int)base, leader);
-    if (p) list[base + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull))] = value;
-}
-
 // the query of lane `lane` of projection wave `wv` (as in kProjectionsCoop)
 __device__ __forceinline__ bool projQuery(const float* __restrict__ pts, const uint32_t* __restrict__ perm, int64_t n,
                                           const Xf& ptXf, int hasPtXf, float up, const float* __restrict__ bound,
@@ -1091,6 +1087,30 @@ __device__ __forceinline__ bool projQuery(const float* __restrict__ pts, const u
         if (bound) { const float b = bound[q]; lim = b < up ? b : up; }
     }
     return valid;
+}
+
+// stores a query's record: the closest point of leaf `leaf` (recomputed as the leaf test computes it), or the
+// reference's empty record with the search limit `lim`
+__device__ __forceinline__ void projStore(const MeshDev& m, int leaf, float lim, float px, float py, float pz,
+                                          ProjRec* __restrict__ out)
+{
+    float4* o = reinterpret_cast<float4*>(out);
+    if (leaf < 0) {
+        o[0] = make_float4(__int_as_float(-1), 0.f, 0.f, 0.f);
+        o[1] = make_float4(__int_as_float(-1), 0.f, 0.f, lim);
+        return;
+    }
+    const Leaf L = loadLeafLanes(m.tri, leaf);
+    const double pd[3] = { px, py, pz };
+    const double ad[3] = { L.a[0], L.a[1], L.a[2] };
+    const double bd[3] = { L.b[0], L.b[1], L.b[2] };
+    const double cd[3] = { L.c[0], L.c[1], L.c[2] };
+    double pr[3], ba, bb;
+    closestPointD(pd, ad, bd, cd, pr, ba, bb);
+    const float qx = (float)pr[0], qy = (float)pr[1], qz = (float)pr[2];
+    const float dx = qx - px, dy = qy - py, dz = qz - pz;
+    o[0] = make_float4(__int_as_float(L.face), qx, qy, qz);
+    o[1] = make_float4(__int_as_float(-1), (float)ba, (float)bb, dx * dx + dy * dy + dz * dz);
 }
 
 // shared tail of the signed-distance kernels: NaN band, winding-number sign, store
