@@ -118,7 +118,7 @@ __global__ __launch_bounds__(kBlock) void kSelfIntersections(MeshDev m, int nLog
 
 // The lane form: every voxel of a 4x4x4 brick walks for itself (laneWalk), one wave per workgroup so that a
 // finished wave's LDS goes to the next one at once.  Measured against the wave-cooperative form with hand-over
-// (both with the winding-number sign): k=8 256^3 98.4 -> 26.4 ms, k=5 64^3 1.50 -> 0.77 ms.  CAPPED: voxels whose cap is below the plain limit and
+// (both with the winding-number sign): k=8 256^3 101 -> 13.4 ms, k=5 64^3 1.48 -> 0.59 ms.  CAPPED: voxels whose cap is below the plain limit and
 // finds nothing walk again without it, counted in failCount.
 template <bool CAPPED>
 __global__ __launch_bounds__(64, 4) void kSdfLane(MeshDev m, int dx, int dy, int zBegin, int zEnd, int nbx, int nby, int nbz,
