@@ -148,7 +148,7 @@ __global__ __launch_bounds__(64, 4) void kSdfLane(MeshDev m, int dx, int dy, int
         }
     }
     waveSync();
-    sdfStore(m, px, py, pz, valid, resSq, o, reinterpret_cast<uint4*>(laneMem), out, idx);
+    sdfStore(m, px, py, pz, valid, resSq, o, out, idx);
 }
 
 // The wave-cooperative form with hand-over, run when a step budget is set.
@@ -182,7 +182,7 @@ __global__ __launch_bounds__(kBlock, 7) void kSdfGridCoop(MeshDev m, int dx, int
         rankCut(m, valid, px, py, pz, sc.order + (size_t)slot * 64);
         return;
     }
-    sdfStore(m, px, py, pz, valid, resSq, o, reinterpret_cast<uint4*>(&stkMem[w]), out, idx);
+    sdfStore(m, px, py, pz, valid, resSq, o, out, idx);
 }
 
 // Second launch of the split form: persistent waves take (handed-over brick, cut subtree) pairs and
@@ -221,12 +221,10 @@ __global__ __launch_bounds__(kBlock) void kSdfSplit(MeshDev m, int dx, int dy, i
 }
 
 // Third launch: the handed-over bricks' results (sign from the winding number, NaN band, store).
-template <int D>
 __global__ __launch_bounds__(kBlock) void kSdfSplitFinish(MeshDev m, int dx, int dy, int zBegin, int zEnd,
                                                             int nbx, int nby, int nbz, Xf xf, DistOpts o,
                                                             SplitScratch sc, float* __restrict__ out)
 {
-    __shared__ float4 stkMem[kWaves][2 * quadStack(D)];
     const int lane = threadIdx.x & 63;
     const int w = threadIdx.x >> 6;
     const uint32_t nHard = sc.counters[0] < sc.cap ? sc.counters[0] : sc.cap;
@@ -242,16 +240,14 @@ __global__ __launch_bounds__(kBlock) void kSdfSplitFinish(MeshDev m, int dx, int
         xfApply(xf, px, py, pz);
         const size_t idx = valid ? ((size_t)(z - zBegin) * dy + y) * dx + x : 0;
         const float resSq = __uint_as_float(sc.best[(size_t)t * 64 + lane]);
-        sdfStore(m, px, py, pz, valid, resSq, o, reinterpret_cast<uint4*>(stkMem[w]), out, idx);
+        sdfStore(m, px, py, pz, valid, resSq, o, out, idx);
     }
 }
 
-template <int D>
 __global__ __launch_bounds__(kBlock) void kFwnGridCoop(MeshDev m, int dx, int dy, int zBegin, int zEnd,
                                                        int nbx, int nby, int nbz, int nLogical, Xf xf,
                                                        float beta, float* __restrict__ out)
 {
-    __shared__ uint4 stkMem[kWaves][D];
     const int lb = gridBlock<kGridChunk>();
     if (lb >= nLogical) return;
     const int lane = threadIdx.x & 63;
@@ -262,18 +258,16 @@ __global__ __launch_bounds__(kBlock) void kFwnGridCoop(MeshDev m, int dx, int dy
     if (!waveBallot(valid)) return;
     float px = (float)x, py = (float)y, pz = (float)z;
     xfApply(xf, px, py, pz);
-    const float wn = coopWinding(m, px, py, pz, valid, beta, -1, stkMem[w]);
+    const float wn = coopWinding(m, px, py, pz, valid, beta, -1);
     if (!valid) return;
     out[((size_t)(z - zBegin) * dy + y) * dx + x] = wn;
 }
 
-template <int D>
 __global__ __launch_bounds__(kBlock) void kFwnPointsCoop(MeshDev m, const float* __restrict__ pts,
                                                          const uint32_t* __restrict__ perm, int64_t n,
                                                          int nLogical, float beta, int32_t skipFace,
                                                          float* __restrict__ out)
 {
-    __shared__ uint4 stkMem[kWaves][D];
     const int lb = logicalBlock(nLogical);
     if (lb >= nLogical) return;
     const int64_t i = (int64_t)lb * kBlock + threadIdx.x;
@@ -282,15 +276,13 @@ __global__ __launch_bounds__(kBlock) void kFwnPointsCoop(MeshDev m, const float*
     const int64_t q = valid ? (perm ? (int64_t)perm[i] : i) : 0;
     float px = 0, py = 0, pz = 0;
     if (valid) { px = pts[3 * q]; py = pts[3 * q + 1]; pz = pts[3 * q + 2]; }
-    const float wn = coopWinding(m, px, py, pz, valid, beta, skipFace, stkMem[threadIdx.x >> 6]);
+    const float wn = coopWinding(m, px, py, pz, valid, beta, skipFace);
     if (valid) out[q] = wn;
 }
 
-template <int D>
 __global__ __launch_bounds__(kBlock) void kSelfIntersectionsCoop(MeshDev m, int nLogical, float beta,
                                                                  uint8_t* __restrict__ out)
 {
-    __shared__ uint4 stkMem[kWaves][D];
     const int lb = logicalBlock(nLogical);
     if (lb >= nLogical) return;
     const int k = lb * kBlock + threadIdx.x;
@@ -301,7 +293,7 @@ __global__ __launch_bounds__(kBlock) void kSelfIntersectionsCoop(MeshDev m, int 
     const float qx = third * ((L.a[0] + L.b[0]) + L.c[0]);
     const float qy = third * ((L.a[1] + L.b[1]) + L.c[1]);
     const float qz = third * ((L.a[2] + L.b[2]) + L.c[2]);
-    const float wn = coopWinding(m, qx, qy, qz, valid, beta, L.face, stkMem[threadIdx.x >> 6]);
+    const float wn = coopWinding(m, qx, qy, qz, valid, beta, L.face);
     if (valid) out[L.face] = (wn < 0 || wn > 1) ? 1 : 0;
 }
 
@@ -364,7 +356,7 @@ __global__ __launch_bounds__(64, 4) void kBatch(const BatchItem* __restrict__ it
                 }
             }
             waveSync();
-            sdfStore(it.m, px, py, pz, valid, resSq, o, reinterpret_cast<uint4*>(laneMem), it.sdf, idx);
+            sdfStore(it.m, px, py, pz, valid, resSq, o, it.sdf, idx);
             waveSync();
         } else {
             const int64_t i = (lu - it.gridUnits) * 64 + lane;
@@ -713,7 +705,7 @@ hipError_t launchSdfGrid(const MeshDev& m, const int32_t dims[3], const Xf& xf, 
         const int blocks = persistentBlocks();
         hipLaunchKernelGGL(splitKernel, dim3(blocks), dim3(kBlock), 0, s, statLaunch(m, 1), dims[0], dims[1], zBegin, zEnd,
                            nbx, nby, nbz, xf, sc);
-        hipLaunchKernelGGL(kSdfSplitFinish<D>, dim3(blocks), dim3(kBlock), 0, s, statLaunch(m, 2), dims[0], dims[1],
+        hipLaunchKernelGGL(kSdfSplitFinish, dim3(blocks), dim3(kBlock), 0, s, statLaunch(m, 2), dims[0], dims[1],
                            zBegin, zEnd, nbx, nby, nbz, xf, o, sc, out);
         return hipGetLastError();
     });
@@ -726,15 +718,16 @@ hipError_t launchFwnGrid(const MeshDev& m, const int32_t dims[3], const Xf& xf, 
     const int64_t bricks = (int64_t)nbx * nby * nbz;
     if (bricks <= 0) return hipSuccess;
     const int nLogical = (int)((bricks + 3) / 4);
-    const bool coop = m.traversal == (int)Traversal::WaveCoop;
+    const dim3 grid(chunkedGrid(nLogical, kGridChunk));
+    if (m.traversal == (int)Traversal::WaveCoop) {
+        hipLaunchKernelGGL(kFwnGridCoop, grid, dim3(kBlock), 0, s, m, dims[0], dims[1], zBegin, zEnd, nbx, nby, nbz,
+                           nLogical, xf, beta, out);
+        return hipGetLastError();
+    }
     return dispatchDepth(stackD, [&](auto Dc) {
         constexpr int D = decltype(Dc)::value;
-        if (coop)
-            hipLaunchKernelGGL(kFwnGridCoop<D>, dim3(chunkedGrid(nLogical, kGridChunk)), dim3(kBlock), 0, s, m, dims[0],
-                               dims[1], zBegin, zEnd, nbx, nby, nbz, nLogical, xf, beta, out);
-        else
-            hipLaunchKernelGGL(kFwnGrid<D>, dim3(chunkedGrid(nLogical, kGridChunk)), dim3(kBlock), 0, s, m, dims[0],
-                               dims[1], zBegin, zEnd, nbx, nby, nbz, nLogical, xf, beta, out);
+        hipLaunchKernelGGL(kFwnGrid<D>, grid, dim3(kBlock), 0, s, m, dims[0], dims[1], zBegin, zEnd, nbx, nby, nbz,
+                           nLogical, xf, beta, out);
         return hipGetLastError();
     });
 }
@@ -744,15 +737,14 @@ hipError_t launchFwnPoints(const MeshDev& m, const float* pts, const uint32_t* p
 {
     if (n <= 0) return hipSuccess;
     const int nLogical = (int)((n + kBlock - 1) / kBlock);
-    const bool coop = m.traversal == (int)Traversal::WaveCoop;
+    const dim3 grid(paddedGrid(nLogical));
+    if (m.traversal == (int)Traversal::WaveCoop) {
+        hipLaunchKernelGGL(kFwnPointsCoop, grid, dim3(kBlock), 0, s, m, pts, perm, n, nLogical, beta, skipFace, out);
+        return hipGetLastError();
+    }
     return dispatchDepth(stackD, [&](auto Dc) {
         constexpr int D = decltype(Dc)::value;
-        if (coop)
-            hipLaunchKernelGGL(kFwnPointsCoop<D>, dim3(paddedGrid(nLogical)), dim3(kBlock), 0, s, m, pts,
-                               perm, n, nLogical, beta, skipFace, out);
-        else
-            hipLaunchKernelGGL(kFwnPoints<D>, dim3(paddedGrid(nLogical)), dim3(kBlock), 0, s, m, pts,
-                               perm, n, nLogical, beta, skipFace, out);
+        hipLaunchKernelGGL(kFwnPoints<D>, grid, dim3(kBlock), 0, s, m, pts, perm, n, nLogical, beta, skipFace, out);
         return hipGetLastError();
     });
 }
@@ -761,15 +753,14 @@ hipError_t launchSelfIntersections(const MeshDev& m, float beta, uint8_t* out, i
 {
     if (m.numFaces <= 0) return hipSuccess;
     const int nLogical = (m.numFaces + kBlock - 1) / kBlock;
-    const bool coop = m.traversal == (int)Traversal::WaveCoop;
+    const dim3 grid(paddedGrid(nLogical));
+    if (m.traversal == (int)Traversal::WaveCoop) {
+        hipLaunchKernelGGL(kSelfIntersectionsCoop, grid, dim3(kBlock), 0, s, m, nLogical, beta, out);
+        return hipGetLastError();
+    }
     return dispatchDepth(stackD, [&](auto Dc) {
         constexpr int D = decltype(Dc)::value;
-        if (coop)
-            hipLaunchKernelGGL(kSelfIntersectionsCoop<D>, dim3(paddedGrid(nLogical)), dim3(kBlock), 0, s, m,
-                               nLogical, beta, out);
-        else
-            hipLaunchKernelGGL(kSelfIntersections<D>, dim3(paddedGrid(nLogical)), dim3(kBlock), 0, s, m,
-                               nLogical, beta, out);
+        hipLaunchKernelGGL(kSelfIntersections<D>, grid, dim3(kBlock), 0, s, m, nLogical, beta, out);
         return hipGetLastError();
     });
 }

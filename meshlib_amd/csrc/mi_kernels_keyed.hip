@@ -286,16 +286,14 @@ __global__ __launch_bounds__(kBlock) void kSdfBandGrid(MeshDev m, BrickSource sr
         return;
     }
     // the winner's true squared distance, or the limit itself when nothing is below it
-    sdfStore(m, px, py, pz, valid, h.distSq, o, reinterpret_cast<uint4*>(&stkMem[w]), out, (size_t)idx);
+    sdfStore(m, px, py, pz, valid, h.distSq, o, out, (size_t)idx);
 }
 
 // Third launch of the split band grid: the handed-over bricks' distances (the winning leaf's test
 // recomputed), then NaN band, sign and store.
-template <int D>
 __global__ __launch_bounds__(kBlock) void kSdfBandFinish(MeshDev m, BrickSource src, DistOpts o, SplitScratch sc,
                                                          float* __restrict__ out)
 {
-    __shared__ uint4 stkMem[kWaves][D];
     const int lane = threadIdx.x & 63;
     const int w = threadIdx.x >> 6;
     const unsigned long long* best = reinterpret_cast<const unsigned long long*>(sc.best);
@@ -315,7 +313,7 @@ __global__ __launch_bounds__(kBlock) void kSdfBandFinish(MeshDev m, BrickSource 
             const int leaf = keyLeaf(m, (uint32_t)b, px, py, pz);
             if (leaf >= 0) resSq = leafDistSq(loadLeafLanes(m.tri, leaf), px, py, pz);
         }
-        sdfStore(m, px, py, pz, valid, resSq, o, stkMem[w], out, (size_t)idx);
+        sdfStore(m, px, py, pz, valid, resSq, o, out, (size_t)idx);
     }
 }
 
@@ -397,7 +395,7 @@ hipError_t launchSdfGridKeyed(const MeshDev& m, const int32_t dims[3], const Xf&
             const int blocks = persistentBlocks();
             hipLaunchKernelGGL((kKeyedSplit<D, BrickSource>), dim3(blocks), dim3(kBlock), 0, s, statLaunch(m, 1), src,
                                sc);
-            hipLaunchKernelGGL(kSdfBandFinish<D>, dim3(blocks), dim3(kBlock), 0, s, statLaunch(m, 2), src, o, sc, out);
+            hipLaunchKernelGGL(kSdfBandFinish, dim3(blocks), dim3(kBlock), 0, s, statLaunch(m, 2), src, o, sc, out);
         }
         return hipGetLastError();
     });

@@ -46,9 +46,7 @@ struct LaneTies {
 inline size_t laneSharedBytes(int depth, bool ties)
 {
     const size_t d = depth > 0 ? (size_t)depth : 1;
-    const size_t walk = sizeof(LaneShared) + (ties ? sizeof(LaneTies) : 0) + d * 64 * 6;
-    const size_t fwn = d * sizeof(uint4);     // the winding-number stack reuses the same memory
-    return walk > fwn ? walk : fwn;
+    return sizeof(LaneShared) + (ties ? sizeof(LaneTies) : 0) + d * 64 * 6;
 }
 
 // the wave's view of its LDS

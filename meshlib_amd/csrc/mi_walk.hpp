@@ -16,6 +16,8 @@
 // v_writelane_b32: `old` with lane `lane` replaced by the wave-uniform `value` (the compiler's
 // intrinsic, reached by name: clang has no builtin for it)
 __device__ int mi_writeLane(int value, int lane, int old) __asm("llvm.amdgcn.writelane");
+// each lane's bit of a wave mask as its predicate, without vector instructions
+__device__ bool mi_inverseBallot(uint64_t mask) __asm("llvm.amdgcn.inverse.ballot.i64");
 
 namespace mi {
 namespace {
@@ -239,15 +241,62 @@ __device__ __forceinline__ Leaf loadLeafLanes(const float4* __restrict__ tri, in
     return L;
 }
 
+// Square roots and quotients of the winding number.  A value between 2^-60 and 2^60 has no intermediate
+// result outside the normal range below, so the scaling and special cases of the general square root and
+// division fall away: Goldschmidt iteration from the raw reciprocal square root with Markstein's final
+// residual steps (fused multiply-adds), which round the square root and the quotient correctly except in
+// about one of 10^7 cases, where they are off by one unit.
+constexpr uint32_t kMidLow = 0x21800000u;                 // 2^-60
+constexpr uint32_t kMidSpan = 0x5d800000u - kMidLow;      // to 2^60
+__device__ __forceinline__ bool midRange(float x) { return __float_as_uint(x) - kMidLow < kMidSpan; }
+
+// sqrt(x) for midRange(x); half = 1 / (2 sqrt(x)) to a few units
+__device__ __forceinline__ float midSqrt(float x, float& half)
+{
+    const float y = __builtin_amdgcn_rsqf(x);
+    float g = x * y, h = 0.5f * y;
+    const float r = __builtin_fmaf(-g, h, 0.5f);
+    g = __builtin_fmaf(g, r, g);
+    h = __builtin_fmaf(h, r, h);
+    half = h;
+    return __builtin_fmaf(__builtin_fmaf(-g, g, x), h, g);
+}
+
+__device__ __forceinline__ float anySqrt(float x)
+{
+    float half;
+    return midRange(x) ? midSqrt(x, half) : sqrtf(x);
+}
+
+// num / (sqrt(dd) dd) for midRange(dd): a dipole's far field (Dipole::addIfGoodApprox, source/MRMesh/MRDipole.h:18-27)
+__device__ __forceinline__ float midDipole(float num, float dd)
+{
+    float h;
+    const float den = midSqrt(dd, h) * dd;
+    const float t = h + h;
+    float y = t * t * t;
+    y = __builtin_fmaf(__builtin_fmaf(-den, y, 1.f), y, y);
+    const float q = num * y;
+    return __builtin_fmaf(__builtin_fmaf(-den, q, num), y, q);
+}
+
+// the same for any dd; nothing at the dipole itself
+__device__ __forceinline__ float anyDipole(float num, float dd)
+{
+    if (midRange(dd)) return midDipole(num, dd);
+    const float dist = sqrtf(dd);
+    return dist > 0 ? num / (dist * dd) : 0.f;
+}
+
 // triangleSolidAngle (source/MRMesh/MRDipole.cpp:81-92), det as MRMatrix3.h:226-232
 __device__ __forceinline__ float solidAngle(float px, float py, float pz, const Leaf& L)
 {
     const float mxx = L.a[0] - px, mxy = L.a[1] - py, mxz = L.a[2] - pz;
     const float myx = L.b[0] - px, myy = L.b[1] - py, myz = L.b[2] - pz;
     const float mzx = L.c[0] - px, mzy = L.c[1] - py, mzz = L.c[2] - pz;
-    const float x = sqrtf(mxx * mxx + mxy * mxy + mxz * mxz);
-    const float y = sqrtf(myx * myx + myy * myy + myz * myz);
-    const float z = sqrtf(mzx * mzx + mzy * mzy + mzz * mzz);
+    const float x = anySqrt(mxx * mxx + mxy * mxy + mxz * mxz);
+    const float y = anySqrt(myx * myx + myy * myy + myz * myz);
+    const float z = anySqrt(mzx * mzx + mzy * mzy + mzz * mzz);
     const float dxy = mxx * myx + mxy * myy + mxz * myz;
     const float dyz = myx * mzx + myy * mzy + myz * mzz;
     const float dzx = mzx * mxx + mzy * mxy + mzz * mxz;
@@ -353,8 +402,7 @@ __device__ __forceinline__ float windingNumber(const MeshDev& m, float qx, float
         const float dpx = d0.x - qx, dpy = d0.y - qy, dpz = d0.z - qz;
         const float dd = dpx * dpx + dpy * dpy + dpz * dpz;
         if (!(dd <= betaSq * d0.w)) {
-            const float dist = sqrtf(dd);
-            if (dist > 0) res += (dpx * d1.x + dpy * d1.y + dpz * d1.z) / (dist * dd);
+            res += anyDipole(dpx * d1.x + dpy * d1.y + dpz * d1.z, dd);
         } else if (cur >= 0) {
             const float4 n3 = cload(m.dnode, 4 * cur + 3);
             stk[sp * kBlock].x = __float_as_int(n3.y);   // right child later
@@ -489,6 +537,9 @@ __device__ __forceinline__ float slotDistSq(const Quad& Q, int i, float px, floa
 
 // lanes with a < b (ordered compare) as a wave mask, straight from the compare
 __device__ __forceinline__ uint64_t ltMask(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, 4); }
+
+// lanes with a <= b (ordered compare)
+__device__ __forceinline__ uint64_t leMask(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, 5); }
 
 // A lower bound of the squared distance from (px, py, pz) to the triangle of leaf slot `slot`, at
 // most the leaf test's own result (the FP64 closest point, rounded).  The slot's record holds a unit
@@ -694,55 +745,70 @@ __device__ __forceinline__ float coopDistance(const MeshDev& m, float px, float 
     return best;
 }
 
+typedef float Dipole8 __attribute__((ext_vector_type(8)));     // (pos, rr), (dirArea, area): one scalar load
+
 // Winding number of each lane's point: the traversal order of calcFastWindingNumber is left-first
 // for every query, so a wave walks one left-first traversal and each entry carries the mask of
 // lanes that still descend there.  Every lane visits exactly its own node sequence in its own
 // order, so the sums are bit-identical to the per-lane traversal.  valid = false opts a lane out.
+//
+// The node, its masks and the stack (one entry per lane of five VGPRs) are wave-uniform and stay in scalar
+// registers, and children are found without memory: the left child has the first half of the leaves
+// (rounded down) and follows its parent in pre-order.  A visit is one 32-byte scalar load and, where a
+// lane takes the dipole, 37 vector operations (62 with a stack in LDS, masks in vector registers and the
+// general square root and division).  Bound by vector issue (82 % of it): 160^3 on 328 k triangles
+// 1.60 -> 1.22 ms; the same with both next records asked for a visit ahead took 1.97 ms (three scalar loads
+// a visit), with vector loads 1.43 ms, with 64-byte records of both children 1.29 ms.
 __device__ __forceinline__ float coopWinding(const MeshDev& m, float qx, float qy, float qz, bool valid,
-                                             float beta, int32_t skipFace, uint4* stk)
+                                             float beta, int32_t skipFace)
 {
     if (m.numFaces <= 0) return 0;
     const float betaSq = beta * beta;
-    const int lane = threadIdx.x & 63;
     float res = 0;
-    uint64_t curMask = waveBallot(valid);
-    int cur = m.rootRef;
-    int sp = 0;
+    uint64_t mask = waveBallot(valid);
+    int node = 0, first = 0, num = uniform(m.numFaces), sp = 0;     // node: internal nodes only (num > 1)
+    int sNode = 0, sFirst = 0, sNum = 0, sLo = 0, sHi = 0;          // lane e: stack entry e
     uint32_t nVisit = 0, nDesc = 0, nLeaf = 0;     // measurement counts
-    while (curMask) {
-        const bool mine = (curMask >> lane) & 1;
-        cur = uniform(cur);
+    while (mask) {
         ++nVisit;
-        float4 d0, d1;
-        if (cur >= 0) { d0 = cload(m.dint, 2 * cur); d1 = cload(m.dint, 2 * cur + 1); }
-        else { d0 = cload(m.dleaf, 2 * (~cur)); d1 = cload(m.dleaf, 2 * (~cur) + 1); }
-        const float dpx = d0.x - qx, dpy = d0.y - qy, dpz = d0.z - qz;
+        const bool leaf = num == 1;
+        const Dipole8 rec = ((const __attribute__((address_space(4))) Dipole8*)(leaf ? m.dleaf : m.dint))[leaf ? first : node];
+        const float dpx = rec[0] - qx, dpy = rec[1] - qy, dpz = rec[2] - qz;
         const float dd = dpx * dpx + dpy * dpy + dpz * dpz;
-        const bool approx = !(dd <= betaSq * d0.w);
-        if (mine && approx) {
-            const float dist = sqrtf(dd);
-            if (dist > 0) res += (dpx * d1.x + dpy * d1.y + dpz * d1.z) / (dist * dd);
+        const uint64_t near = mask & leMask(dd, betaSq * rec[3]);
+        const uint64_t far = mask & ~near;
+        if (far) {
+            const float dot = dpx * rec[4] + dpy * rec[5] + dpz * rec[6];
+            const uint64_t mid = far & __builtin_amdgcn_uicmp(__float_as_uint(dd) - kMidLow, kMidSpan, 36);
+            if (mi_inverseBallot(mid)) res += midDipole(dot, dd);
+            if (far != mid && mi_inverseBallot(far & ~mid)) res += anyDipole(dot, dd);
         }
-        const uint64_t desc = waveBallot(mine && !approx);
-        if (desc) {
-            if (cur >= 0) {
-                const float4 n3 = cload(m.dnode, 4 * cur + 3);
-                stk[sp] = make_uint4(__float_as_uint(n3.y), (uint32_t)desc, (uint32_t)(desc >> 32), 0u);
+        if (near) {
+            if (!leaf) {
+                const int h = num >> 1;
+                sNode = mi_writeLane(node + h, sp, sNode);
+                sFirst = mi_writeLane(first + h, sp, sFirst);
+                sNum = mi_writeLane(num - h, sp, sNum);
+                sLo = mi_writeLane((int)(uint32_t)near, sp, sLo);
+                sHi = mi_writeLane((int)(uint32_t)(near >> 32), sp, sHi);
                 ++sp;
                 ++nDesc;
-                cur = __float_as_int(n3.x);
-                curMask = desc;
+                node += 1;
+                num = h;
+                mask = near;
                 continue;
             }
             ++nLeaf;
-            const Leaf L = loadLeaf(m.tri, ~cur);
-            if (mine && !approx && L.face != skipFace) res += solidAngle(qx, qy, qz, L);
+            const Leaf L = loadLeaf(m.tri, first);
+            if (L.face != skipFace && mi_inverseBallot(near)) res += solidAngle(qx, qy, qz, L);
         }
         if (sp == 0) break;
         --sp;
-        const uint4 e = stk[sp];
-        cur = (int)e.x;
-        curMask = (uint64_t)e.y | ((uint64_t)e.z << 32);
+        node = __builtin_amdgcn_readlane(sNode, sp);
+        first = __builtin_amdgcn_readlane(sFirst, sp);
+        num = __builtin_amdgcn_readlane(sNum, sp);
+        mask = (uint64_t)(uint32_t)__builtin_amdgcn_readlane(sLo, sp) |
+               ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(sHi, sp) << 32);
     }
     if (m.stats) {
         statAdd(m, kStatWalks, 1);
@@ -823,9 +889,6 @@ __device__ __forceinline__ void flushProjLeaves(const MeshDev& m, float px, floa
     bestD = __uint_as_float((uint32_t)(b >> 32));
     bestKey = (uint32_t)b;
 }
-
-// lanes with a <= b (ordered compare)
-__device__ __forceinline__ uint64_t leMask(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, 5); }
 
 // the `<=` pruning limit of a projection walk: its best, with +inf lowered to FLT_MAX so that an
 // empty quad slot (+inf box) never passes; every finite box distance still does
@@ -1116,10 +1179,10 @@ __device__ __forceinline__ void projStore(const MeshDev& m, int leaf, float lim,
 // shared tail of the signed-distance kernels: NaN band, winding-number sign, store
 // (FastWindingNumber::calcWithDistances, source/MRMesh/MRFastWindingNumber.cpp:69-76)
 __device__ __forceinline__ void sdfStore(const MeshDev& m, float px, float py, float pz, bool valid, float resSq,
-                                         const DistOpts& o, uint4* stk, float* out, size_t idx)
+                                         const DistOpts& o, float* out, size_t idx)
 {
     const bool nan = o.nullOutsideMinMax && (resSq < o.minDistSq || resSq >= o.maxDistSq);
-    const float wn = coopWinding(m, px, py, pz, valid && !nan, o.beta, -1, stk);
+    const float wn = coopWinding(m, px, py, pz, valid && !nan, o.beta, -1);
     if (!valid) return;
     if (nan) {
         out[idx] = __int_as_float(0x7fc00000);
