@@ -457,6 +457,7 @@ int finishArena(mi_mesh* m, const ArenaLayout& L)
     DevBuf ranges;
     MI_HIP(ranges.alloc(mi::cylinderScratchBytes(m->nf)));
     m->dev.numFaces = m->nf;
+    m->dev.depth = m->depth;
     MI_HIP(mi::buildCylinders(m->dev, reinterpret_cast<float4*>(base + L.total() - L.cyl), ranges.p, m->stream));
     char* cutBase = base + L.dnode + L.tri + L.dint + L.dleaf + L.dquad;
     mi::CutEntry* cut = reinterpret_cast<mi::CutEntry*>(cutBase);
@@ -587,10 +588,8 @@ int createDeviceBuilt(mi_mesh* m, const float* verts, const int32_t* tris, const
     o.dint = reinterpret_cast<float4*>(base + L.dnode + L.tri);
     o.dleaf = reinterpret_cast<float4*>(base + L.dnode + L.tri + L.dint);
     mi::DeviceTreeInfo info;
-    const hipError_t e = mi::buildDeviceTree(dv.as<float>(), m->nv, dt.as<int32_t>(), m->nf, scratch.p, scratch.bytes,
-                                             o, info, m->stream, ids.as<int32_t>());
-    if (e == hipErrorInvalidValue) return fail(MI_E_INVALID, "triangle vertex index out of range");
-    MI_HIP(e);
+    MI_HIP(mi::buildDeviceTree(dv.as<float>(), dt.as<int32_t>(), m->nf, scratch.p, scratch.bytes, o, info, m->stream,
+                               ids.as<int32_t>()));
     m->depth = info.depth;
     m->stackD = mi::stackDepthFor(m->depth);
     if (m->stackD == 0) return fail(MI_E_LIMIT, "tree deeper than 32 levels");

@@ -3,31 +3,36 @@
 // Tree (source/MRMesh/MRAABBTreeMaker.hpp:50-165): every internal node splits its leaves at the
 // median (left gets num/2) under a total order -- key (min+max) along the node box's dims sorted by
 // extent, largest first, ties to the next dim, last to the face id.  Because the order is total,
-// the left set of each node is unique; the build below finds it for all nodes of one tree level at
-// once, with no per-node selection:
-//   * the leaves of each node stay contiguous, nodes of a level in pre-order (which is also their
-//     array order, since left subtrees precede right subtrees in both);
-//   * per level: segmented box reduction (wave-segmented shuffles + one atomic per run), per-leaf
-//     keys from its node's dims, then a stable LSD radix chain face -> k2 -> k1 -> (node, k0), which
-//     sorts every node's leaves by the full total order without moving them out of their node;
-//   * the first num/2 leaves of a node form its left child; children are numbered root+1 and
-//     root+2*half as in the reference's pre-order layout.
+// the left set of each node is unique, however it is found; and because every node gives num/2 of its
+// leaves to its left child, the shape of the tree, all node numbers (children root+1 and root+2*half)
+// and all leaf ranges follow from the number of faces alone (nodeAt) -- no level waits for the host.
+//   * nodes of more than kSub leaves are split level by level, several blocks a node: box reduction,
+//     three rounds of radix selection on the first key (histograms of 11, 11 and 10 bits), a block per
+//     node that settles equal first keys by the other keys, partition of the leaves into the two halves;
+//   * nodes of at most kSub leaves are finished by one block each in LDS, all their levels in one launch
+//     (a bitonic sort of each node's leaves per level), dipoles included.
+// Four library radix sorts per level were 1,800 launches for a mesh of 328 k faces, bound by the launches; now 90
+// launches, and creating that mesh from host arrays went from 13.0 to 2.1 ms (1.0 ms of it kernels).
 // Leaf boxes, dipoles (source/MRMesh/MRDipole.cpp:23-71) and the flattened arrays repeat the host
 // builder's float expressions in the same order (the library is compiled with -ffp-contract=off and
 // correctly rounded division and square root), so every record equals the host build bit-for-bit.
 #include "mi_tree_gpu.hpp"
 
-#include <hipcub/hipcub.hpp>
-
+#include <algorithm>
 #include <cfloat>
-#include <vector>
 
 namespace mi {
 namespace {
 
 constexpr int kB = 256;
+// leaves of a subtree built in LDS, two a thread: three blocks of 48 KB a CU (2048 leaves in one 96-KB block a CU:
+// 1.3 M faces 1.08 ms against 0.64 ms, one level fewer above)
+constexpr int kSub = 1024;
+constexpr int kSubThreads = 512;
+constexpr int kChunk = 4096;        // leaves of a block of the level kernels
+constexpr int kBins = 2048;         // histogram of one selection round
 
-// leaf record while building: {min.xyz, max.x} {max.y, max.z, face, node}
+// leaf record while building: {min.xyz, max.x} {max.y, max.z, face, 0}
 struct Elem { float4 a, b; };
 
 __device__ __forceinline__ uint32_t ordU(float x)
@@ -58,97 +63,39 @@ __device__ __forceinline__ float nextUp(float x)
     return __uint_as_float(x > 0.0f ? b + 1u : b - 1u);
 }
 
+// a node: its pre-order number, the first of its leaves in left-to-right order and their number
+struct Node { int32_t v, first, num; };
+
+// node i (from the left) of a level all of whose parents have two leaves or more
+__device__ __forceinline__ Node child(const Node& p, bool right)
+{
+    const int32_t h = p.num >> 1;
+    return right ? Node{ p.v + 2 * h, p.first + h, p.num - h } : Node{ p.v + 1, p.first, h };
+}
+__device__ __forceinline__ Node nodeAt(int32_t n, int level, uint32_t i)
+{
+    Node d{ 0, 0, n };
+    for (int l = level - 1; l >= 0; --l) d = child(d, (i >> l) & 1u);
+    return d;
+}
+
 // computeFaceBox + insignificantlyExpanded (source/MRMesh/MRAABBTree.cpp:15-29, MRBox.h:260-270)
-__global__ void kLeafBoxes(const float* __restrict__ verts, int32_t nv, const int32_t* __restrict__ tris,
-                           int32_t n, Elem* __restrict__ el, uint32_t* __restrict__ err)
+__global__ void kLeafBoxes(const float* __restrict__ verts, const int32_t* __restrict__ tris, int32_t n,
+                           Elem* __restrict__ el)
 {
     const int32_t f = blockIdx.x * kB + threadIdx.x;
     if (f >= n) return;
     float mn[3] = { FLT_MAX, FLT_MAX, FLT_MAX }, mx[3] = { -FLT_MAX, -FLT_MAX, -FLT_MAX };
-    bool ok = true;
     for (int k = 0; k < 3; ++k) {
-        const int32_t vi = tris[3 * (int64_t)f + k];
-        if (vi < 0 || vi >= nv) { ok = false; continue; }
-        const float* p = verts + 3 * (int64_t)vi;
+        const float* p = verts + 3 * (int64_t)tris[3 * (int64_t)f + k];
         for (int i = 0; i < 3; ++i) {
             if (p[i] < mn[i]) mn[i] = p[i];
             if (p[i] > mx[i]) mx[i] = p[i];
         }
     }
-    if (!ok) {
-        atomicOr(err, 1u);
-        for (int i = 0; i < 3; ++i) { mn[i] = 0; mx[i] = 0; }
-    }
     for (int i = 0; i < 3; ++i) { mn[i] = nextDown(mn[i]); mx[i] = nextUp(mx[i]); }
     el[f].a = make_float4(mn[0], mn[1], mn[2], mx[0]);
-    el[f].b = make_float4(mx[1], mx[2], __int_as_float(f), __int_as_float(0));
-}
-
-__global__ void kInit(int32_t n, int32_t* segFirst, int32_t* segNum, int32_t* list, uint32_t* iota)
-{
-    const int32_t p = blockIdx.x * kB + threadIdx.x;
-    if (p == 0) { segFirst[0] = 0; segNum[0] = n; list[0] = 0; }
-    if (p < n) iota[p] = (uint32_t)p;
-}
-
-__global__ void kSegInit(const int32_t* __restrict__ list, int32_t count, const int32_t* __restrict__ segNum,
-                         uint32_t* __restrict__ acc)
-{
-    const int32_t i = blockIdx.x * kB + threadIdx.x;
-    if (i >= count) return;
-    const int32_t v = list[i];
-    if (segNum[v] < 2) return;
-    uint32_t* a = acc + 6 * (int64_t)v;
-    a[0] = a[1] = a[2] = 0xffffffffu;      // min accumulators (ordered encoding)
-    a[3] = a[4] = a[5] = 0u;               // max accumulators
-}
-
-// node box = union of its leaves' boxes: segmented min/max within the wave (a node's leaves are
-// contiguous), then one atomic per node-run per wave
-__global__ void kSegBox(const Elem* __restrict__ el, int32_t n, const int32_t* __restrict__ segNum,
-                        uint32_t* __restrict__ acc)
-{
-    const int32_t p = blockIdx.x * kB + threadIdx.x;
-    int v = -1;
-    float b[6] = { FLT_MAX, FLT_MAX, FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX };
-    if (p < n) {
-        const Elem e = el[p];
-        const int vv = __float_as_int(e.b.w);
-        if (segNum[vv] >= 2) {
-            v = vv;
-            b[0] = e.a.x; b[1] = e.a.y; b[2] = e.a.z; b[3] = e.a.w; b[4] = e.b.x; b[5] = e.b.y;
-        }
-    }
-    const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int ov = __shfl_up(v, d);
-        float o[6];
-#pragma unroll
-        for (int i = 0; i < 6; ++i) o[i] = __shfl_up(b[i], d);
-        if (lane >= d && ov == v) {
-#pragma unroll
-            for (int i = 0; i < 3; ++i) {
-                b[i] = fminf(b[i], o[i]);
-                b[i + 3] = fmaxf(b[i + 3], o[i + 3]);
-            }
-        }
-    }
-    const int nv = __shfl_down(v, 1);
-    if (v >= 0 && (lane == 63 || nv != v)) {
-        uint32_t* a = acc + 6 * (int64_t)v;
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            atomicMin(a + i, ordU(b[i]));
-            atomicMax(a + 3 + i, ordU(b[i + 3]));
-        }
-    }
-}
-
-__device__ __forceinline__ void nodeBox(const uint32_t* acc, int v, float mn[3], float mx[3])
-{
-    const uint32_t* a = acc + 6 * (int64_t)v;
-    for (int i = 0; i < 3; ++i) { mn[i] = unordU(a[i]); mx[i] = unordU(a[3 + i]); }
+    el[f].b = make_float4(mx[1], mx[2], __int_as_float(f), 0.f);
 }
 
 // dims by (extent, index), smallest first -- findSortedBoxDims (source/MRMesh/MRBox.h:378-396)
@@ -163,50 +110,297 @@ __device__ __forceinline__ void sortedDims(const float mn[3], const float mx[3],
     if (lessP(sd[1], sd[0])) { t = sd[0]; sd[0] = sd[1]; sd[1] = t; }
 }
 
-__global__ void kKeys(const Elem* __restrict__ el, int32_t n, const int32_t* __restrict__ segNum,
-                      const uint32_t* __restrict__ acc, uint32_t* __restrict__ faceKey, uint32_t* __restrict__ k1,
-                      uint32_t* __restrict__ k2, uint64_t* __restrict__ k64)
+// the four keys of a leaf in its node's order, k = 0 (first) to 3 (the face); sd = sortedDims of the node
+__device__ __forceinline__ uint32_t leafKey(const Elem& e, const int sd[3], int k)
 {
-    const int32_t p = blockIdx.x * kB + threadIdx.x;
-    if (p >= n) return;
-    const Elem e = el[p];
-    const int v = __float_as_int(e.b.w);
-    faceKey[p] = (uint32_t)__float_as_int(e.b.z);
-    uint32_t a0 = 0, a1 = 0, a2 = 0;
-    if (segNum[v] >= 2) {
-        float mn[3], mx[3];
-        nodeBox(acc, v, mn, mx);
+    if (k == 3) return (uint32_t)__float_as_int(e.b.z);
+    const float c[3] = { e.a.x + e.a.w, e.a.y + e.b.x, e.a.z + e.b.y };
+    const int d = sd[2 - k];
+    return keyU(d == 0 ? c[0] : d == 1 ? c[1] : c[2]);
+}
+
+// ---------------------------------------------------------------- levels of large nodes
+//
+// Per node of the level: its box, the histograms of the three rounds, the pivot (the leaf of rank num/2: the
+// leaves before it in the order go left) and the write positions of both halves.
+struct LevelNode {
+    uint32_t box[6];        // ordered encoding: min xyz, max xyz
+    uint32_t pivot[4];      // its keys; those behind the first that no other leaf shares are 0
+    uint32_t left, right;   // leaves written so far
+    uint32_t listed;        // leaves in `list`
+};
+
+struct Level {
+    int32_t n;              // faces
+    int32_t level;
+    int32_t blocksPerNode;
+    Elem* src;
+    Elem* dst;
+    uint32_t* k0;           // first key of the leaf at each position
+    uint32_t* list;         // positions of the leaves left after two rounds, per node from its first
+    LevelNode* nodes;
+    uint32_t* hist;         // 3 * kBins per node
+};
+
+// this block's node and its chunk of leaves
+__device__ __forceinline__ Node blockNode(const Level& L, uint32_t& i, int32_t& begin, int32_t& end)
+{
+    i = blockIdx.x / (uint32_t)L.blocksPerNode;
+    const Node d = nodeAt(L.n, L.level, i);
+    begin = d.first + (int32_t)(blockIdx.x % (uint32_t)L.blocksPerNode) * kChunk;
+    end = min(begin + kChunk, d.first + d.num);
+    return d;
+}
+
+__device__ __forceinline__ void nodeDims(const LevelNode& nd, int sd[3])
+{
+    float mn[3], mx[3];
+    for (int k = 0; k < 3; ++k) { mn[k] = unordU(nd.box[k]); mx[k] = unordU(nd.box[3 + k]); }
+    sortedDims(mn, mx, sd);
+}
+
+__global__ void kLevelInit(Level L, int32_t count)
+{
+    const int64_t t = (int64_t)blockIdx.x * kB + threadIdx.x;
+    if (t < (int64_t)count * 3 * kBins) L.hist[t] = 0u;
+    if (t < count) {
+        LevelNode& nd = L.nodes[t];
+        for (int k = 0; k < 3; ++k) { nd.box[k] = 0xffffffffu; nd.box[3 + k] = 0u; }
+        nd.left = nd.right = nd.listed = 0u;
+    }
+}
+
+__global__ __launch_bounds__(kB) void kLevelBox(Level L)
+{
+    uint32_t i;
+    int32_t begin, end;
+    blockNode(L, i, begin, end);
+    float b[6] = { FLT_MAX, FLT_MAX, FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX };
+    bool any = false;
+    for (int32_t p = begin + (int32_t)threadIdx.x; p < end; p += kB) {
+        const Elem e = L.src[p];
+        const float o[6] = { e.a.x, e.a.y, e.a.z, e.a.w, e.b.x, e.b.y };
+        for (int k = 0; k < 3; ++k) { b[k] = fminf(b[k], o[k]); b[k + 3] = fmaxf(b[k + 3], o[k + 3]); }
+        any = true;
+    }
+    for (int d = 32; d; d >>= 1)
+        for (int k = 0; k < 3; ++k) {
+            b[k] = fminf(b[k], __shfl_xor(b[k], d));
+            b[k + 3] = fmaxf(b[k + 3], __shfl_xor(b[k + 3], d));
+        }
+    if ((threadIdx.x & 63) == 0 && any)
+        for (int k = 0; k < 3; ++k) {
+            atomicMin(&L.nodes[i].box[k], ordU(b[k]));
+            atomicMax(&L.nodes[i].box[3 + k], ordU(b[k + 3]));
+        }
+}
+
+// the bin of a histogram that holds rank `rank` (block-wide): rank becomes the rank inside the bin, count the
+// bin's size
+__device__ __forceinline__ uint32_t pickBin(const uint32_t* hist, uint32_t& rank, uint32_t& count)
+{
+    __shared__ uint32_t sums[kB];
+    __shared__ uint32_t found[3];
+    constexpr int per = kBins / kB;
+    uint32_t h[per], own = 0;
+    for (int k = 0; k < per; ++k) { h[k] = hist[per * threadIdx.x + k]; own += h[k]; }
+    __syncthreads();
+    sums[threadIdx.x] = own;
+    __syncthreads();
+    for (int d = 1; d < kB; d <<= 1) {
+        const uint32_t o = (int)threadIdx.x >= d ? sums[threadIdx.x - d] : 0u;
+        __syncthreads();
+        sums[threadIdx.x] += o;
+        __syncthreads();
+    }
+    uint32_t before = sums[threadIdx.x] - own;
+    if (rank >= before && rank < before + own) {
+        int k = 0;
+        while (rank >= before + h[k]) { before += h[k]; ++k; }
+        found[0] = (uint32_t)(per * threadIdx.x + k);
+        found[1] = rank - before;
+        found[2] = h[k];
+    }
+    __syncthreads();
+    const uint32_t bin = found[0];
+    rank = found[1];
+    count = found[2];
+    __syncthreads();
+    return bin;
+}
+
+// the bits of a 32-bit key in selection round r
+__device__ __forceinline__ uint32_t roundBits(uint32_t key, int r)
+{
+    return r == 0 ? key >> 21 : r == 1 ? (key >> 10) & 2047u : key & 1023u;
+}
+
+// Selection round ROUND on the first key: the histogram of the leaves whose bits of the earlier rounds are
+// the picked ones.  Round 0 also stores the keys, the last round lists its leaves.
+template <int ROUND>
+__global__ __launch_bounds__(kB) void kLevelHist(Level L)
+{
+    __shared__ uint32_t h[kBins];
+    __shared__ uint32_t mine[ROUND == 2 ? kChunk : 1];
+    __shared__ uint32_t count2, base2;
+    uint32_t i;
+    int32_t begin, end;
+    const Node d = blockNode(L, i, begin, end);
+    for (int k = threadIdx.x; k < kBins; k += kB) h[k] = 0u;
+    if (threadIdx.x == 0) count2 = 0u;
+    uint32_t* const hist = L.hist + (size_t)i * 3 * kBins;
+    uint32_t prefix = 0, rank = (uint32_t)(d.num >> 1), count;
+    if (ROUND >= 1) prefix = pickBin(hist, rank, count);
+    if (ROUND >= 2) prefix = (prefix << 11) | pickBin(hist + kBins, rank, count);
+    int sd[3];
+    if (ROUND == 0) nodeDims(L.nodes[i], sd);
+    __syncthreads();
+    for (int32_t p = begin + (int32_t)threadIdx.x; p < end; p += kB) {
+        uint32_t key;
+        if (ROUND == 0) {
+            key = leafKey(L.src[p], sd, 0);
+            L.k0[p] = key;
+        } else {
+            key = L.k0[p];
+            if ((ROUND == 1 ? key >> 21 : key >> 10) != prefix) continue;
+        }
+        atomicAdd(&h[roundBits(key, ROUND)], 1u);
+        if (ROUND == 2) mine[atomicAdd(&count2, 1u)] = (uint32_t)p;
+    }
+    __syncthreads();
+    for (int k = threadIdx.x; k < kBins; k += kB)
+        if (h[k]) atomicAdd(&hist[ROUND * kBins + k], h[k]);
+    if (ROUND == 2) {
+        if (threadIdx.x == 0) base2 = atomicAdd(&L.nodes[i].listed, count2);
+        __syncthreads();
+        for (uint32_t k = threadIdx.x; k < count2; k += kB) L.list[(uint32_t)d.first + base2 + k] = mine[k];
+    }
+}
+
+// One block per node: the pivot's first key, and where several leaves share it the other keys, by the same
+// selection over those leaves.
+__global__ __launch_bounds__(kB) void kLevelPivot(Level L)
+{
+    __shared__ uint32_t h[kBins];
+    __shared__ uint32_t shared;
+    const uint32_t i = blockIdx.x;
+    const Node d = nodeAt(L.n, L.level, i);
+    const uint32_t* const hist = L.hist + (size_t)i * 3 * kBins;
+    uint32_t rank = (uint32_t)(d.num >> 1), count;
+    uint32_t k0 = pickBin(hist, rank, count);
+    k0 = (k0 << 11) | pickBin(hist + kBins, rank, count);
+    k0 = (k0 << 10) | pickBin(hist + 2 * kBins, rank, count);
+    uint32_t piv[4] = { k0, 0u, 0u, 0u };
+    if (count > 1) {
         int sd[3];
-        sortedDims(mn, mx, sd);
-        const float c[3] = { e.a.x + e.a.w, e.a.y + e.b.x, e.a.z + e.b.y };
-        a0 = keyU(c[sd[2]]);
-        a1 = keyU(c[sd[1]]);
-        a2 = keyU(c[sd[0]]);
+        nodeDims(L.nodes[i], sd);
+        const int32_t ties = (int32_t)L.nodes[i].listed;
+        for (int w = 1; w < 4 && count > 1; ++w) {
+            uint32_t prefix = 0;
+            for (int r = 0; r < 3 && count > 1; ++r) {
+                __syncthreads();
+                for (int k = threadIdx.x; k < kBins; k += kB) h[k] = 0u;
+                __syncthreads();
+                for (int32_t q = (int32_t)threadIdx.x; q < ties; q += kB) {
+                    const uint32_t p = L.list[d.first + q];
+                    bool in = L.k0[p] == k0;
+                    if (!in) continue;
+                    const Elem e = L.src[p];
+                    for (int u = 1; u < w; ++u) in = in && leafKey(e, sd, u) == piv[u];
+                    const uint32_t key = leafKey(e, sd, w);
+                    if (r == 1) in = in && (key >> 21) == prefix;
+                    if (r == 2) in = in && (key >> 10) == prefix;
+                    if (in) atomicAdd(&h[roundBits(key, r)], 1u);
+                }
+                __syncthreads();
+                prefix = (prefix << (r == 2 ? 10 : 11)) | pickBin(h, rank, count);
+                // a bin of one leaf is the pivot: its remaining bits are its own
+                if (count == 1 && r < 2) {
+                    __syncthreads();
+                    for (int32_t q = (int32_t)threadIdx.x; q < ties; q += kB) {
+                        const uint32_t p = L.list[d.first + q];
+                        bool in = L.k0[p] == k0;
+                        if (!in) continue;
+                        const Elem e = L.src[p];
+                        for (int u = 1; u < w; ++u) in = in && leafKey(e, sd, u) == piv[u];
+                        const uint32_t key = leafKey(e, sd, w);
+                        if (in && (key >> (r == 0 ? 21 : 10)) == prefix) shared = key;
+                    }
+                    __syncthreads();
+                    prefix = shared;
+                }
+            }
+            piv[w] = prefix;
+        }
     }
-    k1[p] = a1;
-    k2[p] = a2;
-    k64[p] = ((uint64_t)(uint32_t)v << 32) | a0;
-}
-
-template <typename T>
-__global__ void kGather(const T* __restrict__ src, const uint32_t* __restrict__ perm, int32_t n, T* __restrict__ dst)
-{
-    const int32_t p = blockIdx.x * kB + threadIdx.x;
-    if (p < n) dst[p] = src[perm[p]];
-}
-
-__global__ void kGatherElems(const Elem* __restrict__ src, const uint32_t* __restrict__ perm, int32_t n,
-                             Elem* __restrict__ dst)
-{
-    const int32_t p = blockIdx.x * kB + threadIdx.x;
-    if (p < n) {
-        const Elem e = src[perm[p]];
-        dst[p].a = e.a;
-        dst[p].b = e.b;
+    if (threadIdx.x < 4) {
+        const int t = threadIdx.x;
+        L.nodes[i].pivot[t] = t == 0 ? piv[0] : t == 1 ? piv[1] : t == 2 ? piv[2] : piv[3];
     }
 }
 
-__global__ void kZero(uint32_t* p) { if (threadIdx.x == 0 && blockIdx.x == 0) *p = 0; }
+// writes the level's nodes and moves every leaf to its half of the node's range (in any order)
+__global__ __launch_bounds__(kB) void kLevelPartition(Level L, TreeNode* __restrict__ tree, int32_t* __restrict__ firstOf)
+{
+    __shared__ uint32_t sums[kB];
+    __shared__ uint32_t base[2];
+    uint32_t i;
+    int32_t begin, end;
+    const Node d = blockNode(L, i, begin, end);
+    LevelNode& nd = L.nodes[i];
+    const int32_t h = d.num >> 1;
+    if (begin == d.first && threadIdx.x == 0) {
+        TreeNode t;
+        for (int k = 0; k < 3; ++k) { t.box.min[k] = unordU(nd.box[k]); t.box.max[k] = unordU(nd.box[3 + k]); }
+        t.l = d.v + 1;
+        t.r = d.v + 2 * h;
+        tree[d.v] = t;
+        firstOf[d.v] = d.first;
+    }
+    int sd[3];
+    nodeDims(nd, sd);
+    const uint32_t piv[4] = { nd.pivot[0], nd.pivot[1], nd.pivot[2], nd.pivot[3] };
+    constexpr int per = kChunk / kB;
+    uint32_t goLeft = 0, mine = 0;
+    for (int k = 0; k < per; ++k) {
+        const int32_t p = begin + k * kB + (int32_t)threadIdx.x;
+        if (p >= end) break;
+        ++mine;
+        const uint32_t key = L.k0[p];
+        bool left = key < piv[0];
+        if (key == piv[0]) {
+            const Elem e = L.src[p];
+            for (int w = 1; w < 4; ++w) {
+                const uint32_t kw = leafKey(e, sd, w);
+                if (kw != piv[w]) { left = kw < piv[w]; break; }
+            }
+        }
+        if (left) goLeft |= 1u << k;
+    }
+    const uint32_t nl = (uint32_t)__popc(goLeft);
+    // both counts in one scan: 16 bits each (at most kChunk)
+    const uint32_t own = nl | ((mine - nl) << 16);
+    sums[threadIdx.x] = own;
+    __syncthreads();
+    for (int s = 1; s < kB; s <<= 1) {
+        const uint32_t o = (int)threadIdx.x >= s ? sums[threadIdx.x - s] : 0u;
+        __syncthreads();
+        sums[threadIdx.x] += o;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        base[0] = atomicAdd(&nd.left, sums[kB - 1] & 0xffffu);
+        base[1] = atomicAdd(&nd.right, sums[kB - 1] >> 16);
+    }
+    __syncthreads();
+    const uint32_t before = sums[threadIdx.x] - own;
+    int32_t l = d.first + (int32_t)(base[0] + (before & 0xffffu));
+    int32_t r = d.first + h + (int32_t)(base[1] + (before >> 16));
+    for (int k = 0; k < (int)mine; ++k) {
+        const Elem e = L.src[begin + k * kB + (int32_t)threadIdx.x];
+        L.dst[(goLeft >> k) & 1u ? l++ : r++] = e;
+    }
+}
 
 // leaf dipole: dirArea = cross(b-a, c-a)/2, area = |dirArea|, pos = area * centroid
 // (source/MRMesh/MRDipole.cpp:28-45, triCenter / leftDirDblArea in MRMeshMath.cpp:119-149)
@@ -229,79 +423,198 @@ __device__ __forceinline__ Dipole leafDipole(const float* __restrict__ verts, co
     return d;
 }
 
-// writes the nodes of one level; a leaf takes its element's box and face, an internal node its
-// reduced box and children root+1 / root+2*half (MRAABBTreeMaker.hpp:88-89), whose leaf ranges are
-// recorded and appended to the next level's list
-__global__ void kSplit(const int32_t* __restrict__ list, int32_t count, int32_t* __restrict__ segFirst,
-                       int32_t* __restrict__ segNum, const Elem* __restrict__ el, const uint32_t* __restrict__ acc,
-                       const float* __restrict__ verts, const int32_t* __restrict__ tris, TreeNode* __restrict__ nodes,
-                       Dipole* __restrict__ dip, int32_t* __restrict__ nextList, uint32_t* __restrict__ nextCount)
+// sum of the children's dipoles (source/MRMesh/MRDipole.cpp:47-60)
+__device__ __forceinline__ void addDipoles(Dipole* __restrict__ dip, const Node& d)
 {
-    const int32_t i = blockIdx.x * kB + threadIdx.x;
-    if (i >= count) return;
-    const int32_t v = list[i];
-    const int32_t f = segFirst[v], s = segNum[v];
-    TreeNode nd;
-    if (s == 1) {
-        const Elem e = el[f];
-        nd.box.min[0] = e.a.x; nd.box.min[1] = e.a.y; nd.box.min[2] = e.a.z;
-        nd.box.max[0] = e.a.w; nd.box.max[1] = e.b.x; nd.box.max[2] = e.b.y;
-        nd.l = __float_as_int(e.b.z);
-        nd.r = -1;
-        dip[v] = leafDipole(verts, tris, nd.l);
-    } else {
-        const int32_t h = s / 2;
-        nodeBox(acc, v, nd.box.min, nd.box.max);
-        nd.l = v + 1;
-        nd.r = v + 2 * h;
-        segFirst[v + 1] = f;
-        segNum[v + 1] = h;
-        segFirst[v + 2 * h] = f + h;
-        segNum[v + 2 * h] = s - h;
-        const uint32_t slot = atomicAdd(nextCount, 2u);
-        nextList[slot] = v + 1;
-        nextList[slot + 1] = v + 2 * h;
-    }
-    nodes[v] = nd;
-}
-
-__global__ void kRelabel(Elem* __restrict__ el, int32_t n, const int32_t* __restrict__ segFirst,
-                         const int32_t* __restrict__ segNum)
-{
-    const int32_t p = blockIdx.x * kB + threadIdx.x;
-    if (p >= n) return;
-    const int v = __float_as_int(el[p].b.w);
-    const int32_t s = segNum[v];
-    if (s < 2) return;
-    const int32_t h = s / 2;
-    const int child = (p - segFirst[v] < h) ? v + 1 : v + 2 * h;
-    el[p].b.w = __int_as_float(child);
-}
-
-// internal dipoles of one level from their children (source/MRMesh/MRDipole.cpp:47-60)
-__global__ void kInternalDipoles(const int32_t* __restrict__ list, int32_t count, const TreeNode* __restrict__ nodes,
-                                 Dipole* __restrict__ dip)
-{
-    const int32_t i = blockIdx.x * kB + threadIdx.x;
-    if (i >= count) return;
-    const int32_t v = list[i];
-    const TreeNode nd = nodes[v];
-    if (nd.r < 0) return;
-    const Dipole dl = dip[nd.l], dr = dip[nd.r];
-    Dipole d;
+    const Dipole dl = dip[d.v + 1], dr = dip[d.v + 2 * (d.num >> 1)];
+    Dipole o;
     for (int k = 0; k < 3; ++k) {
-        d.pos[k] = dl.pos[k] + dr.pos[k];
-        d.dirArea[k] = dl.dirArea[k] + dr.dirArea[k];
+        o.pos[k] = dl.pos[k] + dr.pos[k];
+        o.dirArea[k] = dl.dirArea[k] + dr.dirArea[k];
     }
-    d.area = dl.area + dr.area;
-    d.rr = 0;
-    dip[v] = d;
+    o.area = dl.area + dr.area;
+    o.rr = 0;
+    dip[d.v] = o;
+}
+
+// ---------------------------------------------------------------- subtrees of at most kSub leaves
+
+struct SubShared {
+    uint64_t key[kSub];            // leaf at each position: first key << 32 | leaf
+    float box[6][kSub];            // by leaf
+    int32_t face[kSub];
+    uint32_t acc[6][kSub / 2];     // node boxes, by half the node's first position (nodes of two leaves or more)
+};
+
+// One block per node of level `level`: all levels below it.  A thread keeps the nodes that cover its two
+// positions; leaves move between positions of one node only.
+__global__ __launch_bounds__(kSubThreads) void kSubtrees(int32_t n, int level, const Elem* __restrict__ el,
+                                                         const float* __restrict__ verts, const int32_t* __restrict__ tris,
+                                                         TreeNode* __restrict__ tree, Dipole* __restrict__ dip,
+                                                         int32_t* __restrict__ firstOf)
+{
+    extern __shared__ __align__(16) unsigned char subMem[];
+    SubShared& S = *reinterpret_cast<SubShared*>(subMem);
+    const Node root = nodeAt(n, level, blockIdx.x);
+    const int s0 = root.num, tid = threadIdx.x, lane = tid & 63;
+    Node nd[2];            // first relative to the root's
+    int leaf[2];
+    for (int q = 0; q < 2; ++q) {
+        const int p = tid + q * kSubThreads;
+        nd[q] = Node{ root.v, 0, p < s0 ? s0 : 0 };
+        leaf[q] = p;
+        if (p < s0) {
+            const Elem e = el[root.first + p];
+            S.box[0][p] = e.a.x; S.box[1][p] = e.a.y; S.box[2][p] = e.a.z;
+            S.box[3][p] = e.a.w; S.box[4][p] = e.b.x; S.box[5][p] = e.b.y;
+            S.face[p] = __float_as_int(e.b.z);
+        }
+    }
+    int levels = 0;
+    for (int maxNum = s0; maxNum > 1; maxNum = (maxNum + 1) >> 1, ++levels) {
+        for (int k = 0; k < 6; ++k) S.acc[k][tid] = k < 3 ? 0xffffffffu : 0u;
+        __syncthreads();
+        // node boxes: runs of equal nodes within the wave, then one atomic per run
+        for (int q = 0; q < 2; ++q) {
+            const bool in = nd[q].num > 1;
+            const int f = in ? nd[q].first : -1;
+            float b[6] = { FLT_MAX, FLT_MAX, FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX };
+            if (in)
+                for (int k = 0; k < 6; ++k) b[k] = S.box[k][leaf[q]];
+            for (int d = 1; d < 64; d <<= 1) {
+                const int of = __shfl_up(f, d);
+                float o[6];
+                for (int k = 0; k < 6; ++k) o[k] = __shfl_up(b[k], d);
+                if (lane >= d && of == f)
+                    for (int k = 0; k < 3; ++k) {
+                        b[k] = fminf(b[k], o[k]);
+                        b[k + 3] = fmaxf(b[k + 3], o[k + 3]);
+                    }
+            }
+            const int nf = __shfl_down(f, 1);
+            if (in && (lane == 63 || nf != f))
+                for (int k = 0; k < 3; ++k) {
+                    atomicMin(&S.acc[k][f >> 1], ordU(b[k]));
+                    atomicMax(&S.acc[3 + k][f >> 1], ordU(b[k + 3]));
+                }
+        }
+        __syncthreads();
+        const auto dims = [&](int f, int sd[3]) {
+            float mn[3], mx[3];
+            for (int k = 0; k < 3; ++k) { mn[k] = unordU(S.acc[k][f >> 1]); mx[k] = unordU(S.acc[3 + k][f >> 1]); }
+            sortedDims(mn, mx, sd);
+        };
+        const auto element = [&](int e) {
+            Elem x;
+            x.a = make_float4(S.box[0][e], S.box[1][e], S.box[2][e], S.box[3][e]);
+            x.b = make_float4(S.box[4][e], S.box[5][e], __int_as_float(S.face[e]), 0.f);
+            return x;
+        };
+        for (int q = 0; q < 2; ++q) {
+            const int p = tid + q * kSubThreads;
+            if (p >= s0) continue;
+            uint64_t key = (uint32_t)leaf[q];
+            if (nd[q].num > 1) {
+                int sd[3];
+                dims(nd[q].first, sd);
+                key |= (uint64_t)leafKey(element(leaf[q]), sd, 0) << 32;
+                if (p == nd[q].first) {
+                    TreeNode t;
+                    for (int k = 0; k < 3; ++k) {
+                        t.box.min[k] = unordU(S.acc[k][p >> 1]);
+                        t.box.max[k] = unordU(S.acc[3 + k][p >> 1]);
+                    }
+                    t.l = nd[q].v + 1;
+                    t.r = nd[q].v + 2 * (nd[q].num >> 1);
+                    tree[nd[q].v] = t;
+                    firstOf[nd[q].v] = root.first + p;
+                }
+            }
+            S.key[p] = key;
+        }
+        __syncthreads();
+        // Every node of the level sorts its own leaves: `half` threads a node, each one pair a stage.  All
+        // comparisons are ascending (a merge starts by comparing mirrored positions), so the positions a node
+        // lacks up to a power of two would hold the largest keys and never move: they are skipped.  Pairs of up
+        // to 64 threads stay within a wave, whose LDS operations are in order.
+        int half = 1;
+        while (2 * half < maxNum) half <<= 1;
+        Node own = Node{ 0, 0, s0 };
+        const int t = tid & (half - 1);
+        for (int b = levels - 1; b >= 0; --b) own = child(own, ((tid / half) >> b) & 1);
+        const bool sorts = tid / half < (1 << levels);
+        const auto sync = [&] {
+            if (half > 64) __syncthreads();
+            else {
+                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+            }
+        };
+        for (int k = 2; k <= 2 * half; k <<= 1)
+            for (int j = k >> 1; j > 0; j >>= 1) {
+                const int block = t / j, in = t - block * j;
+                const int a = block * 2 * j + in, b = j == (k >> 1) ? block * 2 * j + 2 * j - 1 - in : a + j;
+                if (sorts && b < own.num) {
+                    const int pa = own.first + a, pb = own.first + b;
+                    const uint64_t ka = S.key[pa], kb = S.key[pb];
+                    bool swap = kb < ka;
+                    if ((ka >> 32) == (kb >> 32)) {
+                        int sd[3];
+                        dims(own.first, sd);
+                        const Elem xa = element((int)(uint32_t)ka), xb = element((int)(uint32_t)kb);
+                        for (int w = 1; w < 4; ++w) {
+                            const uint32_t va = leafKey(xa, sd, w), vb = leafKey(xb, sd, w);
+                            if (va != vb) { swap = vb < va; break; }
+                        }
+                    }
+                    if (swap) { S.key[pa] = kb; S.key[pb] = ka; }
+                }
+                sync();
+            }
+        __syncthreads();
+        for (int q = 0; q < 2; ++q) {
+            const int p = tid + q * kSubThreads;
+            if (p >= s0) continue;
+            leaf[q] = (int)(uint32_t)S.key[p];
+            if (nd[q].num > 1) nd[q] = child(nd[q], p - nd[q].first >= (nd[q].num >> 1));
+        }
+        __syncthreads();
+    }
+    for (int q = 0; q < 2; ++q) {
+        const int p = tid + q * kSubThreads;
+        if (p >= s0) continue;
+        TreeNode t;
+        for (int k = 0; k < 3; ++k) { t.box.min[k] = S.box[k][leaf[q]]; t.box.max[k] = S.box[3 + k][leaf[q]]; }
+        t.l = S.face[leaf[q]];
+        t.r = -1;
+        tree[nd[q].v] = t;
+        firstOf[nd[q].v] = root.first + p;
+        dip[nd[q].v] = leafDipole(verts, tris, t.l);
+    }
+    for (int l = levels - 1; l >= 0; --l) {
+        __threadfence_block();
+        __syncthreads();
+        if (tid < (1 << l)) {
+            Node d = root;
+            for (int b = l - 1; b >= 0 && d.num > 1; --b) d = child(d, (tid >> b) & 1);
+            if (d.num > 1) addDipoles(dip, d);
+        }
+    }
+}
+
+// the dipoles of the levels above the subtrees, one block for all of them
+__global__ __launch_bounds__(kSubThreads) void kTopDipoles(int32_t n, int level, Dipole* __restrict__ dip)
+{
+    for (int l = level - 1; l >= 0; --l) {
+        for (uint32_t i = threadIdx.x; i < (1u << l); i += kSubThreads) addDipoles(dip, nodeAt(n, l, i));
+        __threadfence_block();
+        __syncthreads();
+    }
 }
 
 // pos /= area (as a multiplication by 1/area), rr = squared distance to the farthest box corner
 // (source/MRMesh/MRDipole.cpp:11-21, 62-70)
-__global__ void kFinalizeDipoles(int32_t nn, const TreeNode* __restrict__ nodes, Dipole* __restrict__ dip,
-                                 int32_t* __restrict__ leafFlag)
+__global__ void kFinalizeDipoles(int32_t nn, const TreeNode* __restrict__ nodes, Dipole* __restrict__ dip)
 {
     const int32_t i = blockIdx.x * kB + threadIdx.x;
     if (i >= nn) return;
@@ -321,18 +634,16 @@ __global__ void kFinalizeDipoles(int32_t nn, const TreeNode* __restrict__ nodes,
     }
     d.rr = rr;
     dip[i] = d;
-    leafFlag[i] = nd.r < 0 ? 1 : 0;
 }
 
-__device__ __forceinline__ int32_t refOf(int32_t i, const int32_t* leafFlag, const int32_t* leafBefore)
-{
-    return leafFlag[i] ? ~leafBefore[i] : i - leafBefore[i];
-}
-
-// the traversal layout (mi_tree.hpp): internal nodes and leaf slots in pre-order
-__global__ void kFlatten(int32_t nn, const TreeNode* __restrict__ nodes, const Dipole* __restrict__ dip,
-                         const int32_t* __restrict__ leafFlag, const int32_t* __restrict__ leafBefore,
-                         const float* __restrict__ verts, const int32_t* __restrict__ tris, float4* __restrict__ dnode,
+// the traversal layout (mi_tree.hpp): internal nodes and leaf slots in pre-order.  Before node i in pre-order
+// there are firstOf[i] leaves, all those to the left of its own.  faceIds (optional): a tree built over the
+// valid faces of a mesh with deleted faces names the packed face index in its leaves; the reference's leaves
+// hold the real FaceId (source/MRMesh/MRAABBTree.cpp:35-49).  Packing keeps the face order, so the tree (whose
+// ties fall to the face index) is the same; only the ids of the leaf nodes and triangle records are mapped back.
+__global__ void kFlatten(int32_t nn, TreeNode* __restrict__ nodes, const Dipole* __restrict__ dip,
+                         const int32_t* __restrict__ firstOf, const float* __restrict__ verts,
+                         const int32_t* __restrict__ tris, const int32_t* __restrict__ faceIds, float4* __restrict__ dnode,
                          float4* __restrict__ tri, float4* __restrict__ dint, float4* __restrict__ dleaf)
 {
     const int32_t i = blockIdx.x * kB + threadIdx.x;
@@ -342,122 +653,75 @@ __global__ void kFlatten(int32_t nn, const TreeNode* __restrict__ nodes, const D
     const float4 d0 = make_float4(d.pos[0], d.pos[1], d.pos[2], d.rr);
     const float4 d1 = make_float4(d.dirArea[0], d.dirArea[1], d.dirArea[2], d.area);
     if (n.r >= 0) {
-        const int32_t j = i - leafBefore[i];
+        const int32_t j = i - firstOf[i];
+        const auto refOf = [&](int32_t c) { return nodes[c].r < 0 ? ~firstOf[c] : c - firstOf[c]; };
         const Box3 L = nodes[n.l].box, R = nodes[n.r].box;
         float4* r = dnode + 4 * (int64_t)j;
         r[0] = make_float4(L.min[0], L.min[1], L.min[2], L.max[0]);
         r[1] = make_float4(L.max[1], L.max[2], R.min[0], R.min[1]);
         r[2] = make_float4(R.min[2], R.max[0], R.max[1], R.max[2]);
-        r[3] = make_float4(__int_as_float(refOf(n.l, leafFlag, leafBefore)),
-                           __int_as_float(refOf(n.r, leafFlag, leafBefore)), 0.f, 0.f);
+        r[3] = make_float4(__int_as_float(refOf(n.l)), __int_as_float(refOf(n.r)), 0.f, 0.f);
         dint[2 * (int64_t)j] = d0;
         dint[2 * (int64_t)j + 1] = d1;
     } else {
-        const int32_t k = leafBefore[i];
+        const int32_t k = firstOf[i];
         const int32_t f = n.l;
         const int32_t* t = tris + 3 * (int64_t)f;
         const float* a = verts + 3 * (int64_t)t[0];
         const float* b = verts + 3 * (int64_t)t[1];
         const float* c = verts + 3 * (int64_t)t[2];
+        const int32_t id = faceIds ? faceIds[f] : f;
         float4* r = tri + 3 * (int64_t)k;
         r[0] = make_float4(a[0], a[1], a[2], b[0]);
         r[1] = make_float4(b[1], b[2], c[0], c[1]);
-        r[2] = make_float4(c[2], __int_as_float(f), 0.f, 0.f);
+        r[2] = make_float4(c[2], __int_as_float(id), 0.f, 0.f);
         dleaf[2 * (int64_t)k] = d0;
         dleaf[2 * (int64_t)k + 1] = d1;
+        if (faceIds) nodes[i].l = id;
     }
 }
 
-// A tree built over the valid faces of a mesh with deleted faces names the packed face index in its
-// leaves; the reference's leaves hold the real FaceId (source/MRMesh/MRAABBTree.cpp:35-49).  Packing
-// keeps the face order, so the tree (whose ties fall to the face index) is the same; only the ids
-// written to the leaf nodes and the triangle records are mapped back.
-__global__ void kRemapFaces(int32_t nn, TreeNode* __restrict__ nodes, const int32_t* __restrict__ leafFlag,
-                            const int32_t* __restrict__ leafBefore, float4* __restrict__ tri,
-                            const int32_t* __restrict__ faceIds)
-{
-    const int32_t i = blockIdx.x * kB + threadIdx.x;
-    if (i >= nn || !leafFlag[i]) return;
-    const int32_t f = faceIds[nodes[i].l];
-    nodes[i].l = f;
-    tri[3 * (int64_t)leafBefore[i] + 2].y = __int_as_float(f);
-}
-
 inline size_t al(size_t b) { return (b + 255) & ~size_t(255); }
-inline int bitsFor(uint64_t x) { int b = 1; while (b < 64 && (x >> b)) ++b; return b; }
 inline unsigned gridFor(int64_t n) { return (unsigned)((n + kB - 1) / kB); }
+
+// levels of nodes of more than kSub leaves (the largest node of level l has ceil(n / 2^l) leaves)
+inline int64_t largest(int32_t n, int level) { return ((int64_t)n + (int64_t(1) << level) - 1) >> level; }
+inline int topLevels(int32_t n)
+{
+    int l = 0;
+    while (largest(n, l) > kSub) ++l;
+    return l;
+}
 
 struct Scratch {
     Elem* el[2];
-    uint32_t *iota, *faceKey, *keyA, *keyB, *permA, *permB, *k1, *k2, *counters;
-    uint64_t *k64, *k64A, *k64B;
-    int32_t *segFirst, *segNum, *lists, *leafFlag, *leafBefore;
-    uint32_t* acc;
-    void* temp;
-    size_t tempBytes;
+    uint32_t *k0, *list, *hist;
+    LevelNode* nodes;
+    int32_t* firstOf;
 };
-
-size_t sortTempBytes(int32_t n)
-{
-    size_t a = 0, b = 0, c = 0;
-    (void)hipcub::DeviceRadixSort::SortPairs(nullptr, a, (const uint32_t*)nullptr, (uint32_t*)nullptr,
-                                             (const uint32_t*)nullptr, (uint32_t*)nullptr, n);
-    (void)hipcub::DeviceRadixSort::SortPairs(nullptr, b, (const uint64_t*)nullptr, (uint64_t*)nullptr,
-                                             (const uint32_t*)nullptr, (uint32_t*)nullptr, n);
-    (void)hipcub::DeviceScan::ExclusiveSum(nullptr, c, (const int32_t*)nullptr, (int32_t*)nullptr, 2 * n);
-    return std::max(a, std::max(b, c));
-}
 
 size_t layout(int32_t nf, Scratch* s, char* base)
 {
     const size_t n = (size_t)nf, nn = 2 * n - 1;
+    const int top = topLevels(nf);
+    const size_t wide = top > 0 ? size_t(1) << (top - 1) : 0;      // nodes of the widest level
     size_t off = 0;
     auto take = [&](size_t bytes) { char* p = base ? base + off : nullptr; off += al(bytes); return p; };
     char* e0 = take(n * sizeof(Elem));
-    char* e1 = take(n * sizeof(Elem));
-    char* iota = take(n * 4);
-    char* faceKey = take(n * 4);
-    char* keyA = take(n * 4);
-    char* keyB = take(n * 4);
-    char* permA = take(n * 4);
-    char* permB = take(n * 4);
-    char* k1 = take(n * 4);
-    char* k2 = take(n * 4);
-    char* counters = take(64);
-    char* k64 = take(n * 8);
-    char* k64A = take(n * 8);
-    char* k64B = take(n * 8);
-    char* segFirst = take(nn * 4);
-    char* segNum = take(nn * 4);
-    char* lists = take(nn * 4);
-    char* leafFlag = take(nn * 4);
-    char* leafBefore = take(nn * 4);
-    char* acc = take(nn * 24);
-    const size_t tb = sortTempBytes(nf);
-    char* temp = take(tb);
+    char* e1 = take(top ? n * sizeof(Elem) : 0);
+    char* k0 = take(top ? n * 4 : 0);
+    char* list = take(top ? n * 4 : 0);
+    char* hist = take(wide * 3 * kBins * 4);
+    char* nodes = take(wide * sizeof(LevelNode));
+    char* firstOf = take(nn * 4);
     if (s) {
         s->el[0] = reinterpret_cast<Elem*>(e0);
         s->el[1] = reinterpret_cast<Elem*>(e1);
-        s->iota = reinterpret_cast<uint32_t*>(iota);
-        s->faceKey = reinterpret_cast<uint32_t*>(faceKey);
-        s->keyA = reinterpret_cast<uint32_t*>(keyA);
-        s->keyB = reinterpret_cast<uint32_t*>(keyB);
-        s->permA = reinterpret_cast<uint32_t*>(permA);
-        s->permB = reinterpret_cast<uint32_t*>(permB);
-        s->k1 = reinterpret_cast<uint32_t*>(k1);
-        s->k2 = reinterpret_cast<uint32_t*>(k2);
-        s->counters = reinterpret_cast<uint32_t*>(counters);
-        s->k64 = reinterpret_cast<uint64_t*>(k64);
-        s->k64A = reinterpret_cast<uint64_t*>(k64A);
-        s->k64B = reinterpret_cast<uint64_t*>(k64B);
-        s->segFirst = reinterpret_cast<int32_t*>(segFirst);
-        s->segNum = reinterpret_cast<int32_t*>(segNum);
-        s->lists = reinterpret_cast<int32_t*>(lists);
-        s->leafFlag = reinterpret_cast<int32_t*>(leafFlag);
-        s->leafBefore = reinterpret_cast<int32_t*>(leafBefore);
-        s->acc = reinterpret_cast<uint32_t*>(acc);
-        s->temp = temp;
-        s->tempBytes = tb;
+        s->k0 = reinterpret_cast<uint32_t*>(k0);
+        s->list = reinterpret_cast<uint32_t*>(list);
+        s->hist = reinterpret_cast<uint32_t*>(hist);
+        s->nodes = reinterpret_cast<LevelNode*>(nodes);
+        s->firstOf = reinterpret_cast<int32_t*>(firstOf);
     }
     return off;
 }
@@ -476,7 +740,7 @@ size_t deviceTreeScratchBytes(int32_t nf)
     return layout(nf, nullptr, nullptr);
 }
 
-hipError_t buildDeviceTree(const float* d_verts, int32_t nv, const int32_t* d_tris, int32_t nf, void* scratch,
+hipError_t buildDeviceTree(const float* d_verts, const int32_t* d_tris, int32_t nf, void* scratch,
                            size_t scratchBytes, const DeviceTreeOut& out, DeviceTreeInfo& info, hipStream_t st,
                            const int32_t* d_faceIds)
 {
@@ -485,71 +749,33 @@ hipError_t buildDeviceTree(const float* d_verts, int32_t nv, const int32_t* d_tr
     Scratch S;
     if (layout(nf, &S, static_cast<char*>(scratch)) > scratchBytes) return hipErrorInvalidValue;
     const int32_t n = nf, nn = 2 * nf - 1;
-    const int faceBits = bitsFor((uint64_t)(n - 1));
-    const int nodeBits = bitsFor((uint64_t)(nn - 1));
-    uint32_t* nextCount = S.counters;
-    uint32_t* err = S.counters + 16;
-
-    kZero<<<1, 64, 0, st>>>(err);
-    kLeafBoxes<<<gridFor(n), kB, 0, st>>>(d_verts, nv, d_tris, n, S.el[0], err);
-    TG_HIP(hipGetLastError());
-    kInit<<<gridFor(n), kB, 0, st>>>(n, S.segFirst, S.segNum, S.lists, S.iota);
-    uint32_t hostErr = 0;
-    TG_HIP(hipMemcpyAsync(&hostErr, err, 4, hipMemcpyDeviceToHost, st));
-    TG_HIP(hipStreamSynchronize(st));
-    if (hostErr) return hipErrorInvalidValue;
-
-    std::vector<int32_t> levelOff, levelCount;
+    while (largest(n, info.depth) > 1) ++info.depth;
+    kLeafBoxes<<<gridFor(n), kB, 0, st>>>(d_verts, d_tris, n, S.el[0]);
+    const int top = topLevels(n);
     int cur = 0;
-    int32_t off = 0, count = 1;
-    int64_t maxSize = n;
-    while (count > 0) {
-        const int32_t* list = S.lists + off;
-        if (maxSize >= 2) {
-            kSegInit<<<gridFor(count), kB, 0, st>>>(list, count, S.segNum, S.acc);
-            kSegBox<<<gridFor(n), kB, 0, st>>>(S.el[cur], n, S.segNum, S.acc);
-            kKeys<<<gridFor(n), kB, 0, st>>>(S.el[cur], n, S.segNum, S.acc, S.faceKey, S.k1, S.k2, S.k64);
-            size_t tb = S.tempBytes;
-            // stable LSD chain: face, k2, k1, then (node, k0)
-            TG_HIP(hipcub::DeviceRadixSort::SortPairs(S.temp, tb, S.faceKey, S.keyB, S.iota, S.permA, n, 0, faceBits, st));
-            kGather<uint32_t><<<gridFor(n), kB, 0, st>>>(S.k2, S.permA, n, S.keyA);
-            tb = S.tempBytes;
-            TG_HIP(hipcub::DeviceRadixSort::SortPairs(S.temp, tb, S.keyA, S.keyB, S.permA, S.permB, n, 0, 32, st));
-            kGather<uint32_t><<<gridFor(n), kB, 0, st>>>(S.k1, S.permB, n, S.keyA);
-            tb = S.tempBytes;
-            TG_HIP(hipcub::DeviceRadixSort::SortPairs(S.temp, tb, S.keyA, S.keyB, S.permB, S.permA, n, 0, 32, st));
-            kGather<uint64_t><<<gridFor(n), kB, 0, st>>>(S.k64, S.permA, n, S.k64A);
-            tb = S.tempBytes;
-            TG_HIP(hipcub::DeviceRadixSort::SortPairs(S.temp, tb, S.k64A, S.k64B, S.permA, S.permB, n, 0,
-                                                      32 + nodeBits, st));
-            kGatherElems<<<gridFor(n), kB, 0, st>>>(S.el[cur], S.permB, n, S.el[cur ^ 1]);
-            cur ^= 1;
-        }
-        kZero<<<1, 64, 0, st>>>(nextCount);
-        kSplit<<<gridFor(count), kB, 0, st>>>(list, count, S.segFirst, S.segNum, S.el[cur], S.acc, d_verts, d_tris,
-                                             out.nodes, out.dipoles, S.lists + off + count, nextCount);
-        if (maxSize >= 2) kRelabel<<<gridFor(n), kB, 0, st>>>(S.el[cur], n, S.segFirst, S.segNum);
+    for (int l = 0; l < top; ++l, cur ^= 1) {
+        const int32_t count = int32_t(1) << l;
+        const Level L{ n, l, (int32_t)((largest(n, l) + kChunk - 1) / kChunk), S.el[cur], S.el[cur ^ 1], S.k0, S.list,
+                       S.nodes, S.hist };
+        const dim3 blocks((unsigned)(count * L.blocksPerNode));
+        kLevelInit<<<gridFor((int64_t)count * 3 * kBins), kB, 0, st>>>(L, count);
+        kLevelBox<<<blocks, kB, 0, st>>>(L);
+        kLevelHist<0><<<blocks, kB, 0, st>>>(L);
+        kLevelHist<1><<<blocks, kB, 0, st>>>(L);
+        kLevelHist<2><<<blocks, kB, 0, st>>>(L);
+        kLevelPivot<<<count, kB, 0, st>>>(L);
+        kLevelPartition<<<blocks, kB, 0, st>>>(L, out.nodes, S.firstOf);
         TG_HIP(hipGetLastError());
-        uint32_t next = 0;
-        TG_HIP(hipMemcpyAsync(&next, nextCount, 4, hipMemcpyDeviceToHost, st));
-        TG_HIP(hipStreamSynchronize(st));
-        levelOff.push_back(off);
-        levelCount.push_back(count);
-        off += count;
-        if ((int64_t)off + next > nn) return hipErrorUnknown;   // cannot happen for a binary tree of nn nodes
-        count = (int32_t)next;
-        maxSize = (maxSize + 1) / 2;
     }
-    info.depth = (int)levelOff.size() - 1;
-    for (int l = (int)levelOff.size() - 2; l >= 0; --l)
-        kInternalDipoles<<<gridFor(levelCount[l]), kB, 0, st>>>(S.lists + levelOff[l], levelCount[l], out.nodes,
-                                                                out.dipoles);
-    kFinalizeDipoles<<<gridFor(nn), kB, 0, st>>>(nn, out.nodes, out.dipoles, S.leafFlag);
-    size_t tb = S.tempBytes;
-    TG_HIP(hipcub::DeviceScan::ExclusiveSum(S.temp, tb, S.leafFlag, S.leafBefore, nn, st));
-    kFlatten<<<gridFor(nn), kB, 0, st>>>(nn, out.nodes, out.dipoles, S.leafFlag, S.leafBefore, d_verts, d_tris,
-                                         out.dnode, out.tri, out.dint, out.dleaf);
-    if (d_faceIds) kRemapFaces<<<gridFor(nn), kB, 0, st>>>(nn, out.nodes, S.leafFlag, S.leafBefore, out.tri, d_faceIds);
+    TG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kSubtrees), hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)sizeof(SubShared)));
+    kSubtrees<<<1u << top, kSubThreads, sizeof(SubShared), st>>>(n, top, S.el[cur], d_verts, d_tris, out.nodes, out.dipoles,
+                                                                 S.firstOf);
+    TG_HIP(hipGetLastError());
+    if (top > 0) kTopDipoles<<<1, kSubThreads, 0, st>>>(n, top, out.dipoles);
+    kFinalizeDipoles<<<gridFor(nn), kB, 0, st>>>(nn, out.nodes, out.dipoles);
+    kFlatten<<<gridFor(nn), kB, 0, st>>>(nn, out.nodes, out.dipoles, S.firstOf, d_verts, d_tris, d_faceIds, out.dnode, out.tri,
+                                         out.dint, out.dleaf);
     TG_HIP(hipGetLastError());
     TreeNode root;
     TG_HIP(hipMemcpyAsync(&root, out.nodes, sizeof(TreeNode), hipMemcpyDeviceToHost, st));
