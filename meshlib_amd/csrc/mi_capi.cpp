@@ -1358,8 +1358,10 @@ int launchPrepared(mi_batch* b, int32_t count, int64_t total, int depth, const m
     mi::DistOpts o{ opts->minDistSq, opts->maxDistSq, opts->nullOutsideMinMax, opts->windingNumberThreshold,
                     opts->windingNumberBeta };
     MI_HIP(mi::fillU32(b->tickets.as<uint32_t>(), 16, 0u, s));
-    MI_HIP(mi::launchBatch(b->items.as<mi::BatchItem>(), count, total, o, up,
-                           b->tickets.as<unsigned long long>(), xcdSplit, b->numCUs * blocksPerCU, depth, capped, s));
+    bool wide = false;
+    for (const mi::BatchItem& it : b->host) wide = wide || it.m.numFaces > (1 << 23);
+    MI_HIP(mi::launchBatch(b->items.as<mi::BatchItem>(), count, total, o, up, b->tickets.as<unsigned long long>(), xcdSplit,
+                           b->numCUs * blocksPerCU, depth, wide, capped, s));
     return MI_OK;
 }
 

@@ -120,7 +120,7 @@ __global__ __launch_bounds__(kBlock) void kSelfIntersections(MeshDev m, int nLog
 // finished wave's LDS goes to the next one at once.  Measured against the wave-cooperative form with hand-over
 // (both with the winding-number sign): k=8 256^3 101 -> 13.4 ms, k=5 64^3 1.48 -> 0.59 ms.  CAPPED: voxels whose cap is below the plain limit and
 // finds nothing walk again without it, counted in failCount.
-template <bool CAPPED>
+template <bool CAPPED, bool WIDE>
 __global__ __launch_bounds__(64, 4) void kSdfLane(MeshDev m, int dx, int dy, int zBegin, int zEnd, int nbx, int nby, int nbz,
                                                   int nBricks, Xf xf, DistOpts o, const float* __restrict__ bound,
                                                   uint32_t* __restrict__ failCount, float* __restrict__ out)
@@ -129,7 +129,7 @@ __global__ __launch_bounds__(64, 4) void kSdfLane(MeshDev m, int dx, int dy, int
     const int brick = gridBlock<64>();
     if (brick >= nBricks) return;
     const int lane = threadIdx.x & 63;
-    const LaneLds l = laneLds<false>(laneMem, m.depth, lane);
+    const LaneLds<false, WIDE> l(laneMem, m.depth);
     int x, y, z;
     const bool valid = brickVoxel(brick, lane, nbx, nby, nbz, dx, dy, zBegin, zEnd, x, y, z);
     float px = (float)x, py = (float)y, pz = (float)z;
@@ -137,13 +137,13 @@ __global__ __launch_bounds__(64, 4) void kSdfLane(MeshDev m, int dx, int dy, int
     const size_t idx = valid ? ((size_t)(z - zBegin) * dy + y) * dx + x : 0;
     float lim = o.maxDistSq;
     if (CAPPED && valid) { const float b = bound[idx]; lim = b < lim ? b : lim; }
-    float resSq = laneWalk<false>(m, l, px, py, pz, lim, valid, kStatQuadSteps, kStatLeafTests);
+    float resSq = laneWalk(m, l, px, py, pz, lim, valid, kStatQuadSteps, kStatLeafTests);
     if (CAPPED) {
         const bool again = valid && lim < o.maxDistSq && !(resSq < lim);
         const uint64_t failed = waveBallot(again);
         if (failed) {
             if (lane == 0) atomicAdd(failCount, (uint32_t)__popcll(failed));
-            const float r = laneWalk<false>(m, l, px, py, pz, o.maxDistSq, again, kStatQuadSteps, kStatLeafTests);
+            const float r = laneWalk(m, l, px, py, pz, o.maxDistSq, again, kStatQuadSteps, kStatLeafTests);
             if (again) resSq = r;
         }
     }
@@ -308,13 +308,14 @@ __global__ __launch_bounds__(kBlock) void kSelfIntersectionsCoop(MeshDev m, int 
 // Queries walk one per lane (laneWalk).  CAPPED: the items' caps apply; lanes that found nothing below a cap
 // smaller than the plain limit walk once more, uncapped (persistent waves take new units meanwhile, so the
 // retries do not form a tail of their own as a separate launch over scattered queries would).
-template <bool CAPPED>
+template <bool CAPPED, bool WIDE>
 __global__ __launch_bounds__(64, 4) void kBatch(const BatchItem* __restrict__ items, int nItems, int64_t total, DistOpts o,
                                                 float up, int depth, unsigned long long* __restrict__ tickets, int xcdSplit)
 {
     extern __shared__ __align__(16) unsigned char laneMem[];
     const int lane = threadIdx.x & 63;
-    const LaneLds l = laneLds<true>(laneMem, depth, lane);
+    const LaneLds<true, WIDE> l(laneMem, depth);
+    const LaneLds<false, WIDE> ld(laneMem, depth);      // grid units: the same memory without ties
     const int parts = xcdSplit ? kXcds : 1;
     int part = xcdSplit ? (int)(blockIdx.x % kXcds) : 0;
     int drained = 0;
@@ -345,13 +346,13 @@ __global__ __launch_bounds__(64, 4) void kBatch(const BatchItem* __restrict__ it
             xfApply(it.xf, px, py, pz);
             float lim = o.maxDistSq;
             if (CAPPED && it.capSdf && valid) { const float c = it.capSdf[idx]; lim = c < lim ? c : lim; }
-            float resSq = laneWalk<false>(it.m, l, px, py, pz, lim, valid, kStatQuadSteps, kStatLeafTests);
+            float resSq = laneWalk(it.m, ld, px, py, pz, lim, valid, kStatQuadSteps, kStatLeafTests);
             if (CAPPED) {
                 const bool retry = valid && !(resSq < lim) && lim < o.maxDistSq;
                 const uint64_t rm = waveBallot(retry);
                 if (rm) {
                     if (lane == 0) atomicAdd(it.rerunCount, (uint32_t)__popcll(rm));
-                    const float r = laneWalk<false>(it.m, l, px, py, pz, o.maxDistSq, retry, kStatQuadSteps, kStatLeafTests);
+                    const float r = laneWalk(it.m, ld, px, py, pz, o.maxDistSq, retry, kStatQuadSteps, kStatLeafTests);
                     if (retry) resSq = r;
                 }
             }
@@ -369,14 +370,14 @@ __global__ __launch_bounds__(64, 4) void kBatch(const BatchItem* __restrict__ it
                 if (CAPPED && it.capProj) { const float c = it.capProj[q]; lim = c < up ? c : up; }
             }
             int leaf = -1;
-            float d = laneWalk<true>(it.m, l, px, py, pz, lim, valid, kStatKeyedSteps, kStatKeyedTests, &leaf);
+            float d = laneWalk(it.m, l, px, py, pz, lim, valid, kStatKeyedSteps, kStatKeyedTests, &leaf);
             if (CAPPED) {
                 const bool retry = valid && leaf < 0 && lim < up;
                 const uint64_t rm = waveBallot(retry);
                 if (rm) {
                     if (lane == 0) atomicAdd(it.rerunCount + 1, (uint32_t)__popcll(rm));
                     int leaf2 = -1;
-                    const float d2 = laneWalk<true>(it.m, l, px, py, pz, up, retry, kStatKeyedSteps, kStatKeyedTests, &leaf2);
+                    const float d2 = laneWalk(it.m, l, px, py, pz, up, retry, kStatKeyedSteps, kStatKeyedTests, &leaf2);
                     if (retry) { leaf = leaf2; d = d2; }
                 }
             }
@@ -556,13 +557,14 @@ __global__ void kFillU32(uint32_t* p, int n, uint32_t v)
 } // namespace
 
 hipError_t launchBatch(const BatchItem* items, int nItems, int64_t totalUnits, const DistOpts& o, float up,
-                       unsigned long long* tickets, int xcdSplit, int blocks, int depth, bool capped,
+                       unsigned long long* tickets, int xcdSplit, int blocks, int depth, bool wide, bool capped,
                        hipStream_t s)
 {
     if (totalUnits <= 0 || nItems <= 0) return hipSuccess;
     if (o.minDistSq > 0 || blocks <= 0 || depth < 0) return hipErrorInvalidValue;
-    const size_t lds = laneSharedBytes(depth, true);
-    const auto kernel = capped ? kBatch<true> : kBatch<false>;
+    const size_t lds = laneSharedBytes(depth, true, wide);
+    const auto kernel = capped ? (wide ? kBatch<true, true> : kBatch<true, false>)
+                               : (wide ? kBatch<false, true> : kBatch<false, false>);
     hipLaunchKernelGGL(kernel, dim3(blocks * kWaves), dim3(64), lds, s, items, nItems, totalUnits, o, up, depth, tickets,
                        xcdSplit);
     return hipGetLastError();
@@ -671,8 +673,10 @@ hipError_t launchSdfGrid(const MeshDev& m, const int32_t dims[3], const Xf& xf, 
     if (o.minDistSq > 0 && m.traversal == (int)Traversal::WaveCoop)
         return launchSdfGridKeyed(m, dims, xf, o, zBegin, zEnd, out, stackD, s, split);
     if (bound || (m.traversal == (int)Traversal::WaveCoop && !(split && split->list && split->budget > 0 && m.nCut > 0))) {
-        const auto kernel = bound ? kSdfLane<true> : kSdfLane<false>;
-        hipLaunchKernelGGL(kernel, dim3(chunkedGrid((int)bricks, 64)), dim3(64), laneSharedBytes(m.depth, false), s, m,
+        const bool wide = laneWide(m.numFaces);
+        const auto kernel = bound ? (wide ? kSdfLane<true, true> : kSdfLane<true, false>)
+                                  : (wide ? kSdfLane<false, true> : kSdfLane<false, false>);
+        hipLaunchKernelGGL(kernel, dim3(chunkedGrid((int)bricks, 64)), dim3(64), laneSharedBytes(m.depth, false, wide), s, m,
                            dims[0], dims[1], zBegin, zEnd, nbx, nby, nbz, (int)bricks, xf, o, bound, failCount, out);
         return hipGetLastError();
     }

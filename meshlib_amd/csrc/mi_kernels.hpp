@@ -107,9 +107,10 @@ struct BatchItem {
 };
 
 // persistent launch over items[0..nItems) (device array); tickets = 8 zeroed 64-bit counters;
-// blocks = number of four-wave groups to keep resident; depth: of the deepest tree; capped: the items' caps apply
+// blocks = number of four-wave groups to keep resident; depth: of the deepest tree; wide: a tree has more than 2^23
+// faces; capped: the items' caps apply
 hipError_t launchBatch(const BatchItem* items, int nItems, int64_t totalUnits, const DistOpts& o, float up,
-                       unsigned long long* tickets, int xcdSplit, int blocks, int depth, bool capped,
+                       unsigned long long* tickets, int xcdSplit, int blocks, int depth, bool wide, bool capped,
                        hipStream_t s);
 
 // small fill kernel (used instead of hipMemsetAsync so streams stay graph-capture safe)

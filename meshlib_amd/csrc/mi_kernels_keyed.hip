@@ -117,7 +117,7 @@ __device__ __forceinline__ int keyLeaf(const MeshDev& m, uint32_t key, float px,
 // the output): a limit per query below `up`.  CAPPED: the bound is a guess; queries that find nothing below a
 // cap smaller than `up` walk again without it, counted in failCount (any cap above the true distance gives the
 // reference's record, so the combination is exact).
-template <bool CAPPED>
+template <bool CAPPED, bool WIDE>
 __global__ __launch_bounds__(64, 4) void kProjectionsLane(MeshDev m, const float* __restrict__ pts,
                                                           const uint32_t* __restrict__ perm, int64_t n, int nWaves, Xf ptXf,
                                                           int hasPtXf, float up, const float* __restrict__ bound,
@@ -127,19 +127,19 @@ __global__ __launch_bounds__(64, 4) void kProjectionsLane(MeshDev m, const float
     const int wv = logicalBlock(nWaves);
     if (wv >= nWaves) return;
     const int lane = threadIdx.x & 63;
-    const LaneLds l = laneLds<true>(laneMem, m.depth, lane);
+    const LaneLds<true, WIDE> l(laneMem, m.depth);
     int64_t q;
     float px, py, pz, lim;
     const bool valid = projQuery(pts, perm, n, ptXf, hasPtXf, up, bound, (uint32_t)wv, lane, q, px, py, pz, lim);
     int leaf = -1;
-    float d = laneWalk<true>(m, l, px, py, pz, lim, valid, kStatKeyedSteps, kStatKeyedTests, &leaf);
+    float d = laneWalk(m, l, px, py, pz, lim, valid, kStatKeyedSteps, kStatKeyedTests, &leaf);
     if (CAPPED) {
         const bool again = valid && leaf < 0 && lim < up;
         const uint64_t failed = waveBallot(again);
         if (failed) {
             if (lane == 0) atomicAdd(failCount, (uint32_t)__popcll(failed));
             int leaf2 = -1;
-            const float d2 = laneWalk<true>(m, l, px, py, pz, up, again, kStatKeyedSteps, kStatKeyedTests, &leaf2);
+            const float d2 = laneWalk(m, l, px, py, pz, up, again, kStatKeyedSteps, kStatKeyedTests, &leaf2);
             if (again) { leaf = leaf2; d = d2; }
         }
     }
@@ -337,8 +337,10 @@ hipError_t launchProjections(const MeshDev& m, const float* pts, const uint32_t*
     // per-lane form
     if (failCount || (coop && !(lo > 0) && !steps)) {
         const int nWaves = (int)((n + 63) / 64);
-        const auto kernel = failCount ? kProjectionsLane<true> : kProjectionsLane<false>;
-        hipLaunchKernelGGL(kernel, dim3(paddedGrid(nWaves)), dim3(64), laneSharedBytes(m.depth, true), s, m, pts, perm, n,
+        const bool wide = laneWide(m.numFaces);
+        const auto kernel = failCount ? (wide ? kProjectionsLane<true, true> : kProjectionsLane<true, false>)
+                                      : (wide ? kProjectionsLane<false, true> : kProjectionsLane<false, false>);
+        hipLaunchKernelGGL(kernel, dim3(paddedGrid(nWaves)), dim3(64), laneSharedBytes(m.depth, true, wide), s, m, pts, perm, n,
                            nWaves, px, ptXf ? 1 : 0, up, bound, failCount, out);
         return hipGetLastError();
     }

@@ -15,7 +15,10 @@
 //
 //  * stack: [entry][lane] in LDS, the child's ref and the top 16 bits of its lower bound (a truncated
 //    non-negative float is a lower bound of itself), so a pop drops what the best has overtaken without
-//    touching memory;
+//    touching memory.  An entry takes 5 bytes (refs of 24 bits; 6 in trees of more than 2^23 faces, WIDE): the
+//    walk waits for its gathers, so waves per CU count, and the stacks limit them (LDS comes in units of 1,280
+//    bytes: depth 21 has 21 waves of distance walks and 18 of projections a CU; the 1.3 M-triangle volume took
+//    11.9 / 14.5 / 16.5 / 20.4 ms with 18 / 14 / 12 / 10);
 //  * leaf tests (FP64) are queued per wave and run one per lane when as many wait as lanes are walking:
 //    dense lanes while the wave is full, no stale bests when only a few long walks are left;
 //  * results are minima over candidates and do not depend on the order of visits: a subtree is dropped
@@ -31,42 +34,67 @@ namespace {
 // no node: neither an internal ref (>= 0) nor a leaf (~slot, slot < 2^30)
 constexpr int kNoNode = (int)0x80000000u;
 
-// LDS of one wave, sized at launch: the fixed part, then int32 ref[depth][64], uint16 bound[depth][64]
+// LDS of one wave, sized at launch: the fixed part, the ties of projections, then the stack, per entry
+// 64 x uint32 and 64 x uint8 (WIDE: uint16)
 struct LaneShared {
     int32_t leaf[128];      // queued leaf tests: leaf slot
-    uint8_t owner[128];     //   and the lane that asked
+    uint8_t owner[128];     //   and the lane whose query it is for; takeovers use 64.. while fewer than 64 wait
     uint32_t best[64];      // each lane's best squared distance (float bits, >= 0)
 };
-constexpr int kLaneTies = 5;
+// idle lanes take over pending subtrees while at most this many lanes have a node
+constexpr int kTakeBelow = 48;
+constexpr int kLaneTies = 4;
 // projections also keep the leaves that tie at the lane's best
 struct LaneTies {
     int32_t leaf[kLaneTies][64];
     uint32_t count[64];
 };
-inline size_t laneSharedBytes(int depth, bool ties)
+constexpr int32_t kNarrowFaces = 1 << 23;      // refs of at most 24 bits with sign
+inline bool laneWide(int32_t numFaces) { return numFaces > kNarrowFaces; }
+inline size_t laneSharedBytes(int depth, bool ties, bool wide)
 {
     const size_t d = depth > 0 ? (size_t)depth : 1;
-    return sizeof(LaneShared) + (ties ? sizeof(LaneTies) : 0) + d * 64 * 6;
+    return sizeof(LaneShared) + (ties ? sizeof(LaneTies) : 0) + d * 64 * (wide ? 6 : 5);
 }
 
 // the wave's view of its LDS
+template <bool TIES, bool WIDE>
 struct LaneLds {
     LaneShared* s;
     LaneTies* ties;          // projections only
-    int32_t* ref;            // + lane, stride 64
-    uint16_t* bound;
+    uint32_t* word;          // WIDE: ref; else upper half of the bound, lower half of the ref
+    uint8_t* rest;           // WIDE: upper half of the bound; else bits 16..23 of the ref
+
+    __device__ __forceinline__ LaneLds(unsigned char* base, int depth)
+    {
+        s = reinterpret_cast<LaneShared*>(base);
+        ties = TIES ? reinterpret_cast<LaneTies*>(base + sizeof(LaneShared)) : nullptr;
+        unsigned char* stack = base + sizeof(LaneShared) + (TIES ? sizeof(LaneTies) : 0);
+        word = reinterpret_cast<uint32_t*>(stack);
+        rest = stack + (size_t)(depth > 0 ? depth : 1) * 256;
+    }
+    // entry at = 64 * index + lane; the bound is stored as its top 16 bits
+    __device__ __forceinline__ void put(int at, int ref, float bound) const
+    {
+        if (WIDE) {
+            word[at] = (uint32_t)ref;
+            reinterpret_cast<uint16_t*>(rest)[at] = stackDist(bound);
+        } else {
+            word[at] = (__float_as_uint(bound) & 0xffff0000u) | ((uint32_t)ref & 0xffffu);
+            rest[at] = (uint8_t)((uint32_t)ref >> 16);
+        }
+    }
+    __device__ __forceinline__ int get(int at, float& bound) const
+    {
+        const uint32_t w = word[at];
+        if (WIDE) {
+            bound = stackDist(reinterpret_cast<const uint16_t*>(rest)[at]);
+            return (int)w;
+        }
+        bound = __uint_as_float(w & 0xffff0000u);
+        return ((int)(int8_t)rest[at] << 16) | (int)(w & 0xffffu);
+    }
 };
-template <bool TIES>
-__device__ __forceinline__ LaneLds laneLds(unsigned char* base, int depth, int lane)
-{
-    LaneLds l;
-    l.s = reinterpret_cast<LaneShared*>(base);
-    l.ties = TIES ? reinterpret_cast<LaneTies*>(base + sizeof(LaneShared)) : nullptr;
-    unsigned char* stack = base + sizeof(LaneShared) + (TIES ? sizeof(LaneTies) : 0);
-    l.ref = reinterpret_cast<int32_t*>(stack) + lane;
-    l.bound = reinterpret_cast<uint16_t*>(stack + (size_t)(depth > 0 ? depth : 1) * 256) + lane;
-    return l;
-}
 
 // Squared distance from the point to a child's cylinder, a lower bound of its triangles' distances up to
 // the rounding that kBoundSlack covers; capped at FLT_MAX so that an overflow never hides a subtree from a
@@ -121,21 +149,21 @@ __device__ __forceinline__ bool visitedFirst(const MeshDev& m, int k1, int k2, f
 }
 
 // leaves a lane's list of `count` tied leaves with its first in the query's order at the front
-__device__ __forceinline__ void resolveTies(const MeshDev& m, const LaneLds& l, float px, float py, float pz, uint32_t count)
+__device__ __forceinline__ void resolveTies(const MeshDev& m, LaneTies* ties, float px, float py, float pz, uint32_t count)
 {
     const int lane = threadIdx.x & 63;
-    int win = l.ties->leaf[0][lane];
+    int win = ties->leaf[0][lane];
     for (uint32_t i = 1; i < count; ++i) {
-        const int k = l.ties->leaf[i][lane];
+        const int k = ties->leaf[i][lane];
         if (visitedFirst(m, k, win, px, py, pz)) win = k;
     }
-    l.ties->leaf[0][lane] = win;
+    ties->leaf[0][lane] = win;
 }
 
 // Runs the last min(qn, 64) queued tests, one per lane, and returns how many stay queued.  TIES: leaves at
 // exactly their owner's best are listed.
-template <bool TIES>
-__device__ __forceinline__ int flushLane(const MeshDev& m, const LaneLds& l, float px, float py, float pz, int qn)
+template <bool TIES, bool WIDE>
+__device__ __forceinline__ int flushLane(const MeshDev& m, const LaneLds<TIES, WIDE>& l, float px, float py, float pz, int qn)
 {
     const int lane = threadIdx.x & 63;
     const int n = qn < 64 ? qn : 64, base = qn - n;
@@ -166,7 +194,7 @@ __device__ __forceinline__ int flushLane(const MeshDev& m, const LaneLds& l, flo
             }
             waveSync();
             if (l.ties->count[lane] > (uint32_t)kLaneTies) {     // a full list keeps only its first in order
-                resolveTies(m, l, px, py, pz, kLaneTies);
+                resolveTies(m, l.ties, px, py, pz, kLaneTies);
                 l.ties->count[lane] = 1;
             }
             waveSync();
@@ -175,16 +203,24 @@ __device__ __forceinline__ int flushLane(const MeshDev& m, const LaneLds& l, flo
     return base;
 }
 
-// Walks every lane's query for the leaves nearer than `up` (squared); lanes with walk = false take part in
-// the wave's work only.  Returns the lane's least squared distance, or `up` where nothing is nearer.
+// Walks every lane's query for the leaves nearer than `up` (squared); lanes with walk = false only help.
+// Returns the lane's least squared distance, or `up` where nothing is nearer.
 // TIES: *leaf = the leaf that the reference's walk would return (the first in the query's own order among
 // those at the least distance), -1 without one.
-template <bool TIES>
-__device__ __forceinline__ float laneWalk(const MeshDev& m, const LaneLds& l, float px, float py, float pz, float up,
+//
+// A lane without a node of its own takes over the oldest pending subtree of another lane's query (`own`: the
+// query a lane works for); bests and ties are kept by query, so the results do not notice.  Walks differ in
+// length -- half the lanes' visits on one grid, ten times the mean near a medial axis -- and a wave took as
+// many steps as its longest.  Without and with (kTakeBelow 48): 1,000 points on 20 k triangles 160 -> 101 us, 64^3
+// on them 0.67 -> 0.39 ms, 2^22 points on 1.3 M triangles 3.31 -> 2.97 ms, 256^3 on them 11.6 -> 11.0 ms; a
+// threshold of 16 gains less, of 60 costs the large launches 4 %.
+template <bool TIES, bool WIDE>
+__device__ __forceinline__ float laneWalk(const MeshDev& m, const LaneLds<TIES, WIDE>& l, float qx, float qy, float qz, float up,
                                           bool walk, int statSteps, int statTests, int* leaf = nullptr)
 {
     const int lane = threadIdx.x & 63;
-    int cur = kNoNode, sp = 0, qn = 0;
+    float px = qx, py = qy, pz = qz;
+    int own = lane, cur = kNoNode, base = 0, sp = 0, qn = 0;      // pending: entries base .. sp - 1
     uint32_t nStep = 0, nVisit = 0, nTest = 0;      // measurement counts
     if (walk && m.numFaces > 0) {
         const float rootd = boxDistSq(m.rootMin[0], m.rootMin[1], m.rootMin[2], m.rootMax[0], m.rootMax[1],
@@ -195,14 +231,16 @@ __device__ __forceinline__ float laneWalk(const MeshDev& m, const LaneLds& l, fl
     waveSync();
     l.s->best[lane] = upBits;
     if (TIES) l.ties->count[lane] = 0;
-    float limit = cur == kNoNode ? -1.f : laneLimit(up);
+    float limit = laneLimit(__uint_as_float(upBits));
+    bool mayTake = true;      // one round of takeovers per step
     for (;;) {
         // next node of every lane without one; leaves go to the queue at once
         for (;;) {
-            while (cur == kNoNode && sp > 0) {
+            while (cur == kNoNode && sp > base) {
                 --sp;
-                const int r = l.ref[64 * sp];
-                if (stackDist(l.bound[64 * sp]) < limit) cur = r;
+                float bound;
+                const int r = l.get(64 * sp + lane, bound);
+                if (bound < limit) cur = r;
             }
             const bool isLeaf = cur < 0 && cur != kNoNode;
             const uint64_t lm = waveBallot(isLeaf);
@@ -211,24 +249,56 @@ __device__ __forceinline__ float laneWalk(const MeshDev& m, const LaneLds& l, fl
                                                               __builtin_amdgcn_mbcnt_lo((uint32_t)lm, 0u));
             if (isLeaf) {
                 l.s->leaf[at] = ~cur;
-                l.s->owner[at] = (uint8_t)lane;
+                l.s->owner[at] = (uint8_t)own;
                 cur = kNoNode;
             }
             qn += __popcll(lm);
-            const int walking = __popcll(waveBallot(cur != kNoNode || sp > 0));
+            const int walking = __popcll(waveBallot(cur != kNoNode || sp > base));
             if (qn >= 64 || qn >= walking) {
                 nTest += (uint32_t)(qn < 64 ? qn : 64);
-                qn = flushLane<TIES>(m, l, px, py, pz, qn);
-                if (limit > 0) limit = laneLimit(__uint_as_float(l.s->best[lane]));
+                qn = flushLane(m, l, qx, qy, qz, qn);
+                limit = laneLimit(__uint_as_float(l.s->best[own]));
             }
         }
         const uint64_t act = waveBallot(cur != kNoNode);
         if (!act) {
             if (!qn) break;
             nTest += (uint32_t)qn;      // the last tests, fewer than 64
-            qn = flushLane<TIES>(m, l, px, py, pz, qn);
+            qn = flushLane(m, l, qx, qy, qz, qn);
             continue;
         }
+        if (mayTake && __popcll(act) <= kTakeBelow) {
+            const bool gives = sp > base;      // lanes with entries have a node too
+            const uint64_t gm = waveBallot(gives);
+            if (gm) {
+                mayTake = false;
+                const uint64_t im = ~act;
+                const int n = __popcll(gm) < __popcll(im) ? __popcll(gm) : __popcll(im);
+                const uint64_t rankOf = gives ? gm : im;
+                const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(rankOf >> 32),
+                                                                __builtin_amdgcn_mbcnt_lo((uint32_t)rankOf, 0u));
+                if (gives) l.s->owner[64 + rank] = (uint8_t)lane;
+                waveSync();
+                const bool takes = cur == kNoNode && rank < n;
+                const int from = takes ? l.s->owner[64 + rank] : lane;
+                const int entry = 64 * __shfl(base, from) + from;
+                const float x = __shfl(px, from), y = __shfl(py, from), z = __shfl(pz, from), lim = __shfl(limit, from);
+                const int o = __shfl(own, from);
+                float bound = 0.f;
+                const int r = takes ? l.get(entry, bound) : kNoNode;
+                if (takes && bound < lim) {
+                    cur = r;
+                    own = o;
+                    px = x; py = y; pz = z;
+                    limit = lim;
+                    base = sp = 0;
+                }
+                if (gives && rank < n) ++base;
+                waveSync();
+                continue;
+            }
+        }
+        mayTake = true;
         ++nStep;
         nVisit += (uint32_t)__popcll(act);
         if (cur != kNoNode) {
@@ -247,8 +317,7 @@ __device__ __forceinline__ float laneWalk(const MeshDev& m, const LaneLds& l, fl
             const bool goNear = dn < limit, goFar = df < limit;
             cur = goNear ? rn : goFar ? rf : kNoNode;
             if (goNear && goFar) {
-                l.ref[64 * sp] = rf;
-                l.bound[64 * sp] = stackDist(df);
+                l.put(64 * sp + lane, rf, df);
                 ++sp;
             }
         }
@@ -261,11 +330,11 @@ __device__ __forceinline__ float laneWalk(const MeshDev& m, const LaneLds& l, fl
     }
     waveSync();
     const uint32_t b = l.s->best[lane];
-    const bool found = limit > 0 && b < upBits;
+    const bool found = b < upBits;
     if (TIES) {
         *leaf = -1;
         if (found) {
-            resolveTies(m, l, px, py, pz, l.ties->count[lane]);
+            resolveTies(m, l.ties, qx, qy, qz, l.ties->count[lane]);
             *leaf = l.ties->leaf[0][lane];
         }
     }

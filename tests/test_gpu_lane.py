@@ -129,3 +129,27 @@ def test_lane_walks_match_cooperative_walks():
     for i in (2, 4):
         for k in range(2):
             assert np.array_equal(out[i + k][0], out[k][0]) and np.array_equal(out[i + k][1], out[k][1])
+
+
+def test_lane_walks_on_more_than_2_23_faces():
+    """The stack entries with full refs (trees of more than 2^23 faces) against the per-lane reference form."""
+    n = 2060
+    rng = np.random.default_rng(1)
+    x, y = np.meshgrid(np.arange(n, dtype=np.float32), np.arange(n, dtype=np.float32), indexing="ij")
+    v = np.stack([x.ravel(), y.ravel(), rng.random(n * n).astype(np.float32)], 1)
+    i, j = (k.ravel() for k in np.meshgrid(np.arange(n - 1), np.arange(n - 1), indexing="ij"))
+    a = i * n + j
+    f = np.concatenate([np.stack([a, a + n, a + n + 1], 1), np.stack([a, a + n + 1, a + 1], 1)]).astype(np.int32)
+    assert len(f) > 1 << 23
+    gm = M.Mesh(v, f)
+    say("faces", len(f), "depth", gm.depth())
+    pr, fwn = M.PointsToMeshProjector(), M.FastWindingNumber(gm)
+    pr.updateMeshData(gm)
+    pts = (rng.random((3000, 3)) * [n, n, 6] - [0, 0, 3]).astype(np.float32)
+    pts[:500] = v[rng.integers(0, len(v), 500)]
+    dims, xf, _ = synth.grid_for_mesh(v, (14, 13, 6))
+    got = pr.findProjections(pts), fwn.calcFromGridWithDistances(dims, xf, M.DistanceToMeshOptions())
+    gm.set_mode("traversal", "per_lane")
+    ref = pr.findProjections(pts), fwn.calcFromGridWithDistances(dims, xf, M.DistanceToMeshOptions())
+    assert np.array_equal(got[0].view(np.uint8), ref[0].view(np.uint8))
+    assert np.array_equal(got[1].view(np.uint32), ref[1].view(np.uint32))
