@@ -41,8 +41,10 @@ struct LaneShared {
     uint8_t owner[128];     //   and the lane whose query it is for; takeovers use 64.. while fewer than 64 wait
     uint32_t best[64];      // each lane's best squared distance (float bits, >= 0)
 };
-// idle lanes take over pending subtrees while at most this many lanes have a node
+// idle lanes take over pending subtrees while at most this many lanes have work left
 constexpr int kTakeBelow = 48;
+// entries a lane without a node may try per step
+constexpr int kPops = 2;
 constexpr int kLaneTies = 4;
 // projections also keep the leaves that tie at the lane's best
 struct LaneTies {
@@ -111,7 +113,7 @@ __device__ __forceinline__ float cylinderDistSq(const float4& a, const float4& b
     const uint32_t tr = __float_as_uint(b.z);
     const float s = fmaxf(fabsf(h) - __uint_as_float(tr & 0xffff0000u), 0.f);
     const float q = fmaxf(rho - __uint_as_float(tr << 16), 0.f);
-    return fminf(__builtin_fmaf(s, s, q * q), FLT_MAX);
+    return __builtin_fmaf(s, s, q * q);
 }
 
 // A lower bound is compared with best * (1 + 2^-17) + 1e-37: the relative part covers the rounding of
@@ -208,12 +210,18 @@ __device__ __forceinline__ int flushLane(const MeshDev& m, const LaneLds<TIES, W
 // TIES: *leaf = the leaf that the reference's walk would return (the first in the query's own order among
 // those at the least distance), -1 without one.
 //
-// A lane without a node of its own takes over the oldest pending subtree of another lane's query (`own`: the
+// A lane without work of its own takes over the oldest pending subtree of another lane's query (`own`: the
 // query a lane works for); bests and ties are kept by query, so the results do not notice.  Walks differ in
 // length -- half the lanes' visits on one grid, ten times the mean near a medial axis -- and a wave took as
-// many steps as its longest.  Without and with (kTakeBelow 48): 1,000 points on 20 k triangles 160 -> 101 us, 64^3
-// on them 0.67 -> 0.39 ms, 2^22 points on 1.3 M triangles 3.31 -> 2.97 ms, 256^3 on them 11.6 -> 11.0 ms; a
-// threshold of 16 gains less, of 60 costs the large launches 4 %.
+// many steps as its longest.  Without and with: 1,000 points on 20 k triangles 160 -> 101 us, 64^3 on them
+// 0.67 -> 0.39 ms, 2^22 points on 1.3 M triangles 3.31 -> 2.97 ms, 256^3 on them 11.6 -> 11.0 ms; thresholds
+// (kTakeBelow) of 40 to 56 are alike, 16 gains less.
+//
+// The vector units bound the large launches (96 % of their cycles on the volume), and whatever one lane needs
+// the wave issues.  So a round is one straight pass: one look for leaves, at most kPops stack entries, one
+// step; a lane that has no internal node by then sits out that step, where a loop until every lane had one
+// issued about 190 vector instructions a step.  With the loop and with rounds of 1 / 2 / 3 entries: 2^22
+// points 2.95 -> 2.39 / 2.33 / 2.53 ms, 256^3 11.1 -> 9.19 / 9.13 / 9.51 ms, 1,000 points 97 -> 71 / 75 / 77 us.
 template <bool TIES, bool WIDE>
 __device__ __forceinline__ float laneWalk(const MeshDev& m, const LaneLds<TIES, WIDE>& l, float qx, float qy, float qz, float up,
                                           bool walk, int statSteps, int statTests, int* leaf = nullptr)
@@ -232,92 +240,91 @@ __device__ __forceinline__ float laneWalk(const MeshDev& m, const LaneLds<TIES, 
     l.s->best[lane] = upBits;
     if (TIES) l.ties->count[lane] = 0;
     float limit = laneLimit(__uint_as_float(upBits));
-    bool mayTake = true;      // one round of takeovers per step
     for (;;) {
-        // next node of every lane without one; leaves go to the queue at once
-        for (;;) {
-            while (cur == kNoNode && sp > base) {
-                --sp;
-                float bound;
-                const int r = l.get(64 * sp + lane, bound);
-                if (bound < limit) cur = r;
-            }
-            const bool isLeaf = cur < 0 && cur != kNoNode;
-            const uint64_t lm = waveBallot(isLeaf);
-            if (!lm) break;
-            const int at = qn + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(lm >> 32),
-                                                              __builtin_amdgcn_mbcnt_lo((uint32_t)lm, 0u));
+        // leaves go to the queue
+        const bool isLeaf = cur < 0 && cur != kNoNode;
+        const uint64_t lm = waveBallot(isLeaf);
+        if (lm) {
             if (isLeaf) {
+                const int at = qn + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(lm >> 32),
+                                                                  __builtin_amdgcn_mbcnt_lo((uint32_t)lm, 0u));
                 l.s->leaf[at] = ~cur;
                 l.s->owner[at] = (uint8_t)own;
                 cur = kNoNode;
             }
             qn += __popcll(lm);
-            const int walking = __popcll(waveBallot(cur != kNoNode || sp > base));
-            if (qn >= 64 || qn >= walking) {
-                nTest += (uint32_t)(qn < 64 ? qn : 64);
-                qn = flushLane(m, l, qx, qy, qz, qn);
-                limit = laneLimit(__uint_as_float(l.s->best[own]));
+        }
+#pragma unroll
+        for (int i = 0; i < kPops; ++i) {
+            if (cur == kNoNode && sp > base) {
+                --sp;
+                float bound;
+                const int r = l.get(64 * sp + lane, bound);
+                if (bound <= limit) cur = r;
             }
         }
-        const uint64_t act = waveBallot(cur != kNoNode);
-        if (!act) {
+        const uint64_t busy = waveBallot(cur != kNoNode || sp > base);
+        const int walking = __popcll(busy);
+        if (qn >= 64 || qn >= walking) {
             if (!qn) break;
-            nTest += (uint32_t)qn;      // the last tests, fewer than 64
+            nTest += (uint32_t)(qn < 64 ? qn : 64);
             qn = flushLane(m, l, qx, qy, qz, qn);
-            continue;
+            limit = laneLimit(__uint_as_float(l.s->best[own]));
         }
-        if (mayTake && __popcll(act) <= kTakeBelow) {
-            const bool gives = sp > base;      // lanes with entries have a node too
+        if (walking <= kTakeBelow) {
+            const bool gives = sp - base > (cur == kNoNode ? 1 : 0);
             const uint64_t gm = waveBallot(gives);
             if (gm) {
-                mayTake = false;
-                const uint64_t im = ~act;
+                const uint64_t im = ~busy;
                 const int n = __popcll(gm) < __popcll(im) ? __popcll(gm) : __popcll(im);
                 const uint64_t rankOf = gives ? gm : im;
                 const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(rankOf >> 32),
                                                                 __builtin_amdgcn_mbcnt_lo((uint32_t)rankOf, 0u));
                 if (gives) l.s->owner[64 + rank] = (uint8_t)lane;
                 waveSync();
-                const bool takes = cur == kNoNode && rank < n;
+                const bool takes = ((im >> lane) & 1) && rank < n;
                 const int from = takes ? l.s->owner[64 + rank] : lane;
                 const int entry = 64 * __shfl(base, from) + from;
                 const float x = __shfl(px, from), y = __shfl(py, from), z = __shfl(pz, from), lim = __shfl(limit, from);
                 const int o = __shfl(own, from);
-                float bound = 0.f;
-                const int r = takes ? l.get(entry, bound) : kNoNode;
-                if (takes && bound < lim) {
-                    cur = r;
-                    own = o;
-                    px = x; py = y; pz = z;
-                    limit = lim;
-                    base = sp = 0;
+                if (takes) {
+                    float bound;
+                    const int r = l.get(entry, bound);
+                    if (bound <= lim) {
+                        cur = r;
+                        own = o;
+                        px = x; py = y; pz = z;
+                        limit = lim;
+                        base = sp = 0;
+                    }
                 }
                 if (gives && rank < n) ++base;
                 waveSync();
-                continue;
             }
         }
-        mayTake = true;
+        const uint64_t act = waveBallot(cur >= 0);
+        if (!act) continue;
         ++nStep;
         nVisit += (uint32_t)__popcll(act);
-        if (cur != kNoNode) {
-            const size_t rec = 4 * (size_t)cur;
-            const float4 a0 = gload(m.cyl, rec), b0 = gload(m.cyl, rec + 1);
-            const float4 a1 = gload(m.cyl, rec + 2), b1 = gload(m.cyl, rec + 3);
+        if (cur >= 0) {
+            float4 a0, b0, a1, b1;
+            if (WIDE) {
+                const size_t rec = 4 * (size_t)cur;
+                a0 = gload(m.cyl, rec); b0 = gload(m.cyl, rec + 1); a1 = gload(m.cyl, rec + 2); b1 = gload(m.cyl, rec + 3);
+            } else {
+                const uint32_t rec = 4u * (uint32_t)cur;
+                a0 = gload(m.cyl, rec); b0 = gload(m.cyl, rec + 1); a1 = gload(m.cyl, rec + 2); b1 = gload(m.cyl, rec + 3);
+            }
             float c0, c1;
             const float d0 = cylinderDistSq(a0, b0, px, py, pz, c0), d1 = cylinderDistSq(a1, b1, px, py, pz, c1);
             const int r0 = __float_as_int(b0.w), r1 = __float_as_int(b1.w);
             // the child with the nearer centre first: while both bounds still hold the point (or nearly), they
             // say little, the centres say on which side the surface is nearer.  Against the nearer bound first:
             // 102 instead of 217 visits and 10 instead of 37 leaf tests per voxel at 1.3 M triangles, 256^3
-            const bool first = c0 <= c1;
-            const float dn = first ? d0 : d1, df = first ? d1 : d0;
-            const int rn = first ? r0 : r1, rf = first ? r1 : r0;
-            const bool goNear = dn < limit, goFar = df < limit;
-            cur = goNear ? rn : goFar ? rf : kNoNode;
-            if (goNear && goFar) {
-                l.put(64 * sp + lane, rf, df);
+            const bool first = c0 <= c1, go0 = d0 <= limit, go1 = d1 <= limit;
+            cur = go0 && (first || !go1) ? r0 : go1 ? r1 : kNoNode;
+            if (go0 && go1) {
+                l.put(64 * sp + lane, first ? r1 : r0, first ? d1 : d0);
                 ++sp;
             }
         }
