@@ -122,16 +122,16 @@ __global__ __launch_bounds__(kBlock) void kSelfIntersections(MeshDev m, int nLog
 // finds nothing walk again without it, counted in failCount.
 template <bool CAPPED, bool WIDE>
 __global__ __launch_bounds__(64, 4) void kSdfLane(MeshDev m, int dx, int dy, int zBegin, int zEnd, int nbx, int nby, int nbz,
-                                                  int nBricks, Xf xf, DistOpts o, const float* __restrict__ bound,
+                                                  int nWaves, int perWave, Xf xf, DistOpts o, const float* __restrict__ bound,
                                                   uint32_t* __restrict__ failCount, float* __restrict__ out)
 {
     extern __shared__ __align__(16) unsigned char laneMem[];
-    const int brick = gridBlock<64>();
-    if (brick >= nBricks) return;
+    const int wv = gridBlock<64>();
+    if (wv >= nWaves) return;
     const int lane = threadIdx.x & 63;
     const LaneLds<false, WIDE> l(laneMem, m.depth);
     int x, y, z;
-    const bool valid = brickVoxel(brick, lane, nbx, nby, nbz, dx, dy, zBegin, zEnd, x, y, z);
+    const bool valid = waveVoxel(wv, lane, perWave, nbx, nby, nbz, dx, dy, zBegin, zEnd, x, y, z);
     float px = (float)x, py = (float)y, pz = (float)z;
     xfApply(xf, px, py, pz);
     const size_t idx = valid ? ((size_t)(z - zBegin) * dy + y) * dx + x : 0;
@@ -245,16 +245,15 @@ __global__ __launch_bounds__(kBlock) void kSdfSplitFinish(MeshDev m, int dx, int
 }
 
 __global__ __launch_bounds__(kBlock) void kFwnGridCoop(MeshDev m, int dx, int dy, int zBegin, int zEnd,
-                                                       int nbx, int nby, int nbz, int nLogical, Xf xf,
+                                                       int nbx, int nby, int nbz, int nLogical, int perWave, Xf xf,
                                                        float beta, float* __restrict__ out)
 {
     const int lb = gridBlock<kGridChunk>();
     if (lb >= nLogical) return;
     const int lane = threadIdx.x & 63;
     const int w = threadIdx.x >> 6;
-    const int brick = lb * kWaves + w;
     int x, y, z;
-    const bool valid = brickVoxel(brick, lane, nbx, nby, nbz, dx, dy, zBegin, zEnd, x, y, z);
+    const bool valid = waveVoxel(lb * kWaves + w, lane, perWave, nbx, nby, nbz, dx, dy, zBegin, zEnd, x, y, z);
     if (!waveBallot(valid)) return;
     float px = (float)x, py = (float)y, pz = (float)z;
     xfApply(xf, px, py, pz);
@@ -266,12 +265,13 @@ __global__ __launch_bounds__(kBlock) void kFwnGridCoop(MeshDev m, int dx, int dy
 __global__ __launch_bounds__(kBlock) void kFwnPointsCoop(MeshDev m, const float* __restrict__ pts,
                                                          const uint32_t* __restrict__ perm, int64_t n,
                                                          int nLogical, float beta, int32_t skipFace,
-                                                         float* __restrict__ out)
+                                                         int perWave, float* __restrict__ out)
 {
     const int lb = logicalBlock(nLogical);
     if (lb >= nLogical) return;
-    const int64_t i = (int64_t)lb * kBlock + threadIdx.x;
-    const bool valid = i < n;
+    const int lane = threadIdx.x & 63;
+    const int64_t i = ((int64_t)lb * kWaves + (threadIdx.x >> 6)) * perWave + lane;
+    const bool valid = lane < perWave && i < n;
     if (!waveBallot(valid)) return;
     const int64_t q = valid ? (perm ? (int64_t)perm[i] : i) : 0;
     float px = 0, py = 0, pz = 0;
@@ -281,14 +281,16 @@ __global__ __launch_bounds__(kBlock) void kFwnPointsCoop(MeshDev m, const float*
 }
 
 __global__ __launch_bounds__(kBlock) void kSelfIntersectionsCoop(MeshDev m, int nLogical, float beta,
-                                                                 uint8_t* __restrict__ out)
+                                                                 int perWave, uint8_t* __restrict__ out)
 {
     const int lb = logicalBlock(nLogical);
     if (lb >= nLogical) return;
-    const int k = lb * kBlock + threadIdx.x;
-    const bool valid = k < m.numFaces;
+    const int lane = threadIdx.x & 63;
+    const int64_t i = ((int64_t)lb * kWaves + (threadIdx.x >> 6)) * perWave + lane;
+    const bool valid = lane < perWave && i < m.numFaces;
+    const int k = valid ? (int)i : 0;
     if (!waveBallot(valid)) return;
-    const Leaf L = loadLeaf(m.tri, valid ? k : 0);
+    const Leaf L = loadLeaf(m.tri, k);
     const float third = 1 / 3.0f;
     const float qx = third * ((L.a[0] + L.b[0]) + L.c[0]);
     const float qy = third * ((L.a[1] + L.b[1]) + L.c[1]);
@@ -676,8 +678,10 @@ hipError_t launchSdfGrid(const MeshDev& m, const int32_t dims[3], const Xf& xf, 
         const bool wide = laneWide(m.numFaces);
         const auto kernel = bound ? (wide ? kSdfLane<true, true> : kSdfLane<true, false>)
                                   : (wide ? kSdfLane<false, true> : kSdfLane<false, false>);
-        hipLaunchKernelGGL(kernel, dim3(chunkedGrid((int)bricks, 64)), dim3(64), laneSharedBytes(m.depth, false, wide), s, m,
-                           dims[0], dims[1], zBegin, zEnd, nbx, nby, nbz, (int)bricks, xf, o, bound, failCount, out);
+        const int perWave = sharedPerWave(64 * bricks, m.numFaces);
+        const int nWaves = (int)(bricks * (64 / perWave));
+        hipLaunchKernelGGL(kernel, dim3(chunkedGrid(nWaves, 64)), dim3(64), laneSharedBytes(m.depth, false, wide), s, m, dims[0],
+                           dims[1], zBegin, zEnd, nbx, nby, nbz, nWaves, perWave, xf, o, bound, failCount, out);
         return hipGetLastError();
     }
     if (m.traversal != (int)Traversal::WaveCoop)
@@ -724,8 +728,10 @@ hipError_t launchFwnGrid(const MeshDev& m, const int32_t dims[3], const Xf& xf, 
     const int nLogical = (int)((bricks + 3) / 4);
     const dim3 grid(chunkedGrid(nLogical, kGridChunk));
     if (m.traversal == (int)Traversal::WaveCoop) {
-        hipLaunchKernelGGL(kFwnGridCoop, grid, dim3(kBlock), 0, s, m, dims[0], dims[1], zBegin, zEnd, nbx, nby, nbz,
-                           nLogical, xf, beta, out);
+        const int perWave = sharedPerWave(64 * bricks, m.numFaces);
+        const int blocks = (int)((bricks * (64 / perWave) + kWaves - 1) / kWaves);
+        hipLaunchKernelGGL(kFwnGridCoop, dim3(chunkedGrid(blocks, kGridChunk)), dim3(kBlock), 0, s, m, dims[0], dims[1], zBegin,
+                           zEnd, nbx, nby, nbz, blocks, perWave, xf, beta, out);
         return hipGetLastError();
     }
     return dispatchDepth(stackD, [&](auto Dc) {
@@ -740,12 +746,15 @@ hipError_t launchFwnPoints(const MeshDev& m, const float* pts, const uint32_t* p
                            float beta, int32_t skipFace, float* out, int stackD, hipStream_t s)
 {
     if (n <= 0) return hipSuccess;
-    const int nLogical = (int)((n + kBlock - 1) / kBlock);
-    const dim3 grid(paddedGrid(nLogical));
     if (m.traversal == (int)Traversal::WaveCoop) {
-        hipLaunchKernelGGL(kFwnPointsCoop, grid, dim3(kBlock), 0, s, m, pts, perm, n, nLogical, beta, skipFace, out);
+        const int perWave = sharedPerWave(n, m.numFaces);
+        const int blocks = (int)((n + (int64_t)kWaves * perWave - 1) / ((int64_t)kWaves * perWave));
+        hipLaunchKernelGGL(kFwnPointsCoop, dim3(paddedGrid(blocks)), dim3(kBlock), 0, s, m, pts, perm, n, blocks, beta, skipFace,
+                           perWave, out);
         return hipGetLastError();
     }
+    const int nLogical = (int)((n + kBlock - 1) / kBlock);
+    const dim3 grid(paddedGrid(nLogical));
     return dispatchDepth(stackD, [&](auto Dc) {
         constexpr int D = decltype(Dc)::value;
         hipLaunchKernelGGL(kFwnPoints<D>, grid, dim3(kBlock), 0, s, m, pts, perm, n, nLogical, beta, skipFace, out);
@@ -756,12 +765,14 @@ hipError_t launchFwnPoints(const MeshDev& m, const float* pts, const uint32_t* p
 hipError_t launchSelfIntersections(const MeshDev& m, float beta, uint8_t* out, int stackD, hipStream_t s)
 {
     if (m.numFaces <= 0) return hipSuccess;
-    const int nLogical = (m.numFaces + kBlock - 1) / kBlock;
-    const dim3 grid(paddedGrid(nLogical));
     if (m.traversal == (int)Traversal::WaveCoop) {
-        hipLaunchKernelGGL(kSelfIntersectionsCoop, grid, dim3(kBlock), 0, s, m, nLogical, beta, out);
+        const int perWave = sharedPerWave(m.numFaces, m.numFaces);
+        const int blocks = (int)(((int64_t)m.numFaces + (int64_t)kWaves * perWave - 1) / ((int64_t)kWaves * perWave));
+        hipLaunchKernelGGL(kSelfIntersectionsCoop, dim3(paddedGrid(blocks)), dim3(kBlock), 0, s, m, blocks, beta, perWave, out);
         return hipGetLastError();
     }
+    const int nLogical = (m.numFaces + kBlock - 1) / kBlock;
+    const dim3 grid(paddedGrid(nLogical));
     return dispatchDepth(stackD, [&](auto Dc) {
         constexpr int D = decltype(Dc)::value;
         hipLaunchKernelGGL(kSelfIntersections<D>, grid, dim3(kBlock), 0, s, m, nLogical, beta, out);

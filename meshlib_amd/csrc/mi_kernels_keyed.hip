@@ -121,7 +121,8 @@ template <bool CAPPED, bool WIDE>
 __global__ __launch_bounds__(64, 4) void kProjectionsLane(MeshDev m, const float* __restrict__ pts,
                                                           const uint32_t* __restrict__ perm, int64_t n, int nWaves, Xf ptXf,
                                                           int hasPtXf, float up, const float* __restrict__ bound,
-                                                          uint32_t* __restrict__ failCount, ProjRec* __restrict__ out)
+                                                          uint32_t* __restrict__ failCount, ProjRec* __restrict__ out,
+                                                          int perWave)
 {
     extern __shared__ __align__(16) unsigned char laneMem[];
     const int wv = logicalBlock(nWaves);
@@ -130,7 +131,8 @@ __global__ __launch_bounds__(64, 4) void kProjectionsLane(MeshDev m, const float
     const LaneLds<true, WIDE> l(laneMem, m.depth);
     int64_t q;
     float px, py, pz, lim;
-    const bool valid = projQuery(pts, perm, n, ptXf, hasPtXf, up, bound, (uint32_t)wv, lane, q, px, py, pz, lim);
+    const bool valid = projQuery(pts, perm, n, ptXf, hasPtXf, up, bound, (uint32_t)wv, lane, q, px, py, pz, lim,
+                                 perWave);
     int leaf = -1;
     float d = laneWalk(m, l, px, py, pz, lim, valid, kStatKeyedSteps, kStatKeyedTests, &leaf);
     if (CAPPED) {
@@ -336,12 +338,13 @@ hipError_t launchProjections(const MeshDev& m, const float* pts, const uint32_t*
     // budget asks for the wave-cooperative form; a non-rigid tree transform (applied per box) keeps the
     // per-lane form
     if (failCount || (coop && !(lo > 0) && !steps)) {
-        const int nWaves = (int)((n + 63) / 64);
+        const int perWave = lanePerWave(n);
+        const int nWaves = (int)((n + perWave - 1) / perWave);
         const bool wide = laneWide(m.numFaces);
         const auto kernel = failCount ? (wide ? kProjectionsLane<true, true> : kProjectionsLane<true, false>)
                                       : (wide ? kProjectionsLane<false, true> : kProjectionsLane<false, false>);
         hipLaunchKernelGGL(kernel, dim3(paddedGrid(nWaves)), dim3(64), laneSharedBytes(m.depth, true, wide), s, m, pts, perm, n,
-                           nWaves, px, ptXf ? 1 : 0, up, bound, failCount, out);
+                           nWaves, px, ptXf ? 1 : 0, up, bound, failCount, out, perWave);
         return hipGetLastError();
     }
     SplitScratch sc;

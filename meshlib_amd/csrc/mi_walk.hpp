@@ -87,6 +87,32 @@ inline int chunkedGrid(int nLogical, int chunk)
     return (nLogical + round - 1) / round * round;
 }
 
+// Queries per wave.  A wave takes as long for a few queries as for 64 -- lane walks are chains of loads, and a
+// shared walk visits the union of its lanes' nodes -- so a launch that cannot fill the chip with full waves
+// spreads its queries over more of them: the smallest power of two that needs no more waves than the chip holds.
+inline int perWaveFor(int64_t n, int64_t waves)
+{
+    int per = 1;
+    while (per < 64 && n > waves * per) per *= 2;
+    return per;
+}
+// Lane walks of separate queries (16 waves a CU; the free lanes take over subtrees).  64 and the rule, whole calls on
+// 82 k triangles: 1,000 points 101 -> 50 us, 16,384 169 -> 87, 65,536 187 -> 133, 262,144 314 -> 295; on 1.3 M
+// triangles 65,536 303 -> 177, 524,288 608 -> 578.  4,096 single queries lose to 2,048 pairs (66 / 57 us), and with
+// more than 2^19 queries full waves win (2^20 on 82 k: 605 / 640 us).
+inline int lanePerWave(int64_t n)
+{
+    if (n > (int64_t)1 << 19) return 64;
+    const int per = perWaveFor(n, 4096);
+    return per == 1 && n > 2048 ? 2 : per < 32 ? per : 32;
+}
+// Winding numbers and grids, whose winding-number walks are shared by a wave: neighbours' walks overlap the
+// less the finer the mesh, so a large mesh takes up to 8,192 waves (32 a CU), a small one 4,096.  64 and the rule:
+// 1,000 points 1126 -> 124 us, 65,536 on 82 k triangles 605 -> 399 us, on 1.3 M 1129 -> 494; 32^3 signed
+// distances on 5 k triangles 234 -> 186 us, on 1.3 M 1053 -> 437; 64^3 there 1171 -> 991, but on 5 k 218 -> 291
+// (32 a wave), hence the limit by faces.
+inline int sharedPerWave(int64_t n, int32_t faces) { return perWaveFor(n, faces < 1 << 17 ? 4096 : 8192); }
+
 // blocks of a persistent launch: enough resident waves to fill every CU
 inline int persistentBlocks()
 {
@@ -432,6 +458,15 @@ __device__ __forceinline__ bool brickVoxel(int brick, int lane, int nbx, int nby
     y = by * 4 + ((lane >> 2) & 3);
     z = zBegin + bz * 4 + (lane >> 4);
     return bz < nbz && x < dx && y < dy && z < zEnd;
+}
+
+// the voxel of a wave that takes `perWave` (a power of two) consecutive voxels of a brick
+__device__ __forceinline__ bool waveVoxel(int wv, int lane, int perWave, int nbx, int nby, int nbz, int dx, int dy,
+                                          int zBegin, int zEnd, int& x, int& y, int& z)
+{
+    const int64_t first = (int64_t)wv * perWave;
+    return brickVoxel((int)(first >> 6), (int)(first & 63) + (lane & (perWave - 1)), nbx, nby, nbz, dx, dy, zBegin, zEnd, x, y, z) &&
+           lane < perWave;
 }
 
 // ---------------------------------------------------------------- wave-cooperative traversals
@@ -1137,10 +1172,11 @@ __device__ __forceinline__ void rankCut(const MeshDev& m, bool valid, float px, 
 // the query of lane `lane` of projection wave `wv` (as in kProjectionsCoop)
 __device__ __forceinline__ bool projQuery(const float* __restrict__ pts, const uint32_t* __restrict__ perm, int64_t n,
                                           const Xf& ptXf, int hasPtXf, float up, const float* __restrict__ bound,
-                                          uint32_t wv, int lane, int64_t& q, float& px, float& py, float& pz, float& lim)
+                                          uint32_t wv, int lane, int64_t& q, float& px, float& py, float& pz, float& lim,
+                                          int perWave = 64)
 {
-    const int64_t i = (int64_t)wv * 64 + lane;
-    const bool valid = i < n;
+    const int64_t i = (int64_t)wv * perWave + lane;
+    const bool valid = lane < perWave && i < n;
     q = valid ? (perm ? (int64_t)perm[i] : i) : 0;
     px = py = pz = 0;
     lim = up;
