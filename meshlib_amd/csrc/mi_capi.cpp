@@ -762,7 +762,7 @@ int mi_fwn_vector_device(mi_mesh* m, const float* d_pts, int64_t n, float beta, 
     hipStream_t s = pick(m, stream);
     if (int rc = ensureWorkspace(m, mi::sortWorkspaceBytes(n))) return rc;
     const uint32_t* perm = nullptr;
-    MI_HIP(mi::sortPointsMorton(d_pts, n, m->sortLo, m->sortHi, m->ws.p, m->ws.bytes, &perm, s));
+    MI_HIP(mi::sortPointsMorton(d_pts, n, m->sortLo, m->sortHi, m->ws.p, m->ws.bytes, &perm, s, mi::PointOrder::Shared));
     MI_HIP(mi::launchFwnPoints(callView(m), d_pts, perm, n, beta, skipFace, d_res, m->stackD, s));
     return MI_OK;
 }
@@ -780,11 +780,12 @@ int mi_proj_find_projections_device(mi_mesh* m, const float* d_pts, int64_t n, c
     if (int rc = ensureWorkspace(m, sortBytes + projSplitBytes(m, n, lo))) return rc;
     mi::SplitScratch sc;
     projSplit(m, m->ws.as<char>() + sortBytes, n, lo, sc);
-    const uint32_t* perm = nullptr;
-    MI_HIP(mi::sortPointsMorton(d_pts, n, m->sortLo, m->sortHi, m->ws.p, m->ws.bytes, &perm, s));
     mi::Xf px, tx;
     if (ptXf) px = toXf(ptXf);
     if (treeXf) tx = toXf(treeXf);
+    const uint32_t* perm = nullptr;
+    MI_HIP(mi::sortPointsMorton(d_pts, n, m->sortLo, m->sortHi, m->ws.p, m->ws.bytes, &perm, s,
+                                mi::projectionOrder(callView(m), treeXf ? &tx : nullptr, lo, &sc)));
     MI_HIP(mi::launchProjections(callView(m), d_pts, perm, n, ptXf ? &px : nullptr, treeXf ? &tx : nullptr, up, lo,
                                  reinterpret_cast<mi::ProjRec*>(d_res), m->stackD, s, nullptr, nullptr, &sc));
     return MI_OK;
@@ -809,11 +810,12 @@ int mi_proj_find_projections_noalloc_device(mi_mesh* m, const float* d_pts, int6
         return fail(MI_E_LIMIT, "the no-allocation scratch is too small for this call");
     mi::SplitScratch sc;
     projSplit(m, static_cast<char*>(scratch) + sortBytes, n, lo, sc);
-    const uint32_t* perm = nullptr;
-    MI_HIP(mi::sortPointsMorton(d_pts, n, m->sortLo, m->sortHi, scratch, sortBytes, &perm, s));
     mi::Xf px, tx;
     if (ptXf) px = toXf(ptXf);
     if (treeXf) tx = toXf(treeXf);
+    const uint32_t* perm = nullptr;
+    MI_HIP(mi::sortPointsMorton(d_pts, n, m->sortLo, m->sortHi, scratch, sortBytes, &perm, s,
+                                mi::projectionOrder(callView(m), treeXf ? &tx : nullptr, lo, &sc)));
     MI_HIP(mi::launchProjections(callView(m), d_pts, perm, n, ptXf ? &px : nullptr, treeXf ? &tx : nullptr, up, lo,
                                  reinterpret_cast<mi::ProjRec*>(d_res), m->stackD, s, nullptr, nullptr, &sc));
     return MI_OK;
@@ -833,11 +835,12 @@ int mi_proj_find_projections_bounded_device(mi_mesh* m, const float* d_pts, int6
     if (int rc = ensureWorkspace(m, sortBytes + projSplitBytes(m, n, lo))) return rc;
     mi::SplitScratch sc;
     projSplit(m, m->ws.as<char>() + sortBytes, n, lo, sc);
-    const uint32_t* perm = nullptr;
-    MI_HIP(mi::sortPointsMorton(d_pts, n, m->sortLo, m->sortHi, m->ws.p, m->ws.bytes, &perm, s));
     mi::Xf px, tx;
     if (ptXf) px = toXf(ptXf);
     if (treeXf) tx = toXf(treeXf);
+    const uint32_t* perm = nullptr;
+    MI_HIP(mi::sortPointsMorton(d_pts, n, m->sortLo, m->sortHi, m->ws.p, m->ws.bytes, &perm, s,
+                                mi::projectionOrder(callView(m), treeXf ? &tx : nullptr, lo, &sc)));
     MI_HIP(mi::launchProjections(callView(m), d_pts, perm, n, ptXf ? &px : nullptr, treeXf ? &tx : nullptr, up, lo,
                                  reinterpret_cast<mi::ProjRec*>(d_res), m->stackD, s, d_upSq, nullptr, &sc));
     return MI_OK;
@@ -858,7 +861,7 @@ int mi_proj_find_projections_capped_device(mi_mesh* m, const float* d_pts, int64
     if (int rc = ensureWorkspace(m, sortBytes + 256)) return rc;
     uint32_t* count = reinterpret_cast<uint32_t*>(m->ws.as<char>() + sortBytes);
     const uint32_t* perm = nullptr;
-    MI_HIP(mi::sortPointsMorton(d_pts, n, m->sortLo, m->sortHi, m->ws.p, sortBytes, &perm, s));
+    MI_HIP(mi::sortPointsMorton(d_pts, n, m->sortLo, m->sortHi, m->ws.p, sortBytes, &perm, s, mi::PointOrder::Lanes));
     MI_HIP(mi::fillU32(count, 1, 0u, s));
     MI_HIP(mi::launchProjections(callView(m), d_pts, perm, n, nullptr, nullptr, up, 0.f,
                                  reinterpret_cast<mi::ProjRec*>(d_res), m->stackD, s, d_capSq, count));
@@ -1121,9 +1124,9 @@ int mi_fwn_calc_from_grid_with_distances_by_parts(mi_mesh* m, mi_grid_part_fn fn
 // and downloaded on its slot's stream while the other slot's part runs.
 constexpr size_t kPartPoints = size_t(1) << 21;
 
-template <class LaunchFn>
-static int pointsHost(mi_mesh* m, const float* pts, int64_t n, size_t outElem, void* res, LaunchFn&& launchFn,
-                      mi_progress_fn cb, void* user, bool split = false, float lo = 0.f)
+template <class OrderFn, class LaunchFn>
+static int pointsHost(mi_mesh* m, const float* pts, int64_t n, size_t outElem, void* res, OrderFn&& orderFn,
+                      LaunchFn&& launchFn, mi_progress_fn cb, void* user, bool split = false, float lo = 0.f)
 {
     std::lock_guard<std::mutex> lk(m->mu);
     MI_HIP(hipSetDevice(m->device));
@@ -1165,7 +1168,8 @@ static int pointsHost(mi_mesh* m, const float* pts, int64_t n, size_t outElem, v
         MI_HIP(hipMemcpyAsync(s.pts.p, pts + 3 * off, sz * 12, hipMemcpyHostToDevice, st));
         float* const dp = static_cast<float*>(s.pts.p);
         const uint32_t* perm = nullptr;
-        MI_HIP(mi::sortPointsMorton(dp, (int64_t)sz, m->sortLo, m->sortHi, s.ws.p, s.ws.bytes, &perm, st));
+        MI_HIP(mi::sortPointsMorton(dp, (int64_t)sz, m->sortLo, m->sortHi, s.ws.p, s.ws.bytes, &perm, st,
+                                    orderFn(&s.sc)));
         MI_HIP(launchFn(dp, perm, (int64_t)sz, s.res.p, &s.sc, st));
         return MI_OK;
     };
@@ -1192,7 +1196,7 @@ int mi_fwn_calc_from_vector(mi_mesh* m, const float* pts, int64_t n, float beta,
                             mi_progress_fn cb, void* user)
 {
     if (!m || n < 0 || (n > 0 && (!pts || !res))) return fail(MI_E_INVALID, "invalid arguments");
-    return pointsHost(m, pts, n, sizeof(float), res,
+    return pointsHost(m, pts, n, sizeof(float), res, [](const mi::SplitScratch*) { return mi::PointOrder::Shared; },
                       [&](const float* dp, const uint32_t* perm, int64_t sz, void* dr, const mi::SplitScratch*,
                           hipStream_t st) {
                           return mi::launchFwnPoints(callView(m), dp, perm, sz, beta, skipFace, static_cast<float*>(dr),
@@ -1240,6 +1244,9 @@ int mi_proj_find_projections(mi_mesh* m, const float* pts, int64_t n, const floa
     if (ptXf) px = toXf(ptXf);
     if (treeXf) tx = toXf(treeXf);
     return pointsHost(m, pts, n, sizeof(mi_projection), res,
+                      [&](const mi::SplitScratch* sc) {
+                          return mi::projectionOrder(callView(m), treeXf ? &tx : nullptr, lo, sc);
+                      },
                       [&](const float* dp, const uint32_t* perm, int64_t sz, void* dr, const mi::SplitScratch* sc,
                           hipStream_t st) {
                           return mi::launchProjections(callView(m), dp, perm, sz, ptXf ? &px : nullptr,
@@ -1341,7 +1348,7 @@ int prepareBatch(mi_batch* b, const mi_batch_item* items, int32_t count, hipStre
             const size_t wsb = align256(mi::sortWorkspaceBytes(it.numPts));
             const uint32_t* perm = nullptr;
             MI_HIP(mi::sortPointsMorton(it.d_pts, it.numPts, it.mesh->sortLo, it.mesh->sortHi,
-                                        b->sortWs.as<char>() + off, wsb, &perm, s));
+                                        b->sortWs.as<char>() + off, wsb, &perm, s, mi::PointOrder::FullWaves));
             d.perm = perm;
             off += wsb;
         }

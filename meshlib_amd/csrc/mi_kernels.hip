@@ -30,6 +30,8 @@
 
 #include <hipcub/hipcub.hpp>
 
+#include <algorithm>
+
 namespace mi {
 namespace {
 
@@ -398,19 +400,102 @@ __device__ __forceinline__ uint32_t spread10(uint32_t v)
     return v;
 }
 
-__global__ void kMorton(const float* __restrict__ pts, int64_t n, float lx, float ly, float lz,
-                        float sx, float sy, float sz, uint32_t* __restrict__ keys,
+// Morton code of a point, 10 bits per axis over the box that (l, s) maps to [0, 1023]; outside points (and NaN)
+// take the nearest cell (the first)
+__device__ __forceinline__ uint32_t mortonKey(const float* __restrict__ pts, int64_t i, float3 l, float3 s)
+{
+    const float fx = fminf(fmaxf((pts[3 * i] - l.x) * s.x, 0.f), 1023.f);
+    const float fy = fminf(fmaxf((pts[3 * i + 1] - l.y) * s.y, 0.f), 1023.f);
+    const float fz = fminf(fmaxf((pts[3 * i + 2] - l.z) * s.z, 0.f), 1023.f);
+    return spread10((uint32_t)fx) | (spread10((uint32_t)fy) << 1) | (spread10((uint32_t)fz) << 2);
+}
+
+__global__ void kMorton(const float* __restrict__ pts, int64_t n, float3 l, float3 s, uint32_t* __restrict__ keys,
                         uint32_t* __restrict__ vals)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const float fx = fminf(fmaxf((pts[3 * i] - lx) * sx, 0.f), 1023.f);
-    const float fy = fminf(fmaxf((pts[3 * i + 1] - ly) * sy, 0.f), 1023.f);
-    const float fz = fminf(fmaxf((pts[3 * i + 2] - lz) * sz, 0.f), 1023.f);
-    keys[i] = spread10((uint32_t)fx) | (spread10((uint32_t)fy) << 1) | (spread10((uint32_t)fz) << 2);
+    keys[i] = mortonKey(pts, i, l, s);
     vals[i] = (uint32_t)i;
 }
 
+// Counting sort of points by the cell that the top bits of their Morton code name, in three launches (clearing the
+// counts is the first): the walks need only that the points of a wave lie together, not an order inside a cell,
+// and at these sizes the 30-bit library sort is a chain of some 18 launches that each leave the chip idle.
+//
+// Counts per cell.  A block counts its chunk in LDS, adds its counts to the global ones with one
+// atomic per cell that it met (equal points cost no more than others), and notes every point's cell and its
+// place among the cell's points.
+constexpr int kCellThreads = 1024;
+constexpr int kCellItems = 8;                 // points per thread, at most
+__global__ __launch_bounds__(kCellThreads) void kCellCount(const float* __restrict__ pts, int64_t n, float3 l, float3 s, int bits,
+                                                           int items, uint32_t* __restrict__ count, uint2* __restrict__ place)
+{
+    extern __shared__ uint4 first4[];
+    uint32_t* const first = reinterpret_cast<uint32_t*>(first4);
+    const int cells = 1 << bits, tid = threadIdx.x;
+    for (int c = tid; c < cells / 4; c += kCellThreads) first4[c] = make_uint4(0, 0, 0, 0);
+    __syncthreads();
+    const int64_t base = (int64_t)blockIdx.x * items * kCellThreads;
+    uint2 own[kCellItems];
+#pragma unroll
+    for (int k = 0; k < kCellItems; ++k) {
+        const int64_t i = base + (int64_t)k * kCellThreads + tid;
+        if (k < items && i < n) {
+            own[k].x = mortonKey(pts, i, l, s) >> (30 - bits);
+            own[k].y = atomicAdd(&first[own[k].x], 1u);
+        }
+    }
+    __syncthreads();
+    for (int c = tid; c < cells; c += kCellThreads) {
+        const uint32_t have = first[c];
+        if (have) first[c] = atomicAdd(&count[c], have);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kCellItems; ++k) {
+        const int64_t i = base + (int64_t)k * kCellThreads + tid;
+        if (k < items && i < n) place[i] = make_uint2(own[k].x, first[own[k].x] + own[k].y);
+    }
+}
+
+// Every block scans the counts for itself (cheaper than one more launch) and scatters its chunk's indices.
+__global__ __launch_bounds__(kCellThreads) void kCellScatter(int64_t n, int bits, int items, const uint32_t* __restrict__ count,
+                                                             const uint2* __restrict__ place, uint32_t* __restrict__ perm)
+{
+    extern __shared__ uint4 start4[];
+    uint32_t* const start = reinterpret_cast<uint32_t*>(start4);
+    __shared__ uint32_t waveSum[kCellThreads / 64];
+    const int quads = 1 << (bits - 2), tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    uint32_t carry = 0;
+    for (int c0 = 0; c0 < quads; c0 += kCellThreads) {
+        const int c = c0 + tid;
+        const uint4 have = c < quads ? reinterpret_cast<const uint4*>(count)[c] : make_uint4(0, 0, 0, 0);
+        const uint32_t mine = have.x + have.y + have.z + have.w;
+        uint32_t sum = mine;
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t o = __shfl_up(sum, d);
+            if (lane >= d) sum += o;
+        }
+        if (lane == 63) waveSum[w] = sum;
+        __syncthreads();
+        uint32_t before = carry + sum - mine, total = 0;
+        for (int k = 0; k < kCellThreads / 64; ++k) {
+            if (k < w) before += waveSum[k];
+            total += waveSum[k];
+        }
+        if (c < quads) start4[c] = make_uint4(before, before + have.x, before + have.x + have.y, before + have.x + have.y + have.z);
+        carry += total;
+        __syncthreads();
+    }
+    const int64_t base = (int64_t)blockIdx.x * items * kCellThreads;
+    for (int k = 0; k < items; ++k) {
+        const int64_t i = base + (int64_t)k * kCellThreads + tid;
+        if (i >= n) break;
+        const uint2 p = place[i];
+        perm[start[p.x] + p.y] = (uint32_t)i;
+    }
+}
 
 } // namespace
 
@@ -782,6 +867,21 @@ hipError_t launchSelfIntersections(const MeshDev& m, float beta, uint8_t* out, i
 
 namespace {
 inline size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
+
+// Bits of the cell number of the counting sort, 0: the 30-bit library sort.  Lane walks only share their caches, so
+// 13 or 14 bits serve them up to 2^21 points: whole calls with the library / counting sort on 82 k triangles 65,536
+// points 135 / 102 us, 2^18 298 / 221, 2^20 605 / 474, 2^21 855 / 764, but 2^22 1368 / 1433.  Waves that
+// share one walk want their queries closer together: winding numbers take 15 bits (128 KB of counts in LDS) up to
+// 2^18 points (on 1.3 M triangles 65,536 524 / 496 us, 2^18 908 / 853; on 82 k alike), above that the library
+// sort is ahead (2^19 614 / 665, 2^20 797 / 855).  Fewer than 512 points: as many counts as the smallest
+// workspace holds.
+int cellBits(int64_t n, PointOrder order)
+{
+    if (n > (order == PointOrder::Shared ? int64_t(1) << 18 : int64_t(1) << 21)) return 0;
+    if (n <= 32768) return n < 512 ? 6 : n <= 8192 ? 9 : 12;
+    return order == PointOrder::Shared ? 15 : n <= 1 << 18 ? 13 : 14;
+}
+
 size_t cubTempBytes(int64_t n)
 {
     size_t bytes = 0;
@@ -798,11 +898,12 @@ size_t sortWorkspaceBytes(int64_t n)
 }
 
 hipError_t sortPointsMorton(const float* pts, int64_t n, const float lo[3], const float hi[3],
-                            void* ws, size_t wsBytes, const uint32_t** permOut, hipStream_t s)
+                            void* ws, size_t wsBytes, const uint32_t** permOut, hipStream_t s, PointOrder order)
 {
     *permOut = nullptr;
     if (n <= 0) return hipSuccess;
     if (n > INT32_MAX || wsBytes < sortWorkspaceBytes(n)) return hipErrorInvalidValue;
+    if (order == PointOrder::Lanes && lanePerWave(n) == 1) return hipSuccess;      // nothing shares a wave
     char* p = static_cast<char*>(ws);
     const size_t a = align256((size_t)n * 4);
     uint32_t* keysIn = reinterpret_cast<uint32_t*>(p);
@@ -811,14 +912,23 @@ hipError_t sortPointsMorton(const float* pts, int64_t n, const float lo[3], cons
     uint32_t* valsOut = reinterpret_cast<uint32_t*>(p + 3 * a);
     void* temp = p + 4 * a;
     size_t tempBytes = cubTempBytes(n);
-    float sc[3];
-    for (int i = 0; i < 3; ++i) {
-        const float ext = hi[i] - lo[i];
-        sc[i] = ext > 0 ? 1023.f / ext : 0.f;
+    auto scale = [&](int i) { const float ext = hi[i] - lo[i]; return ext > 0 ? 1023.f / ext : 0.f; };
+    const float3 l = make_float3(lo[0], lo[1], lo[2]), sc = make_float3(scale(0), scale(1), scale(2));
+    if (const int bits = cellBits(n, order)) {
+        const int items = (int)std::min<int64_t>(kCellItems, 1 + n / (256 * kCellThreads));
+        const int blocks = (int)((n + (int64_t)items * kCellThreads - 1) / ((int64_t)items * kCellThreads));
+        const size_t lds = sizeof(uint32_t) << bits;
+        uint2* const place = reinterpret_cast<uint2*>(keysIn);      // over keysIn and keysOut
+        uint32_t* const count = valsIn;
+        const hipError_t e = fillU32(count, 1 << bits, 0u, s);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(kCellCount, dim3(blocks), dim3(kCellThreads), lds, s, pts, n, l, sc, bits, items, count, place);
+        hipLaunchKernelGGL(kCellScatter, dim3(blocks), dim3(kCellThreads), lds, s, n, bits, items, count, place, valsOut);
+        *permOut = valsOut;
+        return hipGetLastError();
     }
     const int tb = 256;
-    hipLaunchKernelGGL(kMorton, dim3((unsigned)((n + tb - 1) / tb)), dim3(tb), 0, s, pts, n, lo[0], lo[1],
-                       lo[2], sc[0], sc[1], sc[2], keysIn, valsIn);
+    hipLaunchKernelGGL(kMorton, dim3((unsigned)((n + tb - 1) / tb)), dim3(tb), 0, s, pts, n, l, sc, keysIn, valsIn);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     e = hipcub::DeviceRadixSort::SortPairs(temp, tempBytes, keysIn, keysOut, valsIn, valsOut, (int)n, 0,

@@ -179,10 +179,16 @@ hipError_t launchProjections(const MeshDev& m, const float* pts, const uint32_t*
                              int stackD, hipStream_t s, const float* bound = nullptr,
                              uint32_t* failCount = nullptr, const SplitScratch* split = nullptr);
 
-// spatial ordering of query points: Morton codes over box [lo, hi] then a radix sort.
-// workspace layout is private; query its size first with ws == nullptr.
+// how the walks use the order of their points: one query per lane in lanePerWave or in full waves, or one
+// walk shared by a wave
+enum class PointOrder { Lanes, FullWaves, Shared };
+// the order for a projection launch with these arguments
+PointOrder projectionOrder(const MeshDev& m, const Xf* treeXf, float lo, const SplitScratch* split);
+
+// Spatial ordering of query points by their Morton codes over box [lo, hi].  *permOut: indices in the workspace,
+// or null where the given order serves.  The workspace's layout is private.
 size_t sortWorkspaceBytes(int64_t n);
 hipError_t sortPointsMorton(const float* pts, int64_t n, const float lo[3], const float hi[3],
-                            void* ws, size_t wsBytes, const uint32_t** permOut, hipStream_t s);
+                            void* ws, size_t wsBytes, const uint32_t** permOut, hipStream_t s, PointOrder order);
 
 } // namespace mi

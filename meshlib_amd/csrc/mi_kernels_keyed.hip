@@ -321,6 +321,19 @@ __global__ __launch_bounds__(kBlock) void kSdfBandFinish(MeshDev m, BrickSource 
 
 } // namespace
 
+namespace {
+bool stepsSet(const MeshDev& m, const SplitScratch* split) { return split && split->list && split->budget > 0 && m.nCut > 0; }
+} // namespace
+
+// lo > 0: the record depends on the reference's visit order, which the keyed walk reproduces; a step
+// budget asks for the wave-cooperative form; a non-rigid tree transform (applied per box) keeps the
+// per-lane form
+PointOrder projectionOrder(const MeshDev& m, const Xf* treeXf, float lo, const SplitScratch* split)
+{
+    const bool lanes = !treeXf && m.traversal == (int)Traversal::WaveCoop && !(lo > 0) && !stepsSet(m, split);
+    return lanes ? PointOrder::Lanes : PointOrder::Shared;
+}
+
 hipError_t launchProjections(const MeshDev& m, const float* pts, const uint32_t* perm, int64_t n,
                              const Xf* ptXf, const Xf* treeXf, float up, float lo, ProjRec* out,
                              int stackD, hipStream_t s, const float* bound, uint32_t* failCount,
@@ -333,11 +346,8 @@ hipError_t launchProjections(const MeshDev& m, const float* pts, const uint32_t*
     if (treeXf) tx = *treeXf;
     if (failCount && (treeXf || !bound || lo > 0)) return hipErrorInvalidValue;
     const bool coop = !treeXf && m.traversal == (int)Traversal::WaveCoop;
-    const bool steps = split && split->list && split->budget > 0 && m.nCut > 0;
-    // lo > 0: the record depends on the reference's visit order, which the keyed walk reproduces; a step
-    // budget asks for the wave-cooperative form; a non-rigid tree transform (applied per box) keeps the
-    // per-lane form
-    if (failCount || (coop && !(lo > 0) && !steps)) {
+    const bool steps = stepsSet(m, split);
+    if (failCount || projectionOrder(m, treeXf, lo, split) == PointOrder::Lanes) {
         const int perWave = lanePerWave(n);
         const int nWaves = (int)((n + perWave - 1) / perWave);
         const bool wide = laneWide(m.numFaces);
