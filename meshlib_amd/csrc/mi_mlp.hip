@@ -6,10 +6,9 @@
 // softplus = distance / scale.  Parameters live in one FP32 vector (master copy, Adam state) with
 // BF16 copies W (out-major) and W^T (in-major) that the MFMA kernels read.
 //
-// Tile shape: a workgroup of 4 waves owns 64 rows; wave w computes rows [16w, 16w+16) of every
-// layer as 8 output tiles of 16x16, K = 128 in 4 MFMA steps of 32.  Activations stay in LDS between
-// layers; each layer's weights are staged once per workgroup into LDS (rows padded to 136 BF16 so
-// the 16-byte fragment reads of 16 rows fall in distinct banks).
+// Training tile: a workgroup of 16 waves owns 64 rows; a wave computes 32 rows by 16 columns of every layer as two
+// output tiles of 16x16, K = 128 in 4 MFMA steps of 32.  Activations stay in LDS between layers (rows padded to 136
+// BF16 so that the 16-byte fragment reads of 16 rows fall in distinct banks), weight fragments come from L2.
 //
 // MFMA 16x16x32 BF16 fragments (lane l): A row l%16, K elements 8*(l/16)..+7; B column l%16, the
 // same K elements; accumulator element j sits at row 4*(l/16)+j, column l%16.
@@ -29,12 +28,14 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int LDP = kHidden + 8;   // padded LDS row (BF16 elements) for 128-wide rows
 
-__device__ __forceinline__ uint16_t f2bf(float x)
+// two BF16 (round to nearest even) in one instruction, `lo` in the lower half
+__device__ __forceinline__ uint32_t pack2(float lo, float hi)
 {
-    uint32_t u = __float_as_uint(x);
-    u += 0x7FFFu + ((u >> 16) & 1u);     // round to nearest even
-    return (uint16_t)(u >> 16);
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{ lo, hi }), bf16x2));
 }
+__device__ __forceinline__ uint16_t f2bf(float x) { return __builtin_bit_cast(uint16_t, (__bf16)x); }
 __device__ __forceinline__ float bf2f(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
 
 __device__ __forceinline__ bf16x8 frag(const uint16_t* p)
@@ -69,87 +70,120 @@ __device__ __forceinline__ void normalised(const Params& p, const float* pt, flo
     x[2] = (pt[2] - p.center[2]) * p.invScale;
 }
 
-// stages layer l's BF16 weights (128 x 128, rows of `src`) into LDS rows padded to LDP
-__device__ __forceinline__ void stageWeights(const uint16_t* __restrict__ src, uint16_t* Ws)
+// One training step's forward and backward pass over a 64-row tile, in one launch.  loss =
+// 1/(2B) sum (pred/scale - label/scale)^2 over the batch; writes the tile's partial gradient.
+//
+// 16 waves; wave w computes columns [16 (w % 8), + 16) of rows [32 (w / 8), + 32) of every layer, two accumulator
+// tiles (rows 16 t + 4 (l/16) + j, column l%16), so that a SIMD has four waves whose MFMA chains, exponentials
+// and LDS round trips overlap (a batch of 8192 rows has only 128 tiles for 256 CUs: the launch is one tile long).
+// Weights go from L2 straight into fragments, one layer ahead.  SiLU'(Z) of every layer stays in registers (it
+// shares its exponential with SiLU(Z)), and dH with it.  In LDS: the running activations row-major (operand of
+// the next layer), H_{-1} .. H_2 also column-major (rows contiguous) for dW = dZ^T H, dZ both ways, in two
+// buffers, so that a backward layer takes one barrier.
+// Four waves that staged each layer's weights in LDS, gathered columns element by element and computed Z twice
+// took 76 us for 8192 rows, this form 33 (a third of it exponentials and divisions; half the CUs have no tile).
+// Rounding points as the oracle: features, weights, activations and dZ (for the products) in BF16,
+// FP32 accumulation, the bias gradients from FP32 dZ.
+constexpr int kTrainWaves = 16;
+constexpr int LDC = kTileRows + 8;       // padded column of kTileRows rows
+struct TrainShared {
+    uint16_t act[2][kTileRows * LDP];        // forward: H_{l-1}, H_l; backward: dZ, by turns
+    uint16_t actT[kLayers][kHidden * LDC];   // H_{-1} .. H_2
+    uint16_t dzT[2][kHidden * LDC];
+    float du[kTileRows];
+    float red[3][4][kHidden];                // bias gradients, by turns; [2]: dw5
+};
+
+__device__ __forceinline__ void loadWeights(const uint16_t* __restrict__ W, int row, int lk, bf16x8 w[4])
 {
-    const int tid = threadIdx.x;
-    for (int it = 0; it < 8; ++it) {          // 128 x 128 BF16 = 2048 chunks of 16 B
-        const int c = it * 256 + tid, row = c >> 4, c8 = (c & 15) * 8;
-        *reinterpret_cast<uint4*>(&Ws[row * LDP + c8]) = *reinterpret_cast<const uint4*>(&src[row * kHidden + c8]);
+#pragma unroll
+    for (int kc = 0; kc < 4; ++kc) w[kc] = frag(&W[row * kHidden + kc * 32 + lk * 8]);
+}
+
+// acc[t] = rows [r0 + 16 t, + 16) of the row-major A times w
+__device__ __forceinline__ void product(const uint16_t* A, int r0, int lr, int lk, const bf16x8 w[4], f32x4 acc[2])
+{
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        acc[t] = f32x4{ 0.f, 0.f, 0.f, 0.f };
+#pragma unroll
+        for (int kc = 0; kc < 4; ++kc)
+            acc[t] = mfma(frag(&A[(r0 + 16 * t + lr) * LDP + kc * 32 + lk * 8]), w[kc], acc[t]);
     }
 }
 
-// 8 BF16 of column `col` in rows r .. r + 7 of a row-major LDS array (a K-major MFMA fragment)
-__device__ __forceinline__ bf16x8 colFrag(const uint16_t* A, int r, int col)
+// four rows r .. r + 3 of one column, to the row-major and (T) the column-major array
+__device__ __forceinline__ void store4(uint16_t* A, uint16_t* T, int r, int col, const float v[4])
 {
-    uint16_t h[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) h[e] = A[(r + e) * LDP + col];
-    const uint4 v = make_uint4((uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16),
-                               (uint32_t)h[4] | ((uint32_t)h[5] << 16), (uint32_t)h[6] | ((uint32_t)h[7] << 16));
-    return __builtin_bit_cast(bf16x8, v);
+    const uint32_t p0 = pack2(v[0], v[1]), p1 = pack2(v[2], v[3]);
+    A[r * LDP + col] = (uint16_t)p0;
+    A[(r + 1) * LDP + col] = (uint16_t)(p0 >> 16);
+    A[(r + 2) * LDP + col] = (uint16_t)p1;
+    A[(r + 3) * LDP + col] = (uint16_t)(p1 >> 16);
+    if (T) *reinterpret_cast<uint2*>(&T[col * LDC + r]) = make_uint2(p0, p1);
 }
 
-// One training step's forward and backward pass over a 64-row tile, in one launch.  loss =
-// 1/(2B) sum (pred/scale - label/scale)^2 over the batch; writes the tile's partial gradient.
-// The BF16 activations H_{-1} (features) .. H_3 stay in LDS; each layer's pre-activations Z are computed
-// again in the backward pass from the same MFMA inputs in the same order (so the same values) instead
-// of being stored; dH and dZ stay in registers in the accumulator layout (wave w: rows 16w + 4(l/16) + j,
-// column 16 nt + l%16), dZ also in LDS as BF16 for the two products dW = dZ^T H and dH = dZ W.
-// Rounding points as the oracle: features, weights, activations and dZ (for the products) in BF16,
-// FP32 accumulation, the bias gradients from FP32 dZ.
-__global__ __launch_bounds__(256) void kTrainTile(Params p, const float* __restrict__ pts,
-                                                  const float* __restrict__ labels, int64_t n, float invB,
-                                                  float* __restrict__ partial)
+__global__ __launch_bounds__(64 * kTrainWaves) void kTrainTile(Params p, const float* __restrict__ pts,
+                                                               const float* __restrict__ labels, int64_t n, float invB,
+                                                               float* __restrict__ partial)
 {
-    __shared__ __attribute__((aligned(16))) uint16_t Act[kLayers + 1][kTileRows * LDP];
-    __shared__ __attribute__((aligned(16))) uint16_t Ws[kHidden * LDP];
-    __shared__ __attribute__((aligned(16))) uint16_t dZr[kTileRows * LDP];
-    __shared__ float duS[kTileRows];
-    __shared__ float red[4][kHidden];
+    extern __shared__ __align__(16) unsigned char trainMem[];
+    TrainShared& S = *reinterpret_cast<TrainShared*>(trainMem);
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int lr = lane & 15, lk = lane >> 4;
-    const int r0 = 16 * w;
+    const int r0 = 32 * (w >> 3);            // this wave's rows
+    const int col = 16 * (w & 7) + lr;       //   and this lane's column
     const int64_t row0 = (int64_t)blockIdx.x * kTileRows;
     float* part = partial + (size_t)blockIdx.x * kParamsPadded;
 
+    bf16x8 wt[4];
+    loadWeights(p.Wb, col, lk, wt);
     {   // features (rows past n: the features of the origin; their loss weight is 0)
-        const int r = tid >> 2, q4 = tid & 3;
+        const int r = tid & 63, c0 = 8 * (tid >> 6);
         const int64_t gi = row0 + r;
         float x[3] = { 0.f, 0.f, 0.f };
         if (gi < n) normalised(p, pts + 3 * gi, x);
-        for (int j = 0; j < 32; ++j) {
-            const int fi = 32 * q4 + j;
-            Act[0][r * LDP + fi] = f2bf(feature(fi, x, p.piFreq));
-        }
-    }
-    // forward: H_l = BF16(SiLU(H_{l-1} W_l^T + b_l))
-    for (int l = 0; l < kLayers; ++l) {
-        __syncthreads();
-        stageWeights(p.Wb + (size_t)l * kHidden * kHidden, Ws);
-        __syncthreads();
-        bf16x8 a[4];
+        uint32_t h[4];
 #pragma unroll
-        for (int kc = 0; kc < 4; ++kc) a[kc] = frag(&Act[l][(r0 + lr) * LDP + kc * 32 + lk * 8]);
-        const float* bias = p.theta + kOffB + l * kHidden;
+        for (int j = 0; j < 4; ++j) h[j] = pack2(feature(c0 + 2 * j, x, p.piFreq), feature(c0 + 2 * j + 1, x, p.piFreq));
+        *reinterpret_cast<uint4*>(&S.act[0][r * LDP + c0]) = make_uint4(h[0], h[1], h[2], h[3]);
 #pragma unroll
-        for (int nt = 0; nt < 8; ++nt) {
-            f32x4 acc = f32x4{ 0.f, 0.f, 0.f, 0.f };
-#pragma unroll
-            for (int kc = 0; kc < 4; ++kc) acc = mfma(a[kc], frag(&Ws[(nt * 16 + lr) * LDP + kc * 32 + lk * 8]), acc);
-            const int col = nt * 16 + lr;
-            const float bc = bias[col];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) Act[l + 1][(r0 + 4 * lk + j) * LDP + col] = f2bf(siluf(acc[j] + bc));
-        }
+        for (int j = 0; j < 8; ++j) S.actT[0][(c0 + j) * LDC + r] = (uint16_t)(h[j >> 1] >> (16 * (j & 1)));
     }
     __syncthreads();
-    {   // output layer u = sum_c h3[c] w5[c] + b5 and du = dloss/du (four partial sums of 32 per row)
+    // forward: H_l = BF16(SiLU(H_{l-1} W_l^T + b_l)); slope = SiLU'(Z_l)
+    float slope[kLayers][2][4];
+#pragma unroll
+    for (int l = 0; l < kLayers; ++l) {
+        bf16x8 next[4];
+        if (l + 1 < kLayers) loadWeights(p.Wb + (size_t)(l + 1) * kHidden * kHidden, col, lk, next);
+        else loadWeights(p.WbT + (size_t)l * kHidden * kHidden, col, lk, next);      // the first of the backward pass
+        const float bias = p.theta[kOffB + l * kHidden + col];
+        f32x4 acc[2];
+        product(S.act[l & 1], r0, lr, lk, wt, acc);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            float h[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float z = acc[t][j] + bias, e = 1.f + expf(-z);
+                const float sg = 1.f / e;
+                h[j] = z / e;
+                slope[l][t][j] = sg * (1.f + z * (1.f - sg));
+            }
+            store4(S.act[(l + 1) & 1], l + 1 < kLayers ? S.actT[l + 1] : nullptr, r0 + 16 * t + 4 * lk, col, h);
+        }
+#pragma unroll
+        for (int kc = 0; kc < 4; ++kc) wt[kc] = next[kc];
+        __syncthreads();
+    }
+    const uint16_t* H3 = S.act[kLayers & 1];
+    if (tid < 4 * kTileRows) {   // output layer u = sum_c h3[c] w5[c] + b5 and du = dloss/du (four partial sums of 32 per row)
         const int r = tid >> 2, q4 = tid & 3;
         float sum = 0.f;
         for (int j = 0; j < 32; ++j) {
             const int c = 32 * q4 + j;
-            sum += bf2f(Act[kLayers][r * LDP + c]) * bf2f(p.w5b[c]);
+            sum += bf2f(H3[r * LDP + c]) * bf2f(p.w5b[c]);
         }
         sum += __shfl_xor(sum, 1);
         sum += __shfl_xor(sum, 2);
@@ -160,105 +194,75 @@ __global__ __launch_bounds__(256) void kTrainTile(Params p, const float* __restr
                 const float u = sum + p.theta[kOffB5];
                 du = (softplusf(u) - labels[gi] * p.invScale) * invB * sigmoidf(u);
             }
-            duS[r] = du;
+            S.du[r] = du;
         }
     }
     __syncthreads();
-    {   // dw5[c] = sum_r du[r] h3[r][c], db5 = sum_r du[r]
+    if (tid < 2 * kHidden) {   // dw5[c] = sum_r du[r] h3[r][c], db5 = sum_r du[r]
         const int c = tid & 127, half = tid >> 7;
         float sum = 0.f;
         for (int rr = 0; rr < 32; ++rr) {
             const int r = half * 32 + rr;
-            sum += duS[r] * bf2f(Act[kLayers][r * LDP + c]);
+            sum += S.du[r] * bf2f(H3[r * LDP + c]);
         }
-        red[half][c] = sum;
-    }
-    __syncthreads();
-    if (tid < kHidden) part[kOffW5 + tid] = red[0][tid] + red[1][tid];
-    if (tid == 0) {
+        S.red[2][half][c] = sum;
+    } else if (tid == 2 * kHidden) {
         float sum = 0.f;
-        for (int r = 0; r < kTileRows; ++r) sum += duS[r];
+        for (int r = 0; r < kTileRows; ++r) sum += S.du[r];
         part[kOffB5] = sum;
     }
     // dH_3 = du w5^T, in registers
-    float dH[8][4];
+    const float w5 = bf2f(p.w5b[col]);
+    float dH[2][4];
 #pragma unroll
-    for (int nt = 0; nt < 8; ++nt)
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) dH[nt][j] = duS[r0 + 4 * lk + j] * bf2f(p.w5b[nt * 16 + lr]);
+        for (int j = 0; j < 4; ++j) dH[t][j] = S.du[r0 + 16 * t + 4 * lk + j] * w5;
+    // backward.  Layer l takes buffer l & 1 of dZ: layer 3 the one that does not hold H_3
+    static_assert((kLayers & 1) == 0, "H_3 is in act[0]");
+#pragma unroll
     for (int l = kLayers - 1; l >= 0; --l) {
-        __syncthreads();      // the previous layer's readers of Ws, dZr and red are done
-        stageWeights(p.Wb + (size_t)l * kHidden * kHidden, Ws);
-        __syncthreads();
-        // Z_l again, then dZ = dH * SiLU'(Z): FP32 for the bias gradient, BF16 in dZr for the products
-        bf16x8 a[4];
+        uint16_t* dz = S.act[l & 1];
+        uint16_t* dzT = S.dzT[l & 1];
+        float(*red)[kHidden] = S.red[l & 1];
 #pragma unroll
-        for (int kc = 0; kc < 4; ++kc) a[kc] = frag(&Act[l][(r0 + lr) * LDP + kc * 32 + lk * 8]);
-        const float* bias = p.theta + kOffB + l * kHidden;
-#pragma unroll
-        for (int nt = 0; nt < 8; ++nt) {
-            f32x4 acc = f32x4{ 0.f, 0.f, 0.f, 0.f };
-#pragma unroll
-            for (int kc = 0; kc < 4; ++kc) acc = mfma(a[kc], frag(&Ws[(nt * 16 + lr) * LDP + kc * 32 + lk * 8]), acc);
-            const int col = nt * 16 + lr;
-            const float bc = bias[col];
-            float colSum = 0.f;
+        for (int t = 0; t < 2; ++t) {
+            float d[4], colSum = 0.f;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const float z = acc[j] + bc;
-                const float sg = sigmoidf(z);
-                const float dz = dH[nt][j] * (sg * (1.f + z * (1.f - sg)));
-                dZr[(r0 + 4 * lk + j) * LDP + col] = f2bf(dz);
-                colSum += dz;
+                d[j] = dH[t][j] * slope[l][t][j];
+                colSum += d[j];
             }
-            // column sums over the wave's 16 rows (lanes l, l^16, l^32, l^48 hold the same column)
+            store4(dz, dzT, r0 + 16 * t + 4 * lk, col, d);
+            // column sums over 16 rows (lanes l, l^16, l^32, l^48 hold the same column)
             colSum += __shfl_xor(colSum, 16);
             colSum += __shfl_xor(colSum, 32);
-            if (lk == 0) red[w][col] = colSum;
+            if (lk == 0) red[2 * (w >> 3) + t][col] = colSum;
         }
         __syncthreads();
+        if (l == kLayers - 1 && tid >= 128 && tid < 256) part[kOffW5 + tid - 128] = S.red[2][0][tid - 128] + S.red[2][1][tid - 128];
         if (tid < kHidden) part[kOffB + l * kHidden + tid] = ((red[0][tid] + red[1][tid]) + red[2][tid]) + red[3][tid];
-        {   // dW_l (128 out x 128 in) = dZ^T (out x rows) . H_{l-1} (rows x in); wave w: out rows [32w, 32w+32)
-            f32x4 acc[2][8];
+        if (l > 0) {      // dH_{l-1} (rows x in) = dZ (rows x out) . W_l (out x in)
+            f32x4 acc[2];
+            product(dz, r0, lr, lk, wt, acc);
+            if (l > 1) loadWeights(p.WbT + (size_t)(l - 1) * kHidden * kHidden, col, lk, wt);
 #pragma unroll
-            for (int mt = 0; mt < 2; ++mt)
+            for (int t = 0; t < 2; ++t)
 #pragma unroll
-                for (int nt = 0; nt < 8; ++nt) acc[mt][nt] = f32x4{ 0.f, 0.f, 0.f, 0.f };
-#pragma unroll
-            for (int kc = 0; kc < 2; ++kc) {
-                const bf16x8 a0 = colFrag(dZr, 32 * kc + 8 * lk, 32 * w + lr);
-                const bf16x8 a1 = colFrag(dZr, 32 * kc + 8 * lk, 32 * w + 16 + lr);
-#pragma unroll
-                for (int nt = 0; nt < 8; ++nt) {
-                    const bf16x8 b = colFrag(Act[l], 32 * kc + 8 * lk, 16 * nt + lr);
-                    acc[0][nt] = mfma(a0, b, acc[0][nt]);
-                    acc[1][nt] = mfma(a1, b, acc[1][nt]);
-                }
-            }
-            float* dW = part + kOffW + l * kHidden * kHidden;
-#pragma unroll
-            for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-                for (int nt = 0; nt < 8; ++nt)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        dW[(32 * w + 16 * mt + 4 * lk + j) * kHidden + 16 * nt + lr] = acc[mt][nt][j];
+                for (int j = 0; j < 4; ++j) dH[t][j] = acc[t][j];
         }
-        if (l == 0) break;
-        // dH_{l-1} (rows x in) = dZ (rows x out) . W_l (out x in); B(k = out, n = in) = W^T[in][out].  Every
-        // wave finished reading Ws (W_l) before the barrier above.
-        stageWeights(p.WbT + (size_t)l * kHidden * kHidden, Ws);
-        __syncthreads();
-        bf16x8 d[4];
+        // dW_l (128 out x 128 in) = dZ^T (out x rows) . H_{l-1} (rows x in); this wave: out columns [16 (w % 8), + 16),
+        // in columns [64 (w / 8), + 64)
+        float* dW = part + kOffW + l * kHidden * kHidden;
+        const bf16x8 a0 = frag(&dzT[col * LDC + 8 * lk]), a1 = frag(&dzT[col * LDC + 32 + 8 * lk]);
 #pragma unroll
-        for (int kc = 0; kc < 4; ++kc) d[kc] = frag(&dZr[(r0 + lr) * LDP + kc * 32 + lk * 8]);
-#pragma unroll
-        for (int nt = 0; nt < 8; ++nt) {
+        for (int t = 0; t < 4; ++t) {
+            const int in = 64 * (w >> 3) + 16 * t + lr;
             f32x4 acc = f32x4{ 0.f, 0.f, 0.f, 0.f };
+            acc = mfma(a0, frag(&S.actT[l][in * LDC + 8 * lk]), acc);
+            acc = mfma(a1, frag(&S.actT[l][in * LDC + 32 + 8 * lk]), acc);
 #pragma unroll
-            for (int kc = 0; kc < 4; ++kc) acc = mfma(d[kc], frag(&Ws[(nt * 16 + lr) * LDP + kc * 32 + lk * 8]), acc);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) dH[nt][j] = acc[j];
+            for (int j = 0; j < 4; ++j) dW[(16 * (w & 7) + 4 * lk + j) * kHidden + in] = acc[j];
         }
     }
 }
@@ -319,8 +323,7 @@ __device__ __forceinline__ float featureFast(int f, const float x[3], const floa
     return r < 3 ? __builtin_amdgcn_sinf(a) : __builtin_amdgcn_cosf(a);
 }
 
-__device__ __forceinline__ uint32_t pack2(uint16_t lo, uint16_t hi) { return (uint32_t)lo | ((uint32_t)hi << 16); }
-
+// Packing two BF16 per instruction instead of rounding with integers: 2^20 points 319 -> 288 us.
 // out[i]: the predicted distance (capMargin < 0), else the cap radius r = pred (1 + capMargin) + slack, squared
 // when capSquared
 __global__ __launch_bounds__(64 * kPredWaves) void kPredict(Params p, PredSource src, int64_t n,
@@ -370,9 +373,9 @@ __global__ __launch_bounds__(64 * kPredWaves) void kPredict(Params p, PredSource
             }
 #pragma unroll
             for (int kc = 0; kc < 4; ++kc) {
-                uint16_t h[8];
+                float h[8];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) h[e] = f2bf(featureFast(32 * kc + 8 * lg + e, x, halfFreq));
+                for (int e = 0; e < 8; ++e) h[e] = featureFast(32 * kc + 8 * lg + e, x, halfFreq);
                 const uint4 v = make_uint4(pack2(h[0], h[1]), pack2(h[2], h[3]), pack2(h[4], h[5]), pack2(h[6], h[7]));
                 cur[g][kc] = __builtin_bit_cast(bf16x8, v);
             }
@@ -403,11 +406,11 @@ __global__ __launch_bounds__(64 * kPredWaves) void kPredict(Params p, PredSource
                     for (int j = 0; j < 4; ++j) bb[half][j] = bias[l * kHidden + 16 * (2 * c + half) + 4 * lg + j];
 #pragma unroll
                 for (int g = 0; g < kPredGroups; ++g) {
-                    uint16_t h[8];
+                    float h[8];
 #pragma unroll
                     for (int half = 0; half < 2; ++half)
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) h[4 * half + j] = f2bf(siluFast(acc[g][half][j] + bb[half][j]));
+                        for (int j = 0; j < 4; ++j) h[4 * half + j] = siluFast(acc[g][half][j] + bb[half][j]);
                     const uint4 v = make_uint4(pack2(h[0], h[1]), pack2(h[2], h[3]), pack2(h[4], h[5]),
                                                pack2(h[6], h[7]));
                     nxt[g][c] = __builtin_bit_cast(bf16x8, v);
@@ -492,23 +495,27 @@ __device__ __forceinline__ void refresh(const Params& p, int j, float v)
     }
 }
 
-// one Adam step straight from the backward pass's per-tile partial gradients (their sum in four
-// interleaved accumulators, then the update): no separate reduction launch
-__global__ void kAdamPartials(Params p, const float* __restrict__ partial, int nBlocks, float* __restrict__ mom,
-                              float* __restrict__ vel, float lr, float b1, float b2, float eps, float c1, float c2)
+// One Adam step straight from the backward pass's per-tile partial gradients: their sum in four interleaved
+// accumulators, one per wave of the block (64 parameters each), then the update.  Bound by the reads (34 MB at 128
+// tiles): 13.8 us with one thread for all four sums, 7.1 with four.
+__global__ __launch_bounds__(256) void kAdamPartials(Params p, const float* __restrict__ partial, int nBlocks,
+                                                     float* __restrict__ mom, float* __restrict__ vel, float lr, float b1,
+                                                     float b2, float eps, float c1, float c2)
 {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= kParams) return;
-    float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
-    int b = 0;
-    for (; b + 4 <= nBlocks; b += 4) {
-        s0 += partial[(size_t)b * kParamsPadded + j];
-        s1 += partial[(size_t)(b + 1) * kParamsPadded + j];
-        s2 += partial[(size_t)(b + 2) * kParamsPadded + j];
-        s3 += partial[(size_t)(b + 3) * kParamsPadded + j];
-    }
-    for (; b < nBlocks; ++b) s0 += partial[(size_t)b * kParamsPadded + j];
-    const float g = (s0 + s1) + (s2 + s3);
+    __shared__ float sum[4][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int j = blockIdx.x * 64 + lane;      // the grid covers kParamsPadded
+    const int rounds = nBlocks & ~3;           // the remainder goes to the first accumulator
+    float s = 0.f;
+    int b = w;
+#pragma unroll 8
+    for (; b < rounds; b += 4) s += partial[(size_t)b * kParamsPadded + j];
+    if (w == 0)
+        for (b = rounds; b < nBlocks; ++b) s += partial[(size_t)b * kParamsPadded + j];
+    sum[w][lane] = s;
+    __syncthreads();
+    if (w || j >= kParams) return;
+    const float g = (sum[0][lane] + sum[1][lane]) + (sum[2][lane] + sum[3][lane]);
     const float m = b1 * mom[j] + (1.f - b1) * g;
     const float v = b2 * vel[j] + (1.f - b2) * g * g;
     mom[j] = m;
@@ -587,7 +594,7 @@ hipError_t gradient(const Params& p, const float* pts, const float* labels, int6
 {
     if (n <= 0) return hipSuccess;
     const int blocks = (int)((n + kTileRows - 1) / kTileRows);
-    hipLaunchKernelGGL(kTrainTile, dim3(blocks), dim3(256), 0, s, p, pts, labels, n, 1.f / (float)n, tb.partial);
+    hipLaunchKernelGGL(kTrainTile, dim3(blocks), dim3(64 * kTrainWaves), sizeof(TrainShared), s, p, pts, labels, n, 1.f / (float)n, tb.partial);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kReduce, dim3((kParamsPadded + 255) / 256), dim3(256), 0, s, tb.partial, blocks, grad);
@@ -599,13 +606,13 @@ hipError_t trainStep(const Params& p, const float* pts, const float* labels, int
 {
     if (n <= 0) return hipSuccess;
     const int blocks = (int)((n + kTileRows - 1) / kTileRows);
-    hipLaunchKernelGGL(kTrainTile, dim3(blocks), dim3(256), 0, s, p, pts, labels, n, 1.f / (float)n, tb.partial);
+    hipLaunchKernelGGL(kTrainTile, dim3(blocks), dim3(64 * kTrainWaves), sizeof(TrainShared), s, p, pts, labels, n, 1.f / (float)n, tb.partial);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
     const float c1 = (float)(1.0 / (1.0 - std::pow(0.9, step)));
     const float c2 = (float)(1.0 / (1.0 - std::pow(0.999, step)));
-    hipLaunchKernelGGL(kAdamPartials, dim3((kParams + 255) / 256), dim3(256), 0, s, p, tb.partial, blocks, mom, vel,
+    hipLaunchKernelGGL(kAdamPartials, dim3(kParamsPadded / 64), dim3(256), 0, s, p, tb.partial, blocks, mom, vel,
                        lr, b1, b2, eps, c1, c2);
     return hipGetLastError();
 }
