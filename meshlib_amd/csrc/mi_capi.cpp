@@ -80,6 +80,117 @@ size_t memBudget()
     return lim;
 }
 
+// Device memory for the temporaries of one call or of a mesh's creation, and streams, kept for reuse: a hipMalloc and
+// its hipFree cost about 57 and 83 us, a stream 150 and 55, and opening a 328 k-triangle mesh and checking it took
+// ten of the former and two of the latter, 1.4 of its 4.3 ms.  Both pools are bounded (at most kTempKeep buffers
+// of together kTempKeepBytes, kStreamKeep streams), are used under a lock, and take back only what no queued work
+// uses any more.  They live until the process ends (never destroyed, so no HIP call runs from a static destructor).
+constexpr size_t kTempKeep = 8, kTempKeepBytes = size_t(64) << 20, kStreamKeep = 8;
+
+struct TempPool {
+    struct Idle { void* p; size_t bytes; int device; };
+    std::mutex mu;
+    std::vector<Idle> idle;      // oldest first
+    size_t held = 0;
+
+    // a buffer of at least `bytes` on the current device, the smallest idle one that is not far too large
+    hipError_t take(size_t bytes, void** p, size_t* got, int* device)
+    {
+        hipError_t e = hipGetDevice(device);
+        if (e != hipSuccess) return e;
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            size_t best = idle.size();
+            for (size_t i = 0; i < idle.size(); ++i)
+                if (idle[i].device == *device && idle[i].bytes >= bytes && idle[i].bytes / 4 <= bytes + (size_t(1) << 18) &&
+                    (best == idle.size() || idle[i].bytes < idle[best].bytes))
+                    best = i;
+            if (best < idle.size()) {
+                *p = idle[best].p;
+                *got = idle[best].bytes;
+                held -= *got;
+                idle.erase(idle.begin() + (ptrdiff_t)best);
+                return hipSuccess;
+            }
+        }
+        *got = bytes;
+        e = hipMalloc(p, bytes);
+        return e == hipErrorOutOfMemory && release() ? hipMalloc(p, bytes) : e;
+    }
+    // nothing queued may use the buffer any more
+    void give(void* p, size_t bytes, int device)
+    {
+        std::vector<Idle> drop;
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            idle.push_back({ p, bytes, device });
+            held += bytes;
+            while (idle.size() > kTempKeep || held > kTempKeepBytes) {
+                drop.push_back(idle.front());
+                held -= idle.front().bytes;
+                idle.erase(idle.begin());
+            }
+        }
+        for (const Idle& d : drop) (void)hipFree(d.p);
+    }
+    // frees every idle buffer; false if there was none
+    bool release()
+    {
+        std::vector<Idle> drop;
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            drop.swap(idle);
+            held = 0;
+        }
+        for (const Idle& d : drop) (void)hipFree(d.p);
+        return !drop.empty();
+    }
+};
+
+TempPool& tempPool()
+{
+    static TempPool* pool = new TempPool;
+    return *pool;
+}
+
+struct StreamPool {
+    std::mutex mu;
+    std::vector<std::pair<hipStream_t, int>> idle;
+
+    // a non-blocking stream of the device, which must be the current one
+    hipError_t take(int device, hipStream_t* s)
+    {
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            for (size_t i = 0; i < idle.size(); ++i)
+                if (idle[i].second == device) {
+                    *s = idle[i].first;
+                    idle.erase(idle.begin() + (ptrdiff_t)i);
+                    return hipSuccess;
+                }
+        }
+        return hipStreamCreateWithFlags(s, hipStreamNonBlocking);
+    }
+    void give(hipStream_t s, int device)
+    {
+        if (!s) return;
+        if (hipStreamSynchronize(s) == hipSuccess) {
+            std::lock_guard<std::mutex> lk(mu);
+            if (idle.size() < kStreamKeep) {
+                idle.emplace_back(s, device);
+                return;
+            }
+        }
+        (void)hipStreamDestroy(s);
+    }
+};
+
+StreamPool& streamPool()
+{
+    static StreamPool* pool = new StreamPool;
+    return *pool;
+}
+
 // RAII device buffer
 struct DevBuf {
     void* p = nullptr;
@@ -93,7 +204,35 @@ struct DevBuf {
         if (p) { (void)hipFree(p); p = nullptr; bytes = 0; }
         if (b == 0) return hipSuccess;
         hipError_t e = hipMalloc(&p, b);
+        if (e == hipErrorOutOfMemory && tempPool().release()) e = hipMalloc(&p, b);
         if (e == hipSuccess) bytes = b;
+        else p = nullptr;
+        return e;
+    }
+    template <class T> T* as() const { return static_cast<T*>(p); }
+};
+
+// RAII lease of a pooled device buffer that only work queued on `s` uses
+struct TempBuf {
+    void* p = nullptr;
+    size_t bytes = 0;
+    int device = 0;
+    hipStream_t stream = nullptr;
+    TempBuf() = default;
+    TempBuf(const TempBuf&) = delete;
+    TempBuf& operator=(const TempBuf&) = delete;
+    ~TempBuf()
+    {
+        if (!p) return;
+        if (hipStreamSynchronize(stream) == hipSuccess) tempPool().give(p, bytes, device);
+        else (void)hipFree(p);
+    }
+    hipError_t take(size_t b, hipStream_t s)
+    {
+        stream = s;
+        if (b == 0) return hipSuccess;
+        const hipError_t e = tempPool().take(b, &p, &bytes, &device);
+        if (e != hipSuccess) p = nullptr;
         return e;
     }
     template <class T> T* as() const { return static_cast<T*>(p); }
@@ -257,7 +396,7 @@ struct mi_mesh {
     // the mesh's own settings (MI_MODE_*), MI_MODE_DEFAULT = follow the process-wide setting
     std::atomic<int32_t> modes[MI_MODE_COUNT] = { MI_MODE_DEFAULT, MI_MODE_DEFAULT, MI_MODE_DEFAULT,
                                                   MI_MODE_DEFAULT };
-    ~mi_mesh() { if (stream) (void)hipStreamDestroy(stream); }
+    ~mi_mesh() { streamPool().give(stream, device); }
 };
 
 namespace {
@@ -454,8 +593,8 @@ int finishArena(mi_mesh* m, const ArenaLayout& L)
     MI_HIP(mi::buildPrisms(m->dev.tri, m->nf,
                            reinterpret_cast<float4*>(base + L.dnode + L.tri + L.dint + L.dleaf + L.dquad + L.cut),
                            m->stream));
-    DevBuf ranges;
-    MI_HIP(ranges.alloc(mi::cylinderScratchBytes(m->nf)));
+    TempBuf ranges;
+    MI_HIP(ranges.take(mi::cylinderScratchBytes(m->nf), m->stream));
     m->dev.numFaces = m->nf;
     m->dev.depth = m->depth;
     MI_HIP(mi::buildCylinders(m->dev, reinterpret_cast<float4*>(base + L.total() - L.cyl), ranges.p, m->stream));
@@ -499,6 +638,13 @@ struct ValidFaces {
 int validFaces(const int32_t* tris, int32_t nf, int32_t nv, ValidFaces& out)
 {
     out = ValidFaces{};
+    // first a pass that the compiler vectorises: as unsigned numbers, negative indices are beyond nv too
+    uint32_t beyond = 0;
+    for (int64_t i = 0; i < 3 * (int64_t)nf; ++i) beyond |= (uint32_t)((uint32_t)tris[i] >= (uint32_t)nv);
+    if (!beyond) {
+        out.count = nf;
+        return MI_OK;
+    }
     int64_t bad = 0, deleted = 0;
     for (int32_t f = 0; f < nf; ++f) {
         const int32_t* t = tris + 3 * (int64_t)f;
@@ -568,17 +714,17 @@ int createDeviceBuilt(mi_mesh* m, const float* verts, const int32_t* tris, const
     MI_HIP(m->arena.alloc(L.total()));
     bindArena(m, L);
     MI_HIP(m->treeDev.alloc(2 * align256(nn * sizeof(mi::TreeNode))));
-    DevBuf dv, dt, scratch, ids;
-    MI_HIP(dv.alloc(std::max<size_t>((size_t)m->nv * 12, 16)));
-    MI_HIP(dt.alloc((size_t)m->nf * 12));
-    MI_HIP(scratch.alloc(mi::deviceTreeScratchBytes(m->nf)));
-    if (m->nv > 0) MI_HIP(hipMemcpyAsync(dv.p, verts, (size_t)m->nv * 12, hipMemcpyHostToDevice, m->stream));
-    MI_HIP(hipMemcpyAsync(dt.p, vf.ids.empty() ? tris : vf.packed.data(), (size_t)m->nf * 12, hipMemcpyHostToDevice,
-                          m->stream));
-    if (!vf.ids.empty()) {
-        MI_HIP(ids.alloc((size_t)m->nf * 4));
-        MI_HIP(hipMemcpyAsync(ids.p, vf.ids.data(), (size_t)m->nf * 4, hipMemcpyHostToDevice, m->stream));
-    }
+    // the mesh arrays, the face ids where some faces are deleted, and the builder's scratch
+    const size_t vBytes = align256(std::max<size_t>((size_t)m->nv * 12, 16)), tBytes = align256((size_t)m->nf * 12);
+    const size_t idBytes = vf.ids.empty() ? 0 : align256((size_t)m->nf * 4), treeBytes = mi::deviceTreeScratchBytes(m->nf);
+    TempBuf temp;
+    MI_HIP(temp.take(vBytes + tBytes + idBytes + treeBytes, m->stream));
+    float* const dv = temp.as<float>();
+    int32_t* const dt = reinterpret_cast<int32_t*>(temp.as<char>() + vBytes);
+    int32_t* const ids = idBytes ? reinterpret_cast<int32_t*>(temp.as<char>() + vBytes + tBytes) : nullptr;
+    if (m->nv > 0) MI_HIP(hipMemcpyAsync(dv, verts, (size_t)m->nv * 12, hipMemcpyHostToDevice, m->stream));
+    MI_HIP(hipMemcpyAsync(dt, idBytes ? vf.packed.data() : tris, (size_t)m->nf * 12, hipMemcpyHostToDevice, m->stream));
+    if (ids) MI_HIP(hipMemcpyAsync(ids, vf.ids.data(), (size_t)m->nf * 4, hipMemcpyHostToDevice, m->stream));
     char* base = m->arena.as<char>();
     mi::DeviceTreeOut o;
     o.nodes = m->treeDev.as<mi::TreeNode>();
@@ -588,8 +734,8 @@ int createDeviceBuilt(mi_mesh* m, const float* verts, const int32_t* tris, const
     o.dint = reinterpret_cast<float4*>(base + L.dnode + L.tri);
     o.dleaf = reinterpret_cast<float4*>(base + L.dnode + L.tri + L.dint);
     mi::DeviceTreeInfo info;
-    MI_HIP(mi::buildDeviceTree(dv.as<float>(), dt.as<int32_t>(), m->nf, scratch.p, scratch.bytes, o, info, m->stream,
-                               ids.as<int32_t>()));
+    MI_HIP(mi::buildDeviceTree(dv, dt, m->nf, temp.as<char>() + vBytes + tBytes + idBytes, treeBytes, o, info, m->stream,
+                               ids));
     m->depth = info.depth;
     m->stackD = mi::stackDepthFor(m->depth);
     if (m->stackD == 0) return fail(MI_E_LIMIT, "tree deeper than 32 levels");
@@ -618,7 +764,8 @@ int mi_mesh_create(const float* verts, int32_t nv, const int32_t* tris, int32_t 
     m->faceSize = nf;
     m->numNodes = vf.count > 0 ? 2 * vf.count - 1 : 0;
     if (hipGetDevice(&m->device) != hipSuccess) { delete m; return fail(MI_E_HIP, "AMD GPU error: no device"); }
-    if (hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking) != hipSuccess) {
+    if (streamPool().take(m->device, &m->stream) != hipSuccess) {
+        m->stream = nullptr;
         delete m;
         return fail(MI_E_HIP, "AMD GPU error: stream creation failed");
     }
@@ -931,17 +1078,19 @@ static int gridLaunch(mi_mesh* m, const int32_t dims[3], const mi::Xf& x, const 
 // streams drain before the second stream and the events are released.
 struct PartStreams {
     hipStream_t st[2] = { nullptr, nullptr };
+    int device = 0;
     std::vector<hipEvent_t> ev;
     ~PartStreams()
     {
         if (st[0]) (void)hipStreamSynchronize(st[0]);
-        if (st[1]) { (void)hipStreamSynchronize(st[1]); (void)hipStreamDestroy(st[1]); }
+        streamPool().give(st[1], device);
         for (hipEvent_t e : ev) if (e) (void)hipEventDestroy(e);
     }
-    hipError_t init(hipStream_t mainStream, size_t events = 0)
+    hipError_t init(const mi_mesh* m, size_t events = 0)
     {
-        st[0] = mainStream;
-        hipError_t e = hipStreamCreateWithFlags(&st[1], hipStreamNonBlocking);
+        st[0] = m->stream;
+        device = m->device;
+        hipError_t e = streamPool().take(device, &st[1]);
         if (e != hipSuccess) { st[1] = nullptr; return e; }
         ev.assign(events, nullptr);
         for (hipEvent_t& x : ev)
@@ -973,13 +1122,14 @@ static int gridHost(mi_mesh* m, const int32_t dims[3], const float xf[12], const
     const size_t part = std::min(budgetLayers, partLayers(layer, nz));
     const size_t nParts = (nz + part - 1) / part;
     const size_t slots = std::min(budgetLayers / part, nParts);
-    DevBuf out, splitBuf;
-    MI_HIP(out.alloc(slots * part * layer * sizeof(float)));
+    DevBuf splitBuf;
+    TempBuf out;      // both streams of `ps` use it; they drain first
+    MI_HIP(out.take(slots * part * layer * sizeof(float), m->stream));
     mi::SplitScratch sc;
     if (opts)
         if (int rc = splitScratch(m, splitBuf, dims, (int32_t)part, sdfLaneBytes(opts), sc)) return rc;
     PartStreams ps;   // st[0] computes, st[1] copies; events: computed / copied per slot
-    MI_HIP(ps.init(m->stream, 2 * slots));
+    MI_HIP(ps.init(m, 2 * slots));
     hipEvent_t* const computed = ps.ev.data();
     hipEvent_t* const copied = ps.ev.data() + slots;
     if (!report(cb, user, 0.6f)) return fail(MI_E_CANCELED, "Operation was canceled");
@@ -1055,17 +1205,18 @@ static int gridByParts(mi_mesh* m, mi_grid_part_fn fn, void* fnUser, const int32
         nChunks = (nz - (size_t)layerOverlap + step - 1) / step;
     }
     const size_t slots = std::min<size_t>(2, nChunks);
-    DevBuf dbuf[2], splitBuf[2];
+    DevBuf splitBuf[2];
+    TempBuf dbuf[2];      // `ps` drains both streams first
     mi::SplitScratch sc[2];
     PinnedBuf hbuf[2];
     for (size_t i = 0; i < slots; ++i) {
-        MI_HIP(dbuf[i].alloc(chunkLayers * layer * sizeof(float)));
+        MI_HIP(dbuf[i].take(chunkLayers * layer * sizeof(float), m->stream));
         MI_HIP(hbuf[i].take(chunkLayers * layer * sizeof(float)));
         if (opts)
             if (int rc = splitScratch(m, splitBuf[i], dims, (int32_t)chunkLayers, sdfLaneBytes(opts), sc[i])) return rc;
     }
     PartStreams ps;
-    MI_HIP(ps.init(m->stream));
+    MI_HIP(ps.init(m));
     if (!report(cb, user, 0.6f)) return fail(MI_E_CANCELED, "Operation was canceled");
     const mi::Xf x = toXf(xf);
     auto chunkRange = [&](size_t c, int32_t& z0, int32_t& z1) {
@@ -1140,21 +1291,25 @@ static int pointsHost(mi_mesh* m, const float* pts, int64_t n, size_t outElem, v
     const size_t part = std::min({ kPartPoints, (size_t)n, std::max<size_t>(1, budget / 2) });
     const size_t nParts = ((size_t)n + part - 1) / part;
     const size_t slots = std::min({ (size_t)2, budget / part, nParts });
+    // a slot's memory: points, results, sort workspace, split scratch
+    const size_t ptBytes = align256(part * 12), resBytes = align256(part * outElem);
+    const size_t wsBytes = align256(mi::sortWorkspaceBytes((int64_t)part));
+    const size_t splitBytes = split ? projSplitBytes(m, (int64_t)part, lo) : 0;
     struct Slot {
-        DevBuf pts, res, ws, split;
+        TempBuf mem;      // `ps` drains both streams first
+        float* pts = nullptr;
+        char *res = nullptr, *ws = nullptr;
         mi::SplitScratch sc;
     } sl[2];
     for (size_t i = 0; i < slots; ++i) {
-        MI_HIP(sl[i].pts.alloc(part * 12));
-        MI_HIP(sl[i].res.alloc(part * outElem));
-        MI_HIP(sl[i].ws.alloc(mi::sortWorkspaceBytes((int64_t)part)));
-        if (split && projSplitBytes(m, (int64_t)part, lo)) {
-            MI_HIP(sl[i].split.alloc(projSplitBytes(m, (int64_t)part, lo)));
-            projSplit(m, sl[i].split.p, (int64_t)part, lo, sl[i].sc);
-        }
+        MI_HIP(sl[i].mem.take(ptBytes + resBytes + wsBytes + splitBytes, m->stream));
+        sl[i].pts = static_cast<float*>(sl[i].mem.p);
+        sl[i].res = static_cast<char*>(sl[i].mem.p) + ptBytes;
+        sl[i].ws = sl[i].res + resBytes;
+        if (splitBytes) projSplit(m, sl[i].ws + wsBytes, (int64_t)part, lo, sl[i].sc);
     }
     PartStreams ps;
-    MI_HIP(ps.init(m->stream));
+    MI_HIP(ps.init(m));
     if (!report(cb, user, 0.6f)) return fail(MI_E_CANCELED, "Operation was canceled");
     auto range = [&](size_t k, size_t& off, size_t& sz) {
         off = k * part;
@@ -1165,12 +1320,10 @@ static int pointsHost(mi_mesh* m, const float* pts, int64_t n, size_t outElem, v
         const hipStream_t st = ps.st[k % slots];
         size_t off, sz;
         range(k, off, sz);
-        MI_HIP(hipMemcpyAsync(s.pts.p, pts + 3 * off, sz * 12, hipMemcpyHostToDevice, st));
-        float* const dp = static_cast<float*>(s.pts.p);
+        MI_HIP(hipMemcpyAsync(s.pts, pts + 3 * off, sz * 12, hipMemcpyHostToDevice, st));
         const uint32_t* perm = nullptr;
-        MI_HIP(mi::sortPointsMorton(dp, (int64_t)sz, m->sortLo, m->sortHi, s.ws.p, s.ws.bytes, &perm, st,
-                                    orderFn(&s.sc)));
-        MI_HIP(launchFn(dp, perm, (int64_t)sz, s.res.p, &s.sc, st));
+        MI_HIP(mi::sortPointsMorton(s.pts, (int64_t)sz, m->sortLo, m->sortHi, s.ws, wsBytes, &perm, st, orderFn(&s.sc)));
+        MI_HIP(launchFn(s.pts, perm, (int64_t)sz, s.res, &s.sc, st));
         return MI_OK;
     };
     for (size_t k = 0; k < slots; ++k)
@@ -1179,7 +1332,7 @@ static int pointsHost(mi_mesh* m, const float* pts, int64_t n, size_t outElem, v
         size_t off, sz;
         range(k, off, sz);
         const hipStream_t st = ps.st[k % slots];
-        MI_HIP(hipMemcpyAsync(static_cast<char*>(res) + off * outElem, sl[k % slots].res.p, sz * outElem,
+        MI_HIP(hipMemcpyAsync(static_cast<char*>(res) + off * outElem, sl[k % slots].res, sz * outElem,
                               hipMemcpyDeviceToHost, st));
         MI_HIP(hipStreamSynchronize(st));
         if (k + slots < nParts)
@@ -1215,8 +1368,8 @@ int mi_fwn_calc_self_intersections(mi_mesh* m, float beta, uint8_t* res, mi_prog
     // one flag per entry of the caller's triangle array; deleted faces stay 0 (the reference sets bits
     // of valid faces only, source/MRMesh/MRFastWindingNumber.cpp:40-52)
     const int words = (int)(((size_t)m->faceSize + 3) / 4);
-    DevBuf out;
-    MI_HIP(out.alloc((size_t)words * 4));
+    TempBuf out;
+    MI_HIP(out.take((size_t)words * 4, m->stream));
     MI_HIP(mi::fillU32(out.as<uint32_t>(), words, 0u, m->stream));
     MI_HIP(mi::launchSelfIntersections(callView(m), beta, out.as<uint8_t>(), m->stackD, m->stream));
     MI_HIP(hipMemcpyAsync(res, out.p, (size_t)m->faceSize, hipMemcpyDeviceToHost, m->stream));
