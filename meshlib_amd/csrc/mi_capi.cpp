@@ -1425,7 +1425,7 @@ struct mi_batch {
     int blocksPerCU = 4;
     int xcdSplit = 1;
     DevBuf items;        // BatchItem[]
-    DevBuf tickets;      // 8 x u64
+    DevBuf tickets;      // a u64 per XCD, each on a line of its own
     DevBuf sortWs;       // per-item Morton sort workspaces
     DevBuf rerunWs;      // capped form: per-item counters of failed caps
     std::vector<mi::BatchItem> host;     // launch order (see prepareBatch)
@@ -1517,7 +1517,7 @@ int launchPrepared(mi_batch* b, int32_t count, int64_t total, int depth, const m
 {
     mi::DistOpts o{ opts->minDistSq, opts->maxDistSq, opts->nullOutsideMinMax, opts->windingNumberThreshold,
                     opts->windingNumberBeta };
-    MI_HIP(mi::fillU32(b->tickets.as<uint32_t>(), 16, 0u, s));
+    MI_HIP(mi::fillU32(b->tickets.as<uint32_t>(), mi::kTicketWords, 0u, s));
     bool wide = false;
     for (const mi::BatchItem& it : b->host) wide = wide || it.m.numFaces > (1 << 23);
     MI_HIP(mi::launchBatch(b->items.as<mi::BatchItem>(), count, total, o, up, b->tickets.as<unsigned long long>(), xcdSplit,
@@ -1544,7 +1544,7 @@ int mi_batch_create(mi_batch** out)
     if (!b) return fail(MI_E_NOMEM, "out of host memory");
     hipDeviceProp_t prop;
     if (hipGetDevice(&b->device) != hipSuccess || hipGetDeviceProperties(&prop, b->device) != hipSuccess ||
-        b->tickets.alloc(16 * sizeof(uint32_t)) != hipSuccess) {
+        b->tickets.alloc(mi::kTicketWords * sizeof(uint32_t)) != hipSuccess) {
         delete b;
         return fail(MI_E_HIP, "AMD GPU error: cannot set up the batch");
     }

@@ -106,9 +106,10 @@ struct BatchItem {
     uint32_t* rerunCount;
 };
 
-// persistent launch over items[0..nItems) (device array); tickets = 8 zeroed 64-bit counters;
-// blocks = number of four-wave groups to keep resident; depth: of the deepest tree; wide: a tree has more than 2^23
-// faces; capped: the items' caps apply
+// persistent launch over items[0..nItems) (device array); tickets: kTicketWords zeroed words; blocks = number of
+// groups of waves to keep resident; depth: of the deepest tree; wide: a tree has more than 2^23 faces; capped: the
+// items' caps apply
+constexpr int kTicketStride = 32, kTicketWords = 2 * 8 * kTicketStride;      // a counter per XCD, 256 bytes apart
 hipError_t launchBatch(const BatchItem* items, int nItems, int64_t totalUnits, const DistOpts& o, float up,
                        unsigned long long* tickets, int xcdSplit, int blocks, int depth, bool wide, bool capped,
                        hipStream_t s);
