@@ -30,25 +30,8 @@ std::atomic<int> g_treeBuilder{ MI_TREE_BUILDER_DEVICE };
 std::atomic<int> g_splitBudget{ MI_SPLIT_AUTO };       // signed-distance walks
 std::atomic<int> g_splitBudgetProj{ MI_SPLIT_AUTO };   // projection walks
 
-// Automatic step budgets of the keyed walks (a band: loDistLimitSq > 0 or minDistSq > 0), from sweeps on
-// MI355X (bumpy spheres of 20 k to 5.2 M triangles, tree depths 15 to 23).  Signed distance on trees of
-// >= 18 levels: 3072 steps below 64 k waves, 6144 below 1 M, none from 1 M waves on (enough waves to spread
-// the long ones); shallower trees walk less, so the 64 subtree items of a hand-over weigh more and an earlier
-// hand-over spreads the few long waves (512 steps below 16 k waves, 1024 above).  Projections: on trees of
-// >= 20 levels nearly every wave is long and 64 steps is best; on shallower trees most waves finish alone
-// given 1-2 k steps.  Without a band the lane walks need no hand-over: automatic is none.
-int autoSdfBudget(int depth, int64_t waves, bool band)
-{
-    if (!band) return 0;
-    if (depth >= 18) return waves < 65536 ? 3072 : waves < (1 << 20) ? 6144 : 0;
-    return waves < 16384 ? 512 : 1024;
-}
-int autoProjBudget(int depth, bool band)
-{
-    if (!band) return 0;
-    if (depth >= 20) return 64;
-    return depth >= 17 ? 2048 : 1024;
-}
+// The lane walks need no hand-over: an automatic step budget is none.
+int stepBudget(int setting) { return setting >= 0 ? setting : 0; }
 
 int fail(int code, const std::string& msg)
 {
@@ -432,14 +415,13 @@ int sdfLaneBytes(const mi_dist_options* o) { return o && o->minDistSq > 0 ? 8 : 
 size_t sdfBytesPerVoxel(const mi_dist_options* o) { return o ? sizeof(float) + sdfLaneBytes(o) + 2 : sizeof(float); }
 
 // waves of a signed-distance launch over `layers` z-layers and the split budget it runs with
-int64_t sdfSplitPlan(const mi_mesh* m, const int32_t dims[3], int32_t layers, bool band, int32_t* budget)
+int64_t sdfSplitPlan(const mi_mesh* m, const int32_t dims[3], int32_t layers, int32_t* budget)
 {
     *budget = 0;
     if (layers <= 0) return 0;
     const int32_t d[3] = { dims[0], dims[1], layers };
     const int64_t waves = mi::sdfGridWaves(d, 0, layers);
-    const int setting = meshMode(m, MI_MODE_SPLIT_SDF, g_splitBudget.load());
-    *budget = setting >= 0 ? setting : autoSdfBudget(m->depth, waves, band);
+    *budget = stepBudget(meshMode(m, MI_MODE_SPLIT_SDF, g_splitBudget.load()));
     return waves;
 }
 
@@ -448,7 +430,7 @@ int splitScratch(mi_mesh* m, DevBuf& buf, const int32_t dims[3], int32_t layers,
 {
     sc = mi::SplitScratch{};
     int32_t budget = 0;
-    const int64_t waves = sdfSplitPlan(m, dims, layers, laneBytes == 8, &budget);
+    const int64_t waves = sdfSplitPlan(m, dims, layers, &budget);
     if (budget <= 0) return MI_OK;
     const size_t bytes = mi::splitScratchBytes(waves, laneBytes);
     if (buf.bytes < bytes) MI_HIP(buf.alloc(bytes));
@@ -456,23 +438,19 @@ int splitScratch(mi_mesh* m, DevBuf& buf, const int32_t dims[3], int32_t layers,
     return MI_OK;
 }
 
-// split scratch of a projection launch over n points with loDistLimitSq `lo`, placed at `base`
-// (caller-sized with projSplitBytes); no split when the budget is 0
-int projBudget(const mi_mesh* m, float lo)
+// split scratch of a projection launch over n points, placed at `base` (caller-sized with projSplitBytes); no split
+// when the budget is 0
+int projBudget(const mi_mesh* m) { return stepBudget(meshMode(m, MI_MODE_SPLIT_PROJECTIONS, g_splitBudgetProj.load())); }
+
+size_t projSplitBytes(const mi_mesh* m, int64_t n)
 {
-    const int setting = meshMode(m, MI_MODE_SPLIT_PROJECTIONS, g_splitBudgetProj.load());
-    return setting >= 0 ? setting : autoProjBudget(m->depth, lo > 0);
+    return projBudget(m) > 0 ? mi::splitScratchBytes(mi::projectionWaves(n), 8) : 0;
 }
 
-size_t projSplitBytes(const mi_mesh* m, int64_t n, float lo)
-{
-    return projBudget(m, lo) > 0 ? mi::splitScratchBytes(mi::projectionWaves(n), 8) : 0;
-}
-
-void projSplit(const mi_mesh* m, void* base, int64_t n, float lo, mi::SplitScratch& sc)
+void projSplit(const mi_mesh* m, void* base, int64_t n, mi::SplitScratch& sc)
 {
     sc = mi::SplitScratch{};
-    const int budget = projBudget(m, lo);
+    const int budget = projBudget(m);
     if (budget <= 0 || !base) return;
     mi::splitScratchBind(base, mi::projectionWaves(n), 8, budget, sc);
 }
@@ -924,15 +902,15 @@ int mi_proj_find_projections_device(mi_mesh* m, const float* d_pts, int64_t n, c
     MI_HIP(hipSetDevice(m->device));
     hipStream_t s = pick(m, stream);
     const size_t sortBytes = align256(mi::sortWorkspaceBytes(n));
-    if (int rc = ensureWorkspace(m, sortBytes + projSplitBytes(m, n, lo))) return rc;
+    if (int rc = ensureWorkspace(m, sortBytes + projSplitBytes(m, n))) return rc;
     mi::SplitScratch sc;
-    projSplit(m, m->ws.as<char>() + sortBytes, n, lo, sc);
+    projSplit(m, m->ws.as<char>() + sortBytes, n, sc);
     mi::Xf px, tx;
     if (ptXf) px = toXf(ptXf);
     if (treeXf) tx = toXf(treeXf);
     const uint32_t* perm = nullptr;
     MI_HIP(mi::sortPointsMorton(d_pts, n, m->sortLo, m->sortHi, m->ws.p, m->ws.bytes, &perm, s,
-                                mi::projectionOrder(callView(m), treeXf ? &tx : nullptr, lo, &sc)));
+                                mi::projectionOrder(callView(m), treeXf ? &tx : nullptr, &sc)));
     MI_HIP(mi::launchProjections(callView(m), d_pts, perm, n, ptXf ? &px : nullptr, treeXf ? &tx : nullptr, up, lo,
                                  reinterpret_cast<mi::ProjRec*>(d_res), m->stackD, s, nullptr, nullptr, &sc));
     return MI_OK;
@@ -953,16 +931,16 @@ int mi_proj_find_projections_noalloc_device(mi_mesh* m, const float* d_pts, int6
     MI_HIP(mi::noAllocScratch(m->device, &scratch));
     // the same workspace layout as mi_proj_find_projections_device, in the fixed scratch
     const size_t sortBytes = align256(mi::sortWorkspaceBytes(n));
-    if (sortBytes + projSplitBytes(m, n, lo) > mi::kNoAllocScratchBytes)
+    if (sortBytes + projSplitBytes(m, n) > mi::kNoAllocScratchBytes)
         return fail(MI_E_LIMIT, "the no-allocation scratch is too small for this call");
     mi::SplitScratch sc;
-    projSplit(m, static_cast<char*>(scratch) + sortBytes, n, lo, sc);
+    projSplit(m, static_cast<char*>(scratch) + sortBytes, n, sc);
     mi::Xf px, tx;
     if (ptXf) px = toXf(ptXf);
     if (treeXf) tx = toXf(treeXf);
     const uint32_t* perm = nullptr;
     MI_HIP(mi::sortPointsMorton(d_pts, n, m->sortLo, m->sortHi, scratch, sortBytes, &perm, s,
-                                mi::projectionOrder(callView(m), treeXf ? &tx : nullptr, lo, &sc)));
+                                mi::projectionOrder(callView(m), treeXf ? &tx : nullptr, &sc)));
     MI_HIP(mi::launchProjections(callView(m), d_pts, perm, n, ptXf ? &px : nullptr, treeXf ? &tx : nullptr, up, lo,
                                  reinterpret_cast<mi::ProjRec*>(d_res), m->stackD, s, nullptr, nullptr, &sc));
     return MI_OK;
@@ -979,15 +957,15 @@ int mi_proj_find_projections_bounded_device(mi_mesh* m, const float* d_pts, int6
     MI_HIP(hipSetDevice(m->device));
     hipStream_t s = pick(m, stream);
     const size_t sortBytes = align256(mi::sortWorkspaceBytes(n));
-    if (int rc = ensureWorkspace(m, sortBytes + projSplitBytes(m, n, lo))) return rc;
+    if (int rc = ensureWorkspace(m, sortBytes + projSplitBytes(m, n))) return rc;
     mi::SplitScratch sc;
-    projSplit(m, m->ws.as<char>() + sortBytes, n, lo, sc);
+    projSplit(m, m->ws.as<char>() + sortBytes, n, sc);
     mi::Xf px, tx;
     if (ptXf) px = toXf(ptXf);
     if (treeXf) tx = toXf(treeXf);
     const uint32_t* perm = nullptr;
     MI_HIP(mi::sortPointsMorton(d_pts, n, m->sortLo, m->sortHi, m->ws.p, m->ws.bytes, &perm, s,
-                                mi::projectionOrder(callView(m), treeXf ? &tx : nullptr, lo, &sc)));
+                                mi::projectionOrder(callView(m), treeXf ? &tx : nullptr, &sc)));
     MI_HIP(mi::launchProjections(callView(m), d_pts, perm, n, ptXf ? &px : nullptr, treeXf ? &tx : nullptr, up, lo,
                                  reinterpret_cast<mi::ProjRec*>(d_res), m->stackD, s, d_upSq, nullptr, &sc));
     return MI_OK;
@@ -1277,7 +1255,7 @@ constexpr size_t kPartPoints = size_t(1) << 21;
 
 template <class OrderFn, class LaunchFn>
 static int pointsHost(mi_mesh* m, const float* pts, int64_t n, size_t outElem, void* res, OrderFn&& orderFn,
-                      LaunchFn&& launchFn, mi_progress_fn cb, void* user, bool split = false, float lo = 0.f)
+                      LaunchFn&& launchFn, mi_progress_fn cb, void* user, bool split = false)
 {
     std::lock_guard<std::mutex> lk(m->mu);
     MI_HIP(hipSetDevice(m->device));
@@ -1294,7 +1272,7 @@ static int pointsHost(mi_mesh* m, const float* pts, int64_t n, size_t outElem, v
     // a slot's memory: points, results, sort workspace, split scratch
     const size_t ptBytes = align256(part * 12), resBytes = align256(part * outElem);
     const size_t wsBytes = align256(mi::sortWorkspaceBytes((int64_t)part));
-    const size_t splitBytes = split ? projSplitBytes(m, (int64_t)part, lo) : 0;
+    const size_t splitBytes = split ? projSplitBytes(m, (int64_t)part) : 0;
     struct Slot {
         TempBuf mem;      // `ps` drains both streams first
         float* pts = nullptr;
@@ -1306,7 +1284,7 @@ static int pointsHost(mi_mesh* m, const float* pts, int64_t n, size_t outElem, v
         sl[i].pts = static_cast<float*>(sl[i].mem.p);
         sl[i].res = static_cast<char*>(sl[i].mem.p) + ptBytes;
         sl[i].ws = sl[i].res + resBytes;
-        if (splitBytes) projSplit(m, sl[i].ws + wsBytes, (int64_t)part, lo, sl[i].sc);
+        if (splitBytes) projSplit(m, sl[i].ws + wsBytes, (int64_t)part, sl[i].sc);
     }
     PartStreams ps;
     MI_HIP(ps.init(m));
@@ -1398,7 +1376,7 @@ int mi_proj_find_projections(mi_mesh* m, const float* pts, int64_t n, const floa
     if (treeXf) tx = toXf(treeXf);
     return pointsHost(m, pts, n, sizeof(mi_projection), res,
                       [&](const mi::SplitScratch* sc) {
-                          return mi::projectionOrder(callView(m), treeXf ? &tx : nullptr, lo, sc);
+                          return mi::projectionOrder(callView(m), treeXf ? &tx : nullptr, sc);
                       },
                       [&](const float* dp, const uint32_t* perm, int64_t sz, void* dr, const mi::SplitScratch* sc,
                           hipStream_t st) {
@@ -1407,7 +1385,7 @@ int mi_proj_find_projections(mi_mesh* m, const float* pts, int64_t n, const floa
                                                        static_cast<mi::ProjRec*>(dr), m->stackD, st,
                                                        nullptr, nullptr, sc);
                       },
-                      nullptr, nullptr, true, lo);
+                      nullptr, nullptr, true);
 }
 
 size_t mi_proj_heap_bytes(size_t numProjections)

@@ -122,7 +122,7 @@ __global__ __launch_bounds__(kBlock) void kSelfIntersections(MeshDev m, int nLog
 // finished wave's LDS goes to the next one at once.  Measured against the wave-cooperative form with hand-over
 // (both with the winding-number sign): k=8 256^3 101 -> 13.4 ms, k=5 64^3 1.48 -> 0.59 ms.  CAPPED: voxels whose cap is below the plain limit and
 // finds nothing walk again without it, counted in failCount.
-template <bool CAPPED, bool WIDE>
+template <bool CAPPED, bool WIDE, bool BAND>
 __global__ __launch_bounds__(64, 4) void kSdfLane(MeshDev m, int dx, int dy, int zBegin, int zEnd, int nbx, int nby, int nbz,
                                                   int nWaves, int perWave, Xf xf, DistOpts o, const float* __restrict__ bound,
                                                   uint32_t* __restrict__ failCount, float* __restrict__ out)
@@ -139,7 +139,7 @@ __global__ __launch_bounds__(64, 4) void kSdfLane(MeshDev m, int dx, int dy, int
     const size_t idx = valid ? ((size_t)(z - zBegin) * dy + y) * dx + x : 0;
     float lim = o.maxDistSq;
     if (CAPPED && valid) { const float b = bound[idx]; lim = b < lim ? b : lim; }
-    float resSq = laneWalk(m, l, px, py, pz, lim, valid, kStatQuadSteps, kStatLeafTests);
+    float resSq = laneWalk<false, WIDE, BAND>(m, l, px, py, pz, lim, valid, kStatQuadSteps, kStatLeafTests, nullptr, o.minDistSq);
     if (CAPPED) {
         const bool again = valid && lim < o.maxDistSq && !(resSq < lim);
         const uint64_t failed = waveBallot(again);
@@ -769,18 +769,18 @@ hipError_t launchSdfGrid(const MeshDev& m, const int32_t dims[3], const Xf& xf, 
     if (bricks <= 0) return hipSuccess;
     const int nLogical = (int)((bricks + 3) / 4);
     if (bound && (o.minDistSq > 0 || !failCount)) return hipErrorInvalidValue;
-    // the lane walk returns the minimum over candidates; with minDistSq > 0 the reference stops at the
-    // first candidate <= minDistSq in its own visit order, which the keyed walk reproduces
-    // (launchSdfGridKeyed; its split scratch holds 8 bytes per lane)
-    if (o.minDistSq > 0 && m.traversal == (int)Traversal::WaveCoop)
-        return launchSdfGridKeyed(m, dims, xf, o, zBegin, zEnd, out, stackD, s, split);
-    if (bound || (m.traversal == (int)Traversal::WaveCoop && !(split && split->list && split->budget > 0 && m.nCut > 0))) {
+    // with minDistSq > 0 the reference stops at the first candidate <= minDistSq in its own visit order
+    const bool band = o.minDistSq > 0, steps = split && split->list && split->budget > 0 && m.nCut > 0;
+    if (band && steps && m.traversal == (int)Traversal::WaveCoop)
+        return launchSdfGridKeyed(m, dims, xf, o, zBegin, zEnd, out, stackD, s, *split);
+    if (bound || (m.traversal == (int)Traversal::WaveCoop && !steps)) {
         const bool wide = laneWide(m.numFaces);
-        const auto kernel = bound ? (wide ? kSdfLane<true, true> : kSdfLane<true, false>)
-                                  : (wide ? kSdfLane<false, true> : kSdfLane<false, false>);
+        const auto kernel = bound ? (wide ? kSdfLane<true, true, false> : kSdfLane<true, false, false>)
+                          : band  ? (wide ? kSdfLane<false, true, true> : kSdfLane<false, false, true>)
+                                  : (wide ? kSdfLane<false, true, false> : kSdfLane<false, false, false>);
         const int perWave = sharedPerWave(64 * bricks, m.numFaces);
         const int nWaves = (int)(bricks * (64 / perWave));
-        hipLaunchKernelGGL(kernel, dim3(chunkedGrid(nWaves, 64)), dim3(64), laneSharedBytes(m.depth, false, wide), s, m, dims[0],
+        hipLaunchKernelGGL(kernel, dim3(chunkedGrid(nWaves, 64)), dim3(64), laneSharedBytes(m.depth, false, wide, band), s, m, dims[0],
                            dims[1], zBegin, zEnd, nbx, nby, nbz, nWaves, perWave, xf, o, bound, failCount, out);
         return hipGetLastError();
     }

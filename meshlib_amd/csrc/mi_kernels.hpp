@@ -163,11 +163,11 @@ hipError_t launchSdfGrid(const MeshDev& m, const int32_t dims[3], const Xf& xf, 
                          int32_t zBegin, int32_t zEnd, float* out, int stackD, hipStream_t s,
                          const float* bound = nullptr, uint32_t* failCount = nullptr,
                          const SplitScratch* split = nullptr);
-// the same with minDistSq > 0 on the keyed walks (the reference's early exit at minDistSq reproduced
-// exactly); split scratch (optional) bound with 8 bytes per lane
+// the same with minDistSq > 0 and a step budget, on the keyed walks (the reference's early exit at minDistSq
+// reproduced by keys); split scratch bound with 8 bytes per lane
 hipError_t launchSdfGridKeyed(const MeshDev& m, const int32_t dims[3], const Xf& xf, const DistOpts& o,
                               int32_t zBegin, int32_t zEnd, float* out, int stackD, hipStream_t s,
-                              const SplitScratch* split);
+                              const SplitScratch& split);
 hipError_t launchFwnGrid(const MeshDev& m, const int32_t dims[3], const Xf& xf, float beta,
                          int32_t zBegin, int32_t zEnd, float* out, int stackD, hipStream_t s);
 // perm may be null (identity order)
@@ -184,7 +184,7 @@ hipError_t launchProjections(const MeshDev& m, const float* pts, const uint32_t*
 // walk shared by a wave
 enum class PointOrder { Lanes, FullWaves, Shared };
 // the order for a projection launch with these arguments
-PointOrder projectionOrder(const MeshDev& m, const Xf* treeXf, float lo, const SplitScratch* split);
+PointOrder projectionOrder(const MeshDev& m, const Xf* treeXf, const SplitScratch* split);
 
 // Spatial ordering of query points by their Morton codes over box [lo, hi].  *permOut: indices in the workspace,
 // or null where the given order serves.  The workspace's layout is private.

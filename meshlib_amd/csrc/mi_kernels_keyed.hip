@@ -111,16 +111,16 @@ __device__ __forceinline__ int keyLeaf(const MeshDev& m, uint32_t key, float px,
 
 // ---------------------------------------------------------------- projections
 
-// The lane form (loDistLimitSq <= 0): every query walks for itself (laneWalk).  Measured against the
+// The lane form: every query walks for itself (laneWalk).  Measured against the
 // wave-cooperative form with hand-over: 2^22 points on 1.3 M triangles 66 -> 3.8 ms, 300 k ICP samples on
 // 328 k triangles 1.09 -> 0.36 ms, 1000 points on 20 k triangles 1.09 -> 0.15 ms.  bound (optional, indexed like
 // the output): a limit per query below `up`.  CAPPED: the bound is a guess; queries that find nothing below a
 // cap smaller than `up` walk again without it, counted in failCount (any cap above the true distance gives the
 // reference's record, so the combination is exact).
-template <bool CAPPED, bool WIDE>
+template <bool CAPPED, bool WIDE, bool BAND>
 __global__ __launch_bounds__(64, 4) void kProjectionsLane(MeshDev m, const float* __restrict__ pts,
                                                           const uint32_t* __restrict__ perm, int64_t n, int nWaves, Xf ptXf,
-                                                          int hasPtXf, float up, const float* __restrict__ bound,
+                                                          int hasPtXf, float up, float lo, const float* __restrict__ bound,
                                                           uint32_t* __restrict__ failCount, ProjRec* __restrict__ out,
                                                           int perWave)
 {
@@ -134,7 +134,7 @@ __global__ __launch_bounds__(64, 4) void kProjectionsLane(MeshDev m, const float
     const bool valid = projQuery(pts, perm, n, ptXf, hasPtXf, up, bound, (uint32_t)wv, lane, q, px, py, pz, lim,
                                  perWave);
     int leaf = -1;
-    float d = laneWalk(m, l, px, py, pz, lim, valid, kStatKeyedSteps, kStatKeyedTests, &leaf);
+    float d = laneWalk<true, WIDE, BAND>(m, l, px, py, pz, lim, valid, kStatKeyedSteps, kStatKeyedTests, &leaf, lo);
     if (CAPPED) {
         const bool again = valid && leaf < 0 && lim < up;
         const uint64_t failed = waveBallot(again);
@@ -168,7 +168,7 @@ __global__ __launch_bounds__(kBlock) void kProjectionsCoop(MeshDev m, const floa
     BestHit h;
     uint32_t key = 0;
     bool stopped = false;
-    coopProject<D>(m, px, py, pz, lim, valid, &stkMem[w], h, &key, sc.list ? sc.budget : 0, &stopped, lo);
+    coopProject<D>(m, px, py, pz, lim, valid, &stkMem[w], h, &key, sc.budget, &stopped, lo);
     if (stopped) {
         handOver(m, sc, wv, valid, px, py, pz, h.distSq, key);
         return;
@@ -282,7 +282,7 @@ __global__ __launch_bounds__(kBlock) void kSdfBandGrid(MeshDev m, BrickSource sr
     BestHit h;
     uint32_t key = 0;
     bool stopped = false;
-    coopProject<D>(m, px, py, pz, lim, valid, &stkMem[w], h, &key, sc.list ? sc.budget : 0, &stopped, src.lo);
+    coopProject<D>(m, px, py, pz, lim, valid, &stkMem[w], h, &key, sc.budget, &stopped, src.lo);
     if (stopped) {
         handOver(m, sc, brick, valid, px, py, pz, h.distSq, key);
         return;
@@ -325,12 +325,10 @@ namespace {
 bool stepsSet(const MeshDev& m, const SplitScratch* split) { return split && split->list && split->budget > 0 && m.nCut > 0; }
 } // namespace
 
-// lo > 0: the record depends on the reference's visit order, which the keyed walk reproduces; a step
-// budget asks for the wave-cooperative form; a non-rigid tree transform (applied per box) keeps the
-// per-lane form
-PointOrder projectionOrder(const MeshDev& m, const Xf* treeXf, float lo, const SplitScratch* split)
+// a step budget asks for the wave-cooperative form; a non-rigid tree transform (applied per box) keeps the per-lane form
+PointOrder projectionOrder(const MeshDev& m, const Xf* treeXf, const SplitScratch* split)
 {
-    const bool lanes = !treeXf && m.traversal == (int)Traversal::WaveCoop && !(lo > 0) && !stepsSet(m, split);
+    const bool lanes = !treeXf && m.traversal == (int)Traversal::WaveCoop && !stepsSet(m, split);
     return lanes ? PointOrder::Lanes : PointOrder::Shared;
 }
 
@@ -346,19 +344,19 @@ hipError_t launchProjections(const MeshDev& m, const float* pts, const uint32_t*
     if (treeXf) tx = *treeXf;
     if (failCount && (treeXf || !bound || lo > 0)) return hipErrorInvalidValue;
     const bool coop = !treeXf && m.traversal == (int)Traversal::WaveCoop;
-    const bool steps = stepsSet(m, split);
-    if (failCount || projectionOrder(m, treeXf, lo, split) == PointOrder::Lanes) {
+    if (failCount || projectionOrder(m, treeXf, split) == PointOrder::Lanes) {
         const int perWave = lanePerWave(n);
         const int nWaves = (int)((n + perWave - 1) / perWave);
-        const bool wide = laneWide(m.numFaces);
-        const auto kernel = failCount ? (wide ? kProjectionsLane<true, true> : kProjectionsLane<true, false>)
-                                      : (wide ? kProjectionsLane<false, true> : kProjectionsLane<false, false>);
-        hipLaunchKernelGGL(kernel, dim3(paddedGrid(nWaves)), dim3(64), laneSharedBytes(m.depth, true, wide), s, m, pts, perm, n,
-                           nWaves, px, ptXf ? 1 : 0, up, bound, failCount, out, perWave);
+        const bool wide = laneWide(m.numFaces), band = lo > 0;
+        const auto kernel = failCount ? (wide ? kProjectionsLane<true, true, false> : kProjectionsLane<true, false, false>)
+                          : band      ? (wide ? kProjectionsLane<false, true, true> : kProjectionsLane<false, false, true>)
+                                      : (wide ? kProjectionsLane<false, true, false> : kProjectionsLane<false, false, false>);
+        hipLaunchKernelGGL(kernel, dim3(paddedGrid(nWaves)), dim3(64), laneSharedBytes(m.depth, true, wide, band), s, m, pts, perm,
+                           n, nWaves, px, ptXf ? 1 : 0, up, lo, bound, failCount, out, perWave);
         return hipGetLastError();
     }
     SplitScratch sc;
-    if (coop && steps) {
+    if (coop) {
         if ((int64_t)split->cap < projectionWaves(n)) return hipErrorInvalidValue;
         sc = *split;
         hipError_t e = fillU32(sc.counters, 3, 0u, s);
@@ -369,13 +367,10 @@ hipError_t launchProjections(const MeshDev& m, const float* pts, const uint32_t*
         if (coop) {
             hipLaunchKernelGGL(kProjectionsCoop<D>, dim3(paddedGrid(nLogical)), dim3(kBlock), 0, s, m, pts, perm, n,
                                nLogical, px, ptXf ? 1 : 0, up, lo, bound, sc, out);
-            if (sc.list) {
-                const PointSource src{ pts, perm, n, px, ptXf ? 1 : 0, up, lo, bound };
-                const int blocks = persistentBlocks();
-                hipLaunchKernelGGL((kKeyedSplit<D, PointSource>), dim3(blocks), dim3(kBlock), 0, s, statLaunch(m, 1),
-                                   src, sc);
-                hipLaunchKernelGGL(kProjSplitFinish<D>, dim3(blocks), dim3(kBlock), 0, s, statLaunch(m, 2), src, sc, out);
-            }
+            const PointSource src{ pts, perm, n, px, ptXf ? 1 : 0, up, lo, bound };
+            const int blocks = persistentBlocks();
+            hipLaunchKernelGGL((kKeyedSplit<D, PointSource>), dim3(blocks), dim3(kBlock), 0, s, statLaunch(m, 1), src, sc);
+            hipLaunchKernelGGL(kProjSplitFinish<D>, dim3(blocks), dim3(kBlock), 0, s, statLaunch(m, 2), src, sc, out);
         } else if (treeXf)
             hipLaunchKernelGGL((kProjections<true, D>), dim3(paddedGrid(nLogical)), dim3(kBlock), 0, s,
                                m, pts, perm, n, nLogical, px, ptXf ? 1 : 0, tx, up, lo, bound, out);
@@ -388,30 +383,23 @@ hipError_t launchProjections(const MeshDev& m, const float* pts, const uint32_t*
 
 hipError_t launchSdfGridKeyed(const MeshDev& m, const int32_t dims[3], const Xf& xf, const DistOpts& o,
                               int32_t zBegin, int32_t zEnd, float* out, int stackD, hipStream_t s,
-                              const SplitScratch* split)
+                              const SplitScratch& sc)
 {
     const int nbx = (dims[0] + 3) / 4, nby = (dims[1] + 3) / 4, nbz = (zEnd - zBegin + 3) / 4;
     const int64_t bricks = (int64_t)nbx * nby * nbz;
     if (bricks <= 0) return hipSuccess;
     const int nLogical = (int)((bricks + 3) / 4);
-    SplitScratch sc;
-    if (split && split->list && split->budget > 0 && m.nCut > 0) {
-        if ((int64_t)split->cap < sdfGridWaves(dims, zBegin, zEnd)) return hipErrorInvalidValue;
-        sc = *split;
-        hipError_t e = fillU32(sc.counters, 3, 0u, s);
-        if (e != hipSuccess) return e;
-    }
+    if ((int64_t)sc.cap < sdfGridWaves(dims, zBegin, zEnd)) return hipErrorInvalidValue;
+    const hipError_t e = fillU32(sc.counters, 3, 0u, s);
+    if (e != hipSuccess) return e;
     const BrickSource src{ dims[0], dims[1], zBegin, zEnd, nbx, nby, nbz, xf, o.maxDistSq, o.minDistSq };
     return dispatchDepth(stackD, [&](auto Dc) {
         constexpr int D = decltype(Dc)::value;
         hipLaunchKernelGGL(kSdfBandGrid<D>, dim3(chunkedGrid(nLogical, kGridChunk)), dim3(kBlock), 0, s, m, src, nLogical, o, sc,
                            out);
-        if (sc.list) {
-            const int blocks = persistentBlocks();
-            hipLaunchKernelGGL((kKeyedSplit<D, BrickSource>), dim3(blocks), dim3(kBlock), 0, s, statLaunch(m, 1), src,
-                               sc);
-            hipLaunchKernelGGL(kSdfBandFinish, dim3(blocks), dim3(kBlock), 0, s, statLaunch(m, 2), src, o, sc, out);
-        }
+        const int blocks = persistentBlocks();
+        hipLaunchKernelGGL((kKeyedSplit<D, BrickSource>), dim3(blocks), dim3(kBlock), 0, s, statLaunch(m, 1), src, sc);
+        hipLaunchKernelGGL(kSdfBandFinish, dim3(blocks), dim3(kBlock), 0, s, statLaunch(m, 2), src, o, sc, out);
         return hipGetLastError();
     });
 }

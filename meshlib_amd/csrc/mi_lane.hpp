@@ -53,10 +53,11 @@ struct LaneTies {
 };
 constexpr int32_t kNarrowFaces = 1 << 23;      // refs of at most 24 bits with sign
 inline bool laneWide(int32_t numFaces) { return numFaces > kNarrowFaces; }
-inline size_t laneSharedBytes(int depth, bool ties, bool wide)
+// band: firstWithin's stack takes the place of the walk's
+inline size_t laneSharedBytes(int depth, bool ties, bool wide, bool band = false)
 {
     const size_t d = depth > 0 ? (size_t)depth : 1;
-    return sizeof(LaneShared) + (ties ? sizeof(LaneTies) : 0) + d * 64 * (wide ? 6 : 5);
+    return sizeof(LaneShared) + (ties ? sizeof(LaneTies) : 0) + d * 64 * (band ? 8 : wide ? 6 : 5);
 }
 
 // the wave's view of its LDS
@@ -75,6 +76,7 @@ struct LaneLds {
         word = reinterpret_cast<uint32_t*>(stack);
         rest = stack + (size_t)(depth > 0 ? depth : 1) * 256;
     }
+    __device__ __forceinline__ int2* band() const { return reinterpret_cast<int2*>(word); }
     // entry at = 64 * index + lane; the bound is stored as its top 16 bits
     __device__ __forceinline__ void put(int at, int ref, float bound) const
     {
@@ -205,6 +207,46 @@ __device__ __forceinline__ int flushLane(const MeshDev& m, const LaneLds<TIES, W
     return base;
 }
 
+// The reference's walk with a low limit (source/MRMesh/MRMeshProject.cpp:13-103) for one lane: depth-first, nearer box
+// first, ending at the first leaf at most `lo` away.  Returns that distance and leaf, or the least ones.
+__device__ __forceinline__ float firstWithin(const MeshDev& m, int2* stack, float px, float py, float pz, float up, float lo,
+                                             int& leaf)
+{
+    const int lane = threadIdx.x & 63;
+    float best = up;
+    leaf = -1;
+    int cur = m.rootRef, sp = 0;
+    bool have = boxDistSq(m.rootMin[0], m.rootMin[1], m.rootMin[2], m.rootMax[0], m.rootMax[1], m.rootMax[2], px, py, pz) < best;
+    for (;;) {
+        if (!have) {
+            if (sp == 0) break;
+            const int2 e = stack[64 * --sp + lane];
+            cur = e.x;
+            if (__int_as_float(e.y) >= best) continue;
+        }
+        have = false;
+        if (cur < 0) {
+            const float d = leafDistSq(loadLeafLanes(m.tri, ~cur), px, py, pz);
+            if (d < best) {
+                best = d;
+                leaf = ~cur;
+                if (d <= lo) break;
+            }
+            continue;
+        }
+        const size_t rec = 4 * (size_t)cur;
+        const float4 n0 = gload(m.dnode, rec), n1 = gload(m.dnode, rec + 1), n2 = gload(m.dnode, rec + 2), n3 = gload(m.dnode, rec + 3);
+        const float d1 = boxDistSq(n0.x, n0.y, n0.z, n0.w, n1.x, n1.y, px, py, pz);
+        const float d2 = boxDistSq(n1.z, n1.w, n2.x, n2.y, n2.z, n2.w, px, py, pz);
+        const bool leftNear = d1 < d2;
+        const int l = __float_as_int(n3.x), r = __float_as_int(n3.y);
+        const float dn = leftNear ? d1 : d2, df = leftNear ? d2 : d1;
+        if (df < best) stack[64 * sp++ + lane] = make_int2(leftNear ? r : l, __float_as_int(df));
+        if (dn < best) { cur = leftNear ? l : r; have = true; }
+    }
+    return best;
+}
+
 // Walks every lane's query for the leaves nearer than `up` (squared); lanes with walk = false only help.
 // Returns the lane's least squared distance, or `up` where nothing is nearer.
 // TIES: *leaf = the leaf that the reference's walk would return (the first in the query's own order among
@@ -222,9 +264,15 @@ __device__ __forceinline__ int flushLane(const MeshDev& m, const LaneLds<TIES, W
 // step; a lane that has no internal node by then sits out that step, where a loop until every lane had one
 // issued about 190 vector instructions a step.  With the loop and with rounds of 1 / 2 / 3 entries: 2^22
 // points 2.95 -> 2.39 / 2.33 / 2.53 ms, 256^3 11.1 -> 9.19 / 9.13 / 9.51 ms, 1,000 points 97 -> 71 / 75 / 77 us.
-template <bool TIES, bool WIDE>
+//
+// BAND: a query with a leaf at most `lo` away ends there and is answered by firstWithin, whose result depends on the
+// reference's order of visits (a query without one has its least distance in any order).  Its stack (8 bytes an
+// entry) costs a third of the waves, so only launches with a low limit have it.  Against the wave-cooperative walk
+// that carries the order as keys: a band of 1.5 to 4.5 voxels in 190^3 around 1.3 M triangles 6.4 -> 1.4 ms, 48^3
+// 14.1 -> 0.34; 300 k projections there with a limit of 0.03 36 -> 0.77, on 20 k triangles 1.9 -> 0.22 ms.
+template <bool TIES, bool WIDE, bool BAND = false>
 __device__ __forceinline__ float laneWalk(const MeshDev& m, const LaneLds<TIES, WIDE>& l, float qx, float qy, float qz, float up,
-                                          bool walk, int statSteps, int statTests, int* leaf = nullptr)
+                                          bool walk, int statSteps, int statTests, int* leaf = nullptr, float lo = 0.f)
 {
     const int lane = threadIdx.x & 63;
     float px = qx, py = qy, pz = qz;
@@ -269,7 +317,9 @@ __device__ __forceinline__ float laneWalk(const MeshDev& m, const LaneLds<TIES, 
             if (!qn) break;
             nTest += (uint32_t)(qn < 64 ? qn : 64);
             qn = flushLane(m, l, qx, qy, qz, qn);
-            limit = laneLimit(__uint_as_float(l.s->best[own]));
+            const float b = __uint_as_float(l.s->best[own]);
+            limit = laneLimit(b);
+            if (BAND && b < __shfl(up, own) && b <= lo) limit = -1.f;
         }
         if (walking <= kTakeBelow) {
             const bool gives = sp - base > (cur == kNoNode ? 1 : 0);
@@ -338,6 +388,12 @@ __device__ __forceinline__ float laneWalk(const MeshDev& m, const LaneLds<TIES, 
     waveSync();
     const uint32_t b = l.s->best[lane];
     const bool found = b < upBits;
+    if (BAND && found && __uint_as_float(b) <= lo) {
+        int at;
+        const float d = firstWithin(m, l.band(), qx, qy, qz, up, lo, at);
+        if (TIES) *leaf = at;
+        return d;
+    }
     if (TIES) {
         *leaf = -1;
         if (found) {
