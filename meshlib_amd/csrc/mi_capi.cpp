@@ -575,6 +575,7 @@ int finishArena(mi_mesh* m, const ArenaLayout& L)
     MI_HIP(ranges.take(mi::cylinderScratchBytes(m->nf), m->stream));
     m->dev.numFaces = m->nf;
     m->dev.depth = m->depth;
+    m->dev.cylUnit = mi::cylinderUnit(m->dev.rootMin, m->dev.rootMax);
     MI_HIP(mi::buildCylinders(m->dev, reinterpret_cast<float4*>(base + L.total() - L.cyl), ranges.p, m->stream));
     char* cutBase = base + L.dnode + L.tri + L.dint + L.dleaf + L.dquad;
     mi::CutEntry* cut = reinterpret_cast<mi::CutEntry*>(cutBase);

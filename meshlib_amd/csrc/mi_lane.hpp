@@ -101,9 +101,9 @@ struct LaneLds {
 };
 
 // Squared distance from the point to a child's cylinder, a lower bound of its triangles' distances up to
-// the rounding that kBoundSlack covers; capped at FLT_MAX so that an overflow never hides a subtree from a
-// search without a finite best.  a = (c, n.x), b = (n.y, n.z, t and r as bf16, ref).  centerSq: to the centre.
-__device__ __forceinline__ float cylinderDistSq(const float4& a, const float4& b, float px, float py, float pz,
+// the rounding that kBoundSlack covers.  a = (c, n.x), b = (n.y, n.z, t and r as halves in units of `unit`, ref).
+// centerSq: to the centre.
+__device__ __forceinline__ float cylinderDistSq(const float4& a, const float4& b, float unit, float px, float py, float pz,
                                                 float& centerSq)
 {
     const float yx = px - a.x, yy = py - a.y, yz = pz - a.z;
@@ -112,9 +112,10 @@ __device__ __forceinline__ float cylinderDistSq(const float4& a, const float4& b
     const float rr = __builtin_fmaf(vz, vz, __builtin_fmaf(vy, vy, vx * vx));
     const float rho = __builtin_amdgcn_sqrtf(rr);
     centerSq = __builtin_fmaf(h, h, rr);
-    const uint32_t tr = __float_as_uint(b.z);
-    const float s = fmaxf(fabsf(h) - __uint_as_float(tr & 0xffff0000u), 0.f);
-    const float q = fmaxf(rho - __uint_as_float(tr << 16), 0.f);
+    typedef _Float16 half2 __attribute__((ext_vector_type(2)));
+    const half2 tr = __builtin_bit_cast(half2, b.z);      // one mixed-precision fma each
+    const float s = fmaxf(__builtin_fmaf(-(float)tr.y, unit, fabsf(h)), 0.f);
+    const float q = fmaxf(__builtin_fmaf(-(float)tr.x, unit, rho), 0.f);
     return __builtin_fmaf(s, s, q * q);
 }
 
@@ -275,6 +276,7 @@ __device__ __forceinline__ float laneWalk(const MeshDev& m, const LaneLds<TIES, 
                                           bool walk, int statSteps, int statTests, int* leaf = nullptr, float lo = 0.f)
 {
     const int lane = threadIdx.x & 63;
+    const float unit = m.cylUnit;
     float px = qx, py = qy, pz = qz;
     int own = lane, cur = kNoNode, base = 0, sp = 0, qn = 0;      // pending: entries base .. sp - 1
     uint32_t nStep = 0, nVisit = 0, nTest = 0;      // measurement counts
@@ -366,7 +368,8 @@ __device__ __forceinline__ float laneWalk(const MeshDev& m, const LaneLds<TIES, 
                 a0 = gload(m.cyl, rec); b0 = gload(m.cyl, rec + 1); a1 = gload(m.cyl, rec + 2); b1 = gload(m.cyl, rec + 3);
             }
             float c0, c1;
-            const float d0 = cylinderDistSq(a0, b0, px, py, pz, c0), d1 = cylinderDistSq(a1, b1, px, py, pz, c1);
+            const float d0 = cylinderDistSq(a0, b0, unit, px, py, pz, c0);
+            const float d1 = cylinderDistSq(a1, b1, unit, px, py, pz, c1);
             const int r0 = __float_as_int(b0.w), r1 = __float_as_int(b1.w);
             // the child with the nearer centre first: while both bounds still hold the point (or nearly), they
             // say little, the centres say on which side the surface is nearer.  Against the nearer bound first:

@@ -4,8 +4,10 @@
 // moved along n to the middle of its vertices' range; t = half that range, r = the largest distance of a
 // vertex from the axis.  Every vertex lies inside, hence every triangle.
 //
-// The record of internal node j is 64 bytes, 32 per child: (c, n.x), (n.y, n.z, t and r as two bf16, ref).
-// t and r are widened before they are rounded up to bf16:
+// The record of internal node j is 64 bytes, 32 per child: (c, n.x), (n.y, n.z, t and r as two halves, ref).  The
+// halves count in units of MeshDev::cylUnit, a 2^15th of the mesh's diagonal rounded up to a power of two: 11 bits
+// instead of bf16's 8, and a mixed-precision fma reads them as they are.
+// t and r are widened before they are rounded up:
 //  * 1.4 * 2^-23 * M, M the largest coordinate of a vertex: the leaf test rounds its closest point to
 //    float (half a unit of 2^-23 per coordinate, hence at most sqrt(3) / 2 of it in length), the rest is
 //    for the rounding of c and of the vertices' offsets from it;
@@ -13,8 +15,20 @@
 //    from c, and the part of that offset beyond t and r is covered by the walk's own relative slack.
 #include "mi_walk.hpp"
 
+#include <algorithm>
+#include <cmath>
+
 namespace mi {
 namespace {
+
+// Slivers -- strips and fans of long narrow triangles -- are long along an edge, not flat: a node whose triangles
+// cover less than kRodArea of its box's squared diagonal while its middle leaf's longest edge spans half of the
+// diagonal takes that edge as its axis (a rod), and so does a triangle with less than kRodArea of its longest
+// edge's square (a regular triangle has 0.43, a regular patch about 0.5).  50 k points with discs alone, with rods
+// and with rods and halves: a tube of 60 k strips of 1 : 10,000 10.9 / 1.5 / 0.82 ms, 40 k separate triangles
+// of 1 : 250 0.91 / 0.09 / 0.08.  What rods do not help: 50,000 triangles around one vertex 51 / 38 / 35 ms, where
+// the points nearest to that vertex are equally far from all of them.
+constexpr float kRodArea = 0.1f;
 
 struct Frame { float c[3], n[3]; };
 
@@ -31,6 +45,32 @@ __device__ __forceinline__ Frame nodeFrame(const float mn[3], const float mx[3],
         f.n[0] = x / len; f.n[1] = y / len; f.n[2] = z / len;
     }
     return f;
+}
+
+// the longest edge of a triangle and its squared length
+__device__ __forceinline__ float longestEdge(const Leaf& L, float e[3])
+{
+    const float* v[3] = { L.a, L.b, L.c };
+    float best = -1.f;
+    for (int i = 0; i < 3; ++i) {
+        const float* p = v[i];
+        const float* q = v[(i + 1) % 3];
+        const float x = q[0] - p[0], y = q[1] - p[1], z = q[2] - p[2], l = x * x + y * y + z * z;
+        if (l > best) { best = l; e[0] = x; e[1] = y; e[2] = z; }
+    }
+    return best;
+}
+
+// the frame of an internal node with the dipole (dirArea, area) d and the middle leaf `slot`
+__device__ __forceinline__ Frame innerFrame(const MeshDev& m, const float mn[3], const float mx[3], const float4& d, int slot)
+{
+    const float x = mx[0] - mn[0], y = mx[1] - mn[1], z = mx[2] - mn[2], dd = x * x + y * y + z * z;
+    if (d.w < kRodArea * dd) {
+        float e[3];
+        const float l = longestEdge(loadLeafLanes(m.tri, slot), e);
+        if (l >= 0.25f * dd && l < INFINITY) return nodeFrame(mn, mx, e[0], e[1], e[2]);
+    }
+    return nodeFrame(mn, mx, d.x, d.y, d.z);
 }
 
 // offset of a vertex along the axis and its squared distance from it
@@ -53,8 +93,8 @@ __device__ __forceinline__ float unordered(uint32_t u)
     return __uint_as_float((u & 0x80000000u) ? (u & 0x7fffffffu) : ~u);
 }
 
-// per internal node: ordered(max h), ordered(max -h), bits of max rr
-struct Range { uint32_t hi, lo, rr, pad; };
+// per internal node: ordered(max h), ordered(max -h), bits of max rr, its middle leaf
+struct Range { uint32_t hi, lo, rr, middle; };
 
 // Every leaf goes down its own path and adds its corners to each node on it: neighbours share most of the path,
 // so equal nodes are reduced within the wave, and a node that holds the whole block within the block, before
@@ -84,7 +124,9 @@ __global__ __launch_bounds__(kRangeThreads) void kCylinderRanges(MeshDev m, Rang
             num = right ? num - h : h;
             if (child >= 0) {
                 const float4 d = m.dint[2 * (size_t)child + 1];
-                const Frame f = nodeFrame(mn, mx, d.x, d.y, d.z);
+                const int middle = first + (num >> 1);
+                if (slot == middle) range[child].middle = (uint32_t)middle;
+                const Frame f = innerFrame(m, mn, mx, d, middle);
                 const float* v[3] = { L.a, L.b, L.c };
                 for (int i = 0; i < 3; ++i) {
                     float a, b;
@@ -128,26 +170,28 @@ __global__ __launch_bounds__(kRangeThreads) void kCylinderRanges(MeshDev m, Rang
     }
 }
 
-// the smallest bf16 not below x (x >= 0; infinity and NaN give infinity), in the upper half
-__device__ __forceinline__ uint32_t bf16Up(float x)
+// the smallest half not below x (x >= 0; infinity and NaN give infinity)
+__device__ __forceinline__ uint32_t halfUp(float x)
 {
-    if (!(x < INFINITY)) return 0x7f800000u;
-    return (__float_as_uint(x) + 0xffffu) & 0xffff0000u;
+    if (!(x <= 65504.f)) return 0x7c00u;
+    const _Float16 h = (_Float16)x;
+    const uint32_t b = __builtin_bit_cast(uint16_t, h);
+    return (float)h < x ? b + 1u : b;
 }
 
 __device__ __forceinline__ void putCylinder(float4* out, const float c[3], const float n[3], float t, float r, float big,
-                                            int ref)
+                                            float unit, int ref)
 {
     const float wide = big * 0x1.4p-23f + (t + r) * 0x1p-19f;
     bool ok = big < INFINITY && t < INFINITY && r < INFINITY;
     for (int i = 0; i < 3; ++i) ok = ok && fabsf(c[i]) < INFINITY && fabsf(n[i]) < 2.f;
-    const uint32_t tr = ok ? bf16Up(t + wide) | (bf16Up(r + wide) >> 16) : 0x7f807f80u;
+    // a quotient below the normal range is rounded to a multiple of 2^-149, far below the widening
+    const uint32_t tr = ok ? (halfUp((t + wide) / unit) << 16) | halfUp((r + wide) / unit) : 0x7c007c00u;
     out[0] = make_float4(ok ? c[0] : 0.f, ok ? c[1] : 0.f, ok ? c[2] : 0.f, ok ? n[0] : 1.f);
     out[1] = make_float4(ok ? n[1] : 0.f, ok ? n[2] : 0.f, __uint_as_float(tr), __int_as_float(ref));
 }
 
-// a leaf's cylinder: the triangle's normal and smallest enclosing circle (a degenerate triangle takes the
-// x axis and the middle of its longest edge)
+// a leaf's cylinder: the triangle's normal and smallest enclosing circle, or a sliver's longest edge
 __device__ __forceinline__ void leafCylinder(const MeshDev& m, int slot, float4* out)
 {
     const Leaf L = loadLeafLanes(m.tri, slot);
@@ -180,6 +224,9 @@ __device__ __forceinline__ void leafCylinder(const MeshDev& m, int slot, float4*
         if (!(v[0][k] - v[0][k] == 0) || !(v[1][k] - v[1][k] == 0) || !(v[2][k] - v[2][k] == 0)) big = INFINITY;
     }
     Frame f = nodeFrame(c, c, nx, ny, nz);
+    float edge[3];
+    const float l = longestEdge(L, edge);
+    if (0.5f * sqrtf(nx * nx + ny * ny + nz * nz) < kRodArea * l) f = nodeFrame(c, c, edge[0], edge[1], edge[2]);
     for (int k = 0; k < 3; ++k) f.c[k] = c[k];
     float t = 0.f, rr = 0.f;
     for (int i = 0; i < 3; ++i) {
@@ -188,7 +235,7 @@ __device__ __forceinline__ void leafCylinder(const MeshDev& m, int slot, float4*
         t = fmaxf(t, fabsf(h));
         rr = fmaxf(rr, q);
     }
-    putCylinder(out, f.c, f.n, t, sqrtf(rr), big, ~slot);
+    putCylinder(out, f.c, f.n, t, sqrtf(rr), big, m.cylUnit, ~slot);
 }
 
 __global__ __launch_bounds__(kBlock) void kCylinderRecords(MeshDev m, const Range* __restrict__ range, float4* __restrict__ cyl)
@@ -208,7 +255,7 @@ __global__ __launch_bounds__(kBlock) void kCylinderRecords(MeshDev m, const Rang
     const float mn[3] = { right ? n1.z : n0.x, right ? n1.w : n0.y, right ? n2.x : n0.z };
     const float mx[3] = { right ? n2.y : n0.w, right ? n2.z : n1.x, right ? n2.w : n1.y };
     const float4 d = m.dint[2 * (size_t)ref + 1];
-    Frame f = nodeFrame(mn, mx, d.x, d.y, d.z);
+    Frame f = innerFrame(m, mn, mx, d, (int)range[ref].middle);
     const float hi = unordered(range[ref].hi), lo = -unordered(range[ref].lo);
     const float mid = 0.5f * hi + 0.5f * lo;
     float big = 0.f;
@@ -216,7 +263,7 @@ __global__ __launch_bounds__(kBlock) void kCylinderRecords(MeshDev m, const Rang
         f.c[k] = f.c[k] + mid * f.n[k];
         big = fmaxf(big, fmaxf(fabsf(mn[k]), fabsf(mx[k])));
     }
-    putCylinder(out, f.c, f.n, 0.5f * hi - 0.5f * lo, sqrtf(__uint_as_float(range[ref].rr)), big, ref);
+    putCylinder(out, f.c, f.n, 0.5f * hi - 0.5f * lo, sqrtf(__uint_as_float(range[ref].rr)), big, m.cylUnit, ref);
 }
 
 __global__ void kRangeInit(Range* r, int n)
@@ -226,6 +273,15 @@ __global__ void kRangeInit(Range* r, int n)
 }
 
 } // namespace
+
+float cylinderUnit(const float rootMin[3], const float rootMax[3])
+{
+    double dd = 0;
+    for (int i = 0; i < 3; ++i) dd += ((double)rootMax[i] - rootMin[i]) * ((double)rootMax[i] - rootMin[i]);
+    const double diag = std::sqrt(dd);
+    if (!(diag > 0) || !(diag < 1e308)) return 1.f;
+    return (float)std::ldexp(1.0, std::max(std::ilogb(diag) + 1 - 15, -126));
+}
 
 size_t cylinderScratchBytes(int32_t numFaces) { return numFaces > 1 ? (size_t)(numFaces - 1) * sizeof(Range) : 0; }
 

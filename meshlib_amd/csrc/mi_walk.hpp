@@ -107,11 +107,12 @@ inline int lanePerWave(int64_t n)
     return per == 1 && n > 2048 ? 2 : per < 32 ? per : 32;
 }
 // Winding numbers and grids, whose winding-number walks are shared by a wave: neighbours' walks overlap the
-// less the finer the mesh, so a large mesh takes up to 8,192 waves (32 a CU), a small one 4,096.  64 and the rule:
+// less the finer the mesh, so a large mesh takes up to 8,192 waves (32 a CU), a small one 2,048.  64 and the rule:
 // 1,000 points 1126 -> 124 us, 65,536 on 82 k triangles 605 -> 399 us, on 1.3 M 1129 -> 494; 32^3 signed
-// distances on 5 k triangles 234 -> 186 us, on 1.3 M 1053 -> 437; 64^3 there 1171 -> 991, but on 5 k 218 -> 291
-// (32 a wave), hence the limit by faces.
-inline int sharedPerWave(int64_t n, int32_t faces) { return perWaveFor(n, faces < 1 << 17 ? 4096 : 8192); }
+// distances on 1.3 M 1053 -> 437; 64^3 there 1171 -> 991, but on 5 k 218 -> 291 (32 a wave), hence the limits by
+// faces.  Below 2^15 faces 4,096 waves are 10 % ahead on a bumpy sphere (32^3 at 20 k: 268 / 311 us) but 25 % behind
+// where every walk opens most leaves (a tube of 20 k strips 26.8 / 21.0 ms).
+inline int sharedPerWave(int64_t n, int32_t faces) { return perWaveFor(n, faces < 1 << 15 ? 2048 : faces < 1 << 17 ? 4096 : 8192); }
 
 // blocks of a persistent launch: enough resident waves to fill every CU
 inline int persistentBlocks()
