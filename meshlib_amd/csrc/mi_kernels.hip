@@ -560,32 +560,28 @@ __global__ void kBuildQuads(const float4* __restrict__ dnode, int32_t ni, float4
 
 // Subtrees at depth kCutDepth (leaves above it stand for themselves), left to right: one thread
 // walks the top of the tree depth-first.
-__global__ void kBuildCut(const float4* __restrict__ dnode, CutEntry root, CutEntry* __restrict__ cut,
-                          int32_t* __restrict__ nCut)
+// One wave: lane k goes down by the bits of k, highest first (1: right), to its subtree at depth kCutDepth or to a
+// leaf above it, which the lane whose further bits are 0 keeps; lane order is left to right.
+__global__ __launch_bounds__(64) void kBuildCut(const float4* __restrict__ dnode, CutEntry root, CutEntry* __restrict__ cut,
+                                                int32_t* __restrict__ nCut)
 {
-    if (threadIdx.x != 0) return;
-    CutEntry stack[kCutDepth + 2];
-    int sp = 0, n = 0;
-    stack[sp++] = root;
-    while (sp > 0) {
-        const CutEntry e = stack[--sp];
-        if (e.ref < 0 || e.depth == kCutDepth) {
-            cut[n++] = e;
-            continue;
-        }
+    static_assert(kMaxCut == 64 && kCutDepth == 6, "one lane per subtree");
+    const int k = threadIdx.x;
+    CutEntry e = root;
+    while (e.ref >= 0 && e.depth < kCutDepth) {
         const float4 n0 = dnode[4 * (size_t)e.ref], n1 = dnode[4 * (size_t)e.ref + 1];
         const float4 n2 = dnode[4 * (size_t)e.ref + 2], n3 = dnode[4 * (size_t)e.ref + 3];
-        CutEntry l = e, r = e;
-        l.ref = __float_as_int(n3.x);
-        r.ref = __float_as_int(n3.y);
-        l.depth = r.depth = e.depth + 1;
-        r.path = e.path | (1u << e.depth);
-        l.mn[0] = n0.x; l.mn[1] = n0.y; l.mn[2] = n0.z; l.mx[0] = n0.w; l.mx[1] = n1.x; l.mx[2] = n1.y;
-        r.mn[0] = n1.z; r.mn[1] = n1.w; r.mn[2] = n2.x; r.mx[0] = n2.y; r.mx[1] = n2.z; r.mx[2] = n2.w;
-        stack[sp++] = r;     // left first out
-        stack[sp++] = l;
+        const bool right = (k >> (kCutDepth - 1 - e.depth)) & 1;
+        e.ref = __float_as_int(right ? n3.y : n3.x);
+        if (right) e.path |= 1u << e.depth;
+        e.mn[0] = right ? n1.z : n0.x; e.mn[1] = right ? n1.w : n0.y; e.mn[2] = right ? n2.x : n0.z;
+        e.mx[0] = right ? n2.y : n0.w; e.mx[1] = right ? n2.z : n1.x; e.mx[2] = right ? n2.w : n1.y;
+        ++e.depth;
     }
-    *nCut = n;
+    const bool keeps = (k & ((1 << (kCutDepth - e.depth)) - 1)) == 0;
+    const uint64_t all = waveBallot(keeps);
+    if (keeps) cut[__popcll(all & ((1ull << k) - 1))] = e;
+    if (k == 0) *nCut = __popcll(all);
 }
 
 __device__ float roundUpF(double x)

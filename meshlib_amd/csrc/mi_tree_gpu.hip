@@ -6,13 +6,13 @@
 // the left set of each node is unique, however it is found; and because every node gives num/2 of its
 // leaves to its left child, the shape of the tree, all node numbers (children root+1 and root+2*half)
 // and all leaf ranges follow from the number of faces alone (nodeAt) -- no level waits for the host.
-//   * nodes of more than kSub leaves are split level by level, several blocks a node: box reduction,
-//     three rounds of radix selection on the first key (histograms of 11, 11 and 10 bits), a block per
-//     node that settles equal first keys by the other keys, partition of the leaves into the two halves;
+//   * nodes of more than kSub leaves are split level by level, several blocks a node: three rounds of radix
+//     selection on the first key (histograms of 11, 11 and 10 bits), a block per node that settles equal
+//     first keys by the other keys, partition of the leaves into the two halves with their boxes;
 //   * nodes of at most kSub leaves are finished by one block each in LDS, all their levels in one launch
 //     (a bitonic sort of each node's leaves per level), dipoles included.
-// Four library radix sorts per level were 1,800 launches for a mesh of 328 k faces, bound by the launches; now 90
-// launches, and creating that mesh from host arrays went from 13.0 to 2.1 ms (1.0 ms of it kernels).
+// Four library radix sorts per level were 1,800 launches for a mesh of 328 k faces, bound by the launches; now 60
+// launches, and creating that mesh from host arrays went from 13.0 to 1.35 ms (0.9 ms of it kernels).
 // Leaf boxes, dipoles (source/MRMesh/MRDipole.cpp:23-71) and the flattened arrays repeat the host
 // builder's float expressions in the same order (the library is compiled with -ffp-contract=off and
 // correctly rounded division and square root), so every record equals the host build bit-for-bit.
@@ -139,6 +139,7 @@ struct Level {
     uint32_t* k0;           // first key of the leaf at each position
     uint32_t* list;         // positions of the leaves left after two rounds, per node from its first
     LevelNode* nodes;
+    LevelNode* next;        // of the next level; null at the last one
     uint32_t* hist;         // 3 * kBins per node
 };
 
@@ -159,61 +160,83 @@ __device__ __forceinline__ void nodeDims(const LevelNode& nd, int sd[3])
     sortedDims(mn, mx, sd);
 }
 
-__global__ void kLevelInit(Level L, int32_t count)
+__device__ __forceinline__ void clearNode(LevelNode& nd)
 {
-    const int64_t t = (int64_t)blockIdx.x * kB + threadIdx.x;
-    if (t < (int64_t)count * 3 * kBins) L.hist[t] = 0u;
-    if (t < count) {
-        LevelNode& nd = L.nodes[t];
-        for (int k = 0; k < 3; ++k) { nd.box[k] = 0xffffffffu; nd.box[3 + k] = 0u; }
-        nd.left = nd.right = nd.listed = 0u;
-    }
+    for (int k = 0; k < 3; ++k) { nd.box[k] = 0xffffffffu; nd.box[3 + k] = 0u; }
+    nd.left = nd.right = nd.listed = 0u;
 }
 
+// what the first level starts from; the later ones are prepared by the level before
+__global__ void kLevelInit(Level L)
+{
+    const int t = blockIdx.x * kB + threadIdx.x;
+    if (t < 3 * kBins) L.hist[t] = 0u;
+    if (t == 0) clearNode(L.nodes[0]);
+}
+
+// the block's sum of every thread's value before its own, and of all
+__device__ __forceinline__ uint32_t scanBlock(uint32_t own, uint32_t& total)
+{
+    __shared__ uint32_t sums[kB / 64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    uint32_t s = own;
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t o = __shfl_up(s, d);
+        if (lane >= d) s += o;
+    }
+    __syncthreads();      // the last call's sums have been read
+    if (lane == 63) sums[w] = s;
+    __syncthreads();
+    uint32_t before = s - own;
+    total = 0;
+    for (int k = 0; k < kB / 64; ++k) {
+        if (k < w) before += sums[k];
+        total += sums[k];
+    }
+    return before;
+}
+
+// the box of the first level's node (the others' come with the partition above them)
 __global__ __launch_bounds__(kB) void kLevelBox(Level L)
 {
     uint32_t i;
     int32_t begin, end;
     blockNode(L, i, begin, end);
     float b[6] = { FLT_MAX, FLT_MAX, FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX };
-    bool any = false;
     for (int32_t p = begin + (int32_t)threadIdx.x; p < end; p += kB) {
         const Elem e = L.src[p];
         const float o[6] = { e.a.x, e.a.y, e.a.z, e.a.w, e.b.x, e.b.y };
         for (int k = 0; k < 3; ++k) { b[k] = fminf(b[k], o[k]); b[k + 3] = fmaxf(b[k + 3], o[k + 3]); }
-        any = true;
     }
     for (int d = 32; d; d >>= 1)
         for (int k = 0; k < 3; ++k) {
             b[k] = fminf(b[k], __shfl_xor(b[k], d));
             b[k + 3] = fmaxf(b[k + 3], __shfl_xor(b[k + 3], d));
         }
-    if ((threadIdx.x & 63) == 0 && any)
-        for (int k = 0; k < 3; ++k) {
-            atomicMin(&L.nodes[i].box[k], ordU(b[k]));
-            atomicMax(&L.nodes[i].box[3 + k], ordU(b[k + 3]));
-        }
+    __shared__ float part[kB / 64][6];
+    if ((threadIdx.x & 63) == 0)
+        for (int k = 0; k < 6; ++k) part[threadIdx.x >> 6][k] = b[k];
+    __syncthreads();
+    if (threadIdx.x >= 6 || begin >= end) return;
+    const int k = threadIdx.x;
+    float x = part[0][k];
+    for (int w = 1; w < kB / 64; ++w) x = k < 3 ? fminf(x, part[w][k]) : fmaxf(x, part[w][k]);
+    if (k < 3) atomicMin(&L.nodes[i].box[k], ordU(x));
+    else atomicMax(&L.nodes[i].box[k], ordU(x));
 }
 
 // the bin of a histogram that holds rank `rank` (block-wide): rank becomes the rank inside the bin, count the
 // bin's size
 __device__ __forceinline__ uint32_t pickBin(const uint32_t* hist, uint32_t& rank, uint32_t& count)
 {
-    __shared__ uint32_t sums[kB];
     __shared__ uint32_t found[3];
     constexpr int per = kBins / kB;
-    uint32_t h[per], own = 0;
-    for (int k = 0; k < per; ++k) { h[k] = hist[per * threadIdx.x + k]; own += h[k]; }
-    __syncthreads();
-    sums[threadIdx.x] = own;
-    __syncthreads();
-    for (int d = 1; d < kB; d <<= 1) {
-        const uint32_t o = (int)threadIdx.x >= d ? sums[threadIdx.x - d] : 0u;
-        __syncthreads();
-        sums[threadIdx.x] += o;
-        __syncthreads();
-    }
-    uint32_t before = sums[threadIdx.x] - own;
+    static_assert(per == 8, "two vector loads");
+    const uint4 v0 = reinterpret_cast<const uint4*>(hist)[2 * threadIdx.x], v1 = reinterpret_cast<const uint4*>(hist)[2 * threadIdx.x + 1];
+    const uint32_t h[per] = { v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w };
+    uint32_t own = 0, all;
+    for (int k = 0; k < per; ++k) own += h[k];
+    uint32_t before = scanBlock(own, all);
     if (rank >= before && rank < before + own) {
         int k = 0;
         while (rank >= before + h[k]) { before += h[k]; ++k; }
@@ -281,10 +304,11 @@ __global__ __launch_bounds__(kB) void kLevelHist(Level L)
 // selection over those leaves.
 __global__ __launch_bounds__(kB) void kLevelPivot(Level L)
 {
-    __shared__ uint32_t h[kBins];
+    __shared__ __align__(16) uint32_t h[kBins];
     __shared__ uint32_t shared;
     const uint32_t i = blockIdx.x;
     const Node d = nodeAt(L.n, L.level, i);
+    if (L.next && threadIdx.x < 2) clearNode(L.next[2 * i + threadIdx.x]);
     const uint32_t* const hist = L.hist + (size_t)i * 3 * kBins;
     uint32_t rank = (uint32_t)(d.num >> 1), count;
     uint32_t k0 = pickBin(hist, rank, count);
@@ -339,11 +363,13 @@ __global__ __launch_bounds__(kB) void kLevelPivot(Level L)
     }
 }
 
-// writes the level's nodes and moves every leaf to its half of the node's range (in any order)
+// Writes the level's nodes and moves every leaf to its half of the node's range (in any order); on the way the
+// boxes of both halves, and the histograms are cleared for the next level (a box pass and a clearing launch per
+// level more: 12 and 4 us of 79 a level at 328 k faces).
 __global__ __launch_bounds__(kB) void kLevelPartition(Level L, TreeNode* __restrict__ tree, int32_t* __restrict__ firstOf)
 {
-    __shared__ uint32_t sums[kB];
     __shared__ uint32_t base[2];
+    __shared__ float part[kB / 64][12];
     uint32_t i;
     int32_t begin, end;
     const Node d = blockNode(L, i, begin, end);
@@ -379,27 +405,46 @@ __global__ __launch_bounds__(kB) void kLevelPartition(Level L, TreeNode* __restr
     }
     const uint32_t nl = (uint32_t)__popc(goLeft);
     // both counts in one scan: 16 bits each (at most kChunk)
-    const uint32_t own = nl | ((mine - nl) << 16);
-    sums[threadIdx.x] = own;
-    __syncthreads();
-    for (int s = 1; s < kB; s <<= 1) {
-        const uint32_t o = (int)threadIdx.x >= s ? sums[threadIdx.x - s] : 0u;
-        __syncthreads();
-        sums[threadIdx.x] += o;
-        __syncthreads();
-    }
+    uint32_t total;
+    const uint32_t before = scanBlock(nl | ((mine - nl) << 16), total);
     if (threadIdx.x == 0) {
-        base[0] = atomicAdd(&nd.left, sums[kB - 1] & 0xffffu);
-        base[1] = atomicAdd(&nd.right, sums[kB - 1] >> 16);
+        base[0] = atomicAdd(&nd.left, total & 0xffffu);
+        base[1] = atomicAdd(&nd.right, total >> 16);
     }
     __syncthreads();
-    const uint32_t before = sums[threadIdx.x] - own;
     int32_t l = d.first + (int32_t)(base[0] + (before & 0xffffu));
     int32_t r = d.first + h + (int32_t)(base[1] + (before >> 16));
+    float box[12];      // of the left and of the right half
+    for (int k = 0; k < 12; ++k) box[k] = k % 6 < 3 ? FLT_MAX : -FLT_MAX;
     for (int k = 0; k < (int)mine; ++k) {
         const Elem e = L.src[begin + k * kB + (int32_t)threadIdx.x];
-        L.dst[(goLeft >> k) & 1u ? l++ : r++] = e;
+        const bool left = (goLeft >> k) & 1u;
+        L.dst[left ? l++ : r++] = e;
+        const float o[6] = { e.a.x, e.a.y, e.a.z, e.a.w, e.b.x, e.b.y };
+        for (int c = 0; c < 3; ++c) {
+            const float lo = o[c], hi = o[3 + c];
+            if (left) { box[c] = fminf(box[c], lo); box[3 + c] = fmaxf(box[3 + c], hi); }
+            else { box[6 + c] = fminf(box[6 + c], lo); box[9 + c] = fmaxf(box[9 + c], hi); }
+        }
     }
+    if (!L.next) return;
+    for (int k = 0; k < 12; ++k)
+        for (int x = 32; x; x >>= 1) box[k] = k % 6 < 3 ? fminf(box[k], __shfl_xor(box[k], x)) : fmaxf(box[k], __shfl_xor(box[k], x));
+    const int lane = threadIdx.x & 63;
+    if (lane == 0)
+        for (int k = 0; k < 12; ++k) part[threadIdx.x >> 6][k] = box[k];
+    __syncthreads();
+    if (threadIdx.x < 12) {
+        const int k = threadIdx.x % 6;
+        const bool least = k < 3;
+        float x = part[0][threadIdx.x];
+        for (int w = 1; w < kB / 64; ++w) x = least ? fminf(x, part[w][threadIdx.x]) : fmaxf(x, part[w][threadIdx.x]);
+        uint32_t* const to = &L.next[2 * i + threadIdx.x / 6].box[k];
+        const uint32_t moved = threadIdx.x < 6 ? total & 0xffffu : total >> 16;
+        if (moved) { if (least) atomicMin(to, ordU(x)); else atomicMax(to, ordU(x)); }
+    }
+    const size_t words = (size_t)3 * kBins << (L.level + 1);
+    for (size_t t = (size_t)blockIdx.x * kB + threadIdx.x; t < words; t += (size_t)gridDim.x * kB) L.hist[t] = 0u;
 }
 
 // leaf dipole: dirArea = cross(b-a, c-a)/2, area = |dirArea|, pos = area * centroid
@@ -712,7 +757,7 @@ size_t layout(int32_t nf, Scratch* s, char* base)
     char* k0 = take(top ? n * 4 : 0);
     char* list = take(top ? n * 4 : 0);
     char* hist = take(wide * 3 * kBins * 4);
-    char* nodes = take(wide * sizeof(LevelNode));
+    char* nodes = take(2 * wide * sizeof(LevelNode));
     char* firstOf = take(nn * 4);
     if (s) {
         s->el[0] = reinterpret_cast<Elem*>(e0);
@@ -752,14 +797,18 @@ hipError_t buildDeviceTree(const float* d_verts, const int32_t* d_tris, int32_t 
     while (largest(n, info.depth) > 1) ++info.depth;
     kLeafBoxes<<<gridFor(n), kB, 0, st>>>(d_verts, d_tris, n, S.el[0]);
     const int top = topLevels(n);
+    const size_t wide = top > 0 ? size_t(1) << (top - 1) : 0;
     int cur = 0;
     for (int l = 0; l < top; ++l, cur ^= 1) {
         const int32_t count = int32_t(1) << l;
-        const Level L{ n, l, (int32_t)((largest(n, l) + kChunk - 1) / kChunk), S.el[cur], S.el[cur ^ 1], S.k0, S.list,
-                       S.nodes, S.hist };
+        LevelNode* const nodes = S.nodes + (l & 1) * wide;
+        const Level L{ n, l, (int32_t)((largest(n, l) + kChunk - 1) / kChunk), S.el[cur], S.el[cur ^ 1], S.k0, S.list, nodes,
+                       l + 1 < top ? S.nodes + (~l & 1) * wide : nullptr, S.hist };
         const dim3 blocks((unsigned)(count * L.blocksPerNode));
-        kLevelInit<<<gridFor((int64_t)count * 3 * kBins), kB, 0, st>>>(L, count);
-        kLevelBox<<<blocks, kB, 0, st>>>(L);
+        if (l == 0) {
+            kLevelInit<<<gridFor(3 * kBins), kB, 0, st>>>(L);
+            kLevelBox<<<blocks, kB, 0, st>>>(L);
+        }
         kLevelHist<0><<<blocks, kB, 0, st>>>(L);
         kLevelHist<1><<<blocks, kB, 0, st>>>(L);
         kLevelHist<2><<<blocks, kB, 0, st>>>(L);
