@@ -14,11 +14,10 @@ Prints ONE JSON line: value = (voxels + projected points) per second for the who
 * `batched`: the uneven 64-mesh workload in one persistent launch (plain and learned);
 * `offset`: the 512^3 volume of a 5,242,880-triangle mesh (plain, learned, and the band options of
   the offset caller on the device path and through calcFromGridWithDistancesByParts);
-* `roofline` (the dominant call: the signed-distance grid) and `rooflines` (every call): achieved =
-  the bytes of the records the walks read, counted per wave by the kernels themselves (each record a
-  wave reads once for its 64 lanes counts once), divided by the call's event time, against the HBM
-  peak; MLP kernels against the BF16 MFMA peak.  `traffic` / L2 hit rate come from the committed PMC
-  profile (profiles/pmc_*.json) when it was taken on the same kernel sources, else null;
+* `roofline` (the dominant call: the signed-distance grid) and `rooflines` (every call): the walks
+  against the vector units' issue rate, from the committed PMC profile (profiles/pmc_*.json) when it was
+  taken on the same kernel sources, else null, with its HBM traffic and L2 hit rate and the bytes of the
+  records that the kernels themselves count; MLP kernels against the BF16 MFMA peak;
 * `cpu_baseline`: the oracle (a C restatement of the reference CPU path) on the host cores available
   to this process, over contiguous z-slabs / query ranges of the same workload, median of 5 after a
   warm-up.
@@ -54,9 +53,10 @@ BATCH_TRAIN_N, BATCH_TRAIN_STEPS = 1 << 18, 500
 MLP_FWD_FLOP = 2 * (99 * 128 + 3 * 128 * 128 + 128)
 MLP_BWD_FLOP = 2 * (99 * 128 + 3 * 128 * 128 + 128) + 2 * (3 * 128 * 128 + 128)
 COPY_BYTES = 1 << 30
+VALU_PEAK_GIPS = 1024 * 2.4 / 4      # a wave64 instruction occupies a SIMD for four cycles
 
 # bytes of the record each counted event reads (mi_mesh_set_stats slots; layouts in mi_tree.hpp /
-# mi_kernels.hpp): 4-wide quad 128 B, plane record 80 B, triangle 48 B, binary node 48 B of box pair
+# mi_kernels.hpp): a lane walk's node 64 B of cylinders; in walks per wave 4-wide quad 128 B, plane record 80 B, triangle 48 B, binary node 48 B of box pair
 # read by the keyed walk's near/far choice, dipole 32 B, child refs 16 B
 RECORD_BYTES = {"quad_steps": 128, "prism_reads": 80, "leaf_tests": 48, "keyed_steps": 128 + 48,
                 "keyed_tests": 48, "fwn_visits": 32, "fwn_descents": 16, "fwn_leaves": 48}
@@ -120,8 +120,11 @@ def counted(torch, M, meshes, fn):
 
 
 def walk_bytes(cnt):
-    """Record bytes one launch's walks read, from its counters (per-wave counts)."""
-    b = sum(RECORD_BYTES[k] * cnt[k] for k in RECORD_BYTES)
+    """Record bytes one launch's walks read, from its counters.  Lane walks count their waves' steps in the step
+    slots, which then read nothing, and every lane's node apart."""
+    lanes = cnt["lane_visits"] > 0
+    b = 64 * cnt["lane_visits"]
+    b += sum(RECORD_BYTES[k] * cnt[k] for k in RECORD_BYTES if not (lanes and k in ("quad_steps", "keyed_steps")))
     b += cnt["seed_levels"] * 64 + cnt["seeds"] * 48    # greedy descents: a 64-B node record per level + a triangle
     return b
 
@@ -173,21 +176,25 @@ def pmc_call(prof, kernels):
     return out
 
 
-def hbm_roofline(kernel, bytes_per_call, ms, counters, prof=None, prof_state=None, prof_kernels=()):
-    achieved = bytes_per_call / (ms / 1e3) / 1e9
-    r = {"bound": "hbm", "kernel": kernel, "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-         "frac": achieved / HBM_PEAK_GBS, "traffic": None, "bytes_per_call": bytes_per_call, "ms": ms,
-         "bytes_model": "records read per wave (kernels' own counters), each counted once per wave visit",
+def walk_roofline(kernel, bytes_per_call, ms, counters, prof=None, prof_state=None, prof_kernels=()):
+    """The walks are bound by the vector units: wave instructions issued per second (PMC counters of the same
+    sources) against one every four cycles on each of the 1024 SIMDs.  record_bytes (the kernels' own counters) are
+    mostly served by L1 and L2; traffic is what the counters saw of HBM."""
+    r = {"bound": "valu", "kernel": kernel, "achieved": None, "peak": VALU_PEAK_GIPS, "unit": "G wave instructions/s",
+         "frac": None, "traffic": None, "record_bytes_per_call": bytes_per_call, "ms": ms,
+         "bytes_model": "records read (kernels' own counters): per lane in lane walks, once per wave in winding numbers",
          "per_launch_bytes": [c["bytes"] for c in counters], "counters": counters}
     pm = pmc_call(prof, prof_kernels)
     if pm:
         r["traffic"] = pm["traffic"]
         r["hbm_gbs_measured"] = pm["traffic"] / (ms / 1e3) / 1e9
+        r["hbm_frac_measured"] = r["hbm_gbs_measured"] / HBM_PEAK_GBS
         r["l2_hit_rate"] = pm["l2_hit_rate"]
         if "stall_frac" in pm:
             r["stall_frac"] = pm["stall_frac"]
         if "valu_insts" in pm:
-            r["valu_issue_frac"] = pm["valu_insts"] / (ms / 1e3) / (1024 * 2.4e9 / 4)
+            r["achieved"] = pm["valu_insts"] / (ms / 1e3) / 1e9
+            r["frac"] = r["achieved"] / VALU_PEAK_GIPS
     r["pmc_profile"] = prof_state
     return r
 
@@ -382,10 +389,10 @@ def learned_leg(ctx):
                       "proj_node_visit_ratio": steps_p / max(plain_p, 1),
                       "sdf_node_visit_ratio": steps_s / max(plain_s, 1),
                       "reruns": rcp + rcs, "identical": same_cp and same_cs,
-                      "why": "the plain walk is already seeded with a real candidate per query (a greedy descent), "
-                             "so a cap prunes only what lies beyond that seed; the visits left are boxes nearer "
-                             "than the true distance, which no bound can prune. The target of >= 2x over the "
-                             "plain walk is above this ceiling."}
+                      "why": "the plain walk finds a real candidate within a few leaves, so a cap prunes only what "
+                             "it visits before that; the visits left are bounds nearer than the true distance, "
+                             "which no cap can prune. The target of >= 2x over the plain walk is above this "
+                             "ceiling."}
     log(f"ceiling (perfect caps): proj {cp:.2f} ms, sdf {cs:.2f} ms, visits {steps_p / max(plain_p, 1):.3f} / "
         f"{steps_s / max(plain_s, 1):.3f} of plain")
     return out
@@ -445,7 +452,7 @@ def batched_leg(args, M, torch, np, synth, timer):
     # every item reads its own voxels out (4 B) and points in / records out / sorted ids (12 + 32 + 4 B)
     cb = with_bytes(cnts, io_bytes=4 * tot_vox + 48 * tot_pts)
     prof, pstate = pmc_profile("batched")
-    roof = hbm_roofline("kBatch", cb[0]["bytes"], t_batch, cb[:1], prof, pstate, ("kBatch",))
+    roof = walk_roofline("kBatch", cb[0]["bytes"], t_batch, cb[:1], prof, pstate, ("kBatch",))
     log(f"batched: {t_batch:.1f} ms (per-item {t_items:.1f} ms), identical {same}")
     learned = None
     if not args.no_learned:
@@ -512,8 +519,7 @@ def offset_leg(args, M, torch, np, synth, timer):
     cnts = counted(torch, M, [mesh], lambda: run(opts))
     cb = with_bytes(cnts, io_bytes=4 * nvox)
     prof, pstate = pmc_profile("offset")
-    roof = hbm_roofline("kSdfGridCoop+kSdfSplit+kSdfSplitFinish", sum(c["bytes"] for c in cb), sdf_ms, cb, prof,
-                        pstate, ("kSdfGridCoop", "kSdfSplit"))
+    roof = walk_roofline("kSdfLane", sum(c["bytes"] for c in cb), sdf_ms, cb, prof, pstate, ("kSdfLane",))
     log(f"offset plain: {sdf_ms:.1f} ms")
     # band options of mcOffsetMesh (source/MRVoxels/MROffset.cpp:176-183) for an offset of 4 voxels,
     # nullOutsideMinMax false (the by-parts path), on the device path, the per-lane form and by parts
@@ -835,10 +841,9 @@ def main():
     learned = None if args.no_learned else learned_leg(ctx)
 
     prof, pstate = pmc_profile("k8_step")
-    roof_sdf = hbm_roofline("kSdfGridCoop+kSdfSplit+kSdfSplitFinish", sum(c["bytes"] for c in cb_sdf), sdf_avg,
-                            cb_sdf, prof, pstate, ("kSdfGridCoop", "kSdfSplit"))
-    roof_proj = hbm_roofline("kProjectionsCoop+kKeyedSplit+kProjSplitFinish", sum(c["bytes"] for c in cb_proj),
-                             proj_avg, cb_proj, prof, pstate, ("kProjectionsCoop", "kKeyedSplit", "kProjSplitFinish"))
+    roof_sdf = walk_roofline("kSdfLane", sum(c["bytes"] for c in cb_sdf), sdf_avg, cb_sdf, prof, pstate, ("kSdfLane",))
+    roof_proj = walk_roofline("kProjectionsLane", sum(c["bytes"] for c in cb_proj), proj_avg, cb_proj, prof, pstate,
+                             ("kProjectionsLane",))
     rooflines = {"sdf": roof_sdf, "projections": roof_proj}
     if "mlp" in ctx:
         mlp = ctx["mlp"]
@@ -862,8 +867,8 @@ def main():
         log(f"cpu baseline ({time.time() - t:.0f} s): {cpu['voxels_per_s']:.0f} vox/s, {cpu['pts_per_s']:.0f} pts/s "
             f"on {cpu['cores']} threads ({cpu['cpu_model']})")
     roof = {k: roof_sdf[k] for k in ("bound", "kernel", "achieved", "peak", "unit", "frac", "traffic")}
-    roof.update({k: roof_sdf[k] for k in ("l2_hit_rate", "hbm_gbs_measured", "stall_frac", "valu_issue_frac",
-                                            "pmc_profile", "bytes_per_call", "ms") if k in roof_sdf})
+    roof.update({k: roof_sdf[k] for k in ("l2_hit_rate", "hbm_gbs_measured", "hbm_frac_measured", "stall_frac",
+                                            "pmc_profile", "record_bytes_per_call", "ms") if k in roof_sdf})
     out = {
         "metric": "signed-dist voxels/s & projected pts/s; learned-bound vs plain GPU speedup",
         "value": value, "unit": "queries/s (voxels + projected points)",

@@ -92,19 +92,22 @@ int mi_set_memory_limit(size_t bytes);
  *
  * Traversal form of the kernels, process-wide default (no counterpart in the reference; its GPU path
  * has one form, MRCudaFastWindingNumber.cu:31-133).  Results do not depend on it.
- *   MI_TRAVERSAL_PER_LANE  one depth-first walk per query, the reference's form
- *   MI_TRAVERSAL_WAVE_COOP one walk per 64-query wave with uniform node loads (default) */
+ *   MI_TRAVERSAL_PER_LANE  one depth-first walk per query over boxes, the reference's form
+ *   MI_TRAVERSAL_WAVE_COOP the default: distances and projections walk one query per lane over bounding
+ *                          cylinders, idle lanes taking over subtrees of their wave's other queries; winding
+ *                          numbers one walk per wave with uniform node loads.  With a step budget above 0
+ *                          (mi_set_split_budget) distances and projections too walk once per wave. */
 #define MI_TRAVERSAL_PER_LANE 0
 #define MI_TRAVERSAL_WAVE_COOP 1
 int mi_set_traversal(int mode);
 int mi_get_traversal(void);
 
-/* Leaf filter of the wave-cooperative signed-distance walks, process-wide default (no counterpart in the
- * reference).  A queued leaf test is dropped for the lanes where a lower bound of the triangle's
- * distance (its plane slab and edge half-spaces, with rounding margins) already exceeds the lane's
- * best, so results do not depend on it.  MI_LEAF_FILTER_AUTO (default) uses it for grids of more
- * than 2^(depth - 8) waves of 64 voxels (depth = tree levels): on deep trees a small grid leaves too
- * few waves to hide the load it adds to each leaf visit. */
+/* Leaf filter of the signed-distance walks that a step budget selects (mi_set_split_budget), process-wide
+ * default (no counterpart in the reference); the default lane walks do not use it.  A queued leaf test is
+ * dropped for the lanes where a lower bound of the triangle's distance (its plane slab and edge half-spaces,
+ * with rounding margins) already exceeds the lane's best, so results do not depend on it.
+ * MI_LEAF_FILTER_AUTO (default) uses it for grids of more than 2^(depth - 8) waves of 64 voxels (depth = tree
+ * levels): on deep trees a small grid leaves too few waves to hide the load it adds to each leaf visit. */
 #define MI_LEAF_FILTER_OFF 0
 #define MI_LEAF_FILTER_ON 1
 #define MI_LEAF_FILTER_AUTO (-1)
@@ -122,16 +125,12 @@ int mi_get_leaf_filter(void);
 int mi_set_tree_builder(int builder);
 int mi_get_tree_builder(void);
 
-/* Step budgets of the split form of the wave-cooperative walks, process-wide defaults (no counterpart in the
- * reference).  A 64-query wave still walking after `steps` node visits hands its queries, with their
- * best candidates so far, to a second launch that walks the tree's 64 top subtrees for them in
- * parallel; results are identical for every budget.  0 = never split; MI_SPLIT_AUTO (the default)
- * picks per call from the tree depth and the number of waves (signed distance on trees of >= 18
- * levels: 3072 steps below 64 k waves, 6144 below 1 M waves, no split from 1 M waves (a 512^3 grid)
- * on; shallower trees: 512 / 1024 below / above 16 k waves; projections: 64 for trees of >= 20
- * levels, else 2048 (>= 17 levels) or 1024).  The device
- * entry points of one mesh share that mesh's workspace: calls on different streams must not overlap
- * in time. */
+/* Step budgets, process-wide defaults (no counterpart in the reference).  0 and MI_SPLIT_AUTO (the default):
+ * distances and projections run as lane walks, which need no hand-over.  Above 0 they run as walks per wave of
+ * 64 queries; one still walking after `steps` node visits hands its queries, with their best candidates so far, to
+ * a second launch that walks the tree's 64 top subtrees for them in parallel.  Results are identical for every
+ * budget.  The capped entry points always run as lane walks.  The device entry points of one mesh share that
+ * mesh's workspace: calls on different streams must not overlap in time. */
 #define MI_SPLIT_SDF 0
 #define MI_SPLIT_PROJECTIONS 1
 #define MI_SPLIT_AUTO (-1)
@@ -159,14 +158,16 @@ int  mi_mesh_num_nodes(const mi_mesh* m);
  * caller, MI_STAT_LAUNCHES * MI_STAT_STRIDE uint64) is set, the wave-cooperative walks of every
  * later call on this mesh add the records they read: block k counts a call's launch k (0 the first
  * launch, 1 the split form's partial walks, 2 its last launch), slot MI_STAT_* within the block.
- * Counts are per wave (a record read once for 64 lanes counts once).  NULL turns counting off.
- * Counting costs a few scalar additions per step and one atomic per walk; results are unchanged. */
+ * Walks per wave count a record read for 64 lanes once.  Lane walks count every lane's node in
+ * MI_STAT_LANE_VISITS, their waves' steps in the slots QUAD_STEPS (distances) and KEYED_STEPS (projections), and
+ * one leaf test per query and triangle.  NULL turns counting off.  Counting costs a few scalar additions per step
+ * and one atomic per walk; results are unchanged. */
 #define MI_STAT_WALKS 0          /* walks run */
-#define MI_STAT_QUAD_STEPS 1     /* distance walk: 4-wide node visits (128-B quad record) */
+#define MI_STAT_QUAD_STEPS 1     /* distance walk: 4-wide node visits (128-B quad record); lane walks: steps */
 #define MI_STAT_PRISM_READS 2    /* distance walk: leaf visits reading the plane record (80 B) */
 #define MI_STAT_LEAF_TESTS 3     /* distance walk: leaf tests (48-B triangle record each) */
-#define MI_STAT_KEYED_STEPS 4    /* keyed (projection) walk: node visits (128-B quad + 48-B node record) */
-#define MI_STAT_KEYED_TESTS 5    /* keyed walk: leaf tests (48-B triangle record each) */
+#define MI_STAT_KEYED_STEPS 4    /* keyed walk: node visits (128-B quad + 48-B node record); lane walks: steps */
+#define MI_STAT_KEYED_TESTS 5    /* projections: leaf tests (48-B triangle record each) */
 #define MI_STAT_FWN_VISITS 6     /* winding number: node visits (32-B dipole record) */
 #define MI_STAT_FWN_DESCENTS 7   /* winding number: descents into children (16-B child refs) */
 #define MI_STAT_FWN_LEAVES 8     /* winding number: exact solid angles (48-B triangle record) */
@@ -320,7 +321,7 @@ void mi_batch_destroy(mi_batch* b);
 int  mi_batch_run_device(mi_batch* b, const mi_batch_item* items, int32_t count, const mi_dist_options* opts,
                          float upDistLimitSq, void* stream);
 /* the project's autotuner (role of runProfiling, source/MRCuda/MRCudaProfiling.cuh:22-79): times the
- * batch over resident workgroups per CU {2..6} x XCD partitioning {off, on} and keeps the fastest
+ * batch over groups of five waves per CU {2..6} x dealing runs of units to the XCDs {off, on} and keeps the fastest
  * for later runs; *bestMs = its time (the outputs are computed as a side effect) */
 int  mi_batch_autotune(mi_batch* b, const mi_batch_item* items, int32_t count, const mi_dist_options* opts,
                        float upDistLimitSq, void* stream, float* bestMs);

@@ -205,7 +205,8 @@ TRAVERSALS = {"per_lane": 0, "wave_coop": 1}
 
 def set_traversal(mode: str):
     """Kernel traversal form: 'per_lane' (one walk per query, the reference's form) or
-    'wave_coop' (one walk per 64-query wave; default).  Results are identical."""
+    'wave_coop' (default: distances and projections one walk per lane over bounding cylinders with
+    the wave's idle lanes helping, winding numbers one walk per wave).  Results are identical."""
     _check(lib().mi_set_traversal(TRAVERSALS[mode]))
 
 
@@ -218,8 +219,8 @@ LEAF_FILTERS = {"off": 0, "on": 1, "auto": -1}
 
 
 def set_leaf_filter(mode: str):
-    """Leaf filter of the signed-distance walks: 'on', 'off' or 'auto' (default: grids of more than
-    2^(depth - 8) waves of 64 voxels).  Results are identical."""
+    """Leaf filter of the signed-distance walks that a step budget selects: 'on', 'off' or 'auto' (default:
+    grids of more than 2^(depth - 8) waves of 64 voxels).  Results are identical."""
     _check(lib().mi_set_leaf_filter(LEAF_FILTERS[mode]))
 
 
@@ -241,9 +242,9 @@ SPLIT_WALKS = {"sdf": 0, "projections": 1}
 
 
 def set_split_budget(steps: int, walk: str = "both"):
-    """Steps after which a wave hands its walk to the split pass (0 = never, -1 = automatic, the
-    default), for the signed-distance walk ('sdf'), the projection walk ('projections') or both;
-    results do not depend on it."""
+    """0 or -1 (automatic, the default): lane walks.  Above 0: walks per wave of 64 queries that hand over to the
+    split pass after so many steps, for the signed-distance walk ('sdf'), the projection walk
+    ('projections') or both.  Results do not depend on it."""
     for w in (SPLIT_WALKS if walk == "both" else [walk]):
         _check(lib().mi_set_split_budget(SPLIT_WALKS[w], int(steps)))
 

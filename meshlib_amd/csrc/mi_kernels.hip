@@ -8,15 +8,16 @@
 //
 // Execution model (one lane = one query, 64-lane waves):
 //  * queries of a wave are spatially coherent: grid voxels are mapped as 4x4x4
-//    bricks per wave; free points are Morton-sorted first, so the lanes of a wave
-//    walk mostly the same nodes and their loads hit the same cache lines;
+//    bricks per wave; free points are ordered by cells of their Morton code first, so the lanes of a wave
+//    walk mostly the same nodes and their loads hit the same cache lines; launches that cannot fill the
+//    chip with full waves put fewer queries in each (lanePerWave, sharedPerWave);
 //  * lane form (the default of distances and projections; mi_lane.hpp): every lane
 //    walks for itself over oriented bounds, FP64 leaf tests queued per wave;
 //  * per-lane reference form (kSdfGrid, kProjections, ...): each lane keeps the reference's
 //    depth-first order exactly (nearer child first, strict '<' on distances), with
 //    the pending far children on a per-lane stack in LDS laid out [depth][lane];
-//  * wave-cooperative form (winding numbers; the keyed walks of a band; distances and projections
-//    when a step budget is set): one walk per wave with wave-uniform node refs
+//  * wave-cooperative form (winding numbers; distances and projections when a step budget is
+//    set): one walk per wave with wave-uniform node refs
 //    (scalar loads), a stack whose uniform part is held in lanes of a few VGPRs and
 //    whose per-lane part (16-bit lower bounds of box distances) sits in LDS, and leaf
 //    tests queued and run one per lane; results equal the per-lane form's;

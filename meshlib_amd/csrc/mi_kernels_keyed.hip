@@ -1,5 +1,5 @@
-// mi_kernels_keyed.hip -- gfx950 kernels of the keyed closest-point walks: findProjections and the
-// signed distance with a band (minDistSq > 0).
+// mi_kernels_keyed.hip -- gfx950 kernels of findProjections (lane walks; with a step budget the keyed walks per
+// wave) and of the signed distance with a band (minDistSq > 0) and a step budget.
 //
 // "Keyed": the result is the leaf minimising (order value, key), where the key is the leaf's position
 // in the query's own depth-first order (near child first, ties to the right) and the order value is

@@ -14,6 +14,8 @@
 //          {a.xyz, b.x} {b.yz, c.xy} {c.z, face, 0, 0}
 //   dint   2 x float4 per internal node: {pos.xyz, rr} {dirArea.xyz, area}
 //   dleaf  2 x float4 per leaf slot:     {pos.xyz, rr} {dirArea.xyz, area}
+//   cyl    4 x float4 per internal node, two per child (made on the device from these, mi_volume.hip):
+//          {c.xyz, n.x} {n.yz, t | r as halves, child ref}
 #pragma once
 
 #include <cstdint>
