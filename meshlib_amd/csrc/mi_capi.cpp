@@ -67,15 +67,24 @@ size_t memBudget()
 // its hipFree cost about 57 and 83 us, a stream 150 and 55, and opening a 328 k-triangle mesh and checking it took
 // ten of the former and two of the latter, 1.4 of its 4.3 ms.  Both pools are bounded (at most kTempKeep buffers
 // of together kTempKeepBytes, kStreamKeep streams), are used under a lock, and take back only what no queued work
-// uses any more.  They live until the process ends (never destroyed, so no HIP call runs from a static destructor).
+// uses any more.  They allocate no host memory (nothing here throws) and free nothing when the process ends, so no
+// HIP call runs from a static destructor.
 constexpr size_t kTempKeep = 8, kTempKeepBytes = size_t(64) << 20, kStreamKeep = 8;
 
 struct TempPool {
     struct Idle { void* p; size_t bytes; int device; };
     std::mutex mu;
-    std::vector<Idle> idle;      // oldest first
-    size_t held = 0;
+    Idle idle[kTempKeep];      // oldest first
+    size_t count = 0, held = 0;
 
+    Idle remove(size_t i)
+    {
+        const Idle d = idle[i];
+        std::copy(idle + i + 1, idle + count, idle + i);
+        --count;
+        held -= d.bytes;
+        return d;
+    }
     // a buffer of at least `bytes` on the current device, the smallest idle one that is not far too large
     hipError_t take(size_t bytes, void** p, size_t* got, int* device)
     {
@@ -83,16 +92,15 @@ struct TempPool {
         if (e != hipSuccess) return e;
         {
             std::lock_guard<std::mutex> lk(mu);
-            size_t best = idle.size();
-            for (size_t i = 0; i < idle.size(); ++i)
+            size_t best = count;
+            for (size_t i = 0; i < count; ++i)
                 if (idle[i].device == *device && idle[i].bytes >= bytes && idle[i].bytes / 4 <= bytes + (size_t(1) << 18) &&
-                    (best == idle.size() || idle[i].bytes < idle[best].bytes))
+                    (best == count || idle[i].bytes < idle[best].bytes))
                     best = i;
-            if (best < idle.size()) {
-                *p = idle[best].p;
-                *got = idle[best].bytes;
-                held -= *got;
-                idle.erase(idle.begin() + (ptrdiff_t)best);
+            if (best < count) {
+                const Idle d = remove(best);
+                *p = d.p;
+                *got = d.bytes;
                 return hipSuccess;
             }
         }
@@ -103,52 +111,53 @@ struct TempPool {
     // nothing queued may use the buffer any more
     void give(void* p, size_t bytes, int device)
     {
-        std::vector<Idle> drop;
-        {
+        Idle drop[kTempKeep + 1];
+        size_t dropped = 0;
+        if (bytes > kTempKeepBytes) {
+            drop[dropped++] = { p, bytes, device };
+        } else {
             std::lock_guard<std::mutex> lk(mu);
-            idle.push_back({ p, bytes, device });
+            while (count && (count == kTempKeep || held + bytes > kTempKeepBytes)) drop[dropped++] = remove(0);
+            idle[count++] = { p, bytes, device };
             held += bytes;
-            while (idle.size() > kTempKeep || held > kTempKeepBytes) {
-                drop.push_back(idle.front());
-                held -= idle.front().bytes;
-                idle.erase(idle.begin());
-            }
         }
-        for (const Idle& d : drop) (void)hipFree(d.p);
+        for (size_t i = 0; i < dropped; ++i) (void)hipFree(drop[i].p);
     }
     // frees every idle buffer; false if there was none
     bool release()
     {
-        std::vector<Idle> drop;
+        Idle drop[kTempKeep];
+        size_t dropped = 0;
         {
             std::lock_guard<std::mutex> lk(mu);
-            drop.swap(idle);
-            held = 0;
+            while (count) drop[dropped++] = remove(count - 1);
         }
-        for (const Idle& d : drop) (void)hipFree(d.p);
-        return !drop.empty();
+        for (size_t i = 0; i < dropped; ++i) (void)hipFree(drop[i].p);
+        return dropped > 0;
     }
 };
 
 TempPool& tempPool()
 {
-    static TempPool* pool = new TempPool;
-    return *pool;
+    static TempPool pool;
+    return pool;
 }
 
 struct StreamPool {
+    struct Idle { hipStream_t s; int device; };
     std::mutex mu;
-    std::vector<std::pair<hipStream_t, int>> idle;
+    Idle idle[kStreamKeep];
+    size_t count = 0;
 
     // a non-blocking stream of the device, which must be the current one
     hipError_t take(int device, hipStream_t* s)
     {
         {
             std::lock_guard<std::mutex> lk(mu);
-            for (size_t i = 0; i < idle.size(); ++i)
-                if (idle[i].second == device) {
-                    *s = idle[i].first;
-                    idle.erase(idle.begin() + (ptrdiff_t)i);
+            for (size_t i = count; i-- > 0;)
+                if (idle[i].device == device) {
+                    *s = idle[i].s;
+                    idle[i] = idle[--count];
                     return hipSuccess;
                 }
         }
@@ -159,8 +168,8 @@ struct StreamPool {
         if (!s) return;
         if (hipStreamSynchronize(s) == hipSuccess) {
             std::lock_guard<std::mutex> lk(mu);
-            if (idle.size() < kStreamKeep) {
-                idle.emplace_back(s, device);
+            if (count < kStreamKeep) {
+                idle[count++] = { s, device };
                 return;
             }
         }
@@ -170,8 +179,8 @@ struct StreamPool {
 
 StreamPool& streamPool()
 {
-    static StreamPool* pool = new StreamPool;
-    return *pool;
+    static StreamPool pool;
+    return pool;
 }
 
 // RAII device buffer
