@@ -125,7 +125,9 @@ __global__ __launch_bounds__(64, 4) void kProjectionsLane(MeshDev m, const float
                                                           int perWave)
 {
     extern __shared__ __align__(16) unsigned char laneMem[];
-    const int wv = logicalBlock(nWaves);
+    // runs of 64 waves to the XCDs in turn: with an eighth of the ordered points each, the XCD with the points deep inside
+    // finished last (2^22 points on 1.3 M triangles 2.50 -> 2.24 ms; winding numbers are 3 % ahead with eighths)
+    const int wv = gridBlock<64>();
     if (wv >= nWaves) return;
     const int lane = threadIdx.x & 63;
     const LaneLds<true, WIDE> l(laneMem, m.depth);
@@ -351,7 +353,7 @@ hipError_t launchProjections(const MeshDev& m, const float* pts, const uint32_t*
         const auto kernel = failCount ? (wide ? kProjectionsLane<true, true, false> : kProjectionsLane<true, false, false>)
                           : band      ? (wide ? kProjectionsLane<false, true, true> : kProjectionsLane<false, false, true>)
                                       : (wide ? kProjectionsLane<false, true, false> : kProjectionsLane<false, false, false>);
-        hipLaunchKernelGGL(kernel, dim3(paddedGrid(nWaves)), dim3(64), laneSharedBytes(m.depth, true, wide, band), s, m, pts, perm,
+        hipLaunchKernelGGL(kernel, dim3(chunkedGrid(nWaves, 64)), dim3(64), laneSharedBytes(m.depth, true, wide, band), s, m, pts, perm,
                            n, nWaves, px, ptXf ? 1 : 0, up, lo, bound, failCount, out, perWave);
         return hipGetLastError();
     }

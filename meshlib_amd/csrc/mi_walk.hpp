@@ -68,7 +68,7 @@ __device__ __forceinline__ int logicalBlock(int nLogical)
     return (b % kXcds) * per + b / kXcds;
 }
 
-// Grid kernels instead deal chunks of consecutive logical blocks (64 bricks: 16 blocks of four waves) to the XCDs
+// Grid kernels and projections instead deal chunks of consecutive logical blocks (64 bricks: 16 blocks of four waves) to the XCDs
 // in turn: each L2 still sees spatially compact runs, and the costly middle of a grid (voxels deep
 // inside the mesh) is spread over all eight XCDs instead of landing on two of them.  The launch
 // covers whole rounds of chunks (chunkedGrid), so the mapping is a bijection onto its blocks.
