@@ -151,7 +151,7 @@ __global__ __launch_bounds__(64, 4) void kSdfLane(MeshDev m, int dx, int dy, int
         }
     }
     waveSync();
-    sdfStore(m, px, py, pz, valid, resSq, o, out, idx);
+    sdfStore<WIDE>(m, px, py, pz, valid, resSq, o, out, idx);
 }
 
 // The wave-cooperative form with hand-over, run when a step budget is set.
@@ -247,6 +247,7 @@ __global__ __launch_bounds__(kBlock) void kSdfSplitFinish(MeshDev m, int dx, int
     }
 }
 
+template <bool WIDE>
 __global__ __launch_bounds__(kBlock) void kFwnGridCoop(MeshDev m, int dx, int dy, int zBegin, int zEnd,
                                                        int nbx, int nby, int nbz, int nLogical, int perWave, Xf xf,
                                                        float beta, float* __restrict__ out)
@@ -260,11 +261,12 @@ __global__ __launch_bounds__(kBlock) void kFwnGridCoop(MeshDev m, int dx, int dy
     if (!waveBallot(valid)) return;
     float px = (float)x, py = (float)y, pz = (float)z;
     xfApply(xf, px, py, pz);
-    const float wn = coopWinding(m, px, py, pz, valid, beta, -1);
+    const float wn = coopWinding<WIDE>(m, px, py, pz, valid, beta, -1);
     if (!valid) return;
     out[((size_t)(z - zBegin) * dy + y) * dx + x] = wn;
 }
 
+template <bool WIDE>
 __global__ __launch_bounds__(kBlock) void kFwnPointsCoop(MeshDev m, const float* __restrict__ pts,
                                                          const uint32_t* __restrict__ perm, int64_t n,
                                                          int nLogical, float beta, int32_t skipFace,
@@ -279,10 +281,11 @@ __global__ __launch_bounds__(kBlock) void kFwnPointsCoop(MeshDev m, const float*
     const int64_t q = valid ? (perm ? (int64_t)perm[i] : i) : 0;
     float px = 0, py = 0, pz = 0;
     if (valid) { px = pts[3 * q]; py = pts[3 * q + 1]; pz = pts[3 * q + 2]; }
-    const float wn = coopWinding(m, px, py, pz, valid, beta, skipFace);
+    const float wn = coopWinding<WIDE>(m, px, py, pz, valid, beta, skipFace);
     if (valid) out[q] = wn;
 }
 
+template <bool WIDE>
 __global__ __launch_bounds__(kBlock) void kSelfIntersectionsCoop(MeshDev m, int nLogical, float beta,
                                                                  int perWave, uint8_t* __restrict__ out)
 {
@@ -298,7 +301,7 @@ __global__ __launch_bounds__(kBlock) void kSelfIntersectionsCoop(MeshDev m, int 
     const float qx = third * ((L.a[0] + L.b[0]) + L.c[0]);
     const float qy = third * ((L.a[1] + L.b[1]) + L.c[1]);
     const float qz = third * ((L.a[2] + L.b[2]) + L.c[2]);
-    const float wn = coopWinding(m, qx, qy, qz, valid, beta, L.face);
+    const float wn = coopWinding<WIDE>(m, qx, qy, qz, valid, beta, L.face);
     if (valid) out[L.face] = (wn < 0 || wn > 1) ? 1 : 0;
 }
 
@@ -377,7 +380,7 @@ __global__ __launch_bounds__(64, 4) void kBatch(const BatchItem* __restrict__ it
                 }
             }
             waveSync();
-            sdfStore(it.m, px, py, pz, valid, resSq, o, it.sdf, idx);
+            sdfStore<WIDE>(it.m, px, py, pz, valid, resSq, o, it.sdf, idx);
             waveSync();
         } else {
             const int64_t i = (lu - it.gridUnits) * 64 + lane;
@@ -827,7 +830,7 @@ hipError_t launchFwnGrid(const MeshDev& m, const int32_t dims[3], const Xf& xf, 
     if (m.traversal == (int)Traversal::WaveCoop) {
         const int perWave = sharedPerWave(64 * bricks, m.numFaces);
         const int blocks = (int)((bricks * (64 / perWave) + kWaves - 1) / kWaves);
-        hipLaunchKernelGGL(kFwnGridCoop, dim3(chunkedGrid(blocks, kGridChunk)), dim3(kBlock), 0, s, m, dims[0], dims[1], zBegin,
+        hipLaunchKernelGGL(m.numFaces > kNarrowFaces ? kFwnGridCoop<true> : kFwnGridCoop<false>, dim3(chunkedGrid(blocks, kGridChunk)), dim3(kBlock), 0, s, m, dims[0], dims[1], zBegin,
                            zEnd, nbx, nby, nbz, blocks, perWave, xf, beta, out);
         return hipGetLastError();
     }
@@ -846,7 +849,7 @@ hipError_t launchFwnPoints(const MeshDev& m, const float* pts, const uint32_t* p
     if (m.traversal == (int)Traversal::WaveCoop) {
         const int perWave = sharedPerWave(n, m.numFaces);
         const int blocks = (int)((n + (int64_t)kWaves * perWave - 1) / ((int64_t)kWaves * perWave));
-        hipLaunchKernelGGL(kFwnPointsCoop, dim3(paddedGrid(blocks)), dim3(kBlock), 0, s, m, pts, perm, n, blocks, beta, skipFace,
+        hipLaunchKernelGGL(m.numFaces > kNarrowFaces ? kFwnPointsCoop<true> : kFwnPointsCoop<false>, dim3(paddedGrid(blocks)), dim3(kBlock), 0, s, m, pts, perm, n, blocks, beta, skipFace,
                            perWave, out);
         return hipGetLastError();
     }
@@ -865,7 +868,7 @@ hipError_t launchSelfIntersections(const MeshDev& m, float beta, uint8_t* out, i
     if (m.traversal == (int)Traversal::WaveCoop) {
         const int perWave = sharedPerWave(m.numFaces, m.numFaces);
         const int blocks = (int)(((int64_t)m.numFaces + (int64_t)kWaves * perWave - 1) / ((int64_t)kWaves * perWave));
-        hipLaunchKernelGGL(kSelfIntersectionsCoop, dim3(paddedGrid(blocks)), dim3(kBlock), 0, s, m, blocks, beta, perWave, out);
+        hipLaunchKernelGGL(m.numFaces > kNarrowFaces ? kSelfIntersectionsCoop<true> : kSelfIntersectionsCoop<false>, dim3(paddedGrid(blocks)), dim3(kBlock), 0, s, m, blocks, beta, perWave, out);
         return hipGetLastError();
     }
     const int nLogical = (m.numFaces + kBlock - 1) / kBlock;

@@ -792,23 +792,31 @@ typedef float Dipole8 __attribute__((ext_vector_type(8)));     // (pos, rr), (di
 // registers, and children are found without memory: the left child has the first half of the leaves
 // (rounded down) and follows its parent in pre-order.  A visit is one 32-byte scalar load and, where a
 // lane takes the dipole, 37 vector operations (62 with a stack in LDS, masks in vector registers and the
-// general square root and division).  Bound by vector issue (82 % of it): 160^3 on 328 k triangles
-// 1.60 -> 1.22 ms; the same with both next records asked for a visit ahead took 1.97 ms (three scalar loads
-// a visit), with vector loads 1.43 ms, with 64-byte records of both children 1.29 ms.
+// general square root and division).  Bound by vector issue (82 % of it): 160^3 on 328 k triangles 1.60 -> 1.16 ms.
+// Slower: both next records asked for a visit ahead (1.97 ms at 1.22: three scalar loads a visit), vector loads
+// (1.43), 64-byte records of both children (1.29), three stack words that the shape is computed from (1.43).
+// The record's place `at` is kept (and stacked) as it enters the load -- a byte offset from dint, which dleaf follows
+// in the arena -- because the scalar chain from a popped entry to its load counts: with places formed at the visit
+// from node, leaf and a choice of base 1.23 ms.  WIDE (more than 2^23 faces): `at` in records.
+template <bool WIDE>
 __device__ __forceinline__ float coopWinding(const MeshDev& m, float qx, float qy, float qz, bool valid,
                                              float beta, int32_t skipFace)
 {
+    typedef __attribute__((address_space(4))) const char Bytes;
+    constexpr uint32_t unit = WIDE ? 1 : 32;
     if (m.numFaces <= 0) return 0;
     const float betaSq = beta * beta;
     float res = 0;
     uint64_t mask = waveBallot(valid);
-    int node = 0, first = 0, num = uniform(m.numFaces), sp = 0;     // node: internal nodes only (num > 1)
-    int sNode = 0, sFirst = 0, sNum = 0, sLo = 0, sHi = 0;          // lane e: stack entry e
+    const uint32_t leafAt = unit * (uint32_t)((m.dleaf - m.dint) / 2);
+    int first = 0, num = uniform(m.numFaces), sp = 0;
+    uint32_t at = num == 1 ? leafAt : 0u;
+    int sAt = 0, sFirst = 0, sNum = 0, sLo = 0, sHi = 0;          // lane e: stack entry e
     uint32_t nVisit = 0, nDesc = 0, nLeaf = 0;     // measurement counts
     while (mask) {
         ++nVisit;
-        const bool leaf = num == 1;
-        const Dipole8 rec = ((const __attribute__((address_space(4))) Dipole8*)(leaf ? m.dleaf : m.dint))[leaf ? first : node];
+        const Dipole8 rec = *(__attribute__((address_space(4))) const Dipole8*)((Bytes*)m.dint +
+                                                                                (WIDE ? (size_t)at * 32 : (size_t)at));
         const float dpx = rec[0] - qx, dpy = rec[1] - qy, dpz = rec[2] - qz;
         const float dd = dpx * dpx + dpy * dpy + dpz * dpz;
         const uint64_t near = mask & leMask(dd, betaSq * rec[3]);
@@ -820,16 +828,16 @@ __device__ __forceinline__ float coopWinding(const MeshDev& m, float qx, float q
             if (far != mid && mi_inverseBallot(far & ~mid)) res += anyDipole(dot, dd);
         }
         if (near) {
-            if (!leaf) {
-                const int h = num >> 1;
-                sNode = mi_writeLane(node + h, sp, sNode);
+            if (num > 1) {
+                const int h = num >> 1, more = num - h;
+                sAt = mi_writeLane((int)(more == 1 ? leafAt + unit * (uint32_t)(first + h) : at + unit * (uint32_t)h), sp, sAt);
                 sFirst = mi_writeLane(first + h, sp, sFirst);
-                sNum = mi_writeLane(num - h, sp, sNum);
+                sNum = mi_writeLane(more, sp, sNum);
                 sLo = mi_writeLane((int)(uint32_t)near, sp, sLo);
                 sHi = mi_writeLane((int)(uint32_t)(near >> 32), sp, sHi);
                 ++sp;
                 ++nDesc;
-                node += 1;
+                at = h == 1 ? leafAt + unit * (uint32_t)first : at + unit;
                 num = h;
                 mask = near;
                 continue;
@@ -840,7 +848,7 @@ __device__ __forceinline__ float coopWinding(const MeshDev& m, float qx, float q
         }
         if (sp == 0) break;
         --sp;
-        node = __builtin_amdgcn_readlane(sNode, sp);
+        at = (uint32_t)__builtin_amdgcn_readlane(sAt, sp);
         first = __builtin_amdgcn_readlane(sFirst, sp);
         num = __builtin_amdgcn_readlane(sNum, sp);
         mask = (uint64_t)(uint32_t)__builtin_amdgcn_readlane(sLo, sp) |
@@ -1215,11 +1223,12 @@ __device__ __forceinline__ void projStore(const MeshDev& m, int leaf, float lim,
 
 // shared tail of the signed-distance kernels: NaN band, winding-number sign, store
 // (FastWindingNumber::calcWithDistances, source/MRMesh/MRFastWindingNumber.cpp:69-76)
+template <bool WIDE = true>
 __device__ __forceinline__ void sdfStore(const MeshDev& m, float px, float py, float pz, bool valid, float resSq,
                                          const DistOpts& o, float* out, size_t idx)
 {
     const bool nan = o.nullOutsideMinMax && (resSq < o.minDistSq || resSq >= o.maxDistSq);
-    const float wn = coopWinding(m, px, py, pz, valid && !nan, o.beta, -1);
+    const float wn = coopWinding<WIDE>(m, px, py, pz, valid && !nan, o.beta, -1);
     if (!valid) return;
     if (nan) {
         out[idx] = __int_as_float(0x7fc00000);

@@ -77,3 +77,25 @@ def test_self_intersections_in_partly_filled_waves(level):
     finally:
         M.set_traversal("wave_coop")
     assert np.array_equal(got, one)
+
+
+def test_winding_numbers_on_more_than_2_23_faces():
+    """Places of records beyond 32-bit byte offsets: winding numbers of points against the per-lane form."""
+    n = 2060
+    rng = np.random.default_rng(4)
+    x, y = np.meshgrid(np.arange(n, dtype=np.float32), np.arange(n, dtype=np.float32), indexing="ij")
+    v = np.stack([x.ravel(), y.ravel(), rng.random(n * n).astype(np.float32)], 1)
+    i, j = (k.ravel() for k in np.meshgrid(np.arange(n - 1), np.arange(n - 1), indexing="ij"))
+    a = i * n + j
+    f = np.concatenate([np.stack([a, a + n, a + n + 1], 1), np.stack([a, a + n + 1, a + 1], 1)]).astype(np.int32)
+    assert len(f) > 1 << 23
+    mesh = M.Mesh(v, f)
+    fwn = M.FastWindingNumber(mesh)
+    pts = (rng.random((2000, 3)) * [n, n, 6] - [0, 0, 3]).astype(np.float32)
+    dims, xf, _ = synth.grid_for_mesh(v, (9, 8, 5))
+    got = fwn.calcFromVector(pts, 2.0), fwn.calcFromGrid(dims, xf, 2.0)
+    mesh.set_mode("traversal", "per_lane")
+    want = fwn.calcFromVector(pts, 2.0), fwn.calcFromGrid(dims, xf, 2.0)
+    for g, w in zip(got, want):
+        # the wave form's square roots and quotients may be off by one unit in about one of 10^7 cases
+        assert np.allclose(g, w, rtol=0, atol=1e-5)
