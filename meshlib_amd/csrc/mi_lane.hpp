@@ -22,10 +22,11 @@
 //  * leaf tests (FP64) are queued per wave and run one per lane when as many wait as lanes are walking:
 //    dense lanes while the wave is full, no stale bests when only a few long walks are left;
 //  * results are minima over candidates and do not depend on the order of visits: a subtree is dropped
-//    only when its lower bound is above the best by more than all rounding (kBoundSlack, the widening in
-//    mi_volume.hip), so every leaf that could decide the result is tested.
+//    only when its lower bound is above the best by more than all rounding (the margins in
+//    mi_bound.hpp), so every leaf that could decide the result is tested.
 #pragma once
 
+#include "mi_bound.hpp"
 #include "mi_walk.hpp"
 
 namespace mi {
@@ -101,7 +102,7 @@ struct LaneLds {
 };
 
 // Squared distance from the point to a child's cylinder, a lower bound of its triangles' distances up to
-// the rounding that kBoundSlack covers.  a = (c, n.x), b = (n.y, n.z, t and r as halves in units of `unit`, ref).
+// the rounding that kLimitSlack covers.  a = (c, n.x), b = (n.y, n.z, t and r as halves in units of `unit`, ref).
 // centerSq: to the centre.
 __device__ __forceinline__ float cylinderDistSq(const float4& a, const float4& b, float unit, float px, float py, float pz,
                                                 float& centerSq)
@@ -119,10 +120,8 @@ __device__ __forceinline__ float cylinderDistSq(const float4& a, const float4& b
     return __builtin_fmaf(s, s, q * q);
 }
 
-// A lower bound is compared with best * (1 + 2^-17) + 1e-37: the relative part covers the rounding of
-// cylinderDistSq (a few units of 2^-24 on every term, the raw square root's one unit), the absolute one
-// results below the normal range.
-__device__ __forceinline__ float laneLimit(float best) { return __builtin_fmaf(best, 1.f + 0x1p-17f, 1e-37f); }
+// what a lower bound is compared with
+__device__ __forceinline__ float laneLimit(float best) { return __builtin_fmaf(best, 1.f + kLimitSlack, 1e-37f); }
 
 // Orders what lanes of one wave write to and read from each other's LDS: the hardware keeps a wave's LDS
 // operations in order, the fence keeps the compiler from reusing or moving values across.

@@ -7,12 +7,8 @@
 // The record of internal node j is 64 bytes, 32 per child: (c, n.x), (n.y, n.z, t and r as two halves, ref).  The
 // halves count in units of MeshDev::cylUnit, a 2^15th of the mesh's diagonal rounded up to a power of two: 11 bits
 // instead of bf16's 8, and a mixed-precision fma reads them as they are.
-// t and r are widened before they are rounded up:
-//  * 1.4 * 2^-23 * M, M the largest coordinate of a vertex: the leaf test rounds its closest point to
-//    float (half a unit of 2^-23 per coordinate, hence at most sqrt(3) / 2 of it in length), the rest is
-//    for the rounding of c and of the vertices' offsets from it;
-//  * (t + r) * 2^-19: the walk's float dot products, whose error is a few units of 2^-24 of the offset
-//    from c, and the part of that offset beyond t and r is covered by the walk's own relative slack.
+// t and r are widened by kWidenCoord and kWidenSize (mi_bound.hpp) before they are rounded up.
+#include "mi_bound.hpp"
 #include "mi_walk.hpp"
 
 #include <algorithm>
@@ -182,7 +178,7 @@ __device__ __forceinline__ uint32_t halfUp(float x)
 __device__ __forceinline__ void putCylinder(float4* out, const float c[3], const float n[3], float t, float r, float big,
                                             float unit, int ref)
 {
-    const float wide = big * 0x1.4p-23f + (t + r) * 0x1p-19f;
+    const float wide = big * kWidenCoord + (t + r) * kWidenSize;
     bool ok = big < INFINITY && t < INFINITY && r < INFINITY;
     for (int i = 0; i < 3; ++i) ok = ok && fabsf(c[i]) < INFINITY && fabsf(n[i]) < 2.f;
     // a quotient below the normal range is rounded to a multiple of 2^-149, far below the widening
