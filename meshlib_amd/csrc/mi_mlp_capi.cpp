@@ -4,6 +4,7 @@
 #include "meshlib_amd.h"
 
 #include "mi_mlp.hpp"
+#include "mi_pool.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -38,8 +39,9 @@ struct Buf {
     {
         if (bytes >= b) return hipSuccess;
         if (p) { (void)hipFree(p); p = nullptr; bytes = 0; }
-        hipError_t e = hipMalloc(&p, b);
+        const hipError_t e = mi::tempPool().allocate(&p, b);
         if (e == hipSuccess) bytes = b;
+        else p = nullptr;
         return e;
     }
     template <class T> T* as() const { return static_cast<T*>(p); }
