@@ -87,6 +87,23 @@ def build_adapter_driver(verbose: bool = False) -> str:
     return ADAPTER_BIN
 
 
+MID_MATH_SRC = os.path.join(ROOT, "tests", "cpp", "mid_math.hip")
+MID_MATH_LIB = os.path.join(ROOT, "tests", "cpp", "libmid_math.so")
+
+
+def build_mid_math(verbose: bool = False) -> str:
+    """Device checks of the winding number's square root and quotient (loaded by the GPU tests)."""
+    cmd = [hipcc(), *FLAGS, "-I", os.path.join(ROOT, "include"), "-I", CSRC, "-shared", MID_MATH_SRC, "-o", MID_MATH_LIB]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        sys.stderr.write(r.stdout + r.stderr)
+        raise RuntimeError("hipcc failed on mid_math.hip")
+    return MID_MATH_LIB
+
+
 if __name__ == "__main__":
     print(build(verbose=True))
     print(build_adapter_driver(verbose=True))
+    print(build_mid_math(verbose=True))

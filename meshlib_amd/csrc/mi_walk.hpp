@@ -271,8 +271,9 @@ __device__ __forceinline__ Leaf loadLeafLanes(const float4* __restrict__ tri, in
 // Square roots and quotients of the winding number.  A value between 2^-60 and 2^60 has no intermediate
 // result outside the normal range below, so the scaling and special cases of the general square root and
 // division fall away: Goldschmidt iteration from the raw reciprocal square root with Markstein's final
-// residual steps (fused multiply-adds), which round the square root and the quotient correctly except in
-// about one of 10^7 cases, where they are off by one unit.
+// residual steps (fused multiply-adds).  Both are correctly rounded on gfx950: compared for all 1,006,632,960 floats
+// of the range (roots), and for all 2^47 pairs of mantissas of dd in [1, 4) and num in [1, 2) (quotients), from which
+// the others follow by powers of 4 and 2 as long as the quotient and its residual are normal numbers.
 constexpr uint32_t kMidLow = 0x21800000u;                 // 2^-60
 constexpr uint32_t kMidSpan = 0x5d800000u - kMidLow;      // to 2^60
 __device__ __forceinline__ bool midRange(float x) { return __float_as_uint(x) - kMidLow < kMidSpan; }
