@@ -7,7 +7,8 @@
 // The record of internal node j is 64 bytes, 32 per child: (c, n.x), (n.y, n.z, t and r as two halves, ref).  The
 // halves count in units of MeshDev::cylUnit, a 2^15th of the mesh's diagonal rounded up to a power of two: 11 bits
 // instead of bf16's 8, and a mixed-precision fma reads them as they are.
-// t and r are widened by kWidenCoord and kWidenSize (mi_bound.hpp) before they are rounded up.
+// t and r are widened by the rounding of the moved centre and by kWidenCoord and kWidenSize (mi_bound.hpp) before they are
+// rounded up.
 #include "mi_bound.hpp"
 #include "mi_walk.hpp"
 
@@ -255,11 +256,18 @@ __global__ __launch_bounds__(kBlock) void kCylinderRecords(MeshDev m, const Rang
     const float hi = unordered(range[ref].hi), lo = -unordered(range[ref].lo);
     const float mid = 0.5f * hi + 0.5f * lo;
     float big = 0.f;
+    double off = 0, offSq = 0;      // what the rounding of the moved centre shifts it by: along the axis, and squared
     for (int k = 0; k < 3; ++k) {
-        f.c[k] = f.c[k] + mid * f.n[k];
+        const float c = f.c[k] + mid * f.n[k];
+        const double e = c - ((double)f.c[k] + (double)mid * f.n[k]);
+        off += e * f.n[k];
+        offSq += e * e;
+        f.c[k] = c;
         big = fmaxf(big, fmaxf(fabsf(mn[k]), fabsf(mx[k])));
     }
-    putCylinder(out, f.c, f.n, 0.5f * hi - 0.5f * lo, sqrtf(__uint_as_float(range[ref].rr)), big, m.cylUnit, ref);
+    const float shiftT = 1.001f * (float)fabs(off), shiftR = 1.001f * sqrtf((float)fmax(offSq - off * off, 0.0));
+    putCylinder(out, f.c, f.n, 0.5f * hi - 0.5f * lo + shiftT, sqrtf(__uint_as_float(range[ref].rr)) + shiftR, big, m.cylUnit,
+                ref);
 }
 
 __global__ void kRangeInit(Range* r, int n)

@@ -130,8 +130,16 @@ static Cyl inner(const std::vector<Tri>& ts, float unit)
     }
     lo = -lo;
     const float mid = 0.5f * hi + 0.5f * lo;
-    for (int k = 0; k < 3; ++k) f.c[k] = f.c[k] + mid * f.n[k];
-    finish(f, 0.5f * hi - 0.5f * lo, std::sqrt(rr), big, unit);
+    double off = 0, offSq = 0;
+    for (int k = 0; k < 3; ++k) {
+        const float c = f.c[k] + mid * f.n[k];
+        const double e1 = c - ((double)f.c[k] + (double)mid * f.n[k]);
+        off += e1 * f.n[k];
+        offSq += e1 * e1;
+        f.c[k] = c;
+    }
+    finish(f, 0.5f * hi - 0.5f * lo + 1.001f * (float)std::fabs(off),
+           std::sqrt(rr) + 1.001f * std::sqrt((float)std::max(offSq - off * off, 0.0)), big, unit);
     return f;
 }
 
