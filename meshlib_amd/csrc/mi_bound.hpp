@@ -20,6 +20,6 @@ namespace mi {
 
 constexpr float kWidenCoord = 0x1.cp-24f;      // 0.875 * 2^-23
 constexpr float kWidenSize = 0x1p-19f;
-constexpr float kLimitSlack = 0x1p-17f;
+constexpr float kLimitSlack = 0x1.8p-19f;      // 48 u
 
 } // namespace mi

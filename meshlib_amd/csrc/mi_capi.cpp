@@ -426,6 +426,7 @@ int finishArena(mi_mesh* m, const ArenaLayout& L)
     m->dev.numFaces = m->nf;
     m->dev.depth = m->depth;
     m->dev.cylUnit = mi::cylinderUnit(m->dev.rootMin, m->dev.rootMax);
+    m->dev.farSq = mi::farDistSq(m->dev.rootMin, m->dev.rootMax, m->nf);
     MI_HIP(mi::buildCylinders(m->dev, reinterpret_cast<float4*>(base + L.total() - L.cyl), ranges.p, m->stream));
     char* cutBase = base + L.dnode + L.tri + L.dint + L.dleaf + L.dquad;
     mi::CutEntry* cut = reinterpret_cast<mi::CutEntry*>(cutBase);

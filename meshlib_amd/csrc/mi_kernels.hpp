@@ -49,6 +49,7 @@ struct MeshDev {
     const CutEntry* cut;   // nCut subtree roots covering every leaf once
     const float4* cyl;     // 4 per internal node: its children's bounding cylinders (lane walks)
     float cylUnit;         // of their thicknesses and radii
+    float farSq;           // squared distance from the root box beyond which a lane walks over boxes
     const float4* prism;   // 5 per leaf slot: planes bounding the triangle (leaf filter of the walks)
     int32_t nCut;
     float rootMin[3], rootMax[3];
@@ -129,6 +130,8 @@ hipError_t buildQuads(const float4* dnode, int32_t numInternal, float4* dquad, h
 size_t cylinderScratchBytes(int32_t numFaces);
 // MeshDev::cylUnit for the root box: a power of two with which halves hold every length in the mesh
 float cylinderUnit(const float rootMin[3], const float rootMax[3]);
+// MeshDev::farSq for the root box
+float farDistSq(const float rootMin[3], const float rootMax[3], int32_t numFaces);
 hipError_t buildCylinders(const MeshDev& m, float4* cyl, void* scratch, hipStream_t s);
 // the leaf-slot plane records of MeshDev::prism from the triangle records
 hipError_t buildPrisms(const float4* tri, int32_t numLeaves, float4* prism, hipStream_t s);

@@ -207,12 +207,13 @@ __device__ __forceinline__ int flushLane(const MeshDev& m, const LaneLds<TIES, W
     return base;
 }
 
-// The reference's walk with a low limit (source/MRMesh/MRMeshProject.cpp:13-103) for one lane: depth-first, nearer box
-// first, ending at the first leaf at most `lo` away.  Returns that distance and leaf, or the least ones.
-__device__ __forceinline__ float firstWithin(const MeshDev& m, int2* stack, float px, float py, float pz, float up, float lo,
-                                             int& leaf)
+// The reference's walk (source/MRMesh/MRMeshProject.cpp:13-103) for one lane: depth-first over boxes, nearer box first, ending
+// at the first leaf at most `lo` away.  Returns that distance and leaf, or the least ones.  put / get: the lane's stack; a
+// bound that it lowers costs a visit without effect, since a leaf counts only below the best.
+template <class Put, class Get>
+__device__ __forceinline__ float boxWalk(const MeshDev& m, Put put, Get get, float px, float py, float pz, float up, float lo,
+                                         int& leaf, uint32_t& visits)
 {
-    const int lane = threadIdx.x & 63;
     float best = up;
     leaf = -1;
     int cur = m.rootRef, sp = 0;
@@ -220,9 +221,9 @@ __device__ __forceinline__ float firstWithin(const MeshDev& m, int2* stack, floa
     for (;;) {
         if (!have) {
             if (sp == 0) break;
-            const int2 e = stack[64 * --sp + lane];
-            cur = e.x;
-            if (__int_as_float(e.y) >= best) continue;
+            float bound;
+            cur = get(--sp, bound);
+            if (bound >= best) continue;
         }
         have = false;
         if (cur < 0) {
@@ -234,6 +235,7 @@ __device__ __forceinline__ float firstWithin(const MeshDev& m, int2* stack, floa
             }
             continue;
         }
+        ++visits;
         const size_t rec = 4 * (size_t)cur;
         const float4 n0 = gload(m.dnode, rec), n1 = gload(m.dnode, rec + 1), n2 = gload(m.dnode, rec + 2), n3 = gload(m.dnode, rec + 3);
         const float d1 = boxDistSq(n0.x, n0.y, n0.z, n0.w, n1.x, n1.y, px, py, pz);
@@ -241,7 +243,7 @@ __device__ __forceinline__ float firstWithin(const MeshDev& m, int2* stack, floa
         const bool leftNear = d1 < d2;
         const int l = __float_as_int(n3.x), r = __float_as_int(n3.y);
         const float dn = leftNear ? d1 : d2, df = leftNear ? d2 : d1;
-        if (df < best) stack[64 * sp++ + lane] = make_int2(leftNear ? r : l, __float_as_int(df));
+        if (df < best) put(sp++, leftNear ? r : l, df);
         if (dn < best) { cur = leftNear ? l : r; have = true; }
     }
     return best;
@@ -265,7 +267,10 @@ __device__ __forceinline__ float firstWithin(const MeshDev& m, int2* stack, floa
 // issued about 190 vector instructions a step.  With the loop and with rounds of 1 / 2 / 3 entries: 2^22
 // points 2.95 -> 2.39 / 2.33 / 2.53 ms, 256^3 11.1 -> 9.19 / 9.13 / 9.51 ms, 1,000 points 97 -> 71 / 75 / 77 us.
 //
-// BAND: a query with a leaf at most `lo` away ends there and is answered by firstWithin, whose result depends on the
+// Queries farther away than m.farSq are answered by boxWalk: the relative slack of the limit grows with the distance until
+// it holds the whole mesh, while boxes' distances are compared as they are.
+//
+// BAND: a query with a leaf at most `lo` away ends there and is answered by boxWalk, whose result depends on the
 // reference's order of visits (a query without one has its least distance in any order).  Its stack (8 bytes an
 // entry) costs a third of the waves, so only launches with a low limit have it.  Against the wave-cooperative walk
 // that carries the order as keys: a band of 1.5 to 4.5 voxels in 190^3 around 1.3 M triangles 6.4 -> 1.4 ms, 48^3
@@ -279,10 +284,12 @@ __device__ __forceinline__ float laneWalk(const MeshDev& m, const LaneLds<TIES, 
     float px = qx, py = qy, pz = qz;
     int own = lane, cur = kNoNode, base = 0, sp = 0, qn = 0;      // pending: entries base .. sp - 1
     uint32_t nStep = 0, nVisit = 0, nTest = 0;      // measurement counts
+    bool far = false;
     if (walk && m.numFaces > 0) {
         const float rootd = boxDistSq(m.rootMin[0], m.rootMin[1], m.rootMin[2], m.rootMax[0], m.rootMax[1],
                                       m.rootMax[2], px, py, pz);
-        if (rootd < up) cur = m.rootRef;
+        far = rootd < up && rootd > m.farSq;
+        if (rootd < up && !far) cur = m.rootRef;
     }
     const uint32_t upBits = cur == kNoNode ? 0u : __float_as_uint(up);
     waveSync();
@@ -381,18 +388,36 @@ __device__ __forceinline__ float laneWalk(const MeshDev& m, const LaneLds<TIES, 
             }
         }
     }
+    waveSync();
+    const uint32_t b = l.s->best[lane];
+    const bool found = b < upBits;
+    const bool within = BAND && found && __uint_as_float(b) <= lo;
+    const bool boxes = far || within;
+    float d = found ? __uint_as_float(b) : up;
+    int at = -1;
+    uint32_t nBox = 0;
+    if (boxes) {
+        if (BAND) {
+            int2* const stack = l.band();
+            d = boxWalk(m, [=](int sp, int ref, float bound) { stack[64 * sp + lane] = make_int2(ref, __float_as_int(bound)); },
+                        [=](int sp, float& bound) {
+                            const int2 e = stack[64 * sp + lane];
+                            bound = __int_as_float(e.y);
+                            return e.x;
+                        }, qx, qy, qz, up, lo, at, nBox);
+        } else {
+            d = boxWalk(m, [&](int sp, int ref, float bound) { l.put(64 * sp + lane, ref, bound); },
+                        [&](int sp, float& bound) { return l.get(64 * sp + lane, bound); }, qx, qy, qz, up, -1.f, at, nBox);
+        }
+    }
     if (m.stats) {
         statAdd(m, kStatWalks, 1);
         statAdd(m, statSteps, nStep);
         statAdd(m, statTests, nTest);
         statAdd(m, kStatLaneVisits, nVisit);
+        if (boxes) atomicAdd(&m.stats[kStatLaneVisits], (unsigned long long)nBox);
     }
-    waveSync();
-    const uint32_t b = l.s->best[lane];
-    const bool found = b < upBits;
-    if (BAND && found && __uint_as_float(b) <= lo) {
-        int at;
-        const float d = firstWithin(m, l.band(), qx, qy, qz, up, lo, at);
+    if (boxes) {
         if (TIES) *leaf = at;
         return d;
     }
@@ -403,7 +428,7 @@ __device__ __forceinline__ float laneWalk(const MeshDev& m, const LaneLds<TIES, 
             *leaf = l.ties->leaf[0][lane];
         }
     }
-    return found ? __uint_as_float(b) : up;
+    return d;
 }
 
 } // namespace

@@ -13,6 +13,7 @@
 #include "mi_walk.hpp"
 
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
 
 namespace mi {
@@ -278,13 +279,29 @@ __global__ void kRangeInit(Range* r, int n)
 
 } // namespace
 
-float cylinderUnit(const float rootMin[3], const float rootMax[3])
+// Distances from which a lane walks over boxes, in diagonals of the mesh times the root of its number of faces: there the
+// limit's slack is some 17 edges deep.  10,000 points, cylinders / boxes: 1.3 M faces 3,000 diagonals away 2.6 / 13.2 ms,
+// 29,000 24 / 3.4, 290,000 263 / 0.33; 20 k faces 29,000 away 0.41 / 1.05, 290,000 2.5 / 0.34.
+constexpr double kFarSizes = 1.2e7;
+
+static double diagonal(const float rootMin[3], const float rootMax[3])
 {
     double dd = 0;
     for (int i = 0; i < 3; ++i) dd += ((double)rootMax[i] - rootMin[i]) * ((double)rootMax[i] - rootMin[i]);
-    const double diag = std::sqrt(dd);
+    return std::sqrt(dd);
+}
+
+float cylinderUnit(const float rootMin[3], const float rootMax[3])
+{
+    const double diag = diagonal(rootMin, rootMax);
     if (!(diag > 0) || !(diag < 1e308)) return 1.f;
     return (float)std::ldexp(1.0, std::max(std::ilogb(diag) + 1 - 15, -126));
+}
+
+float farDistSq(const float rootMin[3], const float rootMax[3], int32_t numFaces)
+{
+    const double far = kFarSizes / std::sqrt((double)numFaces) * diagonal(rootMin, rootMax);
+    return far * far < (double)FLT_MAX ? (float)(far * far) : INFINITY;      // not a number: infinity
 }
 
 size_t cylinderScratchBytes(int32_t numFaces) { return numFaces > 1 ? (size_t)(numFaces - 1) * sizeof(Range) : 0; }
