@@ -321,10 +321,10 @@ __global__ __launch_bounds__(kBlock) void kSelfIntersectionsCoop(MeshDev m, int 
 // retries do not form a tail of their own as a separate launch over scattered queries would).
 constexpr int kBatchChunk = 64;
 // waves of one "block per CU" of the batch's settings: five groups' worth of registers fit a CU at the default of 4
-// (16 waves a CU: 4.17 ms, 20: 4.03)
+// (16 waves a CU: 4.17 ms, 20: 4.03).  The capped form's second walk takes 10 registers more, which would spill.
 constexpr int kBatchGroup = 5;
 template <bool CAPPED, bool WIDE>
-__global__ __launch_bounds__(64, 4) void kBatch(const BatchItem* __restrict__ items, int nItems, int64_t total, DistOpts o,
+__global__ __launch_bounds__(64, CAPPED ? 4 : kBatchGroup) void kBatch(const BatchItem* __restrict__ items, int nItems, int64_t total, DistOpts o,
                                                 float up, int depth, unsigned long long* __restrict__ tickets, int xcdSplit)
 {
     extern __shared__ __align__(16) unsigned char laneMem[];
