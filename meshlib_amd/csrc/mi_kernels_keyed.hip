@@ -348,7 +348,7 @@ hipError_t launchProjections(const MeshDev& m, const float* pts, const uint32_t*
     const bool coop = !treeXf && m.traversal == (int)Traversal::WaveCoop;
     if (failCount || projectionOrder(m, treeXf, split) == PointOrder::Lanes) {
         const int perWave = lanePerWave(n);
-        const int nWaves = (int)((n + perWave - 1) / perWave);
+        const int nWaves = laneWaves(n, perWave);
         const bool wide = laneWide(m.numFaces), band = lo > 0;
         const auto kernel = failCount ? (wide ? kProjectionsLane<true, true, false> : kProjectionsLane<true, false, false>)
                           : band      ? (wide ? kProjectionsLane<false, true, true> : kProjectionsLane<false, false, true>)

@@ -106,6 +106,20 @@ inline int lanePerWave(int64_t n)
     const int per = perWaveFor(n, 4096);
     return per == 1 && n > 2048 ? 2 : per < 32 ? per : 32;
 }
+// Up to kDealPoints points the ordered queries are dealt to runs of kDealWaves waves in turn.  Queries that walk long lie
+// together -- nearest to a vertex of many triangles, equally far from a whole sphere -- and in one wave they are the end of
+// the launch: 50 k points around a cone of 10,000 triangles a tip 6.4 -> 0.75 ms (runs of 16 waves 1.1), 50 of them at the
+// centre of a sphere of 328 k 73 -> 6.8.  Elsewhere 65,536 points on 1.3 M triangles 141 -> 127 us, 150,000 237 -> 223, on
+// 20 k 124 -> 107; above the limit waves want neighbours for their caches: 400,000 on 1.3 M 386 / 415.
+constexpr int64_t kDealPoints = int64_t(1) << 18;
+constexpr int kDealWaves = 256;
+__host__ __device__ inline bool dealt(int64_t n, int perWave) { return perWave < 64 && n <= kDealPoints; }
+// waves of a launch over n points: whole runs where they are dealt
+inline int laneWaves(int64_t n, int perWave)
+{
+    const int64_t waves = (n + perWave - 1) / perWave;
+    return (int)(dealt(n, perWave) ? (waves + kDealWaves - 1) / kDealWaves * kDealWaves : waves);
+}
 // Winding numbers and grids, whose winding-number walks are shared by a wave: neighbours' walks overlap the
 // less the finer the mesh, so a large mesh takes up to 8,192 waves (32 a CU), a small one 2,048.  64 and the rule:
 // 1,000 points 1126 -> 124 us, 65,536 on 82 k triangles 605 -> 399 us, on 1.3 M 1129 -> 494; 32^3 signed
@@ -1179,13 +1193,14 @@ __device__ __forceinline__ void rankCut(const MeshDev& m, bool valid, float px, 
     if (lane < m.nCut) order[rank] = (uint8_t)lane;
 }
 
-// the query of lane `lane` of projection wave `wv` (as in kProjectionsCoop)
+// the query of lane `lane` of projection wave `wv`
 __device__ __forceinline__ bool projQuery(const float* __restrict__ pts, const uint32_t* __restrict__ perm, int64_t n,
                                           const Xf& ptXf, int hasPtXf, float up, const float* __restrict__ bound,
                                           uint32_t wv, int lane, int64_t& q, float& px, float& py, float& pz, float& lim,
                                           int perWave = 64)
 {
-    const int64_t i = (int64_t)wv * perWave + lane;
+    const int64_t i = dealt(n, perWave) ? (int64_t)(wv / kDealWaves) * (kDealWaves * perWave) + lane * kDealWaves + wv % kDealWaves
+                                        : (int64_t)wv * perWave + lane;
     const bool valid = lane < perWave && i < n;
     q = valid ? (perm ? (int64_t)perm[i] : i) : 0;
     px = py = pz = 0;
