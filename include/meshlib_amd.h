@@ -284,10 +284,10 @@ int mi_proj_find_projections_bounded_device(mi_mesh* m, const float* d_pts, int6
                                             float loDistLimitSq, mi_projection* d_res, void* stream);
 
 /* Exact projections accelerated by per-point caps (no counterpart in the reference; the learned
- * bound of this project feeds it): a first pass searches below min(d_capSq[i], upDistLimitSq), the
- * points that found nothing there are searched again without the cap.  The records equal
+ * bound of this project feeds it): point i is searched below min(d_capSq[i], upDistLimitSq), and a point
+ * that finds nothing there again without the cap, inside the same launch.  The records equal
  * findProjections(upDistLimitSq, loDistLimitSq = 0) whatever the caps; *reruns returns how many
- * points needed the second pass.  Synchronises the stream once to size the second pass. */
+ * points were searched again.  Synchronises the stream once at the end, to read that number. */
 int mi_proj_find_projections_capped_device(mi_mesh* m, const float* d_pts, int64_t n, const float* d_capSq,
                                            float upDistLimitSq, mi_projection* d_res, int64_t* reruns,
                                            void* stream);

@@ -628,7 +628,7 @@ class FastWindingNumber:
     def sdf_grid_capped_device(self, dims, xf, options, d_capSq: int, d_out: int, zBegin=0, zEnd=None,
                                stream: int = 0) -> int:
         """Exact signed-distance slab with per-voxel caps on the search radius (squared); returns how
-        many voxels needed the uncapped second pass."""
+        many voxels were searched again without their cap."""
         d = _dims(dims)
         o = (options or DistanceToMeshOptions())._c()
         zEnd = int(d[2]) if zEnd is None else zEnd
@@ -686,7 +686,7 @@ class PointsToMeshProjector:
     def find_projections_capped_device(self, d_pts: int, n: int, d_capSq: int, d_out: int,
                                        upDistLimitSq: float = FLT_MAX, stream: int = 0) -> int:
         """Exact projections with per-point caps on the search radius (squared); returns how many
-        points needed the uncapped second pass."""
+        points were searched again without their cap."""
         r = C.c_int64(0)
         _check(lib().mi_proj_find_projections_capped_device(
             self.mesh.handle, C.c_void_p(d_pts), n, C.c_void_p(d_capSq), upDistLimitSq, C.c_void_p(d_out),

@@ -10,7 +10,8 @@
 //  * queries of a wave are spatially coherent: grid voxels are mapped as 4x4x4
 //    bricks per wave; free points are ordered by cells of their Morton code first, so the lanes of a wave
 //    walk mostly the same nodes and their loads hit the same cache lines; launches that cannot fill the
-//    chip with full waves put fewer queries in each (lanePerWave, sharedPerWave);
+//    chip with full waves put fewer queries in each (lanePerWave, sharedPerWave), and projections of up to
+//    2^18 points deal neighbours to different waves (kDealPoints);
 //  * lane form (the default of distances and projections; mi_lane.hpp): every lane
 //    walks for itself over oriented bounds, FP64 leaf tests queued per wave;
 //  * per-lane reference form (kSdfGrid, kProjections, ...): each lane keeps the reference's
@@ -25,8 +26,8 @@
 //    walks the tree's top subtrees for them in parallel (results merged by atomic
 //    minimum) and a third that stores them;
 //  * blocks are remapped so that each XCD (blocks are dealt round-robin over the 8
-//    XCDs) gets compact ranges of bricks / one contiguous range of sorted queries, keeping each L2's
-//    working set spatially local.
+//    XCDs) gets compact ranges of bricks and of projections' queries in turn / one contiguous range of
+//    winding numbers' queries, keeping each L2's working set spatially local.
 #include "mi_lane.hpp"
 
 #include <hipcub/hipcub.hpp>
@@ -121,8 +122,8 @@ __global__ __launch_bounds__(kBlock) void kSelfIntersections(MeshDev m, int nLog
 
 // The lane form: every voxel of a 4x4x4 brick walks for itself (laneWalk), one wave per workgroup so that a
 // finished wave's LDS goes to the next one at once.  Measured against the wave-cooperative form with hand-over
-// (both with the winding-number sign): k=8 256^3 101 -> 13.4 ms, k=5 64^3 1.48 -> 0.59 ms.  CAPPED: voxels whose cap is below the plain limit and
-// finds nothing walk again without it, counted in failCount.
+// (both with the winding-number sign): 256^3 on 1.3 M triangles 101 -> 9.0 ms, 64^3 on 20 k 1.48 -> 0.28 ms.  CAPPED: voxels
+// whose cap is below the plain limit and finds nothing walk again without it, counted in failCount.
 template <bool CAPPED, bool WIDE, bool BAND>
 __global__ __launch_bounds__(64, 4) void kSdfLane(MeshDev m, int dx, int dy, int zBegin, int zEnd, int nbx, int nby, int nbz,
                                                   int nWaves, int perWave, Xf xf, DistOpts o, const float* __restrict__ bound,
@@ -562,8 +563,7 @@ __global__ void kBuildQuads(const float4* __restrict__ dnode, int32_t ni, float4
     q[7] = make_float4(__int_as_float(leaf[0]), __int_as_float(leaf[1]), 0.f, 0.f);
 }
 
-// Subtrees at depth kCutDepth (leaves above it stand for themselves), left to right: one thread
-// walks the top of the tree depth-first.
+// Subtrees at depth kCutDepth (leaves above it stand for themselves), left to right.
 // One wave: lane k goes down by the bits of k, highest first (1: right), to its subtree at depth kCutDepth or to a
 // leaf above it, which the lane whose further bits are 0 keeps; lane order is left to right.
 __global__ __launch_bounds__(64) void kBuildCut(const float4* __restrict__ dnode, CutEntry root, CutEntry* __restrict__ cut,

@@ -112,8 +112,8 @@ __device__ __forceinline__ int keyLeaf(const MeshDev& m, uint32_t key, float px,
 // ---------------------------------------------------------------- projections
 
 // The lane form: every query walks for itself (laneWalk).  Measured against the
-// wave-cooperative form with hand-over: 2^22 points on 1.3 M triangles 66 -> 3.8 ms, 300 k ICP samples on
-// 328 k triangles 1.09 -> 0.36 ms, 1000 points on 20 k triangles 1.09 -> 0.15 ms.  bound (optional, indexed like
+// wave-cooperative form with hand-over: 2^22 points on 1.3 M triangles 66 -> 2.2 ms, 300 k ICP samples on
+// 328 k triangles 1.09 -> 0.20 ms, 1000 points on 20 k triangles 1.09 -> 0.03 ms.  bound (optional, indexed like
 // the output): a limit per query below `up`.  CAPPED: the bound is a guess; queries that find nothing below a
 // cap smaller than `up` walk again without it, counted in failCount (any cap above the true distance gives the
 // reference's record, so the combination is exact).

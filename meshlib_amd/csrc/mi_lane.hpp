@@ -5,13 +5,13 @@
 // its triangles), a centre c, the half thickness t along n and the radius r across it (mi_volume.hip).
 // A surface patch is thin along its normal, so the cylinder's distance is within a fraction of the
 // patch's curvature of the true one, where an axis-aligned box of a tilted patch is off by about its
-// size.  Bound tests and leaf tests per query on a 1.3 M-triangle bumpy sphere (256^3 voxels, depth-first on
-// the CPU): 2,590 and 552 with boxes, 249 and 14 with cylinders; with vertex noise of a fifth of the edges
-// 2,216 and 360 against 321 and 25.
+// size.  Bound tests and leaf tests per voxel of 256^3 on a 1.3 M-triangle bumpy sphere: 2,590 and 552 with boxes
+// (depth-first on the CPU), 180 and 8.7 in these walks (90 nodes of two children); with vertex noise of a fifth of the
+// edges 2,216 and 360 against 241 and 20.
 //
 // With so few visits a query no longer needs its wave's company: a wave sharing one walk visits the union
 // of its lanes' nodes (about 2,500 four-wide steps per 64 voxels with boxes), while 64 separate walks
-// take as many steps as the longest of them (123 on that grid), each a 64-byte gather per lane.
+// take as many steps as the longest of them (103 on that grid), each a 64-byte gather per lane.
 //
 //  * stack: [entry][lane] in LDS, the child's ref and the top 16 bits of its lower bound (a truncated
 //    non-negative float is a lower bound of itself), so a pop drops what the best has overtaken without
@@ -59,7 +59,7 @@ struct LaneTies {
 };
 constexpr int32_t kNarrowFaces = 1 << 23;      // refs of at most 24 bits with sign
 inline bool laneWide(int32_t numFaces) { return numFaces > kNarrowFaces; }
-// band: firstWithin's stack takes the place of the walk's
+// band: boxWalk's stack takes the place of the walk's
 inline size_t laneSharedBytes(int depth, bool ties, bool wide, bool band = false)
 {
     const size_t d = depth > 0 ? (size_t)depth : 1;

@@ -50,7 +50,6 @@ __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c)
 }
 
 __device__ __forceinline__ float sigmoidf(float z) { return 1.f / (1.f + expf(-z)); }
-__device__ __forceinline__ float siluf(float z) { return z / (1.f + expf(-z)); }
 __device__ __forceinline__ float softplusf(float u) { return u > 20.f ? u : log1pf(expf(u)); }
 
 // feature `i` (0..127) of the normalised point x
@@ -280,7 +279,7 @@ __global__ __launch_bounds__(64 * kTrainWaves) void kTrainTile(Params p, const f
 // activation leaves its lane.  Layer 0's chunks take the features in natural order (lane group g:
 // features 32c + 8g + 0..7), computed in-lane with the hardware sine / cosine (v_sin_f32, v_cos_f32 take
 // revolutions: sin(pi f x) = v_sin(f x / 2); within 2e-4 of sinf / cosf, far below the features' BF16
-// rounding).  Rounding points as in kForward: features, weights and hidden activations in BF16, FP32
+// rounding).  Rounding points as in training: features, weights and hidden activations in BF16, FP32
 // accumulation, the output layer on BF16 activations and weights.
 constexpr int kPredWaves = 8;
 constexpr int kPredGroups = 4;                        // 16-point groups per wave
