@@ -326,12 +326,13 @@ __device__ __forceinline__ float laneWalk(const MeshDev& m, const LaneLds<TIES, 
     float px = qx, py = qy, pz = qz;
     int own = lane, cur = kNoNode, base = 0, sp = 0, qn = 0;      // pending: entries base .. sp - 1
     uint32_t nStep = 0, nVisit = 0, nTest = 0;      // measurement counts
-    bool far = false;
-    if (walk && m.numFaces > 0) {
-        const float rootd = boxDistSq(m.rootMin[0], m.rootMin[1], m.rootMin[2], m.rootMax[0], m.rootMax[1],
-                                      m.rootMax[2], px, py, pz);
-        far = rootd < up && rootd > m.farSq;
-        if (rootd < up && !far) cur = m.rootRef;
+    const auto rootDistSq = [&] {
+        return boxDistSq(m.rootMin[0], m.rootMin[1], m.rootMin[2], m.rootMax[0], m.rootMax[1], m.rootMax[2], qx, qy, qz);
+    };
+    const bool some = walk && m.numFaces > 0;
+    if (some) {
+        const float d = rootDistSq();
+        if (d < up && !(d > m.farSq)) cur = m.rootRef;
     }
     const uint32_t upBits = cur == kNoNode ? 0u : __float_as_uint(up);
     waveSync();
@@ -434,6 +435,11 @@ __device__ __forceinline__ float laneWalk(const MeshDev& m, const LaneLds<TIES, 
     const uint32_t b = l.s->best[lane];
     const bool found = b < upBits;
     const bool within = BAND && found && __uint_as_float(b) <= lo;
+    bool far = false;      // found again: kept across the loop it cost small volumes 1 %
+    if (some && upBits == 0u) {
+        const float r = rootDistSq();
+        far = r < up && r > m.farSq;
+    }
     const bool boxes = far || within;
     float d = found ? __uint_as_float(b) : up;
     int at = -1;
